@@ -1,5 +1,6 @@
 // fft.hip -- batched, LDS-staged mixed-radix Stockham 3D real FFT for gfx950, with the
-// Fourier-space viscous / Stokes solve fused into the z-pencil pass.
+// Fourier-space viscous / Stokes solve fused into the z-pencil pass: the runtime-size kernels,
+// for every grid whose lengths are 2^a 3^b (fft_fast.hip holds the size-specialised ones).
 //
 // Replaces the cufftExecZ2Z calls + kernelShift + kernelUpdateV* chain of fluam
 // (src/runSchemeIncompressible.cu:111-138, src/runSchemeStokesLimit.cu:198-259,
@@ -14,120 +15,162 @@
 //   C  xy-inverse : inverse of A, with an epilogue that blends the result with another field.
 // Half-spectrum layout in HBM: spec[c][ky][z][kx], kx in [0, mx/2], row pitch P = mx/2 + 1, so
 // a pass-B tile (fixed ky, a run of kx, every z) is one compact block of rows.
+//
+// The workgroup is sized to its data: 256, 512 or 1024 lanes for up to 2112, 4224 or 8448 complex
+// elements in LDS, so a lane never holds more than 9 elements (64 VGPRs, the CU full of waves in
+// every class), every load of a lane is in flight at once, and the butterflies a lane may hold in
+// a stage are a constant per radix.  The radices go up to 16 (at most three stages for any length
+// up to 256), the divisions by runtime extents are multiplications by host-made reciprocals.
+// Bound by LDS and barrier latency, like the size-specialised passes.  Per launch (HIP events,
+// which add about 4 us), with 256 lanes, radices up to 8 and a load-wait-store loop per element
+// before, and now: 108 x 54 x 72 forward 33.6 -> 13.1, z 37.4 -> 15.0, inverse 34.8 -> 13.8 us;
+// 128 x 64 x 32 forward 28.9 -> 13.8 us; 256-point columns of 128 x 128 planes 181 -> 58 us.
+// Where a size-specialised instance exists it stays ahead (128^3: 20.7 / 28.0 / 19.2 against
+// 23.6 / 34.2 / 23.2 us; 64^3: 9.6 / 11.3 / 8.9 against 13.8 / 14.0 / 13.3), so those shapes keep it.
 #include "fhd_device.h"
 #include "fhd_kernels.h"
 #include "fft_common.h"
 
 namespace fhd {
 
-// Lines in LDS: line l starts at (l / L1) * S1 + (l % L1) * S0, element stride es.
-struct LineMap {
-  int lines, L1, S1, S0, es;
-  FHD_DEV int base(int l) const { return (l / L1) * S1 + (l % L1) * S0; }
+constexpr int kClassElems[3] = {2112, 4224, 8448};  // complex elements of a 256-, 512-, 1024-lane workgroup
+constexpr int kPerLane = 9;                          // ceil(8448 / 1024)
+constexpr int kmax_for(int R) { return (2112 + R * 256 - 1) / (R * 256); }
+
+// Lines of one transform in LDS: line l at l * ls, element stride es; ml = fast_div's reciprocal
+// of the line count.
+struct Lines {
+  int count;
+  uint32_t ml;
+  int ls, es;
 };
 
-// One Stockham radix-R stage over all lines (Govindaraju et al., SC'08 formulation):
+// One radix-R Stockham stage over all lines (Govindaraju et al., SC'08 formulation):
 // butterfly j of a line reads x[j + r n/R], twiddles by w^{(j mod Ns) r}, w = e^{s 2 pi i/(Ns R)},
-// and writes to (j / Ns) Ns R + (j mod Ns) + r Ns.  In place: every thread reads its
-// butterflies into registers, the workgroup synchronises, then writes.  Consecutive lanes take
-// butterfly j of consecutive lines, which keeps the early stages' strided writes out of each
-// other's LDS banks (consecutive butterflies of one line would collide R ways).
-template <int R, int KMAX>
-FHD_DEV void stockham_stage(float2* buf, const LineMap& lm, int n, int Ns, const float2* tw, int twmul,
+// and writes to (j / Ns) Ns R + (j mod Ns) + r Ns.  In place: every lane reads its butterflies
+// into registers, the workgroup synchronises, then writes.  Consecutive lanes take butterfly j of
+// consecutive lines, which lie an odd number of elements apart or next to each other, so the
+// lanes of a wave use different LDS banks and share one twiddle.
+template <int R, int NT>
+FHD_DEV void stockham_stage(float2* buf, const Lines& ln, int n, int Ns, uint32_t mns, const float2* tw, int twmul,
                             float s) {
+  constexpr int KMAX = kmax_for(R);
   const int nbl = n / R;
-  const int total = lm.lines * nbl;
+  const int total = ln.count * nbl;
+  const int twstep = n / (Ns * R) * twmul;
+  // opaque to the compiler, which otherwise hoists the lane indices of every radix's stage out of
+  // the stage loop and spills them (150 VGPRs)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
   float2 v[KMAX][R];
   int wbase[KMAX];
-  const int stride = n / (Ns * R);
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
-    int b = threadIdx.x + k * blockDim.x;
+    const int b = tid + k * NT;
     wbase[k] = -1;
     if (b < total) {
-      int j = b / lm.lines;
-      int l = b - j * lm.lines;
-      int base = lm.base(l);
-      int kk = j % Ns;
+      const int j = fast_div(b, ln.ml), l = b - j * ln.count;
+      const int base = l * ln.ls;
+      const int step = nbl * ln.es;
+      int at = base + j * ln.es;
+      if (Ns == 1) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float2 x = buf[base + (j + r * nbl) * lm.es];
-        if (r > 0 && kk > 0) {
-          float2 w = tw[(kk * r * stride) * twmul];
-          if (s > 0.0f) w.y = -w.y;
-          x = cmul(x, w);
+        for (int r = 0; r < R; ++r, at += step) v[k][r] = buf[at];
+        wbase[k] = base + j * R * ln.es;
+      } else {
+        const int jn = fast_div(j, mns), kk = j - jn * Ns;
+        const int t1 = kk * twstep;
+#pragma unroll
+        for (int r = 0; r < R; ++r, at += step) {
+          float2 x = buf[at];
+          if (r > 0) {
+            float2 w = tw[r * t1];
+            w.y = s > 0.0f ? -w.y : w.y;
+            x = cmul(x, w);
+          }
+          v[k][r] = x;
         }
-        v[k][r] = x;
+        wbase[k] = base + (jn * Ns * R + kk) * ln.es;
       }
       Dft<R>::run(v[k], s);
-      wbase[k] = base + ((j / Ns) * Ns * R + kk) * lm.es;
     }
   }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     if (wbase[k] >= 0) {
+      int at = wbase[k];
+      const int step = Ns * ln.es;
 #pragma unroll
-      for (int r = 0; r < R; ++r) buf[wbase[k] + r * Ns * lm.es] = v[k][r];
+      for (int r = 0; r < R; ++r, at += step) buf[at] = v[k][r];
     }
   }
   __syncthreads();
 }
 
-// Maximum complex elements staged in LDS by one workgroup.
-constexpr int kLdsElems = 8448;
-constexpr int kThreads = 256;
-constexpr int kmax_for(int R) { return (kLdsElems + R * kThreads - 1) / (R * kThreads); }
-
-// Full FFT of length n on all lines described by lm (radix plan packed 4 bits per stage).
-FHD_DEV void lds_fft(float2* buf, const LineMap& lm, int n, uint32_t plan, int nstages, const float2* tw,
-                     int twmul, float s) {
+// Full FFT of every line: at most three stages.
+template <int NT>
+FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const float2* tw, int twmul, float s) {
   int Ns = 1;
-  for (int st = 0; st < nstages; ++st) {
-    int R = (plan >> (4 * st)) & 15;
+  for (int st = 0; st < p.nst; ++st) {
+    const int R = p.radix[st];
+    const uint32_t mns = p.mns[st];
     switch (R) {
-      case 8: stockham_stage<8, kmax_for(8)>(buf, lm, n, Ns, tw, twmul, s); break;
-      case 4: stockham_stage<4, kmax_for(4)>(buf, lm, n, Ns, tw, twmul, s); break;
-      case 3: stockham_stage<3, kmax_for(3)>(buf, lm, n, Ns, tw, twmul, s); break;
-      default: stockham_stage<2, kmax_for(2)>(buf, lm, n, Ns, tw, twmul, s); break;
+      case 16: stockham_stage<16, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
+      case 9: stockham_stage<9, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
+      case 8: stockham_stage<8, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
+      case 6: stockham_stage<6, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
+      case 4: stockham_stage<4, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
+      case 3: stockham_stage<3, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
+      default: stockham_stage<2, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
     }
     Ns *= R;
   }
 }
 
 // ---------------------------------------------------------------------------------------
-// Pass A: real plane -> half spectrum along x -> FFT along y.
+// Pass A: real plane -> half spectrum along x -> FFT along y.  LDS rows of PS = P | 1 elements
+// (odd, so that the rows of an x stage start in different banks).
 // ---------------------------------------------------------------------------------------
+template <int NT, int ELEMS>
 FHD_BODY void body_fft_xy_fwd(const FftArgs& a, const float* __restrict__ in, float2* __restrict__ spec,
                               const Blk& b) {
-  __shared__ float2 buf[kLdsElems];
+  __shared__ float2 buf[ELEMS];
   __shared__ float2 twx[kMaxFftLen];
   __shared__ float2 twy[kMaxFftLen];
   const int z = b.x, c = b.y;
-  const int mx = a.g.mx, my = a.g.my, mz = a.g.mz, P = a.g.P, h = mx / 2;
-  for (int i = threadIdx.x; i < mx; i += blockDim.x) twx[i] = a.twx[i];
-  for (int i = threadIdx.x; i < my; i += blockDim.x) twy[i] = a.twy[i];
-  float* fbuf = reinterpret_cast<float*>(buf);
-  const float* src = in + ((size_t)c * mz + z) * (size_t)my * mx;
-  for (int e = threadIdx.x; e < mx * my; e += blockDim.x) {
-    int y = e / mx, x = e - y * mx;
-    fbuf[y * 2 * P + x] = src[e];
+  const int mx = a.g.mx, my = a.g.my, mz = a.g.mz, P = a.g.P, h = mx / 2, PS = P | 1;
+  const float2* src = reinterpret_cast<const float2*>(in + ((size_t)c * mz + z) * (size_t)my * mx);
+  float2 v[kPerLane];
+#pragma unroll
+  for (int k = 0; k < kPerLane; ++k) {
+    const int e = threadIdx.x + k * NT;
+    if (e < h * my) v[k] = src[e];
+  }
+  for (int i = threadIdx.x; i < mx; i += NT) twx[i] = a.twx[i];
+  for (int i = threadIdx.x; i < my; i += NT) twy[i] = a.twy[i];
+#pragma unroll
+  for (int k = 0; k < kPerLane; ++k) {
+    const int e = threadIdx.x + k * NT;
+    if (e < h * my) {
+      const int y = fast_div(e, a.mdh);
+      buf[e + y * (PS - h)] = v[k];
+    }
   }
   __syncthreads();
   // x: h-point complex FFT of the even/odd-packed rows
-  LineMap rows = {my, my, 0, P, 1};
-  lds_fft(buf, rows, h, a.plan_h, a.nst_h, twx, 2, -1.0f);
+  lds_fft<NT>(buf, Lines{my, a.mdy, PS, 1}, a.lx, twx, 2, -1.0f);
   // even/odd split: X[k] = E + w^k O, X[h-k] = conj(E - w^k O)
   const int npair = h / 2 + 1;
-  for (int e = threadIdx.x; e < my * npair; e += blockDim.x) {
-    int y = e / npair, k = e - y * npair;
-    float2* row = buf + y * P;
-    float2 A = row[k];
-    float2 B = cconj(row[(h - k) % h]);
-    float2 E = cscale(cadd(A, B), 0.5f);
-    float2 D = csub(A, B);
-    float2 O = make_float2(0.5f * D.y, -0.5f * D.x);  // (A - B) / (2i)
-    float2 wO = cmul(twx[k], O);
+  for (int e = threadIdx.x; e < my * npair; e += NT) {
+    const int k = fast_div(e, a.mdy), y = e - k * my;
+    float2* row = buf + y * PS;
+    const float2 A = row[k];
+    const float2 B = cconj(row[k == 0 ? 0 : h - k]);
+    const float2 E = cscale(cadd(A, B), 0.5f);
+    const float2 D = csub(A, B);
+    const float2 O = make_float2(0.5f * D.y, -0.5f * D.x);  // (A - B) / (2i)
+    const float2 wO = cmul(twx[k], O);
     if (k == 0) {
       row[0] = make_float2(E.x + O.x, 0.0f);
       row[h] = make_float2(E.x - O.x, 0.0f);
@@ -138,172 +181,230 @@ FHD_BODY void body_fft_xy_fwd(const FftArgs& a, const float* __restrict__ in, fl
   }
   __syncthreads();
   // y: columns kx = 0..P-1
-  LineMap cols = {P, P, 0, 1, P};
-  lds_fft(buf, cols, my, a.plan_y, a.nst_y, twy, 1, -1.0f);
-  for (int e = threadIdx.x; e < P * my; e += blockDim.x) {
-    int ky = e / P, kx = e - ky * P;
-    spec[(((size_t)c * my + ky) * mz + z) * P + kx] = buf[e];
+  lds_fft<NT>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1, -1.0f);
+  float2* dst = spec + ((size_t)c * my * mz + z) * P;
+#pragma unroll
+  for (int k = 0; k < kPerLane; ++k) {
+    const int e = threadIdx.x + k * NT;
+    if (e < P * my) {
+      const int ky = fast_div(e, a.mdp), kx = e - ky * P;
+      dst[(size_t)ky * mz * P + kx] = buf[ky * PS + kx];
+    }
   }
 }
-FHD_KERNEL_PAIR((), kThreads, k_fft_xy_fwd, FftPass, body_fft_xy_fwd(a.f, a.in, a.spec, b))
+FHD_KERNEL_PAIR_OCC((template <int NT, int ELEMS>), NT, 8, k_fft_xy_fwd, FftPass,
+                    body_fft_xy_fwd<NT, ELEMS>(a.f, a.in, a.spec, b))
 
 // ---------------------------------------------------------------------------------------
 // Pass B: FFT along z, Fourier-space operator, inverse FFT along z, for all three components.
+// The P columns of a ky row are cut into b.nx tiles whose widths differ by at most one; a tile's
+// columns lie on a grid of T (the widest tile) per component, lines of LS = mz | 1 elements.
 // ---------------------------------------------------------------------------------------
-FHD_BODY void body_fft_z_solve(const FftArgs& a, float2* __restrict__ spec, const Blk& b) {
-  __shared__ float2 buf[kLdsElems];
-  __shared__ float2 twz[kMaxFftLen];
-  __shared__ float2 ezs[kMaxFftLen];
+template <int NT, int ELEMS>
+FHD_BODY void body_fft_z_solve(const FftArgs& a, float2* __restrict__ spec, int T, const Blk& b) {
+  __shared__ float2 buf[ELEMS];
+  __shared__ float2 twz[kMaxFftLen], ezs[kMaxFftLen];
   __shared__ float gzs[kMaxFftLen];
-  const int T = a.ztile;
-  const int kx0 = b.x * T, ky = b.y;
-  const int my = a.g.my, mz = a.g.mz, P = a.g.P;
-  for (int i = threadIdx.x; i < mz; i += blockDim.x) {
+  const int my = a.g.my, mz = a.g.mz, P = a.g.P, LS = mz | 1;
+  // neighbouring column tiles share the 128-byte lines of each z row: keep them on one XCD
+  const int item = xcd_item(b.x + b.nx * b.y, b.nx * b.ny);
+  const int ky = item / b.nx, tile = item - ky * b.nx;
+  const int wide = P / b.nx, rem = P - wide * b.nx;
+  const int kx0 = tile * wide + min(tile, rem), w = wide + (tile < rem ? 1 : 0);
+  const uint32_t mt = fast_div_magic(T), mlz = fast_div_magic(mz);
+  const int tot = a.ncomp * mz * T;
+  const size_t cstride = (size_t)my * mz * P;
+  float2* base = spec + (size_t)ky * mz * P + kx0;
+  float2 v[kPerLane];
+#pragma unroll
+  for (int k = 0; k < kPerLane; ++k) {
+    const int e = threadIdx.x + k * NT;
+    const int r = fast_div(e, mt), t = e - r * T, c = fast_div(r, mlz), z = r - c * mz;
+    if (e < tot && t < w) v[k] = base[c * cstride + z * P + t];
+  }
+  for (int i = threadIdx.x; i < mz; i += NT) {
     twz[i] = a.twz[i];
     ezs[i] = a.ez[i];
     gzs[i] = a.gz[i];
   }
-  const int tot = a.ncomp * mz * T;
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int c = e / (mz * T), r = e - c * mz * T, z = r / T, t = r - z * T;
-    int kx = kx0 + t;
-    float2 val = make_float2(0.0f, 0.0f);
-    if (kx < P) val = spec[(((size_t)c * my + ky) * mz + z) * P + kx];
-    buf[e] = val;
+#pragma unroll
+  for (int k = 0; k < kPerLane; ++k) {
+    const int e = threadIdx.x + k * NT;
+    const int r = fast_div(e, mt), t = e - r * T, c = fast_div(r, mlz), z = r - c * mz;
+    if (e < tot && t < w) buf[(c * T + t) * LS + z] = v[k];
   }
   __syncthreads();
-  LineMap zl = {a.ncomp * T, T, mz * T, 1, T};
-  if (a.zmode != 2) lds_fft(buf, zl, mz, a.plan_z, a.nst_z, twz, 1, -1.0f);
-  if (a.zmode != 0) {
-    // transform-only modes (building blocks for the parity tests): no operator, no scaling
-    if (a.zmode == 2) lds_fft(buf, zl, mz, a.plan_z, a.nst_z, twz, 1, 1.0f);
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-      int c = e / (mz * T), r = e - c * mz * T, z = r / T, t = r - z * T;
-      int kx = kx0 + t;
-      if (kx < P) spec[(((size_t)c * my + ky) * mz + z) * P + kx] = buf[e];
+  const Lines zl{a.ncomp * T, fast_div_magic(a.ncomp * T), LS, 1};
+  if (a.zmode != 2) lds_fft<NT>(buf, zl, a.lz, twz, 1, -1.0f);
+  if (a.zmode == 0) {
+    // Fourier-space operator in the staggered (shifted) basis; 1/N normalisation folded in.
+    const float gy = a.gy[ky];
+    const float2 ey = a.ey[ky];
+    const Key key = a.knoise ? resolve_key(a.key) : a.key;
+    for (int e = threadIdx.x; e < mz * w; e += NT) {
+      const int t = fast_div(e, mlz), z = e - t * mz, kx = kx0 + t;
+      const float gx = a.gx[kx];
+      const float2 ex = a.ex[kx];
+      const float gz = gzs[z];
+      const float2 ez = ezs[z];
+      const int i0 = t * LS + z, i1 = i0 + T * LS, i2 = i1 + T * LS;
+      float2 b0 = buf[i0], b1 = buf[i1], b2 = buf[i2];
+      if (a.knoise) {
+        // the kept part of the stochastic stress divergence, drawn in Fourier space (Stokes limit)
+        float2 nw[3];
+        kspace_noise(key, kx, ky, z, a.g.mx, my, mz, a.knoise, a.kn_f4, a.kn_sqrt_half_n, gx, gy, gz, ex, ey, ez, nw);
+        b0 = cadd(b0, nw[0]);
+        b1 = cadd(b1, nw[1]);
+        b2 = cadd(b2, nw[2]);
+      }
+      const float2 w0 = cmul(b0, cconj(ex));
+      const float2 w1 = cmul(b1, cconj(ey));
+      const float2 w2 = cmul(b2, cconj(ez));
+      const float L = -(gx * gx + gy * gy + gz * gz);
+      float2 o0, o1, o2;
+      if (kx == 0 && ky == 0 && z == 0) {
+        const float keep = a.stokes ? 0.0f : a.inv_n;
+        o0 = cscale(w0, keep);
+        o1 = cscale(w1, keep);
+        o2 = cscale(w2, keep);
+      } else {
+        const float2 GW = make_float2(gx * w0.x + gy * w1.x + gz * w2.x, gx * w0.y + gy * w1.y + gz * w2.y);
+        const float den = a.stokes ? (-a.eta * L) : (1.0f - a.cn_coef * L);
+        const float sc = a.inv_n / den;
+        const float iL = 1.0f / L;
+        o0 = cscale(make_float2(w0.x + gx * GW.x * iL, w0.y + gx * GW.y * iL), sc);
+        o1 = cscale(make_float2(w1.x + gy * GW.x * iL, w1.y + gy * GW.y * iL), sc);
+        o2 = cscale(make_float2(w2.x + gz * GW.x * iL, w2.y + gz * GW.y * iL), sc);
+      }
+      buf[i0] = cmul(o0, ex);
+      buf[i1] = cmul(o1, ey);
+      buf[i2] = cmul(o2, ez);
     }
-    return;
+    __syncthreads();
   }
-  // Fourier-space operator in the staggered (shifted) basis; 1/N normalisation folded in.
-  const float gy = a.gy[ky];
-  const float2 ey = a.ey[ky];
-  const Key key = a.knoise ? resolve_key(a.key) : a.key;
-  for (int e = threadIdx.x; e < mz * T; e += blockDim.x) {
-    int z = e / T, t = e - z * T;
-    int kx = kx0 + t;
-    if (kx >= P) continue;
-    float gx = a.gx[kx];
-    float2 ex = a.ex[kx];
-    float gz = gzs[z];
-    float2 ez = ezs[z];
-    float2 b0 = buf[e], b1 = buf[mz * T + e], b2 = buf[2 * mz * T + e];
-    if (a.knoise) {
-      // the kept part of the stochastic stress divergence, drawn in Fourier space (Stokes limit)
-      float2 nw[3];
-      kspace_noise(key, kx, ky, z, a.g.mx, my, mz, a.knoise, a.kn_f4, a.kn_sqrt_half_n, gx, gy, gz,
-                        ex, ey, ez, nw);
-      b0 = cadd(b0, nw[0]);
-      b1 = cadd(b1, nw[1]);
-      b2 = cadd(b2, nw[2]);
-    }
-    float2 w0 = cmul(b0, cconj(ex));
-    float2 w1 = cmul(b1, cconj(ey));
-    float2 w2 = cmul(b2, cconj(ez));
-    float L = -(gx * gx + gy * gy + gz * gz);
-    float2 o0, o1, o2;
-    if (kx == 0 && ky == 0 && z == 0) {
-      float keep = a.stokes ? 0.0f : a.inv_n;
-      o0 = cscale(w0, keep);
-      o1 = cscale(w1, keep);
-      o2 = cscale(w2, keep);
-    } else {
-      float2 GW = make_float2(gx * w0.x + gy * w1.x + gz * w2.x, gx * w0.y + gy * w1.y + gz * w2.y);
-      float den = a.stokes ? (-a.eta * L) : (1.0f - a.cn_coef * L);
-      float sc = a.inv_n / den;
-      float iL = 1.0f / L;
-      o0 = cscale(make_float2(w0.x + gx * GW.x * iL, w0.y + gx * GW.y * iL), sc);
-      o1 = cscale(make_float2(w1.x + gy * GW.x * iL, w1.y + gy * GW.y * iL), sc);
-      o2 = cscale(make_float2(w2.x + gz * GW.x * iL, w2.y + gz * GW.y * iL), sc);
-    }
-    buf[e] = cmul(o0, ex);
-    buf[mz * T + e] = cmul(o1, ey);
-    buf[2 * mz * T + e] = cmul(o2, ez);
-  }
-  __syncthreads();
-  lds_fft(buf, zl, mz, a.plan_z, a.nst_z, twz, 1, 1.0f);
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int c = e / (mz * T), r = e - c * mz * T, z = r / T, t = r - z * T;
-    int kx = kx0 + t;
-    if (kx < P) spec[(((size_t)c * my + ky) * mz + z) * P + kx] = buf[e];
+  if (a.zmode != 1) lds_fft<NT>(buf, zl, a.lz, twz, 1, 1.0f);
+  // the lane index, opaque to the compiler: the store indices are recomputed here rather than
+  // kept live in registers from the loads through both transforms
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+#pragma unroll
+  for (int k = 0; k < kPerLane; ++k) {
+    const int e = tid + k * NT;
+    const int r = fast_div(e, mt), t = e - r * T, c = fast_div(r, mlz), z = r - c * mz;
+    if (e < tot && t < w) base[c * cstride + z * P + t] = buf[(c * T + t) * LS + z];
   }
 }
-FHD_KERNEL_PAIR((), kThreads, k_fft_z_solve, FftPass, body_fft_z_solve(a.f, a.spec, b))
+FHD_KERNEL_PAIR_OCC((template <int NT, int ELEMS>), NT, 8, k_fft_z_solve, FftPass,
+                    body_fft_z_solve<NT, ELEMS>(a.f, a.spec, a.T, b))
 
 // ---------------------------------------------------------------------------------------
 // Pass C: inverse FFT along y, C2R along x; out = alpha * result + beta * aux.
 // ---------------------------------------------------------------------------------------
+template <int NT, int ELEMS>
 FHD_BODY void body_fft_xy_inv(const FftArgs& a, const float2* __restrict__ spec, float* __restrict__ out,
                               const float* __restrict__ aux, float alpha, float beta, const Blk& b) {
-  __shared__ float2 buf[kLdsElems];
+  __shared__ float2 buf[ELEMS];
   __shared__ float2 twx[kMaxFftLen];
   __shared__ float2 twy[kMaxFftLen];
   const int z = b.x, c = b.y;
-  const int mx = a.g.mx, my = a.g.my, mz = a.g.mz, P = a.g.P, h = mx / 2;
-  for (int i = threadIdx.x; i < mx; i += blockDim.x) twx[i] = a.twx[i];
-  for (int i = threadIdx.x; i < my; i += blockDim.x) twy[i] = a.twy[i];
-  for (int e = threadIdx.x; e < P * my; e += blockDim.x) {
-    int ky = e / P, kx = e - ky * P;
-    buf[e] = spec[(((size_t)c * my + ky) * mz + z) * P + kx];
+  const int mx = a.g.mx, my = a.g.my, mz = a.g.mz, P = a.g.P, h = mx / 2, PS = P | 1;
+  const float2* src = spec + ((size_t)c * my * mz + z) * P;
+  {
+    float2 v[kPerLane];
+#pragma unroll
+    for (int k = 0; k < kPerLane; ++k) {
+      const int e = threadIdx.x + k * NT;
+      const int ky = fast_div(e, a.mdp), kx = e - ky * P;
+      if (e < P * my) v[k] = src[(size_t)ky * mz * P + kx];
+    }
+    for (int i = threadIdx.x; i < mx; i += NT) twx[i] = a.twx[i];
+    for (int i = threadIdx.x; i < my; i += NT) twy[i] = a.twy[i];
+#pragma unroll
+    for (int k = 0; k < kPerLane; ++k) {
+      const int e = threadIdx.x + k * NT;
+      const int ky = fast_div(e, a.mdp), kx = e - ky * P;
+      if (e < P * my) buf[ky * PS + kx] = v[k];
+    }
   }
   __syncthreads();
-  LineMap cols = {P, P, 0, 1, P};
-  lds_fft(buf, cols, my, a.plan_y, a.nst_y, twy, 1, 1.0f);
+  lds_fft<NT>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1, 1.0f);
   // C2R packing: Z[k] = (X[k] + conj X[h-k]) + i (X[k] - conj X[h-k]) e^{+2 pi i k / mx}
   const int npair = h / 2 + 1;
-  for (int e = threadIdx.x; e < my * npair; e += blockDim.x) {
-    int y = e / npair, k = e - y * npair;
-    float2* row = buf + y * P;
-    float2 Xk = row[k], Xh = row[h - k];
-    float2 wk = cconj(twx[k]);  // e^{+2 pi i k / mx}
-    float2 B = cconj(Xh);
-    float2 Zk = cadd(cadd(Xk, B), cmul_si(cmul(csub(Xk, B), wk), 1.0f));
+  for (int e = threadIdx.x; e < my * npair; e += NT) {
+    const int k = fast_div(e, a.mdy), y = e - k * my;
+    float2* row = buf + y * PS;
+    const float2 Xk = row[k], Xh = row[h - k];
+    const float2 wk = cconj(twx[k]);  // e^{+2 pi i k / mx}
+    const float2 B = cconj(Xh);
+    const float2 Zk = cadd(cadd(Xk, B), cmul_si(cmul(csub(Xk, B), wk), 1.0f));
     if (k != 0 && h - k != k) {
-      float2 B2 = cconj(Xk);
-      float2 wk2 = make_float2(-wk.x, wk.y);  // e^{+2 pi i (h-k)/mx} = -conj(e^{+2 pi i k/mx})
-      float2 Zh = cadd(cadd(Xh, B2), cmul_si(cmul(csub(Xh, B2), wk2), 1.0f));
-      row[h - k] = Zh;
+      const float2 B2 = cconj(Xk);
+      const float2 wk2 = make_float2(-wk.x, wk.y);  // e^{+2 pi i (h-k)/mx} = -conj(e^{+2 pi i k/mx})
+      row[h - k] = cadd(cadd(Xh, B2), cmul_si(cmul(csub(Xh, B2), wk2), 1.0f));
     }
     row[k] = Zk;
   }
   __syncthreads();
-  LineMap rows = {my, my, 0, P, 1};
-  lds_fft(buf, rows, h, a.plan_h, a.nst_h, twx, 2, 1.0f);
-  const float* fbuf = reinterpret_cast<const float*>(buf);
+  lds_fft<NT>(buf, Lines{my, a.mdy, PS, 1}, a.lx, twx, 2, 1.0f);
   const size_t off = ((size_t)c * mz + z) * (size_t)my * mx;
-  for (int e = threadIdx.x; e < mx * my; e += blockDim.x) {
-    int y = e / mx, x = e - y * mx;
-    float val = alpha * fbuf[y * 2 * P + x];
-    if (aux) val += beta * aux[off + e];
-    out[off + e] = val;
+  float2* dst = reinterpret_cast<float2*>(out + off);
+  const float2* ax = reinterpret_cast<const float2*>(aux + off);
+  float2 q[kPerLane];
+  if (aux) {
+#pragma unroll
+    for (int k = 0; k < kPerLane; ++k) {
+      const int e = threadIdx.x + k * NT;
+      if (e < h * my) q[k] = ax[e];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kPerLane; ++k) {
+    const int e = threadIdx.x + k * NT;
+    if (e < h * my) {
+      const int y = fast_div(e, a.mdh);
+      const float2 p = buf[e + y * (PS - h)];
+      float2 r = make_float2(alpha * p.x, alpha * p.y);
+      if (aux) {
+        r.x += beta * q[k].x;
+        r.y += beta * q[k].y;
+      }
+      dst[e] = r;
+    }
   }
 }
-FHD_KERNEL_PAIR((), kThreads, k_fft_xy_inv, FftPass, body_fft_xy_inv(a.f, a.spec, a.out, a.aux, a.alpha, a.beta, b))
+FHD_KERNEL_PAIR_OCC((template <int NT, int ELEMS>), NT, 8, k_fft_xy_inv, FftPass,
+                    body_fft_xy_inv<NT, ELEMS>(a.f, a.spec, a.out, a.aux, a.alpha, a.beta, b))
+
+// Workgroup class of a pass that holds `elems` complex elements.
+static int lds_class(int elems) { return elems <= kClassElems[0] ? 0 : elems <= kClassElems[1] ? 1 : 2; }
+
+#define FHD_LAUNCH_CLASS(cls, kern, fam, grid, x, s)                                                     \
+  do {                                                                                                   \
+    if ((cls) == 0) launch(kern<256, kClassElems[0]>, kern##_b<256, kClassElems[0]>, fam, grid, 256, x, s); \
+    else if ((cls) == 1) launch(kern<512, kClassElems[1]>, kern##_b<512, kClassElems[1]>, fam, grid, 512, x, s); \
+    else launch(kern<1024, kClassElems[2]>, kern##_b<1024, kClassElems[2]>, fam, grid, 1024, x, s);      \
+  } while (0)
 
 void launch_fft_xy_fwd(const FftArgs& a, const float* in, float2* spec, hipStream_t s) {
   if (!a.generic && fast_fft_xy_fwd(a, in, spec, s)) return;
   const FftPass x{a, in, spec, nullptr, nullptr, 0.0f, 0.0f, 0};
-  launch(k_fft_xy_fwd, k_fft_xy_fwd_b, FAM_FFT_XY_FWD, dim3(a.g.mz, a.ncomp), kThreads, x, s);
+  FHD_LAUNCH_CLASS(lds_class(a.g.my * (a.g.P | 1)), k_fft_xy_fwd, FAM_FFT_XY_FWD, dim3(a.g.mz, a.ncomp), x, s);
 }
+// Columns per z-pass workgroup: the schedule's tile, as far as the largest class holds it.
 void launch_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s) {
   if (!a.generic && fast_fft_z_solve(a, spec, s)) return;
-  const FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, 0};
-  launch(k_fft_z_solve, k_fft_z_solve_b, FAM_FFT_Z, dim3((a.g.P + a.ztile - 1) / a.ztile, a.g.my), kThreads, x, s);
+  const int LS = a.g.mz | 1;
+  const int most = kClassElems[2] / (3 * LS);  // >= 10: mz is at most 256
+  const int want = a.btile < most ? a.btile : most;
+  const int ntile = (a.g.P + want - 1) / want, T = (a.g.P + ntile - 1) / ntile;
+  const FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, T};
+  FHD_LAUNCH_CLASS(lds_class(3 * T * LS), k_fft_z_solve, FAM_FFT_Z, dim3(ntile, a.g.my), x, s);
 }
 void launch_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha, float beta,
                        hipStream_t s) {
   if (!a.generic && fast_fft_xy_inv(a, spec, out, aux, alpha, beta, s)) return;
   const FftPass x{a, nullptr, const_cast<float2*>(spec), out, aux, alpha, beta, 0};
-  launch(k_fft_xy_inv, k_fft_xy_inv_b, FAM_FFT_XY_INV, dim3(a.g.mz, a.ncomp), kThreads, x, s);
+  FHD_LAUNCH_CLASS(lds_class(a.g.my * (a.g.P | 1)), k_fft_xy_inv, FAM_FFT_XY_INV, dim3(a.g.mz, a.ncomp), x, s);
 }
 
 }  // namespace fhd

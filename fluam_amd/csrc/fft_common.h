@@ -44,6 +44,50 @@ template <> struct Dft<4> {
     v[3] = csub(t1, t3);
   }
 };
+template <> struct Dft<6> {
+  static FHD_DEV void run(float2* v, float s) {
+    float2 e[3] = {v[0], v[2], v[4]}, o[3] = {v[1], v[3], v[5]};
+    Dft<3>::run(e, s);
+    Dft<3>::run(o, s);
+    // w^k = e^{s 2 pi i k / 6}
+    const float c3 = 0.86602540378443864676f;
+    const float2 o1 = cmul(o[1], make_float2(0.5f, s * c3)), o2 = cmul(o[2], make_float2(-0.5f, s * c3));
+    v[0] = cadd(e[0], o[0]);
+    v[3] = csub(e[0], o[0]);
+    v[1] = cadd(e[1], o1);
+    v[4] = csub(e[1], o1);
+    v[2] = cadd(e[2], o2);
+    v[5] = csub(e[2], o2);
+  }
+};
+template <> struct Dft<9> {
+  static FHD_DEV void run(float2* v, float s) {
+    // three 3-point transforms of every third element, twiddles e^{s 2 pi i b k / 9}, three more
+    float2 y[3][3];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+      y[b][0] = v[b];
+      y[b][1] = v[b + 3];
+      y[b][2] = v[b + 6];
+      Dft<3>::run(y[b], s);
+    }
+    const float c1 = 0.76604444311897803520f, s1 = 0.64278760968653932632f;  // 2 pi / 9
+    const float c2 = 0.17364817766693034885f, s2 = 0.98480775301220805937f;  // 4 pi / 9
+    const float c4 = -0.93969262078590838405f, s4 = 0.34202014332566873304f;  // 8 pi / 9
+    y[1][1] = cmul(y[1][1], make_float2(c1, s * s1));
+    y[1][2] = cmul(y[1][2], make_float2(c2, s * s2));
+    y[2][1] = cmul(y[2][1], make_float2(c2, s * s2));
+    y[2][2] = cmul(y[2][2], make_float2(c4, s * s4));
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      float2 t[3] = {y[0][k], y[1][k], y[2][k]};
+      Dft<3>::run(t, s);
+      v[k] = t[0];
+      v[k + 3] = t[1];
+      v[k + 6] = t[2];
+    }
+  }
+};
 template <> struct Dft<8> {
   static FHD_DEV void run(float2* v, float s) {
     float2 e[4] = {v[0], v[2], v[4], v[6]};

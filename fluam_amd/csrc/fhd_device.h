@@ -15,6 +15,10 @@ FHD_DEV int xcd_item(int b, int n) {
   return (b % kXcd) * (n / kXcd) + b / kXcd;
 }
 
+// n / d for n d < 2^32 by multiplication with ceil(2^32 / d) (0 stands for d = 1).
+__host__ FHD_DEV uint32_t fast_div_magic(int d) { return 0xFFFFFFFFu / (uint32_t)d + 1u; }
+FHD_DEV int fast_div(int n, uint32_t magic) { return magic ? (int)__umulhi((uint32_t)n, magic) : n; }
+
 // Device error flags (bits of the context's error word; cf. fluam's errorKernel,
 // src/allocateErrorArray.cu:22-32): a non-finite particle displacement, and a displacement of
 // 2^24 cells or more that was not applied.

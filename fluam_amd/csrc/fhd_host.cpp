@@ -46,23 +46,47 @@ bool g_params_loaded = false;
     }                                                                                  \
   } while (0)
 
-// Radix plan for an n-point complex FFT: stages of 8, then 4, 2, 3, packed 4 bits each.
-bool make_plan(int n, uint32_t* plan, int* nst) {
-  uint32_t p = 0;
-  int k = 0;
-  int m = n;
-  const int rs[4] = {8, 4, 2, 3};
-  for (int r : rs)
-    while (m % r == 0) {
-      if (k >= 8) return false;
-      p |= (uint32_t)r << (4 * k);
-      ++k;
-      m /= r;
-    }
-  if (m != 1) return false;
-  *plan = p;
-  *nst = k;
+// Radix plan for an n-point complex FFT: the fewest stages of radix at most 16, and among those
+// the one whose largest radix is smallest (fewer registers).  False when n is not 2^a 3^b.
+bool make_plan(int n, LinePlan* p) {
+  const int rs[7] = {2, 3, 4, 6, 8, 9, 16};
+  p->n = n;
+  p->nst = 0;
+  for (int k = 0; k < 3; ++k) p->radix[k] = 1;
+  if (n == 1) return true;
+  int best[3] = {0, 0, 0}, most = 99;
+  for (int nst = 1; nst <= 3 && !best[0]; ++nst)
+    for (int r0 : rs)
+      for (int r1 : rs) {
+        if (nst < 2 && r1 != rs[0]) continue;
+        for (int r2 : rs) {
+          if (nst < 3 && r2 != rs[0]) continue;
+          const int q0 = r0, q1 = nst > 1 ? r1 : 1, q2 = nst > 2 ? r2 : 1;
+          // the largest radix first: the first stage has no twiddles
+          if (q0 * q1 * q2 != n || q0 < q1 || q1 < q2 || q0 >= most) continue;
+          most = q0;
+          best[0] = q0; best[1] = q1; best[2] = q2;
+          p->nst = nst;
+        }
+      }
+  if (!best[0]) return false;
+  int Ns = 1;
+  for (int k = 0; k < p->nst; ++k) {
+    p->radix[k] = best[k];
+    p->mns[k] = fast_div_magic(Ns);
+    Ns *= best[k];
+  }
   return true;
+}
+
+// The runtime-size kernels' plans and reciprocals for an mx x my x mz grid.
+void fill_plans(FftArgs& a, int mx, int my, int mz) {
+  make_plan(mx / 2, &a.lx);
+  make_plan(my, &a.ly);
+  make_plan(mz, &a.lz);
+  a.mdh = fast_div_magic(mx / 2);
+  a.mdp = fast_div_magic(mx / 2 + 1);
+  a.mdy = fast_div_magic(my);
 }
 
 int tile_edge(int m) {
@@ -253,9 +277,8 @@ void validate(const fhd_params& p) {
   if (p.mx % 2) throw std::runtime_error("mx must be even (real-to-complex FFT along x)");
   if (p.mx > kMaxFftLen || p.my > kMaxFftLen || p.mz > kMaxFftLen)
     throw std::runtime_error("cells per axis must be <= 256");
-  uint32_t pl;
-  int ns;
-  if (!make_plan(p.mx / 2, &pl, &ns) || !make_plan(p.my, &pl, &ns) || !make_plan(p.mz, &pl, &ns))
+  LinePlan pl;
+  if (!make_plan(p.mx / 2, &pl) || !make_plan(p.my, &pl) || !make_plan(p.mz, &pl))
     throw std::runtime_error("cells per axis must be of the form 2^a 3^b");
   if ((p.mx / 2 + 1) * p.my > 8448) throw std::runtime_error("xy plane too large for one workgroup");
   if (3 * p.mz > 8448) throw std::runtime_error("mz too large");
@@ -335,10 +358,7 @@ void build_tables(fhd_ctx* c) {
   a.twx = c->twx; a.twy = c->twy; a.twz = c->twz;
   a.gx = c->gx; a.gy = c->gy; a.gz = c->gz;
   a.ex = c->ex; a.ey = c->ey; a.ez = c->ez;
-  make_plan(mx / 2, &a.plan_h, &a.nst_h);
-  make_plan(my, &a.plan_y, &a.nst_y);
-  make_plan(mz, &a.plan_z, &a.nst_z);
-  a.ztile = std::max(1, std::min(16, 8448 / (3 * mz)));
+  fill_plans(a, mx, my, mz);
   a.btile = 8;
   a.plan_xy = 0;
   a.plan_xy_inv = 0;
@@ -2340,10 +2360,7 @@ int fhd_fft_r2c_noalloc(int mx, int my, int mz, const float* in, float* out_spec
     a.ex = tab + 3 * kMaxFftLen; a.ey = tab + 4 * kMaxFftLen; a.ez = tab + 5 * kMaxFftLen;
     const float* gt = reinterpret_cast<const float*>(tab + 6 * kMaxFftLen);
     a.gx = gt; a.gy = gt + kMaxFftLen; a.gz = gt + 2 * kMaxFftLen;
-    make_plan(mx / 2, &a.plan_h, &a.nst_h);
-    make_plan(my, &a.plan_y, &a.nst_y);
-    make_plan(mz, &a.plan_z, &a.nst_z);
-    a.ztile = std::max(1, std::min(16, 8448 / (3 * mz)));
+    fill_plans(a, mx, my, mz);
     a.btile = 8;
     a.zmode = 1;
     a.ncomp = 1;

@@ -9,15 +9,22 @@ namespace fhd {
 
 constexpr int kMaxFftLen = 256;
 
+// Radix plan of one transform length of the runtime-size FFT kernels (at most three stages up to
+// 256 points) and fast_div's reciprocal of each stage's sub-transform length.
+struct LinePlan {
+  int n, nst;
+  int radix[3];
+  uint32_t mns[3];
+};
+
 struct FftArgs {
   GridDev g;
   const float2 *twx, *twy, *twz;  // e^{-2 pi i m / m_a}, m < m_a
   const float *gx, *gy, *gz;      // g_a(k) = (2/h_a) sin(pi k / m_a)
   const float2 *ex, *ey, *ez;     // e^{+i pi k / m_a}
-  uint32_t plan_h, plan_y, plan_z;  // radices, 4 bits per stage
-  int nst_h, nst_y, nst_z;
-  int ztile;                      // kx columns per pass-B workgroup (generic kernels)
-  int btile;                      // kx columns per pass-B workgroup (size-specialised: 2, 4, 8 or 16)
+  LinePlan lx, ly, lz;            // transforms of mx/2, my and mz points (runtime-size kernels)
+  uint32_t mdh, mdp, mdy;         // fast_div's reciprocals of mx/2, P and my
+  int btile;                      // kx columns per pass-B workgroup (2, 4, 8 or 16)
   int plan_xy;                    // radix plans of the forward xy pass (96 x 96, 128 x 128 planes): px + 3 py, 0 default
   int plan_xy_inv;                // the same for the inverse xy pass
   int plan_zs;                    // radix plan of the z pass (128-point columns), 0 default

@@ -36,6 +36,24 @@ def test_generic_fft_matches_numpy(shape):
     assert np.abs(back - a * a.size).max() < 1e-5 * np.abs(a * a.size).max()
 
 
+# (mz, my, mx): the smallest box; every radix (2, 3, 4, 6, 8, 9, 16) first and later in a plan, two and
+# three stages; planes at the edges of the workgroup classes (2112, 4224, 8448 elements), with an odd
+# and an even row length; the longest columns.  FP32 transforms of n points are off by about
+# log2(n) 2^-24 relative to the largest mode, below 2e-6 here; the bound is 1e-5.
+@pytest.mark.parametrize("shape", [(1, 1, 2), (2, 3, 6), (9, 27, 18), (16, 81, 54), (243, 6, 162), (256, 16, 32),
+                                   (12, 64, 64), (8, 128, 64), (4, 256, 64), (3, 64, 256), (216, 12, 108),
+                                   (162, 96, 162), (144, 72, 12)])
+def test_generic_fft_radices_and_workgroup_classes(shape):
+    print(f"[gpu-case] generic fft {shape}", flush=True)
+    rng = np.random.default_rng(11 + sum(shape))
+    a = rng.standard_normal(shape)
+    got = F.fft_r2c(a)
+    ref = np.fft.rfftn(a)
+    assert np.abs(got - ref).max() < 1e-5 * np.abs(ref).max()
+    back = F.fft_c2r(ref, shape[2])
+    assert np.abs(back - a * a.size).max() < 1e-5 * np.abs(a * a.size).max()
+
+
 def _run(p, nsteps):
     print(f"[gpu-case] generic scheme={p.scheme} cells=({p.mx},{p.my},{p.mz}) np={p.np} k={p.kernel_points}",
           flush=True)

@@ -26,27 +26,22 @@ def algorithmic_bytes(N, npart):
 
 
 def kernel_bytes(name, mx, my, mz, npart):
-    """Algorithmic HBM bytes of one launch of a kernel group: the per-pass figures of the
-    whole-step formula (FP32, 3 components, per Stokes solve), split by the kernel that does the
-    pass.  Per cell: spread writes 12 B; the W + xy-forward pass reads 12 and writes 12 (its noise
-    is generated in registers); the z pass reads and writes the half spectrum, 24; the xy-inverse
-    pass 24; the interpolation reads 12.  Per particle: sort 32, force 24, spread 24,
-    interpolation and update 24 (the "wca" group is one launch that also holds the gated sort,
-    which runs only when a particle left its tile's skin).  Passes the formula does not charge
-    (the spreading records;
-    the W pass of the other schemes) get 0 B; their cost is time a fused pipeline would not
-    spend.  The Stokes step's noise is drawn in registers inside the z pass."""
+    """Algorithmic HBM bytes of one launch of a kernel group (FP32, 3 components, per Stokes solve).
+    Per cell: the forward xy pass spreads the sources into its own planes and writes the half
+    spectrum, 12 B; the z pass reads and writes it, 24; the xy-inverse pass 24; the interpolation
+    reads 12.  Per particle: spread 24, sort 32, force 24, interpolation and update 24 (the "wca"
+    group is one launch that also holds the gated sort, which runs only when a particle left its
+    tile's skin).  The W pass of the other schemes gets 0 B.  The Stokes step's noise is drawn in
+    registers inside the z pass."""
     N = mx * my * mz
     per = {
-        "spread": 12 * N + 24 * npart,
-        "fft_xy_fwd": 24 * N,
+        "fft_xy_fwd": 12 * N + 24 * npart,
         "fft_z_solve": 24 * N,
         "fft_xy_inv": 24 * N,
         "interp": 12 * N + 24 * npart,
         "sort": 32 * npart,
         "wca": 24 * npart,
         "fluid_w": 0,
-        "src_prep": 0,
     }
     return per.get(name)
 

@@ -27,9 +27,14 @@
 // 128 x 64 x 32 forward 28.9 -> 13.8 us; 256-point columns of 128 x 128 planes 181 -> 58 us.
 // Where a size-specialised instance exists it stays ahead (128^3: 20.7 / 28.0 / 19.2 against
 // 23.6 / 34.2 / 23.2 us; 64^3: 9.6 / 11.3 / 8.9 against 13.8 / 14.0 / 13.3), so those shapes keep it.
+// The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
+// on the one alone and on the other in a merged batch), so the compiler must not choose which
+// products become fused multiply-adds: the fused ones are written out.
+#pragma clang fp contract(off)
 #include "fhd_device.h"
 #include "fhd_kernels.h"
 #include "fft_common.h"
+#include "plane_spread.h"
 
 namespace fhd {
 
@@ -46,15 +51,16 @@ struct Lines {
 };
 
 // One radix-R Stockham stage over all lines (Govindaraju et al., SC'08 formulation):
-// butterfly j of a line reads x[j + r n/R], twiddles by w^{(j mod Ns) r}, w = e^{s 2 pi i/(Ns R)},
+// butterfly j of a line reads x[j + r n/R], twiddles by w^{(j mod Ns) r}, w = e^{-2 pi i/(Ns R)},
 // and writes to (j / Ns) Ns R + (j mod Ns) + r Ns.  In place: every lane reads its butterflies
 // into registers, the workgroup synchronises, then writes.  Consecutive lanes take butterfly j of
 // consecutive lines, which lie an odd number of elements apart or next to each other, so the
-// lanes of a wave use different LDS banks and share one twiddle.
-template <int R, int NT>
-FHD_DEV void stockham_stage(float2* buf, const Lines& ln, int n, int Ns, uint32_t mns, const float2* tw, int twmul,
-                            float s) {
+// lanes of a wave use different LDS banks and share one twiddle.  INV: the adjoint stage of the
+// inverse transform (fft_stages.h).
+template <int R, int NT, bool INV>
+FHD_DEV void stockham_stage(float2* buf, const Lines& ln, int n, int Ns, uint32_t mns, const float2* tw, int twmul) {
   constexpr int KMAX = kmax_for(R);
+  constexpr float s = INV ? 1.0f : -1.0f;
   const int nbl = n / R;
   const int total = ln.count * nbl;
   const int twstep = n / (Ns * R) * twmul;
@@ -63,44 +69,38 @@ FHD_DEV void stockham_stage(float2* buf, const Lines& ln, int n, int Ns, uint32_
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
   float2 v[KMAX][R];
-  int wbase[KMAX];
+  int to[KMAX];  // first element of the butterfly's outputs, -1: none
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     const int b = tid + k * NT;
-    wbase[k] = -1;
+    to[k] = -1;
     if (b < total) {
       const int j = fast_div(b, ln.ml), l = b - j * ln.count;
       const int base = l * ln.ls;
-      const int step = nbl * ln.es;
-      int at = base + j * ln.es;
-      if (Ns == 1) {
+      const int jn = Ns == 1 ? j : fast_div(j, mns), kk = j - jn * Ns;
+      const int t1 = kk * twstep;
+      const int spread = base + j * ln.es, packed = base + (jn * Ns * R + kk) * ln.es;
+      int at = INV ? packed : spread;
+      const int step = (INV ? Ns : nbl) * ln.es;
 #pragma unroll
-        for (int r = 0; r < R; ++r, at += step) v[k][r] = buf[at];
-        wbase[k] = base + j * R * ln.es;
-      } else {
-        const int jn = fast_div(j, mns), kk = j - jn * Ns;
-        const int t1 = kk * twstep;
-#pragma unroll
-        for (int r = 0; r < R; ++r, at += step) {
-          float2 x = buf[at];
-          if (r > 0) {
-            float2 w = tw[r * t1];
-            w.y = s > 0.0f ? -w.y : w.y;
-            x = cmul(x, w);
-          }
-          v[k][r] = x;
-        }
-        wbase[k] = base + (jn * Ns * R + kk) * ln.es;
+      for (int r = 0; r < R; ++r, at += step) {
+        v[k][r] = buf[at];
+        if (!INV && Ns > 1 && r > 0) v[k][r] = cmul(v[k][r], tw[r * t1]);
       }
       Dft<R>::run(v[k], s);
+      if (INV && Ns > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[k][r] = cmul(v[k][r], cconj(tw[r * t1]));
+      }
+      to[k] = INV ? spread : packed;
     }
   }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
-    if (wbase[k] >= 0) {
-      int at = wbase[k];
-      const int step = Ns * ln.es;
+    if (to[k] >= 0) {
+      int at = to[k];
+      const int step = (INV ? nbl : Ns) * ln.es;
 #pragma unroll
       for (int r = 0; r < R; ++r, at += step) buf[at] = v[k][r];
     }
@@ -108,23 +108,25 @@ FHD_DEV void stockham_stage(float2* buf, const Lines& ln, int n, int Ns, uint32_
   __syncthreads();
 }
 
-// Full FFT of every line: at most three stages.
-template <int NT>
-FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const float2* tw, int twmul, float s) {
-  int Ns = 1;
-  for (int st = 0; st < p.nst; ++st) {
+// Full FFT of every line: at most three stages, undone in reverse order by the inverse.
+template <int NT, bool INV>
+FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const float2* tw, int twmul) {
+  int Ns = INV ? p.n : 1;
+  for (int k = 0; k < p.nst; ++k) {
+    const int st = INV ? p.nst - 1 - k : k;
     const int R = p.radix[st];
     const uint32_t mns = p.mns[st];
+    if (INV) Ns /= R;
     switch (R) {
-      case 16: stockham_stage<16, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
-      case 9: stockham_stage<9, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
-      case 8: stockham_stage<8, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
-      case 6: stockham_stage<6, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
-      case 4: stockham_stage<4, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
-      case 3: stockham_stage<3, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
-      default: stockham_stage<2, NT>(buf, ln, p.n, Ns, mns, tw, twmul, s); break;
+      case 16: stockham_stage<16, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
+      case 9: stockham_stage<9, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
+      case 8: stockham_stage<8, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
+      case 6: stockham_stage<6, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
+      case 4: stockham_stage<4, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
+      case 3: stockham_stage<3, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
+      default: stockham_stage<2, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
     }
-    Ns *= R;
+    if (!INV) Ns *= R;
   }
 }
 
@@ -132,34 +134,71 @@ FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const floa
 // Pass A: real plane -> half spectrum along x -> FFT along y.  LDS rows of PS = P | 1 elements
 // (odd, so that the rows of an x stage start in different banks).
 // ---------------------------------------------------------------------------------------
-template <int NT, int ELEMS>
+// SP: the plane is the sources' spread field (plane_spread.h) plus `in` (null: none).
+template <int NT, int ELEMS, bool SP>
 FHD_BODY void body_fft_xy_fwd(const FftArgs& a, const float* __restrict__ in, float2* __restrict__ spec,
-                              const Blk& b) {
+                              const Blk& b, const PlaneSrc* src_sp) {
   __shared__ float2 buf[ELEMS];
-  __shared__ float2 twx[kMaxFftLen];
-  __shared__ float2 twy[kMaxFftLen];
-  const int z = b.x, c = b.y;
+  // the twiddles of both transforms; before they are stored, plane_spread's lists
+  constexpr int kTw = 2 * kMaxFftLen * sizeof(float2);
+  __shared__ __align__(16) unsigned char side[SP && (int)sizeof(PlaneLds) > kTw ? (int)sizeof(PlaneLds) : kTw];
+  float2* const twx = reinterpret_cast<float2*>(side);
+  float2* const twy = twx + kMaxFftLen;
+  // with spreading, the three components and the neighbouring planes, which read the same sources,
+  // are kept on one XCD
+  const int item = SP ? xcd_item(b.x + b.nx * b.y, b.nx * b.ny) : 0;
+  const int z = SP ? item / b.ny : b.x, c = SP ? item - z * b.ny : b.y;
   const int mx = a.g.mx, my = a.g.my, mz = a.g.mz, P = a.g.P, h = mx / 2, PS = P | 1;
   const float2* src = reinterpret_cast<const float2*>(in + ((size_t)c * mz + z) * (size_t)my * mx);
-  float2 v[kPerLane];
+  if constexpr (!SP) {
+    float2 v[kPerLane];
 #pragma unroll
-  for (int k = 0; k < kPerLane; ++k) {
-    const int e = threadIdx.x + k * NT;
-    if (e < h * my) v[k] = src[e];
+    for (int k = 0; k < kPerLane; ++k) {
+      const int e = threadIdx.x + k * NT;
+      if (e < h * my) v[k] = src[e];
+    }
+#pragma unroll
+    for (int k = 0; k < kPerLane; ++k) {
+      const int e = threadIdx.x + k * NT;
+      if (e < h * my) buf[e + fast_div(e, a.mdh) * (PS - h)] = v[k];
+    }
+  } else {
+    PlaneLds& pl = *reinterpret_cast<PlaneLds*>(side);
+    // the integers become the plane in place; between two sweeps the first sums wait in this
+    // workgroup's own rows of the spectrum (at least mx floats each), written later
+    float* part = reinterpret_cast<float*>(spec + ((size_t)c * my * mz + z) * P);
+    int* acc = reinterpret_cast<int*>(buf);
+    float inv2, rest;
+    const float inv = plane_spread<NT>(acc, 2 * my * PS, 2 * PS, a.g, *src_sp, z, c, pl, 0, &inv2);
+    if (inv2 != 0.0f) {
+      for (int e = threadIdx.x; e < h * my; e += NT) {
+        const int y = fast_div(e, a.mdh);
+        const int2 q = *reinterpret_cast<const int2*>(&buf[e + y * (PS - h)]);
+        float* at = part + (size_t)y * mz * 2 * P + 2 * (e - y * h);
+        at[0] = inv * (float)q.x;
+        at[1] = inv * (float)q.y;
+      }
+      __syncthreads();
+      plane_spread<NT>(acc, 2 * my * PS, 2 * PS, a.g, *src_sp, z, c, pl, 1, &rest);
+    }
+    const float f = inv2 != 0.0f ? inv2 : inv;
+    for (int e = threadIdx.x; e < h * my; e += NT) {
+      const int y = fast_div(e, a.mdh);
+      float2* at_e = &buf[e + y * (PS - h)];
+      const int2 q = *reinterpret_cast<const int2*>(at_e);
+      float2 r = make_float2(f * (float)q.x, f * (float)q.y);
+      if (inv2 != 0.0f) {
+        const float* at = part + (size_t)y * mz * 2 * P + 2 * (e - y * h);
+        r = cadd(r, make_float2(at[0], at[1]));
+      }
+      *at_e = in ? cadd(r, src[e]) : r;
+    }
   }
   for (int i = threadIdx.x; i < mx; i += NT) twx[i] = a.twx[i];
   for (int i = threadIdx.x; i < my; i += NT) twy[i] = a.twy[i];
-#pragma unroll
-  for (int k = 0; k < kPerLane; ++k) {
-    const int e = threadIdx.x + k * NT;
-    if (e < h * my) {
-      const int y = fast_div(e, a.mdh);
-      buf[e + y * (PS - h)] = v[k];
-    }
-  }
   __syncthreads();
   // x: h-point complex FFT of the even/odd-packed rows
-  lds_fft<NT>(buf, Lines{my, a.mdy, PS, 1}, a.lx, twx, 2, -1.0f);
+  lds_fft<NT, false>(buf, Lines{my, a.mdy, PS, 1}, a.lx, twx, 2);
   // even/odd split: X[k] = E + w^k O, X[h-k] = conj(E - w^k O)
   const int npair = h / 2 + 1;
   for (int e = threadIdx.x; e < my * npair; e += NT) {
@@ -181,7 +220,7 @@ FHD_BODY void body_fft_xy_fwd(const FftArgs& a, const float* __restrict__ in, fl
   }
   __syncthreads();
   // y: columns kx = 0..P-1
-  lds_fft<NT>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1, -1.0f);
+  lds_fft<NT, false>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1);
   float2* dst = spec + ((size_t)c * my * mz + z) * P;
 #pragma unroll
   for (int k = 0; k < kPerLane; ++k) {
@@ -193,7 +232,9 @@ FHD_BODY void body_fft_xy_fwd(const FftArgs& a, const float* __restrict__ in, fl
   }
 }
 FHD_KERNEL_PAIR_OCC((template <int NT, int ELEMS>), NT, 8, k_fft_xy_fwd, FftPass,
-                    body_fft_xy_fwd<NT, ELEMS>(a.f, a.in, a.spec, b))
+                    body_fft_xy_fwd<NT, ELEMS, false>(a.f, a.in, a.spec, b, nullptr))
+FHD_KERNEL_PAIR_OCC((template <int NT, int ELEMS>), NT, 8, k_fft_spread_xy_fwd, FftSpread,
+                    body_fft_xy_fwd<NT, ELEMS, true>(a.p.f, a.p.in, a.p.spec, b, &a.s))
 
 // ---------------------------------------------------------------------------------------
 // Pass B: FFT along z, Fourier-space operator, inverse FFT along z, for all three components.
@@ -235,7 +276,7 @@ FHD_BODY void body_fft_z_solve(const FftArgs& a, float2* __restrict__ spec, int 
   }
   __syncthreads();
   const Lines zl{a.ncomp * T, fast_div_magic(a.ncomp * T), LS, 1};
-  if (a.zmode != 2) lds_fft<NT>(buf, zl, a.lz, twz, 1, -1.0f);
+  if (a.zmode != 2) lds_fft<NT, false>(buf, zl, a.lz, twz, 1);
   if (a.zmode == 0) {
     // Fourier-space operator in the staggered (shifted) basis; 1/N normalisation folded in.
     const float gy = a.gy[ky];
@@ -249,40 +290,14 @@ FHD_BODY void body_fft_z_solve(const FftArgs& a, float2* __restrict__ spec, int 
       const float2 ez = ezs[z];
       const int i0 = t * LS + z, i1 = i0 + T * LS, i2 = i1 + T * LS;
       float2 b0 = buf[i0], b1 = buf[i1], b2 = buf[i2];
-      if (a.knoise) {
-        // the kept part of the stochastic stress divergence, drawn in Fourier space (Stokes limit)
-        float2 nw[3];
-        kspace_noise(key, kx, ky, z, a.g.mx, my, mz, a.knoise, a.kn_f4, a.kn_sqrt_half_n, gx, gy, gz, ex, ey, ez, nw);
-        b0 = cadd(b0, nw[0]);
-        b1 = cadd(b1, nw[1]);
-        b2 = cadd(b2, nw[2]);
-      }
-      const float2 w0 = cmul(b0, cconj(ex));
-      const float2 w1 = cmul(b1, cconj(ey));
-      const float2 w2 = cmul(b2, cconj(ez));
-      const float L = -(gx * gx + gy * gy + gz * gz);
-      float2 o0, o1, o2;
-      if (kx == 0 && ky == 0 && z == 0) {
-        const float keep = a.stokes ? 0.0f : a.inv_n;
-        o0 = cscale(w0, keep);
-        o1 = cscale(w1, keep);
-        o2 = cscale(w2, keep);
-      } else {
-        const float2 GW = make_float2(gx * w0.x + gy * w1.x + gz * w2.x, gx * w0.y + gy * w1.y + gz * w2.y);
-        const float den = a.stokes ? (-a.eta * L) : (1.0f - a.cn_coef * L);
-        const float sc = a.inv_n / den;
-        const float iL = 1.0f / L;
-        o0 = cscale(make_float2(w0.x + gx * GW.x * iL, w0.y + gx * GW.y * iL), sc);
-        o1 = cscale(make_float2(w1.x + gy * GW.x * iL, w1.y + gy * GW.y * iL), sc);
-        o2 = cscale(make_float2(w2.x + gz * GW.x * iL, w2.y + gz * GW.y * iL), sc);
-      }
-      buf[i0] = cmul(o0, ex);
-      buf[i1] = cmul(o1, ey);
-      buf[i2] = cmul(o2, ez);
+      solve_mode(a, key, kx, ky, z, gx, gy, gz, ex, ey, ez, b0, b1, b2);
+      buf[i0] = b0;
+      buf[i1] = b1;
+      buf[i2] = b2;
     }
     __syncthreads();
   }
-  if (a.zmode != 1) lds_fft<NT>(buf, zl, a.lz, twz, 1, 1.0f);
+  if (a.zmode != 1) lds_fft<NT, true>(buf, zl, a.lz, twz, 1);
   // the lane index, opaque to the compiler: the store indices are recomputed here rather than
   // kept live in registers from the loads through both transforms
   int tid = threadIdx.x;
@@ -327,7 +342,7 @@ FHD_BODY void body_fft_xy_inv(const FftArgs& a, const float2* __restrict__ spec,
     }
   }
   __syncthreads();
-  lds_fft<NT>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1, 1.0f);
+  lds_fft<NT, true>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1);
   // C2R packing: Z[k] = (X[k] + conj X[h-k]) + i (X[k] - conj X[h-k]) e^{+2 pi i k / mx}
   const int npair = h / 2 + 1;
   for (int e = threadIdx.x; e < my * npair; e += NT) {
@@ -345,7 +360,7 @@ FHD_BODY void body_fft_xy_inv(const FftArgs& a, const float2* __restrict__ spec,
     row[k] = Zk;
   }
   __syncthreads();
-  lds_fft<NT>(buf, Lines{my, a.mdy, PS, 1}, a.lx, twx, 2, 1.0f);
+  lds_fft<NT, true>(buf, Lines{my, a.mdy, PS, 1}, a.lx, twx, 2);
   const size_t off = ((size_t)c * mz + z) * (size_t)my * mx;
   float2* dst = reinterpret_cast<float2*>(out + off);
   const float2* ax = reinterpret_cast<const float2*>(aux + off);
@@ -365,8 +380,8 @@ FHD_BODY void body_fft_xy_inv(const FftArgs& a, const float2* __restrict__ spec,
       const float2 p = buf[e + y * (PS - h)];
       float2 r = make_float2(alpha * p.x, alpha * p.y);
       if (aux) {
-        r.x += beta * q[k].x;
-        r.y += beta * q[k].y;
+        r.x = fmaf(beta, q[k].x, r.x);
+        r.y = fmaf(beta, q[k].y, r.y);
       }
       dst[e] = r;
     }
@@ -385,24 +400,38 @@ static int lds_class(int elems) { return elems <= kClassElems[0] ? 0 : elems <= 
     else launch(kern<1024, kClassElems[2]>, kern##_b<1024, kClassElems[2]>, fam, grid, 1024, x, s);      \
   } while (0)
 
+// A merged batch takes the runtime-size passes also where size-specialised ones exist (planes with
+// edges up to 64): its replicas' shapes then share one dispatch per workgroup class instead of one
+// per shape (32 boxes with edges 16-64: 22 dispatches of a few planes each per pass and round, four
+// at a time).
+static bool merged_plane(const FftArgs& a) { return t_recorder && fast_edge(a.g.mx) && fast_edge(a.g.my); }
+
 void launch_fft_xy_fwd(const FftArgs& a, const float* in, float2* spec, hipStream_t s) {
-  if (!a.generic && fast_fft_xy_fwd(a, in, spec, s)) return;
+  if (!a.generic && !merged_plane(a) && fast_fft_xy_fwd(a, in, spec, s)) return;
   const FftPass x{a, in, spec, nullptr, nullptr, 0.0f, 0.0f, 0};
   FHD_LAUNCH_CLASS(lds_class(a.g.my * (a.g.P | 1)), k_fft_xy_fwd, FAM_FFT_XY_FWD, dim3(a.g.mz, a.ncomp), x, s);
 }
+void launch_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc& src, float2* spec, hipStream_t s) {
+  if (!a.generic && !merged_plane(a) && fast_fft_spread_xy_fwd(a, in, src, spec, s)) return;
+  const FftSpread x{{a, in, spec, nullptr, nullptr, 0.0f, 0.0f, 0}, src};
+  FHD_LAUNCH_CLASS(lds_class(a.g.my * (a.g.P | 1)), k_fft_spread_xy_fwd, FAM_FFT_XY_FWD, dim3(a.g.mz, a.ncomp), x, s);
+}
 // Columns per z-pass workgroup: the schedule's tile, as far as the largest class holds it.
 void launch_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s) {
-  if (!a.generic && fast_fft_z_solve(a, spec, s)) return;
+  const bool merged = t_recorder && fast_edge(a.g.mz);
+  if (!a.generic && !merged && fast_fft_z_solve(a, spec, s)) return;
   const int LS = a.g.mz | 1;
   const int most = kClassElems[2] / (3 * LS);  // >= 10: mz is at most 256
   const int want = a.btile < most ? a.btile : most;
   const int ntile = (a.g.P + want - 1) / want, T = (a.g.P + ntile - 1) / ntile;
-  const FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, T};
+  FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, T};
+  // the radices the schedule chose for the context alone (48-point columns: fft_common.h's kPlan48)
+  if (merged && a.g.mz == 48 && a.plan_zs) x.f.lz = a.plan_zs == 1 ? line_plan(48, 3, 16, 1) : line_plan(48, 4, 4, 3);
   FHD_LAUNCH_CLASS(lds_class(3 * T * LS), k_fft_z_solve, FAM_FFT_Z, dim3(ntile, a.g.my), x, s);
 }
 void launch_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha, float beta,
                        hipStream_t s) {
-  if (!a.generic && fast_fft_xy_inv(a, spec, out, aux, alpha, beta, s)) return;
+  if (!a.generic && !merged_plane(a) && fast_fft_xy_inv(a, spec, out, aux, alpha, beta, s)) return;
   const FftPass x{a, nullptr, const_cast<float2*>(spec), out, aux, alpha, beta, 0};
   FHD_LAUNCH_CLASS(lds_class(a.g.my * (a.g.P | 1)), k_fft_xy_inv, FAM_FFT_XY_INV, dim3(a.g.mz, a.ncomp), x, s);
 }

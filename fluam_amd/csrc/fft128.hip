@@ -16,6 +16,10 @@
 // and imaginary parts of one complex transform, separated afterwards).  512 lanes per plane:
 // every lane has work in both transforms.  Same layouts, tables and results (to FP32
 // rounding) as the Stockham passes; the schedule autotuner times the two and keeps the faster.
+// The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
+// on the one alone and on the other in a merged batch), so the compiler must not choose which
+// products become fused multiply-adds: the fused ones are written out.
+#pragma clang fp contract(off)
 #include "fhd_device.h"
 #include "fhd_kernels.h"
 #include "fft_common.h"

@@ -2,16 +2,35 @@
 // the size-specialised Stockham FFT kernels.
 #pragma once
 #include "fhd_device.h"
+#include "fhd_kernels.h"
 
 namespace fhd {
 
 FHD_DEV float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
 FHD_DEV float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
-FHD_DEV float2 cmul(float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+FHD_DEV float2 cmul(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
+}
 FHD_DEV float2 cconj(float2 a) { return make_float2(a.x, -a.y); }
 FHD_DEV float2 cscale(float2 a, float s) { return make_float2(a.x * s, a.y * s); }
 // a * (s i), s = +-1
 FHD_DEV float2 cmul_si(float2 a, float s) { return make_float2(-s * a.y, s * a.x); }
+
+// t sqrt(1/2) and t sqrt(3)/2 with the constants' low parts: the rounded constants alone (2e-8 small)
+// shrink every forward and inverse transform a little, which adds up over the steps of a run.
+FHD_DEV float mul_r2(float t) { return fmaf(1.2101617e-8f, t, 0.70710678118654752440f * t); }
+FHD_DEV float mul_r3(float t) { return fmaf(1.5543628e-8f, t, 0.86602540378443864676f * t); }
+// a e^{s i pi/4} and a e^{s 3 i pi/4}
+FHD_DEV float2 turn1(float2 a, float s) { return make_float2(mul_r2(fmaf(-s, a.y, a.x)), mul_r2(fmaf(s, a.x, a.y))); }
+FHD_DEV float2 turn3(float2 a, float s) { return make_float2(mul_r2(fmaf(-s, a.y, -a.x)), mul_r2(fmaf(s, a.x, -a.y))); }
+
+// a (p c + i s d) with (c, d) = (cos, sin) of pi/8, or exchanged (swap), and their low parts.
+FHD_DEV float2 turn16(float2 a, float p, float s, bool swap) {
+  const float c = 0.92387953251128675613f, d = 0.38268343236508977173f, cl = 2.8307490e-8f, dl = 6.2233509e-9f;
+  const float u = p * (swap ? d : c), ul = p * (swap ? dl : cl), v = s * (swap ? c : d), vl = s * (swap ? cl : dl);
+  return make_float2(fmaf(a.x, u, -(a.y * v)) + fmaf(a.x, ul, -(a.y * vl)),
+                     fmaf(a.x, v, a.y * u) + fmaf(a.x, vl, a.y * ul));
+}
 
 // In-register DFTs with kernel e^{s 2 pi i / R}.
 template <int R> struct Dft;
@@ -24,11 +43,10 @@ template <> struct Dft<2> {
 };
 template <> struct Dft<3> {
   static FHD_DEV void run(float2* v, float s) {
-    const float c3 = 0.86602540378443864676f;
     float2 t = cadd(v[1], v[2]);
     float2 u = csub(v[1], v[2]);
-    float2 m = make_float2(v[0].x - 0.5f * t.x, v[0].y - 0.5f * t.y);
-    float2 r = cmul_si(cscale(u, c3), s);
+    float2 m = make_float2(fmaf(-0.5f, t.x, v[0].x), fmaf(-0.5f, t.y, v[0].y));
+    float2 r = cmul_si(make_float2(mul_r3(u.x), mul_r3(u.y)), s);
     v[0] = cadd(v[0], t);
     v[1] = cadd(m, r);
     v[2] = csub(m, r);
@@ -94,11 +112,10 @@ template <> struct Dft<8> {
     float2 o[4] = {v[1], v[3], v[5], v[7]};
     Dft<4>::run(e, s);
     Dft<4>::run(o, s);
-    const float h = 0.70710678118654752440f;
     // w^k = e^{s 2 pi i k / 8}
-    float2 o1 = cmul(o[1], make_float2(h, s * h));
+    float2 o1 = turn1(o[1], s);
     float2 o2 = cmul_si(o[2], s);
-    float2 o3 = cmul(o[3], make_float2(-h, s * h));
+    float2 o3 = turn3(o[3], s);
     v[0] = cadd(e[0], o[0]);
     v[4] = csub(e[0], o[0]);
     v[1] = cadd(e[1], o1);
@@ -120,20 +137,61 @@ template <> struct Dft<16> {
     }
     Dft<8>::run(e, s);
     Dft<8>::run(o, s);
-    // w^k = e^{s 2 pi i k / 16}: cos and sin of k pi / 8
-    const float c1 = 0.92387953251128675613f, s1 = 0.38268343236508977173f;
-    const float h = 0.70710678118654752440f;
-    const float2 w[8] = {make_float2(1.0f, 0.0f), make_float2(c1, s * s1), make_float2(h, s * h),
-                         make_float2(s1, s * c1), make_float2(0.0f, s), make_float2(-s1, s * c1),
-                         make_float2(-h, s * h), make_float2(-c1, s * s1)};
+    // w^k = e^{s 2 pi i k / 16}
+    const float2 t[8] = {o[0],
+                         turn16(o[1], 1.0f, s, false),
+                         turn1(o[2], s),
+                         turn16(o[3], 1.0f, s, true),
+                         cmul_si(o[4], s),
+                         turn16(o[5], -1.0f, s, true),
+                         turn3(o[6], s),
+                         turn16(o[7], -1.0f, s, false)};
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const float2 t = k == 0 ? o[0] : cmul(o[k], w[k]);
-      v[k] = cadd(e[k], t);
-      v[k + 8] = csub(e[k], t);
+      v[k] = cadd(e[k], t[k]);
+      v[k + 8] = csub(e[k], t[k]);
     }
   }
 };
+
+// The Fourier-space operator at one mode of the z pass (the transforms b0, b1, b2 of the three
+// components, replaced by the solution's): the kept part of the stochastic stress divergence is
+// added (Stokes limit), then shift to the staggered basis, project, apply the viscous or Stokes
+// operator with the 1/N normalisation folded in, shift back.
+FHD_DEV void solve_mode(const FftArgs& a, const Key& key, int kx, int ky, int z, float gx, float gy, float gz, float2 ex,
+                        float2 ey, float2 ez, float2& b0, float2& b1, float2& b2) {
+  if (a.knoise) {
+    float2 nw[3];
+    kspace_noise(key, kx, ky, z, a.g.mx, a.g.my, a.g.mz, a.knoise, a.kn_f4, a.kn_sqrt_half_n, gx, gy, gz, ex, ey, ez, nw);
+    b0 = cadd(b0, nw[0]);
+    b1 = cadd(b1, nw[1]);
+    b2 = cadd(b2, nw[2]);
+  }
+  const float2 w0 = cmul(b0, cconj(ex));
+  const float2 w1 = cmul(b1, cconj(ey));
+  const float2 w2 = cmul(b2, cconj(ez));
+  const float L = -fmaf(gz, gz, fmaf(gy, gy, gx * gx));
+  if (kx == 0 && ky == 0 && z == 0) {
+    const float keep = a.stokes ? 0.0f : a.inv_n;
+    b0 = cscale(b0, keep);
+    b1 = cscale(b1, keep);
+    b2 = cscale(b2, keep);
+  } else {
+    const float iL = 1.0f / L;
+    const float2 GW = make_float2(fmaf(gz, w2.x, fmaf(gy, w1.x, gx * w0.x)) * iL, fmaf(gz, w2.y, fmaf(gy, w1.y, gx * w0.y)) * iL);
+    const float den = a.stokes ? (-a.eta * L) : fmaf(-a.cn_coef, L, 1.0f);
+    const float sc = a.inv_n / den;
+    // sc (b_a + e_a g_a GW): the unprojected part keeps its phase, so the shift there and back (|e|^2,
+    // not quite 1) does not touch it
+    const auto part = [&](float2 b, float2 e, float g) {
+      const float2 q = cmul(e, make_float2(g * GW.x, g * GW.y));
+      return cscale(cadd(b, q), sc);
+    };
+    b0 = part(b0, ex, gx);
+    b1 = part(b1, ey, gy);
+    b2 = part(b2, ez, gz);
+  }
+}
 
 // Radix plan of the size-specialised kernels: 16s first, then 8, 4, 2, 3 (fewest LDS stages).
 constexpr int plan_radix(int n, int st) {

@@ -5,135 +5,21 @@
 // lengths in {16, 24, 32, 48, 64} or mx = my in {96, 128}, and z pencils of any of those
 // lengths; other shapes use the generic kernels, which share the spectrum layout
 // spec[c][ky][z][kx].
+// The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
+// on the one alone and on the other in a merged batch), so the compiler must not choose which
+// products become fused multiply-adds: the fused ones are written out.
+#pragma clang fp contract(off)
 #include "fhd_device.h"
 #include "fhd_kernels.h"
 #include "fft_common.h"
+#include "fft_stages.h"
 
 
 namespace fhd {
 
-// One radix-R Stockham stage, lines l = 0..lines-1 (lines <= MAXL) at base l * LS, element
-// stride ES.  Consecutive lanes take butterfly j of consecutive lines: the lines are either
-// adjacent elements (ES > 1, LS = 1) or an odd number of elements apart (ES = 1), so the lanes
-// of a wave read and write different LDS banks in every stage, and share one twiddle.  (Taking
-// consecutive butterflies of one line instead makes the writes of the early stages R-way bank
-// conflicts.)
-template <int N, int R, int NS, int ES, int NT, int MAXL, int TWM>
-FHD_DEV void fstage(float2* buf, int lines, int LS, const float2* tw, float s) {
-  constexpr int NBL = N / R;
-  constexpr int KMAX = (MAXL * NBL + NT - 1) / NT;
-  constexpr int STRIDE = N / (NS * R);
-  float2 v[KMAX][R];
-  int wb[KMAX];
-#pragma unroll
-  for (int k = 0; k < KMAX; ++k) {
-    const int b = threadIdx.x + k * NT;
-    const int j = b / MAXL;
-    const int l = b - j * MAXL;
-    wb[k] = -1;
-    if (j < NBL && l < lines) {
-      const int base = l * LS;
-      const int kk = j % NS;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float2 x = buf[base + (j + r * NBL) * ES];
-        if (NS > 1 && r > 0) {
-          float2 w = tw[(kk * r * STRIDE) * TWM];
-          w.y = s > 0.0f ? -w.y : w.y;
-          x = cmul(x, w);
-        }
-        v[k][r] = x;
-      }
-      Dft<R>::run(v[k], s);
-      wb[k] = base + ((j / NS) * NS * R + kk) * ES;
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < KMAX; ++k)
-    if (wb[k] >= 0) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) buf[wb[k] + r * NS * ES] = v[k][r];
-    }
-  __syncthreads();
-}
-
-template <int N, int ST, int NS, int ES, int NT, int MAXL, int TWM, uint32_t PLAN>
-struct FStages {
-  static FHD_DEV void run(float2* buf, int lines, int LS, const float2* tw, float s) {
-    constexpr int R = NS >= N ? 1 : plan_at(PLAN, N, ST);
-    if constexpr (R > 1) {
-      fstage<N, R, NS, ES, NT, MAXL, TWM>(buf, lines, LS, tw, s);
-      FStages<N, ST + 1, NS * R, ES, NT, MAXL, TWM, PLAN>::run(buf, lines, LS, tw, s);
-    }
-  }
-};
-
-template <int N, int ES, int NT, int MAXL, int TWM, uint32_t PLAN = 0u>
-FHD_DEV void ffft(float2* buf, int lines, int LS, const float2* tw, float s) {
-  FStages<N, 0, 1, ES, NT, MAXL, TWM, PLAN>::run(buf, lines, LS, tw, s);
-}
-
-// ---------------- pass A: real plane -> half spectrum (x) -> FFT along y ----------------
-template <int MX, int MY, int NT, int PX = 0, int PY = 0>
-FHD_BODY void body_fftA(const FftArgs& a, const float* __restrict__ in, float2* __restrict__ spec, const Blk& b) {
-  constexpr int H = MX / 2, P = H + 1;
-  __shared__ float2 buf[MY * P];
-  __shared__ float2 twx[MX];
-  __shared__ float2 twy[MY];
-  const int z = b.x, c = b.y, mz = a.g.mz;
-  for (int i = threadIdx.x; i < MX; i += NT) twx[i] = a.twx[i];
-  for (int i = threadIdx.x; i < MY; i += NT) twy[i] = a.twy[i];
-  const float4* src = reinterpret_cast<const float4*>(in + ((size_t)c * mz + z) * (size_t)(MX * MY));
-  constexpr int Q = MX / 4;
-  // every load of this lane in flight at once, then into LDS (a load-store loop would wait out
-  // one HBM round trip per element)
-  constexpr int NL = (MY * Q + NT - 1) / NT;
-  float4 v[NL];
-#pragma unroll
-  for (int k = 0; k < NL; ++k) {
-    const int e = threadIdx.x + k * NT;
-    if (e < MY * Q) v[k] = src[e];
-  }
-#pragma unroll
-  for (int k = 0; k < NL; ++k) {
-    const int e = threadIdx.x + k * NT;
-    if (e < MY * Q) {
-      const int y = e / Q, x4 = e - y * Q;
-      buf[y * P + 2 * x4] = make_float2(v[k].x, v[k].y);
-      buf[y * P + 2 * x4 + 1] = make_float2(v[k].z, v[k].w);
-    }
-  }
-  __syncthreads();
-  ffft<H, 1, NT, MY, 2, plan_choice(H, PX)>(buf, MY, P, twx, -1.0f);
-  constexpr int NP = H / 2 + 1;
-  for (int e = threadIdx.x; e < MY * NP; e += NT) {
-    const int y = e / NP, k = e - y * NP;
-    float2* row = buf + y * P;
-    const float2 A = row[k];
-    const float2 B = cconj(row[k == 0 ? 0 : H - k]);
-    const float2 E = cscale(cadd(A, B), 0.5f);
-    const float2 D = csub(A, B);
-    const float2 O = make_float2(0.5f * D.y, -0.5f * D.x);
-    const float2 wO = cmul(twx[k], O);
-    if (k == 0) {
-      row[0] = make_float2(E.x + O.x, 0.0f);
-      row[H] = make_float2(E.x - O.x, 0.0f);
-    } else {
-      row[k] = cadd(E, wO);
-      if (H - k != k) row[H - k] = cconj(csub(E, wO));
-    }
-  }
-  __syncthreads();
-  ffft<MY, P, NT, P, 1, plan_choice(MY, PY)>(buf, P, 1, twy, -1.0f);
-  float2* dst = spec + (size_t)c * MY * mz * P + (size_t)z * P;
-  for (int e = threadIdx.x; e < MY * P; e += NT) {
-    const int ky = e / P, kx = e - ky * P;
-    dst[(size_t)ky * mz * P + kx] = buf[e];
-  }
-}
+// ---------------- pass A ----------------
 FHD_KERNEL_PAIR((template <int MX, int MY, int NT, int PX, int PY>), NT, k_fftA, FftPass,
-                body_fftA<MX, MY, NT, PX, PY>(a.f, a.in, a.spec, b))
+                body_fftA<MX, MY, NT, PX, PY, false>(a.f, a.in, a.spec, b, nullptr))
 
 // ---------------- pass C: FFT along y (inverse) -> C2R along x -> out = alpha r + beta aux ----
 template <int MX, int MY, int NT, int PX = 0, int PY = 0>
@@ -165,7 +51,7 @@ FHD_BODY void body_fftC(const FftArgs& a, const float2* __restrict__ spec, float
     }
   }
   __syncthreads();
-  ffft<MY, P, NT, P, 1, plan_choice(MY, PY)>(buf, P, 1, twy, 1.0f);
+  ffft<MY, P, NT, P, 1, true, plan_choice(MY, PY)>(buf, P, 1, twy);
   constexpr int NP = H / 2 + 1;
   for (int e = threadIdx.x; e < MY * NP; e += NT) {
     const int y = e / NP, k = e - y * NP;
@@ -182,7 +68,7 @@ FHD_BODY void body_fftC(const FftArgs& a, const float2* __restrict__ spec, float
     row[k] = Zk;
   }
   __syncthreads();
-  ffft<H, 1, NT, MY, 2, plan_choice(H, PX)>(buf, MY, P, twx, 1.0f);
+  ffft<H, 1, NT, MY, 2, true, plan_choice(H, PX)>(buf, MY, P, twx);
   const size_t off = ((size_t)c * mz + z) * (size_t)(MX * MY);
   float4* dst = reinterpret_cast<float4*>(out + off);
   const float4* ax = aux ? reinterpret_cast<const float4*>(aux + off) : nullptr;
@@ -204,10 +90,10 @@ FHD_BODY void body_fftC(const FftArgs& a, const float2* __restrict__ spec, float
       const float2 p0 = buf[y * P + 2 * x4], p1 = buf[y * P + 2 * x4 + 1];
       float4 r = make_float4(alpha * p0.x, alpha * p0.y, alpha * p1.x, alpha * p1.y);
       if (ax) {
-        r.x += beta * q[k].x;
-        r.y += beta * q[k].y;
-        r.z += beta * q[k].z;
-        r.w += beta * q[k].w;
+        r.x = fmaf(beta, q[k].x, r.x);
+        r.y = fmaf(beta, q[k].y, r.y);
+        r.z = fmaf(beta, q[k].z, r.z);
+        r.w = fmaf(beta, q[k].w, r.w);
       }
       dst[e] = r;
     }
@@ -264,7 +150,7 @@ FHD_BODY void body_fftB(const FftArgs& a, float2* __restrict__ spec, int T, cons
   }
   __syncthreads();
   const int lines = a.ncomp * TM;
-  if (a.zmode != 2) ffft<MZ, 1, NT, 3 * TM, 1, plan_choice(MZ, PZ)>(buf, lines, LS, twz, -1.0f);
+  if (a.zmode != 2) ffft<MZ, 1, NT, 3 * TM, 1, false, plan_choice(MZ, PZ)>(buf, lines, LS, twz);
   if (a.zmode == 0) {
     const float gy = a.gy[ky];
     const float2 ey = a.ey[ky];
@@ -278,40 +164,14 @@ FHD_BODY void body_fftB(const FftArgs& a, float2* __restrict__ spec, int T, cons
       const float2 ez = ezs[z];
       const int i0 = (0 * TM + t) * LS + z, i1 = (1 * TM + t) * LS + z, i2 = (2 * TM + t) * LS + z;
       float2 b0 = buf[i0], b1 = buf[i1], b2 = buf[i2];
-      if (a.knoise) {
-        float2 nw[3];
-        kspace_noise(key, kx, ky, z, a.g.mx, my, MZ, a.knoise, a.kn_f4, a.kn_sqrt_half_n, gx, gy,
-                          gz, ex, ey, ez, nw);
-        b0 = cadd(b0, nw[0]);
-        b1 = cadd(b1, nw[1]);
-        b2 = cadd(b2, nw[2]);
-      }
-      const float2 w0 = cmul(b0, cconj(ex));
-      const float2 w1 = cmul(b1, cconj(ey));
-      const float2 w2 = cmul(b2, cconj(ez));
-      const float L = -(gx * gx + gy * gy + gz * gz);
-      float2 o0, o1, o2;
-      if (kx == 0 && ky == 0 && z == 0) {
-        const float keep = a.stokes ? 0.0f : a.inv_n;
-        o0 = cscale(w0, keep);
-        o1 = cscale(w1, keep);
-        o2 = cscale(w2, keep);
-      } else {
-        const float2 GW = make_float2(gx * w0.x + gy * w1.x + gz * w2.x, gx * w0.y + gy * w1.y + gz * w2.y);
-        const float den = a.stokes ? (-a.eta * L) : (1.0f - a.cn_coef * L);
-        const float sc = a.inv_n / den;
-        const float iL = 1.0f / L;
-        o0 = cscale(make_float2(w0.x + gx * GW.x * iL, w0.y + gx * GW.y * iL), sc);
-        o1 = cscale(make_float2(w1.x + gy * GW.x * iL, w1.y + gy * GW.y * iL), sc);
-        o2 = cscale(make_float2(w2.x + gz * GW.x * iL, w2.y + gz * GW.y * iL), sc);
-      }
-      buf[i0] = cmul(o0, ex);
-      buf[i1] = cmul(o1, ey);
-      buf[i2] = cmul(o2, ez);
+      solve_mode(a, key, kx, ky, z, gx, gy, gz, ex, ey, ez, b0, b1, b2);
+      buf[i0] = b0;
+      buf[i1] = b1;
+      buf[i2] = b2;
     }
     __syncthreads();
   }
-  if (a.zmode != 1) ffft<MZ, 1, NT, 3 * TM, 1, plan_choice(MZ, PZ)>(buf, lines, LS, twz, 1.0f);
+  if (a.zmode != 1) ffft<MZ, 1, NT, 3 * TM, 1, true, plan_choice(MZ, PZ)>(buf, lines, LS, twz);
   // the lane index, opaque to the compiler: the store indices are recomputed here rather than
   // kept live in registers from the loads through both transforms
   int tid = threadIdx.x;

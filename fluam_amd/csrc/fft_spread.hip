@@ -1,0 +1,51 @@
+// fft_spread.hip -- the forward xy pass with spreading for the plane shapes of fft_fast.hip: mx x my
+// with both lengths in {16, 24, 32, 48, 64} or mx = my in {96, 128}, default radix plans.
+// The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
+// on the one alone and on the other in a merged batch), so the compiler must not choose which
+// products become fused multiply-adds: the fused ones are written out.
+#pragma clang fp contract(off)
+#include "fft_stages.h"
+
+namespace fhd {
+
+FHD_KERNEL_PAIR_OCC((template <int MX, int MY, int NT>), NT, 8, k_spread_fftA, FftSpread,
+                    body_fftA<MX, MY, NT, 0, 0, true>(a.p.f, a.p.in, a.p.spec, b, &a.s))
+
+
+// Lanes per plane workgroup as in the plain pass of a context launched alone; batched dispatches
+// take the same, so a replica's kernel does not depend on the batch.
+template <int MX, int MY>
+static bool launch_plane(const FftSpread& x, hipStream_t s) {
+  constexpr int NT = MX * MY >= 64 * 64 ? 1024 : 256;
+  launch(k_spread_fftA<MX, MY, NT>, k_spread_fftA_b<MX, MY, NT>, FAM_FFT_XY_FWD, dim3(x.p.f.g.mz, x.p.f.ncomp), NT, x, s);
+  return true;
+}
+template <int MX>
+static bool launch_rect(const FftSpread& x, hipStream_t s) {
+  switch (x.p.f.g.my) {
+    case 16: return launch_plane<MX, 16>(x, s);
+    case 24: return launch_plane<MX, 24>(x, s);
+    case 32: return launch_plane<MX, 32>(x, s);
+    case 48: return launch_plane<MX, 48>(x, s);
+    case 64: return launch_plane<MX, 64>(x, s);
+    default: return false;
+  }
+}
+
+bool fast_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc& src, float2* spec, hipStream_t s) {
+  const FftSpread x{{a, in, spec, nullptr, nullptr, 0.0f, 0.0f, 0}, src};
+  if (a.g.mx == a.g.my) {
+    if (a.g.mx == 96) return launch_plane<96, 96>(x, s);
+    if (a.g.mx == 128) return launch_plane<128, 128>(x, s);
+  }
+  switch (a.g.mx) {
+    case 16: return launch_rect<16>(x, s);
+    case 24: return launch_rect<24>(x, s);
+    case 32: return launch_rect<32>(x, s);
+    case 48: return launch_rect<48>(x, s);
+    case 64: return launch_rect<64>(x, s);
+    default: return false;
+  }
+}
+
+}  // namespace fhd

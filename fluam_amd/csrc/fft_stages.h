@@ -1,0 +1,179 @@
+// fft_stages.h -- the Stockham stages and the forward xy pass of the size-specialised FFT kernels,
+// shared by the plain passes (fft_fast.hip) and the passes with spreading (fft_spread.hip).
+#pragma once
+#include "fhd_device.h"
+#include "fhd_kernels.h"
+#include "fft_common.h"
+#include "plane_spread.h"
+
+namespace fhd {
+
+// One radix-R Stockham stage, lines l = 0..lines-1 (lines <= MAXL) at base l * LS, element
+// stride ES.  Consecutive lanes take butterfly j of consecutive lines: the lines are either
+// adjacent elements (ES > 1, LS = 1) or an odd number of elements apart (ES = 1), so the lanes
+// of a wave read and write different LDS banks in every stage, and share one twiddle.  (Taking
+// consecutive butterflies of one line instead makes the writes of the early stages R-way bank
+// conflicts.)
+// INV: the stage of the inverse transform, which undoes the forward stages in reverse order (reads
+// where the forward stage writes, twiddles after the butterfly, writes where it reads).  The
+// inverse is then the exact adjoint of the forward transform with the table's rounded twiddles, so
+// their phase errors cancel over the round trip of a solve instead of adding up over the steps.
+template <int N, int R, int NS, int ES, int NT, int MAXL, int TWM, bool INV>
+FHD_DEV void fstage(float2* buf, int lines, int LS, const float2* tw) {
+  constexpr int NBL = N / R;
+  constexpr int KMAX = (MAXL * NBL + NT - 1) / NT;
+  constexpr int STRIDE = N / (NS * R);
+  constexpr float s = INV ? 1.0f : -1.0f;
+  float2 v[KMAX][R];
+  int to[KMAX];  // first element of the butterfly's outputs, -1: none
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const int b = threadIdx.x + k * NT;
+    const int j = b / MAXL;
+    const int l = b - j * MAXL;
+    to[k] = -1;
+    if (j < NBL && l < lines) {
+      const int base = l * LS;
+      const int kk = j % NS;
+      // spread: elements NBL apart; packed: elements NS apart in the sub-transform's block
+      const int spread = base + j * ES, packed = base + ((j / NS) * NS * R + kk) * ES;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float2 x = INV ? buf[packed + r * NS * ES] : buf[spread + r * NBL * ES];
+        if (!INV && NS > 1 && r > 0) x = cmul(x, tw[(kk * r * STRIDE) * TWM]);
+        v[k][r] = x;
+      }
+      Dft<R>::run(v[k], s);
+      if (INV && NS > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[k][r] = cmul(v[k][r], cconj(tw[(kk * r * STRIDE) * TWM]));
+      }
+      to[k] = INV ? spread : packed;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k)
+    if (to[k] >= 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) buf[to[k] + r * (INV ? NBL : NS) * ES] = v[k][r];
+    }
+  __syncthreads();
+}
+
+template <int N, int ST, int NS, int ES, int NT, int MAXL, int TWM, uint32_t PLAN, bool INV>
+struct FStages {
+  static FHD_DEV void run(float2* buf, int lines, int LS, const float2* tw) {
+    constexpr int R = NS >= N ? 1 : plan_at(PLAN, N, ST);
+    if constexpr (R > 1) {
+      if constexpr (!INV) fstage<N, R, NS, ES, NT, MAXL, TWM, INV>(buf, lines, LS, tw);
+      FStages<N, ST + 1, NS * R, ES, NT, MAXL, TWM, PLAN, INV>::run(buf, lines, LS, tw);
+      if constexpr (INV) fstage<N, R, NS, ES, NT, MAXL, TWM, INV>(buf, lines, LS, tw);
+    }
+  }
+};
+
+template <int N, int ES, int NT, int MAXL, int TWM, bool INV, uint32_t PLAN>
+FHD_DEV void ffft(float2* buf, int lines, int LS, const float2* tw) {
+  FStages<N, 0, 1, ES, NT, MAXL, TWM, PLAN, INV>::run(buf, lines, LS, tw);
+}
+
+// ---------------- pass A: real plane -> half spectrum (x) -> FFT along y ----------------
+// SP: the plane is the sources' spread field (plane_spread.h) plus `in` (null: none).
+template <int MX, int MY, int NT, int PX, int PY, bool SP>
+FHD_BODY void body_fftA(const FftArgs& a, const float* __restrict__ in, float2* __restrict__ spec, const Blk& b,
+                        const PlaneSrc* src_sp) {
+  constexpr int H = MX / 2, P = H + 1;
+  __shared__ float2 buf[MY * P];
+  // the twiddles; before they are stored, plane_spread's lists
+  constexpr int kTw = (MX + MY) * sizeof(float2);
+  __shared__ __align__(16) unsigned char side[SP && (int)sizeof(PlaneLds) > kTw ? (int)sizeof(PlaneLds) : kTw];
+  float2* const twx = reinterpret_cast<float2*>(side);
+  float2* const twy = twx + MX;
+  const int mz = a.g.mz;
+  // with spreading, the three components and the neighbouring planes, which read the same sources,
+  // are kept on one XCD
+  const int item = SP ? xcd_item(b.x + b.nx * b.y, b.nx * b.ny) : 0;
+  const int z = SP ? item / b.ny : b.x, c = SP ? item - z * b.ny : b.y;
+  const float4* src = reinterpret_cast<const float4*>(in + ((size_t)c * mz + z) * (size_t)(MX * MY));
+  constexpr int Q = MX / 4;
+  // every load of this lane in flight at once, then into LDS (a load-store loop would wait out
+  // one HBM round trip per element)
+  constexpr int NL = (MY * Q + NT - 1) / NT;
+  if constexpr (!SP) {
+    float4 v[NL];
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      const int e = threadIdx.x + k * NT;
+      if (e < MY * Q) v[k] = src[e];
+    }
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      const int e = threadIdx.x + k * NT;
+      if (e < MY * Q) {
+        const int y = e / Q, x4 = e - y * Q;
+        buf[y * P + 2 * x4] = make_float2(v[k].x, v[k].y);
+        buf[y * P + 2 * x4 + 1] = make_float2(v[k].z, v[k].w);
+      }
+    }
+  } else {
+    PlaneLds& pl = *reinterpret_cast<PlaneLds*>(side);
+    // the integers become the plane in place; between two sweeps the first sums wait in this
+    // workgroup's own rows of the spectrum (at least MX floats each), written later
+    float* part = reinterpret_cast<float*>(spec + (size_t)c * MY * mz * P + (size_t)z * P);
+    const auto at = [&](int e) { return (size_t)(e / (MX / 2)) * mz * 2 * P + 2 * (e % (MX / 2)); };
+    int* acc = reinterpret_cast<int*>(buf);
+    const float2* src2 = reinterpret_cast<const float2*>(src);
+    float inv2, rest;
+    const float inv = plane_spread<NT>(acc, 2 * MY * P, 2 * P, a.g, *src_sp, z, c, pl, 0, &inv2);
+    if (inv2 != 0.0f) {
+      for (int e = threadIdx.x; e < MY * H; e += NT) {
+        const int2 q = *reinterpret_cast<const int2*>(&buf[e / H * P + e % H]);
+        part[at(e)] = inv * (float)q.x;
+        part[at(e) + 1] = inv * (float)q.y;
+      }
+      __syncthreads();
+      plane_spread<NT>(acc, 2 * MY * P, 2 * P, a.g, *src_sp, z, c, pl, 1, &rest);
+    }
+    const float f = inv2 != 0.0f ? inv2 : inv;
+#pragma unroll 2
+    for (int e = threadIdx.x; e < MY * H; e += NT) {
+      float2* at_e = &buf[e / H * P + e % H];
+      const int2 q = *reinterpret_cast<const int2*>(at_e);
+      float2 r = make_float2(f * (float)q.x, f * (float)q.y);
+      if (inv2 != 0.0f) r = cadd(r, make_float2(part[at(e)], part[at(e) + 1]));
+      *at_e = in ? cadd(r, src2[e]) : r;
+    }
+  }
+  for (int i = threadIdx.x; i < MX; i += NT) twx[i] = a.twx[i];
+  for (int i = threadIdx.x; i < MY; i += NT) twy[i] = a.twy[i];
+  __syncthreads();
+  ffft<H, 1, NT, MY, 2, false, plan_choice(H, PX)>(buf, MY, P, twx);
+  constexpr int NP = H / 2 + 1;
+  for (int e = threadIdx.x; e < MY * NP; e += NT) {
+    const int y = e / NP, k = e - y * NP;
+    float2* row = buf + y * P;
+    const float2 A = row[k];
+    const float2 B = cconj(row[k == 0 ? 0 : H - k]);
+    const float2 E = cscale(cadd(A, B), 0.5f);
+    const float2 D = csub(A, B);
+    const float2 O = make_float2(0.5f * D.y, -0.5f * D.x);
+    const float2 wO = cmul(twx[k], O);
+    if (k == 0) {
+      row[0] = make_float2(E.x + O.x, 0.0f);
+      row[H] = make_float2(E.x - O.x, 0.0f);
+    } else {
+      row[k] = cadd(E, wO);
+      if (H - k != k) row[H - k] = cconj(csub(E, wO));
+    }
+  }
+  __syncthreads();
+  ffft<MY, P, NT, P, 1, false, plan_choice(MY, PY)>(buf, P, 1, twy);
+  float2* dst = spec + (size_t)c * MY * mz * P + (size_t)z * P;
+  for (int e = threadIdx.x; e < MY * P; e += NT) {
+    const int ky = e / P, kx = e - ky * P;
+    dst[(size_t)ky * mz * P + kx] = buf[e];
+  }
+}
+
+}  // namespace fhd

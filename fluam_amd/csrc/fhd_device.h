@@ -19,6 +19,28 @@ FHD_DEV int xcd_item(int b, int n) {
 __host__ FHD_DEV uint32_t fast_div_magic(int d) { return 0xFFFFFFFFu / (uint32_t)d + 1u; }
 FHD_DEV int fast_div(int n, uint32_t magic) { return magic ? (int)__umulhi((uint32_t)n, magic) : n; }
 
+// (c, s) of the unit circle in FP32, chosen among the neighbours within an ulp or so of the nearest
+// pair for the length closest to 1: rounded to nearest the table's entries are 2e-8 short on
+// average, and each transform multiplies by them on the way there and back.
+inline float2 unit_pair(double c, double s) {
+  const float c0 = (float)c, s0 = (float)s;
+  const double uc = ldexp(1.0, ilogb(fabs(c) > 1e-9 ? c : 1e-9) - 23), us = ldexp(1.0, ilogb(fabs(s) > 1e-9 ? s : 1e-9) - 23);
+  float2 best = make_float2(c0, s0);
+  if (fabs(c) < 1e-9 || fabs(s) < 1e-9) return best;
+  double least = 1.0;
+  for (int i = -4; i <= 4; ++i)
+    for (int j = -4; j <= 4; ++j) {
+      const float x = (float)(c0 + i * uc), y = (float)(s0 + j * us);
+      const double off = sqrt((x - c) * (x - c) + (y - s) * (y - s));
+      const double cost = fabs((double)x * x + (double)y * y - 1.0) + 0.1 * off;
+      if (off <= 6e-8 && cost < least) {
+        least = cost;
+        best = make_float2(x, y);
+      }
+    }
+  return best;
+}
+
 // Device error flags (bits of the context's error word; cf. fluam's errorKernel,
 // src/allocateErrorArray.cu:22-32): a non-finite particle displacement, and a displacement of
 // 2^24 cells or more that was not applied.
@@ -240,6 +262,14 @@ struct PartPos {
   float4* off;   // x, y, z, w unused
 };
 
+// Square root of x in [0.25, 4] to within half an ulp or so: the hardware reciprocal root and one
+// Newton step (sqrtf's correct rounding over the full range costs three times the instructions).
+FHD_DEV float root_near_one(float x) {
+  const float r = __builtin_amdgcn_rsqf(x);
+  const float s = x * r;
+  return fmaf(fmaf(-s, s, x), 0.5f * r, s);
+}
+
 // 1D weights of one axis for one velocity component: nodes base .. base+np-1 (unwrapped).
 struct AxisWeights {
   int base;
@@ -265,7 +295,7 @@ FHD_DEV void axis_weights(int c, float frac, int stag, AxisWeights& aw) {
     else if (frac >= 0.0f) { j0 = c; f = frac - 0.5f; }
     else { j0 = c - 1; f = frac + 0.5f; }
     aw.base = j0 - 1;
-    const float w0 = (1.0f + sqrtf(fmaxf(1.0f - 3.0f * f * f, 0.0f))) * (1.0f / 3.0f);
+    const float w0 = (1.0f + root_near_one(1.0f - 3.0f * f * f)) * (1.0f / 3.0f);
     aw.w[0] = 0.5f * (1.0f - w0 - f);  // node j0 - 1, distance f + 1
     aw.w[1] = w0;
     aw.w[2] = 0.5f * (1.0f - w0 + f);  // node j0 + 1, distance f - 1
@@ -279,7 +309,7 @@ FHD_DEV void axis_weights(int c, float frac, int stag, AxisWeights& aw) {
       j0 = c - 1; f = frac + 0.5f;
     }
     aw.base = j0 - 1;
-    const float s = 0.125f * (3.0f - 2.0f * f + sqrtf(fmaxf(1.0f + 4.0f * f * (1.0f - f), 0.0f)));
+    const float s = 0.125f * (3.0f - 2.0f * f + root_near_one(1.0f + 4.0f * f * (1.0f - f)));
     aw.w[0] = 0.75f - 0.5f * f - s;  // distance f + 1
     aw.w[1] = s;                      // distance f
     aw.w[2] = 0.5f * f - 0.25f + s;  // distance f - 1

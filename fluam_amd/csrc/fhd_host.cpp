@@ -25,6 +25,7 @@
 
 #include "../../include/fhd.h"
 #include "fhd_kernels.h"
+#include "fft_common.h"
 
 using namespace fhd;
 
@@ -50,9 +51,7 @@ bool g_params_loaded = false;
 // the one whose largest radix is smallest (fewer registers).  False when n is not 2^a 3^b.
 bool make_plan(int n, LinePlan* p) {
   const int rs[7] = {2, 3, 4, 6, 8, 9, 16};
-  p->n = n;
-  p->nst = 0;
-  for (int k = 0; k < 3; ++k) p->radix[k] = 1;
+  *p = line_plan(n, 1, 1, 1);
   if (n == 1) return true;
   int best[3] = {0, 0, 0}, most = 99;
   for (int nst = 1; nst <= 3 && !best[0]; ++nst)
@@ -66,24 +65,26 @@ bool make_plan(int n, LinePlan* p) {
           if (q0 * q1 * q2 != n || q0 < q1 || q1 < q2 || q0 >= most) continue;
           most = q0;
           best[0] = q0; best[1] = q1; best[2] = q2;
-          p->nst = nst;
         }
       }
   if (!best[0]) return false;
-  int Ns = 1;
-  for (int k = 0; k < p->nst; ++k) {
-    p->radix[k] = best[k];
-    p->mns[k] = fast_div_magic(Ns);
-    Ns *= best[k];
-  }
+  *p = line_plan(n, best[0], best[1], best[2]);
   return true;
 }
 
-// The runtime-size kernels' plans and reciprocals for an mx x my x mz grid.
+// The runtime-size kernels' plans and reciprocals for an mx x my x mz grid.  Where a
+// size-specialised pass exists too they take its radices, so that a replica of a merged batch
+// (whose passes are the runtime-size ones) gets the bits it would get alone.
 void fill_plans(FftArgs& a, int mx, int my, int mz) {
   make_plan(mx / 2, &a.lx);
   make_plan(my, &a.ly);
   make_plan(mz, &a.lz);
+  const auto as_fast = [](int n) { return line_plan(n, plan_radix(n, 0), plan_radix(n, 1), plan_radix(n, 2)); };
+  if (fast_edge(mx) && fast_edge(my)) {
+    a.lx = as_fast(mx / 2);
+    a.ly = as_fast(my);
+  }
+  if (fast_edge(mz)) a.lz = as_fast(mz);
   a.mdh = fast_div_magic(mx / 2);
   a.mdp = fast_div_magic(mx / 2 + 1);
   a.mdy = fast_div_magic(my);
@@ -138,21 +139,15 @@ float2* noalloc_scratch() {
   return g_noalloc_ptr[dev];
 }
 
-// The transform tables of build_tables, computed on the device from the same FP64 formulas:
-// twiddles e^{-2 pi i k/m} (x, y, z), shifts e^{i pi k/m} (x, y, z), then the real symbols
-// g(k) = 2 sin(pi k/m) (unit cells), kMaxFftLen entries per table.
+// The twiddles e^{-2 pi i k/m} of the three axes (block 0: x, 1: y, 2: z), computed on the device,
+// kMaxFftLen entries per table.  The shifts and symbols that follow them in the array belong to the
+// solve, which a plain transform does not run.
 __global__ void k_noalloc_tables(float2* tab, int mx, int my, int mz) {
-  const int k = threadIdx.x;
-  const int m[3] = {mx, my, mz};
-  float* gt = reinterpret_cast<float*>(tab + 6 * kMaxFftLen);
-  for (int ax = 0; ax < 3; ++ax) {
-    if (k >= m[ax]) continue;
-    const double a = -2.0 * M_PI * (double)k / (double)m[ax];
-    tab[ax * kMaxFftLen + k] = make_float2((float)cos(a), (float)sin(a));
-    const double e = M_PI * (double)k / (double)m[ax];
-    tab[(3 + ax) * kMaxFftLen + k] = make_float2((float)cos(e), (float)sin(e));
-    gt[ax * kMaxFftLen + k] = (float)(2.0 / 1.0 * sin(M_PI * (double)k / (double)m[ax]));
-  }
+  const int k = threadIdx.x, m = blockIdx.x == 0 ? mx : blockIdx.x == 1 ? my : mz;
+  if (k >= m) return;
+  double s, c;
+  sincospi(-2.0 * (double)k / (double)m, &s, &c);
+  tab[blockIdx.x * kMaxFftLen + k] = make_float2((float)c, (float)s);
 }
 
 // Half spectrum from the passes' layout [ky][z][kx] to the caller's [z][ky][kx].
@@ -211,8 +206,9 @@ struct fhd_ctx {
   int* sid[2] = {nullptr, nullptr};
   int4* scell[2] = {nullptr, nullptr};
   float4* soff[2] = {nullptr, nullptr};
-  SrcRec* rec[2] = {nullptr, nullptr};   // spreading source records per group (2 np each)
-  int* cull[2] = {nullptr, nullptr};
+  unsigned* key[2] = {nullptr, nullptr};  // plane_key of each sorted slot
+  float margin = 0.0f;     // most that a source's stencil is displaced along z
+  float4* rfd = nullptr;   // normals of the RFD displacement, by sorted slot of set 0
   int* errd = nullptr;
   // harmonic bonds (bondedForces); null when the run has none
   int *bpp_start = nullptr, *bfp_start = nullptr;
@@ -319,7 +315,7 @@ void build_tables(fhd_ctx* c) {
     std::vector<float2> t(n);
     for (int k = 0; k < n; ++k) {
       double a = -2.0 * M_PI * (double)k / (double)n;
-      t[k] = make_float2((float)cos(a), (float)sin(a));
+      t[k] = unit_pair(cos(a), sin(a));
     }
     return t;
   };
@@ -332,7 +328,7 @@ void build_tables(fhd_ctx* c) {
     std::vector<float2> t(n);
     for (int k = 0; k < n; ++k) {
       double a = M_PI * (double)k / (double)n;
-      t[k] = make_float2((float)cos(a), (float)sin(a));
+      t[k] = unit_pair(cos(a), sin(a));
     }
     return t;
   };
@@ -381,8 +377,8 @@ void free_ctx(fhd_ctx* c) {
   void* ptrs[] = {c->v, c->v2, c->W, c->SF, c->adv[0], c->adv[1], c->div, c->spec, c->twx, c->twy, c->twz,
                   c->ex, c->ey, c->ez, c->gx, c->gy, c->gz, c->cell[0], c->cell[1], c->off[0], c->off[1],
                   c->F[0], c->F[1], c->u, c->count, c->slot, c->tmp, c->start[0], c->start[1], c->sid[0],
-                  c->sid[1], c->scell[0], c->scell[1], c->soff[0], c->soff[1], c->errd, c->rec[0], c->rec[1],
-                  c->cull[0], c->cull[1], c->bpp_start, c->bfp_start, c->bpp, c->bfpc, c->bfpo, c->sk_acc,
+                  c->sid[1], c->scell[0], c->scell[1], c->soff[0], c->soff[1], c->errd, c->key[0], c->key[1], c->rfd,
+                  c->bpp_start, c->bfp_start, c->bpp, c->bfpc, c->bfpo, c->sk_acc,
                   c->slot_of, c->sflag, c->M1, c->dulag, c->du, c->dp, c->jvt, c->ms, c->nb_idx, c->nb_cnt,
                   c->nb_flag, c->nb_ref_cell, c->nb_ref_off, c->sbar};
   for (void* q : ptrs)
@@ -614,6 +610,8 @@ SortArgs sort_args(fhd_ctx* c, int k) {
   a.sid = c->sid[k];
   a.scell = c->scell[k];
   a.soff = c->soff[k];
+  a.key = c->key[k];
+  a.margin = c->margin;
   a.bar = c->sbar;
   a.err = c->errd;
   a.np = c->np;
@@ -713,29 +711,25 @@ void sort_and_wca(fhd_ctx* c, int k, float4* F) {
   sort_set(c, k);
   wca(c, k, F);
 }
-// Attach the per-group record buffers, then prepare the source records and spread.
-void run_spread(fhd_ctx* c, SpreadArgs& sa) {
-  for (int k = 0; k < sa.ngroups; ++k) {
-    sa.grp[k].nsrc = c->np;
-    sa.grp[k].rec = c->rec[k];
-    sa.grp[k].cull = c->cull[k];
-  }
-  launch_src_prep(sa, c->s);
-  mark(c, "src_prep");
-  launch_spread(sa, c->s);
-  mark(c, "spread");
+// Forward transform of the spread field S F (plus `in`, null: none).
+void spread_forward(fhd_ctx* c, const PlaneSrc& src, const float* in) {
+  launch_fft_spread_xy_fwd(c->fa, in, src, c->spec, c->s);
+  mark(c, "fft_xy_fwd");
 }
-
-SpreadArgs spread_base(fhd_ctx* c) {
-  SpreadArgs a;
-  memset(&a, 0, sizeof(a));
-  a.g = c->g;
-  a.t = c->t;
-  a.kernel_points = c->p.kernel_points;
-  a.key = make_key(c);
-  a.out_coef = (float)(1.0 / c->dV);
-  a.out = c->SF;
-  return a;
+// One group of vector values by id, spread at position set k; more groups are added by the caller.
+PlaneSrc spread_values(fhd_ctx* c, int k, const float4* val, float coef) {
+  PlaneSrc p;
+  memset(&p, 0, sizeof(p));
+  p.t = c->t;
+  p.kernel_points = c->p.kernel_points;
+  p.out_coef = (float)(1.0 / c->dV);
+  p.ngroups = 1;
+  p.grp[0].set = sset(c, k);
+  p.grp[0].key = c->key[k];
+  p.grp[0].mode = SRC_VALUE;
+  p.grp[0].val = val;
+  p.grp[0].coef = coef;
+  return p;
 }
 InterpArgs interp_base(fhd_ctx* c, int eval_set) {
   InterpArgs a;
@@ -762,6 +756,8 @@ void skin_to_half(fhd_ctx* c, InterpArgs& ia) {
   SkinArgs& k = ia.sk;
   k.s_cell = c->scell[1];
   k.s_off = c->soff[1];
+  k.s_key = c->key[1];
+  k.margin = c->margin;
   k.s_slot = nullptr;
   k.skin_flag = c->sflag + 1;
   k.clear_flag = c->sflag;
@@ -774,6 +770,8 @@ void skin_to_full(fhd_ctx* c, InterpArgs& ia) {
   SkinArgs& k = ia.sk;
   k.s_cell = c->scell[0];
   k.s_off = c->soff[0];
+  k.s_key = c->key[0];
+  k.margin = c->margin;
   k.s_slot = c->slot_of;
   k.skin_flag = c->sflag;
   k.clear_flag = c->sflag + 1;
@@ -840,19 +838,11 @@ void step_stokes(fhd_ctx* c) {
   // solve 1: W = S F^n, and the kept part of sqrt(2) D.Sigma_1, drawn in Fourier space
   if (c->np > 0) {
     sort_and_wca(c, 0, c->F[0]);
-    SpreadArgs sa = spread_base(c);
-    sa.ngroups = 1;
-    sa.grp[0].set = sset(c, 0);
-    sa.grp[0].mode = SRC_VALUE;
-    sa.grp[0].val = c->F[0];
-    sa.grp[0].coef = 1.0f;
-    sa.out = c->W;
-    sa.out_add = nullptr;
-    run_spread(c, sa);
+    spread_forward(c, spread_values(c, 0, c->F[0], 1.0f), nullptr);
   } else {
     launch_zero_f(c->W, 3 * (size_t)c->g.N, c->s);
+    fft_forward(c, c->W);
   }
-  fft_forward(c, c->W);
   fft_solve_stokes(c, 1, (float)(sqrt(2.0) * f1), (float)(sqrt(2.0) * f4));
   fft_inverse(c, c->v, nullptr, 1.0f, 0.0f);
   if (c->np > 0) {
@@ -864,6 +854,7 @@ void step_stokes(fhd_ctx* c) {
     skin_to_half(c, ia);
     ia.f1 = c->v;
     ia.a1 = (float)(0.5 * dt);
+    ia.rfd = c->rfd;
     if (xm) {
       ia.F = c->F[0];
       ia.aF = (float)(0.5 * dt * p.extra_mobility);
@@ -873,25 +864,23 @@ void step_stokes(fhd_ctx* c) {
     launch_interp(ia, c->s);
     mark(c, "interp");
     sort_and_wca(c, 1, c->F[1]);
-    SpreadArgs sa = spread_base(c);
-    sa.ngroups = 2;
-    sa.grp[0].set = sset(c, 1);
-    sa.grp[0].mode = SRC_VALUE;
-    sa.grp[0].val = c->F[1];
-    sa.grp[0].coef = 1.0f;
-    sa.grp[1].set = sset(c, 0);
-    sa.grp[1].mode = SRC_RFD;
-    sa.grp[1].coef = (float)(p.temperature / p.rfd_delta);
-    sa.grp[1].disp = (float)(0.5 * p.rfd_delta);
-    sa.grp[1].rfd_quirk = p.rfd_mode == FHD_RFD_REFERENCE;
-    sa.out = c->W;
-    sa.out_add = nullptr;
-    run_spread(c, sa);
+    // solve 2: W = S F^{n+1/2} + RFD drift, and the kept part of sqrt(1/2) D.(Sigma_1 + Sigma_2)
+    PlaneSrc sp = spread_values(c, 1, c->F[1], 1.0f);
+    sp.ngroups = 2;
+    SpreadGroup& r = sp.grp[1];
+    r.set = sset(c, 0);
+    r.key = c->key[0];
+    r.mode = SRC_RFD;
+    r.val = c->rfd;
+    r.coef = (float)(p.temperature / p.rfd_delta);
+    r.disp = (float)(0.5 * p.rfd_delta);
+    r.rfd_quirk = p.rfd_mode == FHD_RFD_REFERENCE;
+    r.wide = (int)std::min(64.0, std::ceil(2.0 * c->margin / c->dz));
+    spread_forward(c, sp, nullptr);
   } else {
     launch_zero_f(c->W, 3 * (size_t)c->g.N, c->s);
+    fft_forward(c, c->W);
   }
-  // solve 2: W = S F^{n+1/2} + RFD drift, and the kept part of sqrt(1/2) D.(Sigma_1 + Sigma_2)
-  fft_forward(c, c->W);
   fft_solve_stokes(c, 2, (float)(sqrt(0.5) * f1), (float)(sqrt(0.5) * f4));
   fft_inverse(c, c->v, nullptr, 1.0f, 0.0f);
   if (c->np > 0) {
@@ -965,16 +954,8 @@ void qnb_mass_correction(fhd_ctx* c, bool lag, bool update_u) {
   a.out2 = c->jvt;
   pvec(c, a);
   const double f = 1.5 * Vp / (1.5 * Vp * dV * rho + me);  // src/quasiNeutrallyBuoyantFunctions2.cu:1332-1335
-  SpreadArgs sa = spread_base(c);
-  sa.ngroups = 1;
-  sa.grp[0].set = sset(c, 1);
-  sa.grp[0].mode = SRC_VALUE;
-  sa.grp[0].val = c->dp;
-  sa.grp[0].coef = (float)(f * dV);  // the pass scales by 1/dV: sum phi f dp
-  sa.out = c->W;
-  sa.out_add = nullptr;
-  run_spread(c, sa);
-  fft_forward(c, c->W);
+  // the spread scales by 1/dV: sum phi f dp
+  spread_forward(c, spread_values(c, 1, c->dp, (float)(f * dV)), nullptr);
   fft_solve(c, 0, 0.0f);  // projectionDivergenceFree (mode 0 kept)
   fft_inverse(c, c->M1, nullptr, 1.0f, 0.0f);
   a = pvec_base(c);
@@ -992,10 +973,8 @@ void qnb_mass_correction(fhd_ctx* c, bool lag, bool update_u) {
     a.out2 = c->u;
   }
   pvec(c, a);
-  sa.grp[0].val = c->ms;
-  sa.grp[0].coef = (float)(1.0 / rho);  // S(s) / rho = sum phi s / (rho dV)
-  run_spread(c, sa);
-  fft_forward(c, c->W);
+  // S(s) / rho = sum phi s / (rho dV)
+  spread_forward(c, spread_values(c, 1, c->ms, (float)(1.0 / rho)), nullptr);
   fft_solve(c, 0, cn);
   fft_inverse(c, c->W, nullptr, 1.0f, 0.0f);
 }
@@ -1037,6 +1016,12 @@ void step_qnb(fhd_ctx* c) {
   w.f1 = (float)sqrt(4.0 * p.temperature * p.shearviscosity * dt / (dV * rho * rho));
   w.f4 = (float)sqrt(2.0 * p.temperature * p.shearviscosity * dt / (dV * rho * rho));
   const float cn = (float)(0.5 * dt * p.shearviscosity / rho);
+  // W + dt/rho (S F + thermal drift), transformed
+  PlaneSrc src;
+  auto forward = [&] {
+    if (c->np > 0) spread_forward(c, src, c->W);
+    else fft_forward(c, c->W);
+  };
   if (c->np > 0) {
     sort_set(c, 0);
     InterpArgs ia = interp_base(c, 0);
@@ -1052,18 +1037,9 @@ void step_qnb(fhd_ctx* c) {
     sort_and_wca(c, 1, c->F[1]);
     const double mf = 1.5 * dV * p.volume_particle * rho;
     const double ratio = (p.mass + mf) != 0.0 ? mf / (p.mass + mf) : 1.0;
-    SpreadArgs sa = spread_base(c);
-    sa.ngroups = 2;
-    sa.grp[0].set = sset(c, 1);
-    sa.grp[0].mode = SRC_VALUE;
-    sa.grp[0].val = c->F[1];
-    sa.grp[0].coef = 1.0f;
-    sa.grp[1].set = sset(c, 1);
-    sa.grp[1].mode = SRC_DRIFT;
-    sa.grp[1].coef = (float)(p.temperature * ratio);
-    run_spread(c, sa);
-    w.force = c->SF;
-    w.force_coef = (float)(dt / rho);
+    src = spread_values(c, 1, c->F[1], 1.0f);
+    src.grp[0].drift = (float)(p.temperature * ratio);
+    src.out_coef = (float)(dt / (rho * dV));
     c->last_force_set = 1;
   }
   const bool mass = c->M1 != nullptr;
@@ -1074,7 +1050,7 @@ void step_qnb(fhd_ctx* c) {
     w.adv_store = c->adv[c->adv_cur];
     launch_fluid_w(w, c->s);
     mark(c, "fluid_w");
-    fft_forward(c, c->W);
+    forward();
     fft_solve(c, 0, cn);
     if (!mass) {
       fft_inverse(c, c->v2, c->v, 0.5f, 0.5f);  // v^{n+1/2}
@@ -1114,7 +1090,7 @@ void step_qnb(fhd_ctx* c) {
     launch_fluid_w(w, c->s);
     mark(c, "fluid_w");
   }
-  fft_forward(c, c->W);
+  forward();
   fft_solve(c, 0, cn);
   fft_inverse(c, c->v2, nullptr, 1.0f, 0.0f);  // v~^{n+1}
   if (mass) {
@@ -1841,8 +1817,7 @@ fhd_ctx* fhd_create(const fhd_params* pin) {
         c->sid[k] = dalloc<int>(c->np);
         c->scell[k] = dalloc<int4>(c->np);
         c->soff[k] = dalloc<float4>(c->np);
-        c->rec[k] = dalloc<SrcRec>(2 * (size_t)c->np);
-        c->cull[k] = dalloc<int>(2 * (size_t)c->np);
+        c->key[k] = dalloc<unsigned>(c->np);
         HIPCHK(hipMemset(c->F[k], 0, sizeof(float4) * c->np));
         // the sorted sets start empty and in range (every tile empty, every slot particle 0),
         // so a sort that never completes (its grid barrier gave up and raised the device error)
@@ -1851,6 +1826,12 @@ fhd_ctx* fhd_create(const fhd_params* pin) {
         HIPCHK(hipMemset(c->sid[k], 0, sizeof(int) * c->np));
         HIPCHK(hipMemset(c->scell[k], 0, sizeof(int4) * c->np));
         HIPCHK(hipMemset(c->soff[k], 0, sizeof(float4) * c->np));
+        HIPCHK(hipMemset(c->key[k], 0, sizeof(unsigned) * c->np));
+      }
+      if (p.scheme == FHD_SCHEME_STOKES_LIMIT) {
+        c->margin = (float)(0.5 * std::fabs(p.rfd_delta) * 5.8);  // the normals are below 5.8 (24-bit uniforms)
+        c->rfd = dalloc<float4>(c->np);
+        HIPCHK(hipMemset(c->rfd, 0, sizeof(float4) * c->np));
       }
       c->u = dalloc<float4>(c->np);
       HIPCHK(hipMemset(c->u, 0, sizeof(float4) * c->np));
@@ -2345,7 +2326,7 @@ int fhd_fft_r2c_noalloc(int mx, int my, int mz, const float* in, float* out_spec
     float2* spec = sc;
     float2* tab = sc + kNoAllocSpecMax;
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_noalloc_tables, dim3(1), dim3(kMaxFftLen), 0, s, tab, mx, my, mz);
+    hipLaunchKernelGGL(k_noalloc_tables, dim3(3), dim3(kMaxFftLen), 0, s, tab, mx, my, mz);
     HIPCHK(hipGetLastError());
     FftArgs a;
     memset(&a, 0, sizeof(a));
@@ -2457,7 +2438,8 @@ long long ctx_bytes(const fhd_params& p) {
     for (int a = 0; a < 3; ++a) nt *= te[a] > 0 ? m[a] / te[a] : 1;
     b += 2 * np * (16 + 16 + 16 + 4 + 16 + 16) + 2 * (nt + 1) * 4;  // positions, forces, sorted sets
     b += np * 16 + nt * 4 + 2 * np * 4;                               // u, counts, slots, scratch
-    b += 2 * 2 * np * ((long long)sizeof(SrcRec) + 4);                // spreading records
+    b += 2 * np * 4;                                                  // plane keys
+    if (p.scheme == FHD_SCHEME_STOKES_LIMIT) b += np * 16;            // RFD normals
     if (p.scheme == FHD_SCHEME_QUASI_NEUTRALLY_BUOYANT && p.mass != 0.0) b += N3 * 4 + 5 * np * 16;
   }
   return b;

@@ -17,6 +17,18 @@ struct LinePlan {
   uint32_t mns[3];
 };
 
+// The plan of given radices (1: no more stages).
+inline LinePlan line_plan(int n, int r0, int r1, int r2) {
+  LinePlan p{n, 0, {r0, r1, r2}, {0, 0, 0}};
+  for (int Ns = 1; p.nst < 3 && p.radix[p.nst] > 1; ++p.nst) {
+    p.mns[p.nst] = fast_div_magic(Ns);
+    Ns *= p.radix[p.nst];
+  }
+  return p;
+}
+// Lengths of the size-specialised passes: planes with both edges up to 64, columns up to 128.
+inline bool fast_edge(int m) { return m == 16 || m == 24 || m == 32 || m == 48 || m == 64; }
+
 struct FftArgs {
   GridDev g;
   const float2 *twx, *twy, *twz;  // e^{-2 pi i m / m_a}, m < m_a
@@ -51,8 +63,6 @@ struct FluidWArgs {
   const float* adv_prev;   // W += adv_prev_coef * adv_prev (nullptr: off)
   float adv_prev_coef;
   float* adv_store;        // stores A(vadv) when non-null
-  const float* force;      // W += force_coef * force (nullptr: off)
-  float force_coef;
   int noise;               // 0 none, 1 Sigma_1, 2 Sigma_1 + Sigma_2
   int trace_free;
   float f1, f4;            // diagonal / off-diagonal noise prefactors
@@ -105,6 +115,8 @@ struct SortArgs {
   int* sid;             // sorted outputs
   int4* scell;          // wrapped cell, w = the tile the slot is listed in
   float4* soff;
+  unsigned* key;        // per slot: plane_key
+  float margin;         // its margin
   int* slot_of;         // optional: sorted slot of each particle id
   const int* gate;      // optional: the sort runs only when *gate != 0 (the count clearing always runs)
   unsigned long long* bar;  // grid-barrier counter of the one-launch sort (only grows; zero at creation)
@@ -119,42 +131,25 @@ struct SortedSet {
   const int* start;     // tile_start[ntiles + 1]
 };
 
-// Source groups for the spreading kernel.
-enum { SRC_VALUE = 0, SRC_RFD = 1, SRC_DRIFT = 2 };
-// Stencil record of one spreading source (128 bytes): per axis the centred weights and the face
-// weights multiplied by the value's component along that axis (component a is the only one
-// sampled on the a-faces, so each component's stencil is a product of one face row and two
-// centred rows), then the first node of each stencil.
-struct SrcRec {
-  float w[2][3][4];     // [0: centred, 1: face x value][axis][k]
-  int base[2][3];
-  int pad[2];
-};
-
+// Sources spread into the forward xy transform (plane_spread.h).
+enum { SRC_VALUE = 0, SRC_RFD = 1 };
 struct SpreadGroup {
   SortedSet set;
-  int nsrc;             // sorted slots in the set (particles)
+  const unsigned* key;  // per sorted slot: plane_key
   int mode;
-  const float4* val;    // SRC_VALUE: per-particle vector value (by id)
-  float coef;           // multiplies the value (SRC_RFD: kT/delta; SRC_DRIFT: kT ratio)
+  const float4* val;    // SRC_VALUE: vector value by particle id; SRC_RFD: the displacement's normals by sorted slot
+  float coef;           // multiplies the value (SRC_RFD: kT/delta)
+  float drift;          // SRC_VALUE: coefficient of the thermal drift's derivative weights (0: none)
   float disp;           // SRC_RFD: displacement magnitude delta/2
+  int wide;             // most half cells along z between a source's sorted position and its stencil's
   int rfd_quirk;        // SRC_RFD: weights at the undisplaced position
-  SrcRec* rec;          // nsrc x (1 or 2) records, in sorted order
-  int* cull;            // per record: bits 0-8 tile reach mask (3 bits per axis), bits 16-24 e + 192 where
-                        // the record's largest face weight x value is below 2^e
 };
-
-struct SpreadArgs {
-  GridDev g;
+struct PlaneSrc {
   Tiles t;
   int kernel_points;
   int ngroups;
   SpreadGroup grp[2];
-  Key key;
-  float out_coef;       // multiplies the accumulated field (1/dV)
-  float* out;           // 3N field, every node written: out = out_add + coef * sum (out_add may be null)
-  const float* out_add; // may alias out (each node is read, then written, by one thread)
-  int nrec0, nrec_tot;  // records of group 0 and of both groups (set by launch_src_prep)
+  float out_coef;       // multiplies the accumulated field
 };
 
 // Verlet neighbour lists of the WCA pass: every pair closer than rc + list skin when the list
@@ -176,6 +171,8 @@ struct NbList {
 struct SkinArgs {
   int4* s_cell;          // sorted copy to update (wrapped cell; w = listed tile, kept)
   float4* s_off;
+  unsigned* s_key;
+  float margin;
   const int* s_slot;     // slot of each id in s_cell (null: the evaluated slot itself)
   int* skin_flag;        // set to 1 when a particle leaves its tile's skin
   int* clear_flag;       // set to 0 by the pass (a flag consumed by the sort before it)
@@ -200,6 +197,7 @@ struct InterpArgs {
   float4* u_out;         // J f2 (or J f1 when f2 is null), optional
   const float4* F; float aF;           // extra mobility: + aF F
   float aN; int nnoise;                // + aN (Z_1 [+ Z_2]) particle noise
+  float4* rfd;           // optional: the RFD displacement's normals of this step, by evaluated slot
   Key key;
   int* err;
   NbList nb;             // neighbour lists to invalidate when a particle moves (flag null: none)
@@ -292,14 +290,23 @@ struct BondArgs {
   int np;
 };
 
+// The forward xy pass with spreading: the plane of `p.in` (null: none) plus the sources' field.
+struct FftSpread {
+  FftPass p;
+  PlaneSrc s;
+};
+
 // Size-specialised FFT passes (fft_fast.hip); return false when the shape has no specialisation.
 bool fast_fft_xy_fwd(const FftArgs& a, const float* in, float2* spec, hipStream_t s);
+bool fast_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc& src, float2* spec, hipStream_t s);
 bool fast_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s);
 bool fast_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha, float beta,
                      hipStream_t s);
 
 // Launch helpers (defined in the .hip files).
 void launch_fft_xy_fwd(const FftArgs& a, const float* in, float2* spec, hipStream_t s);
+// The same for the field of the sources plus `in` (null: none).
+void launch_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc& src, float2* spec, hipStream_t s);
 // The 128 x 128 xy passes with the transforms in registers (which 0: forward, 1: inverse).
 void launch_fft128_xy(const FftPass& x, int which, int mz, hipStream_t s);
 void launch_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s);
@@ -323,8 +330,6 @@ void launch_sort_wca(const SortArgs& s, const WcaArgs& w, hipStream_t st);
 void launch_wca(const WcaArgs& a, hipStream_t s);
 void launch_wca_list(const WcaArgs& a, hipStream_t s);
 void launch_bonded(const BondArgs& a, hipStream_t s);  // F += bond forces (after the WCA pass)
-void launch_src_prep(const SpreadArgs& a, hipStream_t s);  // per-source records (run first)
-void launch_spread(const SpreadArgs& a, hipStream_t s);    // tile accumulation
 void launch_interp(const InterpArgs& a, hipStream_t s);
 void launch_pvec(const PVecArgs& a, hipStream_t s);
 void launch_lag2(const Lag2Args& a, hipStream_t s);

@@ -160,11 +160,6 @@ FHD_BODY void body_fluid_w(const FluidWArgs& a, const Blk& b) {
         wy += a.adv_prev_coef * a.adv_prev[i + N];
         wz += a.adv_prev_coef * a.adv_prev[i + 2 * (size_t)N];
       }
-      if (a.force) {
-        wx += a.force_coef * a.force[i];
-        wy += a.force_coef * a.force[i + N];
-        wz += a.force_coef * a.force[i + 2 * (size_t)N];
-      }
       a.W[i] = wx;
       a.W[i + N] = wy;
       a.W[i + 2 * (size_t)N] = wz;

@@ -8,11 +8,7 @@
 //  * WCA forces, one workgroup per tile, from the particles of the neighbouring tiles staged
 //    in LDS (fluam's cell-list pair loop, src/stokesLimitFunctions.cu:160-653, with the
 //    analytic potential instead of the float texture table of src/initForcesNonBonded.cu:21-66).
-//  * spreading S F: one workgroup per tile adds the contributions of every source whose
-//    stencil reaches the tile into a 64-bit fixed-point LDS accumulator.  Integer addition is
-//    associative, so the field is bit-identical whatever order the contributions arrive in:
-//    deterministic without float atomics.  Replaces the 27-slot scatter + per-cell gather of
-//    src/stokesLimitFunctions.cu:659-1158,1198-1681 and src/kernelSpreadParticles.cu:3012-4082.
+//  * spreading S F is part of the forward xy transform (plane_spread.h).
 //  * interpolation J v and the particle position updates (src/stokesLimitFunctions.cu:
 //    2479-2892,3513-3894; src/quasiNeutrallyBuoyantFunctions.cu:2448-2853,4481-4862).
 //
@@ -20,6 +16,7 @@
 // and pair distances are computed from small offsets and exact integer cell differences.
 #include "fhd_device.h"
 #include "fhd_kernels.h"
+#include "plane_spread.h"
 
 namespace fhd {
 
@@ -45,7 +42,9 @@ FHD_DEV void place(const SortArgs& a, int i, int pos, int tile) {
   const int4 c = a.cell[i];
   a.sid[pos] = i;
   a.scell[pos] = make_int4(wrapi(c.x, a.g.mx), wrapi(c.y, a.g.my), wrapi(c.z, a.g.mz), tile);
-  a.soff[pos] = a.off[i];
+  const float4 d = a.off[i];
+  a.soff[pos] = d;
+  a.key[pos] = plane_key(a.g, wrapi(c.x, a.g.mx), wrapi(c.y, a.g.my), wrapi(c.z, a.g.mz), d.z, a.margin);
   if (a.slot_of) a.slot_of[i] = pos;
 }
 
@@ -226,18 +225,6 @@ FHD_DEV int wave_incl_scan(int v) {
   for (int o = 1; o < 64; o <<= 1) {
     const int t = __shfl_up(v, o);
     if (lane >= o) v += t;
-  }
-  return v;
-}
-
-// Largest value over the wave, in every lane (butterfly over lane-index bits).  An LDS
-// atomicMax with per-lane values would do the same, but the compiler expands it into a
-// 64-iteration scalar read-lane loop per wave, which saturates the CU's one scalar unit.
-FHD_DEV unsigned wave_max_u32(unsigned v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    const unsigned t = (unsigned)__shfl_xor((int)v, o);
-    v = v > t ? v : t;
   }
   return v;
 }
@@ -642,16 +629,6 @@ FHD_BODY void body_bonded(const BondArgs& a, const Blk& b) {
 }
 FHD_KERNEL_PAIR((), kBondThreads, k_bonded, BondArgs, body_bonded(a, b))
 
-// Weights of one axis at an explicit node base (used for the reference-quirk RFD variant):
-// node k sits at integer position base + k in node units; the particle at c + frac - stag/2.
-template <int NPTS>
-FHD_DEV void axis_weights_at(int base, int c, float frac, int stag, AxisWeights& aw) {
-  aw.base = base;
-  float f = (float)(c - base) + frac - 0.5f * (float)stag;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) aw.w[k] = (k < NPTS) ? (NPTS == 3 ? phi3(f - (float)k) : phi4(f - (float)k)) : 0.0f;
-}
-
 struct SrcWeights {
   AxisWeights cen[3], stg[3];   // centred and face weights per axis
 };
@@ -667,460 +644,6 @@ FHD_DEV void source_weights(int4 c, float3 frac, SrcWeights& w, bool deriv) {
     else axis_weights<NPTS>(cc[ax], ff[ax], 1, w.stg[ax]);
   }
 }
-
-constexpr int kTileEdge = 8;         // largest spreading tile edge (cells)
-constexpr int kSpreadThreads = 256;
-
-// Fold a node index offset into [0, m) (the offsets here stay within a few boxes of the tile).
-// Offsets passed here lie in (-m, 2m) whenever m >= 8 (wrapped cells, stencils within three
-// cells, tiles of at least four cells); smaller boxes take the loop.
-FHD_DEV int fold(int l, int m) {
-  if (l < 0) l += m;
-  else if (l >= m) l -= m;
-  if (m < 8) {
-    while (l < 0) l += m;
-    while (l >= m) l -= m;
-  }
-  return l;
-}
-
-FHD_DEV float3 f3(float4 a) { return make_float3(a.x, a.y, a.z); }
-
-// Position (cell, offset) of source `sub` of a particle, plus its value.
-FHD_DEV void rfd_normal(const Key& key, int id, float n[4]) {
-  draw_normals4(key, (uint32_t)id, FHD_STREAM_RFD, 0, n);
-}
-
-// Does a stencil whose nodes span [lo, lo + NPTS] (both staggerings) reach the tile [o, o+T)?
-template <int NPTS>
-FHD_DEV bool reaches(int lo, int o, int T, int m, int ntiles) {
-  if (ntiles == 1) return true;
-  const int l0 = fold(lo - o, m);
-  return l0 < T || l0 + NPTS >= m;
-}
-
-// One record per source (sorted slot x sub-source): weights, bases, value and the cull data.
-// One launch covers every group: threads [0, n0) build group 0's records, the rest group 1's.
-template <int NPTS>
-FHD_BODY void body_src_prep(const SpreadArgs& a, const Blk& b) {
-  const int n0 = a.nrec0, ntot = a.nrec_tot;
-  int r = b.x * blockDim.x + threadIdx.x;
-  if (r >= ntot) return;
-  const int gi = r < n0 ? 0 : 1;
-  if (gi) r -= n0;
-  const SpreadGroup& G = a.grp[gi];
-  const GridDev& g = a.g;
-  const int nsub = G.mode == SRC_RFD ? 2 : 1;
-  const int sidx = nsub == 2 ? r >> 1 : r, sub = r - sidx * nsub;
-  const int id = G.set.id[sidx];
-  const int4 c = G.set.cell[sidx];
-  const float4 d = G.set.off[sidx];
-  float3 val;
-  int4 cw = c;
-  float3 dw = make_float3(d.x, d.y, d.z);
-  if (G.mode == SRC_VALUE) {
-    const float4 v = G.val[id];
-    val = make_float3(v.x * G.coef, v.y * G.coef, v.z * G.coef);
-    if (val.x == 0.0f && val.y == 0.0f && val.z == 0.0f) {
-      // a zero source (e.g. a particle with no WCA neighbour) adds exactly zero to every node:
-      // an empty reach mask makes every tile cull it, and its record is never read
-      G.cull[r] = 0;
-      return;
-    }
-  } else if (G.mode == SRC_DRIFT) {
-    val = make_float3(G.coef * g.idx, G.coef * g.idy, G.coef * g.idz);
-  } else {
-    float nrm[4];
-    rfd_normal(resolve_key(a.key), id, nrm);
-    const float sg = sub == 0 ? 1.0f : -1.0f;
-    val = make_float3(sg * G.coef * nrm[0], sg * G.coef * nrm[1], sg * G.coef * nrm[2]);
-    dw = make_float3(d.x + sg * G.disp * nrm[0], d.y + sg * G.disp * nrm[1], d.z + sg * G.disp * nrm[2]);
-    renorm_axis(cw.x, dw.x, g.dx, g.idx);
-    renorm_axis(cw.y, dw.y, g.dy, g.idy);
-    renorm_axis(cw.z, dw.z, g.dz, g.idz);
-  }
-  SrcWeights w;
-  source_weights<NPTS>(cw, make_float3(dw.x * g.idx, dw.y * g.idy, dw.z * g.idz), w, G.mode == SRC_DRIFT);
-  if (G.mode == SRC_RFD && G.rfd_quirk) {
-    // nodes from the displaced position, weights at the undisplaced one
-    const int cc[3] = {c.x, c.y, c.z};
-    const float ff[3] = {d.x * g.idx, d.y * g.idy, d.z * g.idz};
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-      axis_weights_at<NPTS>(w.cen[ax].base, cc[ax], ff[ax], 0, w.cen[ax]);
-      axis_weights_at<NPTS>(w.stg[ax].base, cc[ax], ff[ax], 1, w.stg[ax]);
-    }
-  }
-  const float vv[3] = {val.x, val.y, val.z};
-  SrcRec rec;
-#pragma unroll
-  for (int ax = 0; ax < 3; ++ax) {
-    rec.base[0][ax] = w.cen[ax].base;
-    rec.base[1][ax] = w.stg[ax].base;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      rec.w[0][ax][q] = w.cen[ax].w[q];
-      // an overflowed source (non-finite or beyond 3e38) is stored as +-3e38, NaN as -3e38:
-      // its tile's bound then reaches 2^127, and the spreading pass writes that tile's field as
-      // non-finite, which the interpolation pass flags
-      const float fw = w.stg[ax].w[q] * vv[ax];
-      rec.w[1][ax][q] = fabsf(fw) <= 3.0e38f ? fw : (fw > 0.0f ? 3.0e38f : -3.0e38f);
-    }
-  }
-  rec.pad[0] = rec.pad[1] = 0;
-  const float4* src4 = reinterpret_cast<const float4*>(&rec);
-  float4* dst4 = reinterpret_cast<float4*>(G.rec + r);
-#pragma unroll
-  for (int k = 0; k < (int)(sizeof(SrcRec) / 16); ++k) dst4[k] = src4[k];
-  // bound on one contribution: centred weights are at most 1, so the largest face weight x value
-  float m = 0.0f;
-#pragma unroll
-  for (int ax = 0; ax < 3; ++ax)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) m = fmaxf(m, fabsf(rec.w[1][ax][q]));  // <= 3e38
-  // reach mask: per axis, bit e + 1 set when the stencils (nodes lo .. lo + NPTS, both
-  // staggerings) reach the tile at offset e in {-1, 0, 1} from the source's sorting tile
-  const int lo[3] = {min(w.cen[0].base, w.stg[0].base), min(w.cen[1].base, w.stg[1].base),
-                     min(w.cen[2].base, w.stg[2].base)};
-  const Tiles& t = a.t;
-  const int T[3] = {t.tx, t.ty, t.tz}, NT[3] = {t.ntx, t.nty, t.ntz}, MM[3] = {g.mx, g.my, g.mz};
-  // the tile the source is listed in (the sorted copy's w): the spreading pass looks for it in
-  // the lists of that tile's neighbours, which its stencil may reach while it stays within the
-  // skin of that tile
-  const int lt[3] = {c.w % t.ntx, (c.w / t.ntx) % t.nty, c.w / (t.ntx * t.nty)};
-  int mask = 0;
-#pragma unroll
-  for (int ax = 0; ax < 3; ++ax) {
-    const int own = lt[ax];
-#pragma unroll
-    for (int e = -1; e <= 1; ++e) {
-      int tt = own + e;  // in [-1, NT]
-      tt += tt < 0 ? NT[ax] : (tt >= NT[ax] ? -NT[ax] : 0);
-      if (reaches<NPTS>(lo[ax], tt * T[ax], T[ax], MM[ax], NT[ax])) mask |= 1 << (3 * ax + e + 1);
-    }
-  }
-  // the bound enters the spreading pass only through its binary exponent: m < 2^e (e = -191
-  // for m = 0, below any other record's), stored biased by 192 in bits 16-24
-  int e = -191;
-  if (m > 0.0f) frexpf(m, &e);
-  G.cull[r] = mask | ((e + 192) << 16);
-}
-FHD_KERNEL_PAIR((template <int NPTS>), 256, k_src_prep, SpreadArgs, body_src_prep<NPTS>(a, b))
-
-// Fixed-point image of one contribution, as a 64-bit two's-complement addend.  Integer sums are
-// exact, so the accumulated field does not depend on the order in which the contributions
-// arrive.  The records are finite with face weights of at most 3e38 < 2^128, and the tile's
-// scale 2^(30 - e) puts its largest face weight below 2^30; centred weights are at most 1, so
-// |x| <= 2^30 and the conversion is always defined without a clamp.
-FHD_DEV unsigned long long fixed64(float x) {
-  // truncation toward zero: at the 2^30 scale its bias (< 1 unit) is far below FP32 rounding
-  const int q = (int)x;
-  return (unsigned long long)(long long)q;
-}
-
-// Candidate-record reference: group in bit 30, record index below.
-constexpr int kItemCap = 1024;
-// Accumulator z-row stride (64-bit words): the 8 x 8 plane plus 2, so the rows that the four
-// lanes of one candidate update start in different LDS banks.
-constexpr int kRowStride = kTileEdge * kTileEdge + 2;
-
-// Contributions of stencil row kz (nodes base_z + kz) of one source record to the three
-// components of the tile accumulator acc[component][z row][y][x] (x, y: the 8 x 8 tile columns).
-// Only nodes inside the tile are added: a lane whose row lies outside skips it, and out-of-tile
-// columns are masked off, so no LDS atomic is spent on a node the tile does not own.  FAST: the
-// first node relative to the tile comes from one periodic fold; otherwise (small boxes) every
-// node is folded periodically and tested against the tile.
-template <int NPTS, bool FAST>
-FHD_DEV void add_source_row(unsigned long long* acc, const SrcRec* __restrict__ R, int kz, int ox, int oy, int oz,
-                            const GridDev& g, const Tiles& t, float scale) {
-  constexpr int H = NPTS - 1;
-  constexpr int ZS = kTileEdge;
-  constexpr int PL = kRowStride;
-  const float4 cx = *reinterpret_cast<const float4*>(R->w[0][0]);
-  const float4 cy = *reinterpret_cast<const float4*>(R->w[0][1]);
-  const float4 fx = *reinterpret_cast<const float4*>(R->w[1][0]);
-  const float4 fy = *reinterpret_cast<const float4*>(R->w[1][1]);
-  const float cz = R->w[0][2][kz], fz = R->w[1][2][kz];
-  const int4 b0 = *reinterpret_cast<const int4*>(&R->base[0][0]);  // cen x, y, z, face x
-  const int2 b1 = *reinterpret_cast<const int2*>(&R->base[1][1]);  // face y, z
-#pragma unroll
-  for (int C = 0; C < 3; ++C) {
-    const int bx = C == 0 ? b0.w : b0.x, by = C == 1 ? b1.x : b0.y, bz = C == 2 ? b1.y : b0.z;
-    const float4 w4x = C == 0 ? fx : cx, w4y = C == 1 ? fy : cy;
-    const float wx[4] = {w4x.x, w4x.y, w4x.z, w4x.w}, wy[4] = {w4y.x, w4y.y, w4y.z, w4y.w};
-    const float wzs = (C == 2 ? fz : cz) * scale;
-    if (FAST) {
-      // first stencil node relative to the tile, folded to [-H, m - H)
-      int dx = bx - ox, dy = by - oy, dz = bz - oz;
-      dx += dx < -H ? g.mx : (dx >= g.mx - H ? -g.mx : 0);
-      dy += dy < -H ? g.my : (dy >= g.my - H ? -g.my : 0);
-      dz += dz < -H ? g.mz : (dz >= g.mz - H ? -g.mz : 0);
-      const int lz = dz + kz;
-      if ((unsigned)lz >= (unsigned)kTileEdge) continue;  // this row misses the tile
-      const int rb = (C * ZS + lz) * PL;
-#pragma unroll
-      for (int ky = 0; ky < NPTS; ++ky) {
-        const float wyz = wy[ky] * wzs;
-        const int ly = dy + ky;
-#pragma unroll
-        for (int kx = 0; kx < NPTS; ++kx) {
-          const int lx = dx + kx;
-          if ((unsigned)ly < (unsigned)kTileEdge && (unsigned)lx < (unsigned)kTileEdge)
-            atomicAdd(&acc[rb + ly * kTileEdge + lx], fixed64(wx[kx] * wyz));
-        }
-      }
-    } else {
-      const int lz = fold(bz + kz - oz, g.mz);
-      if (lz >= t.tz) continue;
-      unsigned long long* row = acc + (C * ZS + lz) * PL;
-#pragma unroll
-      for (int ky = 0; ky < NPTS; ++ky) {
-        const int ly = fold(by + ky - oy, g.my);
-        if (ly >= t.ty) continue;
-        const float wyz = wy[ky] * wzs;
-#pragma unroll
-        for (int kx = 0; kx < NPTS; ++kx) {
-          const int lx = fold(bx + kx - ox, g.mx);
-          if (lx < t.tx) atomicAdd(&row[ly * kTileEdge + lx], fixed64(wx[kx] * wyz));
-        }
-      }
-    }
-  }
-}
-
-// The narrow accumulator of 8 x 8 x 8 tiles with at most kNarrowCand candidates: 32-bit
-// fixed point, rows of kRow32 words covering x = -3 .. 10 (a halo of three columns each side,
-// so every node of a stencil row that starts in [-3, 7] has a slot and the atomics need no
-// column test; the halo is never read), planes of kPlane32 words (the 8 rows plus 1, so the
-// rows of the four lanes of one candidate start in different LDS banks).  A node's sum has at
-// most one contribution per candidate, so with contributions below 2^(30 - floor(log2 n)) for n
-// candidates it stays below 2^31.
-constexpr int kNarrowCand = 255;
-constexpr int kRow32 = kTileEdge + 6;
-constexpr int kPlane32 = kTileEdge * kRow32 + 1;
-constexpr int kComp32 = kTileEdge * kPlane32;
-
-template <int NPTS>
-FHD_DEV void add_source_row32(unsigned* acc, const SrcRec* __restrict__ R, int kz, int ox, int oy, int oz,
-                              const GridDev& g, float scale) {
-  constexpr int H = NPTS - 1;
-  const float4 cx = *reinterpret_cast<const float4*>(R->w[0][0]);
-  const float4 cy = *reinterpret_cast<const float4*>(R->w[0][1]);
-  const float4 fx = *reinterpret_cast<const float4*>(R->w[1][0]);
-  const float4 fy = *reinterpret_cast<const float4*>(R->w[1][1]);
-  const float cz = R->w[0][2][kz], fz = R->w[1][2][kz];
-  const int4 b0 = *reinterpret_cast<const int4*>(&R->base[0][0]);  // cen x, y, z, face x
-  const int2 b1 = *reinterpret_cast<const int2*>(&R->base[1][1]);  // face y, z
-#pragma unroll
-  for (int C = 0; C < 3; ++C) {
-    const int bx = C == 0 ? b0.w : b0.x, by = C == 1 ? b1.x : b0.y, bz = C == 2 ? b1.y : b0.z;
-    const float4 w4x = C == 0 ? fx : cx, w4y = C == 1 ? fy : cy;
-    const float wx[4] = {w4x.x, w4x.y, w4x.z, w4x.w}, wy[4] = {w4y.x, w4y.y, w4y.z, w4y.w};
-    const float wzs = (C == 2 ? fz : cz) * scale;
-    // first stencil node relative to the tile, folded to [-H, m - H)
-    int dx = bx - ox, dy = by - oy, dz = bz - oz;
-    dx += dx < -H ? g.mx : (dx >= g.mx - H ? -g.mx : 0);
-    dy += dy < -H ? g.my : (dy >= g.my - H ? -g.my : 0);
-    dz += dz < -H ? g.mz : (dz >= g.mz - H ? -g.mz : 0);
-    const int lz = dz + kz;
-    // this row misses the tile, or its columns do (then dx lies outside [-H, 7])
-    if ((unsigned)lz >= (unsigned)kTileEdge || dx > kTileEdge - 1) continue;
-    // word index of the stencil's first node; the stencil's rows and columns are constant
-    // offsets from it
-    const int first = C * kComp32 + lz * kPlane32 + dy * kRow32 + dx + 3;
-#pragma unroll
-    for (int ky = 0; ky < NPTS; ++ky) {
-      if ((unsigned)(dy + ky) >= (unsigned)kTileEdge) continue;
-      const float wyz = wy[ky] * wzs;
-#pragma unroll
-      for (int kx = 0; kx < NPTS; ++kx)
-        atomicAdd(&acc[first + ky * kRow32 + kx], (unsigned)(int)(wx[kx] * wyz));
-    }
-  }
-}
-
-FHD_DEV const SrcRec* rec_of(const SpreadArgs& a, int ref) {
-  return a.grp[ref >> 30].rec + (ref & ((1 << 30) - 1));
-}
-
-// Spreading, one workgroup per tile.  The records of the sources in the neighbouring tiles are
-// culled against the tile into a candidate list; four lanes take each candidate, one stencil
-// z-row each, and add its contributions to the three components into a 64-bit fixed-point LDS
-// accumulator (scale 2^(30 - e) per tile, from the largest face weight x value of its
-// candidates).  Integer addition is associative, so the result is bit-identical whatever order
-// the lanes' atomics land in.  FAST: tiles of 8 x 8 x 8 cells and at least two tiles per axis.
-template <int NPTS, bool FAST>
-FHD_BODY void body_spread(const SpreadArgs& a, const Blk& b) {
-  constexpr int ZS = kTileEdge;
-  constexpr int NACC = 3 * ZS * kRowStride;
-  static_assert(3 * kComp32 <= 2 * NACC, "the narrow accumulator shares the 64-bit one's LDS");
-  constexpr int LPC = 4;  // lanes per candidate (one stencil z-row each)
-  __shared__ unsigned long long acc[NACC];
-  __shared__ int nb_start[64], nb_pref[65], nb_sel[64];
-  __shared__ int items[kItemCap];
-  __shared__ int nitem;
-  __shared__ unsigned int maxbits;
-  const GridDev& g = a.g;
-  const Tiles& t = a.t;
-  const int tid = threadIdx.x;
-  const int tile = xcd_item(b.x, t.n);
-  const int tx = tile % t.ntx, ty = (tile / t.ntx) % t.nty, tz = tile / (t.ntx * t.nty);
-  const int ox = tx * t.tx, oy = ty * t.ty, oz = tz * t.tz;
-  // FAST tiles: each thread's output nodes are e = tid + k * kSpreadThreads, k < kOutPer; their
-  // out_add values are loaded now, so the loads complete under the accumulation
-  constexpr int kOutPer = 3 * kTileEdge * kTileEdge * kTileEdge / kSpreadThreads;
-  float pre[kOutPer];
-  if (FAST && a.out_add) {
-#pragma unroll
-    for (int k = 0; k < kOutPer; ++k) {
-      const int e = tid + k * kSpreadThreads;
-      const int C = e >> 9, lx = e & 7, ly = (e >> 3) & 7, lz = (e >> 6) & 7;
-      pre[k] = a.out_add[(size_t)C * g.N + (ox + lx) + (size_t)g.mx * ((oy + ly) + (size_t)g.my * (oz + lz))];
-    }
-  }
-  for (int e = tid; e < NACC; e += kSpreadThreads) acc[e] = 0ull;
-  // neighbour-tile table: lane k of wave 0 loads the record range of (group, neighbour) k
-  int lox, hix, loy, hiy, loz, hiz;
-  nb_range(t.ntx, lox, hix);
-  nb_range(t.nty, loy, hiy);
-  nb_range(t.ntz, loz, hiz);
-  const int nx = hix - lox + 1, ny = hiy - loy + 1, nz = hiz - loz + 1;
-  const int nnb = nx * ny * nz;
-  const int ntab = a.ngroups * nnb;  // <= 54
-  if (tid < 64) {
-    int cnt = 0;
-    if (tid < ntab) {
-      const int gi = tid / nnb, k = tid - gi * nnb;
-      const int nsub = a.grp[gi].mode == SRC_RFD ? 2 : 1;
-      const int dx = lox + k % nx, dy = loy + (k / nx) % ny, dz = loz + k / (nx * ny);
-      const int nt = wrapi(tx + dx, t.ntx) + t.ntx * (wrapi(ty + dy, t.nty) + t.nty * wrapi(tz + dz, t.ntz));
-      const int s0 = a.grp[gi].set.start[nt];
-      nb_start[tid] = s0 * nsub;
-      cnt = (a.grp[gi].set.start[nt + 1] - s0) * nsub;
-      // this tile sits at offset -d from the source tile: the reach-mask bits to test
-      nb_sel[tid] = (1 << (1 - dx)) | (1 << (4 - dy)) | (1 << (7 - dz));
-    }
-    const int incl = wave_incl_scan(cnt);
-    nb_pref[tid + 1] = incl;
-    if (tid == 0) {
-      nb_pref[0] = 0;
-      nitem = 0;
-      maxbits = 0u;
-    }
-  }
-  __syncthreads();
-  const int nall = nb_pref[ntab];
-  // record index e -> reference; -1 when the record's stencils miss the tile
-  auto cull = [&](int e, int& mx) -> int {
-    // largest lo with nb_pref[lo] <= e: fixed-step search (no divergent loop); entries past
-    // ntab hold nall, which no record index reaches
-    int lo = 0;
-#pragma unroll
-    for (int step = 32; step >= 1; step >>= 1)
-      if (nb_pref[lo + step] <= e) lo += step;
-    const int gi = lo >= nnb;
-    const int ri = nb_start[lo] + (e - nb_pref[lo]);
-    const int cu = a.grp[gi].cull[ri];
-    const int sel = nb_sel[lo];
-    if ((cu & sel) != sel) return -1;
-    mx = max(mx, cu >> 16);
-    return (gi << 30) | ri;
-  };
-  // pass 1: cull every record, keep the first kItemCap candidates, largest magnitude; each wave
-  // appends its survivors with one LDS atomic
-  int lmax = 0;  // largest biased exponent of the candidates' bounds
-  const int lane = tid & 63;
-  const unsigned long long below = (1ull << lane) - 1ull;
-  for (int e0 = 0; e0 < nall; e0 += kSpreadThreads) {
-    const int e = e0 + tid;
-    const int ref = e < nall ? cull(e, lmax) : -1;
-    const unsigned long long bal = __ballot(ref >= 0);
-    int base = 0;
-    if (lane == 0 && bal) base = atomicAdd(&nitem, __popcll(bal));
-    base = __shfl(base, 0);
-    if (ref >= 0) {
-      const int k = base + __popcll(bal & below);
-      if (k < kItemCap) items[k] = ref;
-    }
-  }
-  const unsigned wmax = wave_max_u32((unsigned)lmax);
-  if (lane == 0) atomicMax(&maxbits, wmax);
-  __syncthreads();
-  const int ntot = nitem;
-  // every candidate's largest face weight x value is below 2^e2
-  const int e2 = max((int)maxbits - 192, -90);
-  // narrow tiles: contributions below 2^S with S = 30 - floor(log2 ntot); others 2^30 in 64 bits
-  const bool narrow = FAST && ntot <= kNarrowCand;
-  const int S = narrow ? 30 - (31 - __clz(ntot > 0 ? ntot : 1)) : 30;
-  const float scale = ldexpf(1.0f, S - e2);
-  // a bound of 2^127 or more means an overflowed source among the candidates (the record pass
-  // stores those as +-3e38): the tile's field is written non-finite (every node +-inf or NaN),
-  // so the step is flagged
-  const float inv = e2 >= 128 ? __builtin_inff() : ldexpf(1.0f, e2 - S) * a.out_coef;
-  const int kz = tid % LPC;
-  unsigned* const acc32 = reinterpret_cast<unsigned*>(acc);
-  if (narrow) {
-    if (kz < NPTS)
-      for (int c = tid / LPC; c < ntot; c += kSpreadThreads / LPC)
-        add_source_row32<NPTS>(acc32, rec_of(a, items[c]), kz, ox, oy, oz, g, scale);
-  } else if (ntot <= kItemCap) {
-    if (kz < NPTS)
-      for (int c = tid / LPC; c < ntot; c += kSpreadThreads / LPC)
-        add_source_row<NPTS, FAST>(acc, rec_of(a, items[c]), kz, ox, oy, oz, g, t, scale);
-  } else {
-    // more candidates than the list holds: rounds over disjoint record ranges, re-culled
-    for (int b0 = 0; b0 < nall; b0 += kItemCap) {
-      __syncthreads();
-      if (tid == 0) nitem = 0;
-      __syncthreads();
-      int dummy = 0;
-      for (int e = b0 + tid; e < min(nall, b0 + kItemCap); e += kSpreadThreads) {
-        const int ref = cull(e, dummy);
-        if (ref >= 0) items[atomicAdd(&nitem, 1)] = ref;
-      }
-      __syncthreads();
-      if (kz < NPTS)
-        for (int c = tid / LPC; c < nitem; c += kSpreadThreads / LPC)
-          add_source_row<NPTS, FAST>(acc, rec_of(a, items[c]), kz, ox, oy, oz, g, t, scale);
-    }
-  }
-  __syncthreads();
-  // interior nodes -> field (8 x 8 x 8 tiles: index arithmetic by shifts)
-  const int ncell = t.tx * t.ty * t.tz;
-  if (FAST) {
-#pragma unroll
-    for (int k = 0; k < kOutPer; ++k) {
-      const int e = tid + k * kSpreadThreads;
-      const int C = e >> 9, lx = e & 7, ly = (e >> 3) & 7, lz = (e >> 6) & 7;
-      const size_t gi = (size_t)C * g.N + (ox + lx) + (size_t)g.mx * ((oy + ly) + (size_t)g.my * (oz + lz));
-      const float q = narrow ? (float)(int)acc32[C * kComp32 + lz * kPlane32 + ly * kRow32 + lx + 3]
-                             : (float)(long long)acc[(C * ZS + lz) * kRowStride + ly * kTileEdge + lx];
-      const float val = q * inv;
-      a.out[gi] = a.out_add ? pre[k] + val : val;
-    }
-    return;
-  }
-  for (int e = tid; e < 3 * ncell; e += kSpreadThreads) {
-    int C, lx, ly, lz;
-    if (FAST) {
-      C = e >> 9;
-      lx = e & 7;
-      ly = (e >> 3) & 7;
-      lz = (e >> 6) & 7;
-    } else {
-      C = e / ncell;
-      const int l = e - C * ncell;
-      lx = l % t.tx;
-      ly = (l / t.tx) % t.ty;
-      lz = l / (t.tx * t.ty);
-    }
-    const int ai = (C * ZS + lz) * kRowStride + ly * kTileEdge + lx;
-    const size_t gi = (size_t)C * g.N + (ox + lx) + (size_t)g.mx * ((oy + ly) + (size_t)g.my * (oz + lz));
-    const float val = (float)(long long)acc[ai] * inv;
-    a.out[gi] = a.out_add ? a.out_add[gi] + val : val;
-  }
-}
-FHD_KERNEL_PAIR((template <int NPTS, bool FAST>), kSpreadThreads, k_spread, SpreadArgs, body_spread<NPTS, FAST>(a, b))
 
 // Sum over the NPTS x NPTS nodes of one z-row (kz) of a particle's stencil.
 template <int NPTS>
@@ -1287,6 +810,7 @@ FHD_DEV void interp_finish(const InterpArgs& a, int s, const InterpPre& pre, con
       if (out) *a.sk.skin_flag = 1;
       a.sk.s_cell[slot] = make_int4(wc[0], wc[1], wc[2], lt);
       a.sk.s_off[slot] = make_float4(ox, oy, oz, 0.0f);
+      a.sk.s_key[slot] = plane_key(g, wc[0], wc[1], wc[2], oz, a.sk.margin);
       if (a.sk.sid_dst) a.sk.sid_dst[s] = id;
     }
   }
@@ -1326,7 +850,14 @@ FHD_BODY void body_interp(const InterpArgs& a, const Blk& b) {
       for (int k = gid; k <= a.t.n; k += nth) a.sk.start_dst[k] = a.sk.start_src[k];
     if (gid == 0 && a.sk.clear_flag) *a.sk.clear_flag = 0;
   }
-  if (s >= a.np || q != 0) return;
+  if (s >= a.np) return;
+  if (q == 1 && a.rfd) {
+    // an idle lane draws the normals that displace this particle's RFD sources
+    float n[4];
+    draw_normals4(resolve_key(a.key), (uint32_t)a.eval.id[s], FHD_STREAM_RFD, 0, n);
+    a.rfd[s] = make_float4(n[0], n[1], n[2], 0.0f);
+  }
+  if (q != 0) return;
   interp_finish(a, s, pre, u1, u2);
 }
 FHD_KERNEL_PAIR((template <int NPTS>), 256, k_interp, InterpArgs, body_interp<NPTS>(a, b))
@@ -1459,29 +990,6 @@ void launch_wca_list(const WcaArgs& a, hipStream_t s) {
 }
 void launch_bonded(const BondArgs& a, hipStream_t s) {
   if (a.np > 0) launch(k_bonded, k_bonded_b, FAM_BONDED, dim3((a.np + kBondThreads - 1) / kBondThreads), kBondThreads, a, s);
-}
-void launch_src_prep(const SpreadArgs& a, hipStream_t s) {
-  int nrec[2] = {0, 0};
-  for (int gi = 0; gi < a.ngroups; ++gi) nrec[gi] = a.grp[gi].nsrc * (a.grp[gi].mode == SRC_RFD ? 2 : 1);
-  SpreadArgs x = a;
-  x.nrec0 = nrec[0];
-  x.nrec_tot = nrec[0] + nrec[1];
-  if (x.nrec_tot <= 0) return;
-  const dim3 grid(nblk(x.nrec_tot, 256));
-  if (a.kernel_points == 4) launch(k_src_prep<4>, k_src_prep_b<4>, FAM_SRC_PREP, grid, 256, x, s);
-  else launch(k_src_prep<3>, k_src_prep_b<3>, FAM_SRC_PREP, grid, 256, x, s);
-}
-void launch_spread(const SpreadArgs& a, hipStream_t s) {
-  const bool fast = a.t.tx == kTileEdge && a.t.ty == kTileEdge && a.t.tz == kTileEdge && a.t.ntx >= 2 &&
-                    a.t.nty >= 2 && a.t.ntz >= 2;
-  const dim3 grid(a.t.n);
-  if (a.kernel_points == 4) {
-    if (fast) launch(k_spread<4, true>, k_spread_b<4, true>, FAM_SPREAD, grid, kSpreadThreads, a, s);
-    else launch(k_spread<4, false>, k_spread_b<4, false>, FAM_SPREAD, grid, kSpreadThreads, a, s);
-  } else {
-    if (fast) launch(k_spread<3, true>, k_spread_b<3, true>, FAM_SPREAD, grid, kSpreadThreads, a, s);
-    else launch(k_spread<3, false>, k_spread_b<3, false>, FAM_SPREAD, grid, kSpreadThreads, a, s);
-  }
 }
 void launch_pvec(const PVecArgs& a, hipStream_t s) {
   if (a.np <= 0) return;

@@ -245,6 +245,20 @@ FHD_DEV int wrapi(int i, int m) {
   return r < 0 ? r + m : r;
 }
 
+// Fold an index within a few boxes of [0, m) into it.  Indices within one box of it (wrapped cells
+// and their stencils, m >= 8) need no loop; narrower boxes (SMALL) do.
+template <bool SMALL>
+FHD_DEV int fold_in(int l, int m) {
+  l += l < 0 ? m : 0;
+  l -= l >= m ? m : 0;
+  if (SMALL) {
+    while (l < 0) l += m;
+    while (l >= m) l -= m;
+  }
+  return l;
+}
+FHD_DEV int fold(int l, int m) { return m < 8 ? fold_in<true>(l, m) : fold_in<false>(l, m); }
+
 // ---------------------------------------------------------------------------------------
 // Grid description passed by value to kernels.
 // ---------------------------------------------------------------------------------------

@@ -645,40 +645,73 @@ FHD_DEV void source_weights(int4 c, float3 frac, SrcWeights& w, bool deriv) {
   }
 }
 
-// Sum over the NPTS x NPTS nodes of one z-row (kz) of a particle's stencil.
+FHD_DEV float4 load4(const float* p) {
+  typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+  const f4u v = *reinterpret_cast<const f4u*>(p);
+  return make_float4(v.x, v.y, v.z, v.w);
+}
+
+// One component's stencil as lane q of a particle's four reads it: its z-row, four x nodes per row in
+// one 16-byte load.  A stencil row that ends at the box's edge or wraps is covered by the last four
+// nodes of the row, with shifted weights, and by the first three (v), which only waves that hold such
+// a particle load.
 template <int NPTS>
-FHD_DEV float interp_row(const float* __restrict__ f, const GridDev& g, const AxisWeights& wx,
-                         const AxisWeights& wy, const AxisWeights& wz, int kz) {
-  const int z = fold(wz.base + kz, g.mz);
-  int xs[NPTS];
+struct Rows {
+  int row[NPTS];  // first node of each row (y nodes)
+  int x;
+  float w[4], v[3];
+  float4 n[NPTS];
+};
+template <int NPTS, bool SMALL>
+FHD_DEV void set_rows(Rows<NPTS>& r, const GridDev& g, const AxisWeights& wx, int by, int bz, int q) {
+  const int plane = g.mx * g.my * fold_in<SMALL>(bz + q, g.mz);
 #pragma unroll
-  for (int kx = 0; kx < NPTS; ++kx) xs[kx] = fold(wx.base + kx, g.mx);
-  // a stencil row that does not wrap around the box and ends inside it is read as one 16-byte
-  // load (global loads need only 4-byte alignment); otherwise node by node
-  const bool vec = wx.base >= 0 && wx.base + 4 <= g.mx;
-  float sy = 0.0f;
+  for (int k = 0; k < NPTS; ++k) r.row[k] = plane + g.mx * fold_in<SMALL>(by + k, g.my);
+  r.x = fold_in<SMALL>(wx.base, g.mx);
 #pragma unroll
-  for (int ky = 0; ky < NPTS; ++ky) {
-    const int y = fold(wy.base + ky, g.my);
-    const float* row = f + (size_t)g.mx * (y + (size_t)g.my * z);
-    float r[4];
-    if (vec) {
-      typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-      const f4u v = *reinterpret_cast<const f4u*>(row + wx.base);
-      r[0] = v.x;
-      r[1] = v.y;
-      r[2] = v.z;
-      r[3] = v.w;
-    } else {
+  for (int k = 0; k < 4; ++k) r.w[k] = k < NPTS ? wx.w[k] : 0.0f;
+  r.v[0] = r.v[1] = r.v[2] = 0.0f;
+  if (!SMALL) {
+    const int sh = r.x - (g.mx - 4);
+    if (__any(sh > 0)) {
+      const float w[7] = {0.0f, 0.0f, 0.0f, wx.w[0], wx.w[1], wx.w[2], NPTS > 3 ? wx.w[3] : 0.0f};
+      const auto at = [&](int k) { return k >= 0 && k < 7 ? w[k] : 0.0f; };
 #pragma unroll
-      for (int kx = 0; kx < NPTS; ++kx) r[kx] = row[xs[kx]];
+      for (int k = 0; k < 4; ++k)
+        r.w[k] = sh <= 0 ? at(k + 3) : sh == 1 ? at(k + 2) : sh == 2 ? at(k + 1) : at(k);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) r.v[k] = sh <= 0 ? 0.0f : sh == 1 ? at(k + 6) : sh == 2 ? at(k + 5) : at(k + 4);
+      r.x = min(r.x, g.mx - 4);
     }
-    float sx = 0.0f;
-#pragma unroll
-    for (int kx = 0; kx < NPTS; ++kx) sx += wx.w[kx] * r[kx];
-    sy += wy.w[ky] * sx;
   }
-  return sy;  // weighted by wz.w[kz] when the rows are combined (static indices, no scratch)
+}
+template <int NPTS, bool SMALL>
+FHD_DEV void load_rows(Rows<NPTS>& r, const GridDev& g, const float* __restrict__ f) {
+#pragma unroll
+  for (int k = 0; k < NPTS; ++k) {
+    const float* row = f + r.row[k];
+    if (SMALL)
+      r.n[k] = make_float4(row[r.x], row[fold_in<true>(r.x + 1, g.mx)], row[fold_in<true>(r.x + 2, g.mx)],
+                           row[fold_in<true>(r.x + 3, g.mx)]);
+    else
+      r.n[k] = load4(row + r.x);
+  }
+}
+// Weighted sum of the rows; `f` again for the wrapped part.
+template <int NPTS, bool SMALL>
+FHD_DEV float sum_rows(const Rows<NPTS>& r, const float* __restrict__ f, const AxisWeights& wy) {
+  float s = 0.0f;
+#pragma unroll
+  for (int k = 0; k < NPTS; ++k)
+    s += wy.w[k] * (r.w[0] * r.n[k].x + r.w[1] * r.n[k].y + r.w[2] * r.n[k].z + r.w[3] * r.n[k].w);
+  if (!SMALL && __any(r.v[0] != 0.0f)) {
+    float4 n[NPTS];
+#pragma unroll
+    for (int k = 0; k < NPTS; ++k) n[k] = load4(f + r.row[k]);
+#pragma unroll
+    for (int k = 0; k < NPTS; ++k) s += wy.w[k] * (r.v[0] * n[k].x + r.v[1] * n[k].y + r.v[2] * n[k].z);
+  }
+  return s;  // weighted by wz.w[q] when the rows are combined (static indices, no scratch)
 }
 
 // Combine the four z-rows held by lanes 4p .. 4p+3 (every lane gets the sum): sum_k wz[k] row_k
@@ -693,41 +726,81 @@ FHD_DEV float combine_rows(float row, const AxisWeights& wz) {
   return ((wz.w[0] * r0 + wz.w[1] * r1) + wz.w[2] * r2) + wz.w[3] * r3;
 }
 
-// Four lanes per particle: lane q sums z-row q of the stencil; the rows are combined by a fixed
-// xor-shuffle tree, then lane 0 applies the position update.
+// J f at one stencil; lane q of the particle's four takes z-row q, every lane gets the full sums.
+// DEEP: the rows of all components are in flight before the first is summed; `under` runs after the
+// first loads are issued.  Otherwise component by component, with a third of the registers.
+template <int NPTS, bool SMALL, bool DEEP, class Under>
+FHD_DEV void interp3(const float* f, const GridDev& g, const SrcWeights& w, int q, float out[3], const Under& under) {
+  Rows<NPTS> r[3];
+  const auto load = [&](int c) {
+    set_rows<NPTS, SMALL>(r[c], g, c == 0 ? w.stg[0] : w.cen[0], (c == 1 ? w.stg[1] : w.cen[1]).base,
+                          (c == 2 ? w.stg[2] : w.cen[2]).base, q);
+    load_rows<NPTS, SMALL>(r[c], g, f + (size_t)c * g.N);
+  };
+  const auto sum = [&](int c) {
+    out[c] = combine_rows(sum_rows<NPTS, SMALL>(r[c], f + (size_t)c * g.N, c == 1 ? w.stg[1] : w.cen[1]),
+                          c == 2 ? w.stg[2] : w.cen[2]);
+  };
+  if (DEEP) {
+    load(0);
+    load(1);
+    load(2);
+    under();
+    sum(0);
+    sum(1);
+    sum(2);
+  } else {
+    load(0);
+    under();
+    sum(0);
+    load(1);
+    sum(1);
+    load(2);
+    sum(2);
+  }
+}
+struct Nothing {
+  FHD_DEV void operator()() const {}
+};
+
+// Four lanes per particle: lane q sums z-row q of the stencil, the rows are combined across the quad,
+// then lane 0 applies the position update.  Below ~32,000 particles the launch is a chain of memory
+// round trips (position, rows, update): with the rows of all three components in flight, no branch
+// around the loads and the update's loads under them, 32^3 with 1,024 particles went from 10.6 to
+// 6.0 us per launch, 64^3 with 4,096 from 8.4 to 6.9 (two fields 16 to 10), 64^3 with 16,384 (4-point)
+// from 11.3 to 8.7.  Above, line traffic bounds it: 128^3 with 65,536 21.6 -> 19.9 us (all rows in
+// flight: 21.8; at 128 VGPRs with spills: 27).
 // Position update of sorted particle s from its interpolated velocities u1 = J f1, u2 = J f2:
 // out = base + a1 u1 + a2 u2 + extra mobility + particle noise (by particle index).
 // Per-particle values the position update needs, loaded when the pass starts so that their
 // latency hides under the gathers: the id, the base position and the neighbour-list reference.
 struct InterpPre {
-  int id;
   int4 bc, rc;
-  float4 bo, ro;
+  float4 bo, ro, F;
+  int slot, lt;  // the updated sorted copy's slot and listed tile
 };
-FHD_DEV InterpPre interp_pre(const InterpArgs& a, int s) {
-  InterpPre p;
-  p.id = a.eval.id[s];
-  p.bc = p.rc = make_int4(0, 0, 0, 0);
-  p.bo = p.ro = make_float4(0.f, 0.f, 0.f, 0.f);
+FHD_DEV void interp_pre(const InterpArgs& a, int s, int id, int lt, InterpPre& p) {
+  p.slot = s;
+  p.lt = lt;
   if (a.out_cell) {
-    p.bc = a.base_cell[p.id];
-    p.bo = a.base_off[p.id];
+    p.bc = a.base_cell[id];
+    p.bo = a.base_off[id];
     if (a.nb.flag) {
-      p.rc = a.nb.ref_cell[p.id];
-      p.ro = a.nb.ref_off[p.id];
+      p.rc = a.nb.ref_cell[id];
+      p.ro = a.nb.ref_off[id];
     }
+    if (a.sk.s_slot) p.slot = a.sk.s_slot[id];
   }
-  return p;
+  if (a.F) p.F = a.F[id];
 }
 
-FHD_DEV void interp_finish(const InterpArgs& a, int s, const InterpPre& pre, const float u1[3], const float u2[3]) {
+FHD_DEV void interp_finish(const InterpArgs& a, int s, int id, const InterpPre& pre, const float u1[3], const float u2[3]) {
   const GridDev& g = a.g;
-  const int id = pre.id;
   float disp[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) disp[k] = a.a1 * u1[k] + a.a2 * u2[k];
   if (a.F) {
-    float4 F = a.F[id];
+    const float4 F = pre.F;
     disp[0] += a.aF * F.x;
     disp[1] += a.aF * F.y;
     disp[2] += a.aF * F.z;
@@ -789,8 +862,7 @@ FHD_DEV void interp_finish(const InterpArgs& a, int s, const InterpPre& pre, con
     if (a.sk.s_cell) {
       // the sorted copy of the new position, in the slot of the set it replaces; the particle
       // stays listed in that slot's tile unless it left the tile's skin
-      const int slot = a.sk.s_slot ? a.sk.s_slot[id] : s;
-      const int lt = (a.sk.s_slot ? a.sk.s_cell[slot] : a.eval.cell[s]).w;
+      const int slot = pre.slot, lt = pre.lt;
       const int wc[3] = {wrapi(bc.x, g.mx), wrapi(bc.y, g.my), wrapi(bc.z, g.mz)};
       const int lto[3] = {(lt % a.t.ntx) * a.t.tx, ((lt / a.t.ntx) % a.t.nty) * a.t.ty,
                           (lt / (a.t.ntx * a.t.nty)) * a.t.tz};
@@ -816,93 +888,74 @@ FHD_DEV void interp_finish(const InterpArgs& a, int s, const InterpPre& pre, con
   }
 }
 
-template <int NPTS>
+template <int NPTS, bool SMALL, bool DEEP>
 FHD_BODY void body_interp(const InterpArgs& a, const Blk& b) {
   const int gid = xcd_item(b.x, b.nx) * blockDim.x + threadIdx.x;
   const int s = gid >> 2, q = gid & 3;
   const GridDev& g = a.g;
-  float u1[3] = {0, 0, 0}, u2[3] = {0, 0, 0};
+  // every lane reads a valid particle and row, so that no load waits for a branch
+  const int se = min(s, a.np - 1), qe = q < NPTS ? q : 0;
+  const int4 c = a.eval.cell[se];
+  const float4 d = a.eval.off[se];
+  const int id = a.eval.id[se];
+  // bookkeeping of the kept sort: the tile starts of the set this pass fills in (stored at the end),
+  // and the flag that the sort before it consumed
+  const bool book = a.sk.s_cell && a.sk.start_dst;
+  const int st0 = book ? a.sk.start_src[min(gid, a.t.n)] : 0;
   SrcWeights w;
-  const bool act = s < a.np && q < NPTS;
+  source_weights<NPTS>(c, make_float3(d.x * g.idx, d.y * g.idy, d.z * g.idz), w, false);
   InterpPre pre;
-  if (s < a.np) {
-    const int4 c = a.eval.cell[s];
-    const float4 d = a.eval.off[s];
-    if (q == 0) pre = interp_pre(a, s);
-    source_weights<NPTS>(c, make_float3(d.x * g.idx, d.y * g.idy, d.z * g.idz), w, false);
-  }
-#pragma unroll
-  for (int comp = 0; comp < 3; ++comp) {
-    const AxisWeights& wx = comp == 0 ? w.stg[0] : w.cen[0];
-    const AxisWeights& wy = comp == 1 ? w.stg[1] : w.cen[1];
-    const AxisWeights& wz = comp == 2 ? w.stg[2] : w.cen[2];
-    float r1 = 0.0f, r2 = 0.0f;
-    if (act && a.f1) r1 = interp_row<NPTS>(a.f1 + (size_t)comp * g.N, g, wx, wy, wz, q);
-    if (act && a.f2) r2 = interp_row<NPTS>(a.f2 + (size_t)comp * g.N, g, wx, wy, wz, q);
-    u1[comp] = combine_rows(r1, wz);
-    u2[comp] = a.f2 ? combine_rows(r2, wz) : 0.0f;
-  }
-  if (a.sk.s_cell) {
-    // bookkeeping of the kept sort: the tile starts of the set this pass fills in, and the flag
-    // that the sort before this pass consumed
+  float u1[3], u2[3] = {0.0f, 0.0f, 0.0f};
+  interp3<NPTS, SMALL, DEEP>(a.f1, g, w, qe, u1, [&] { interp_pre(a, se, id, c.w, pre); });
+  const auto listed_tile = [&] {
+    if (a.sk.s_slot) pre.lt = a.sk.s_cell[pre.slot].w;
+  };
+  if (a.f2) interp3<NPTS, SMALL, DEEP>(a.f2, g, w, qe, u2, listed_tile);
+  else listed_tile();
+  if (book) {
+    if (gid <= a.t.n) a.sk.start_dst[gid] = st0;
     const int nth = b.nx * blockDim.x;
-    if (a.sk.start_dst)
-      for (int k = gid; k <= a.t.n; k += nth) a.sk.start_dst[k] = a.sk.start_src[k];
-    if (gid == 0 && a.sk.clear_flag) *a.sk.clear_flag = 0;
+    for (int k = gid + nth; k <= a.t.n; k += nth) a.sk.start_dst[k] = a.sk.start_src[k];
   }
+  if (a.sk.s_cell && gid == 0 && a.sk.clear_flag) *a.sk.clear_flag = 0;
   if (s >= a.np) return;
   if (q == 1 && a.rfd) {
     // an idle lane draws the normals that displace this particle's RFD sources
     float n[4];
-    draw_normals4(resolve_key(a.key), (uint32_t)a.eval.id[s], FHD_STREAM_RFD, 0, n);
+    draw_normals4(resolve_key(a.key), (uint32_t)id, FHD_STREAM_RFD, 0, n);
     a.rfd[s] = make_float4(n[0], n[1], n[2], 0.0f);
   }
   if (q != 0) return;
-  interp_finish(a, s, pre, u1, u2);
+  interp_finish(a, s, id, pre, u1, u2);
 }
-FHD_KERNEL_PAIR((template <int NPTS>), 256, k_interp, InterpArgs, body_interp<NPTS>(a, b))
+FHD_KERNEL_PAIR((template <int NPTS, bool SMALL, bool DEEP>), 256, k_interp, InterpArgs,
+                body_interp<NPTS, SMALL, DEEP>(a, b))
 
 
 // ---------------- inertial coupling with excess mass ----------------
-// Interpolation of the three components of f at one stencil (weights w): every lane of the
-// particle's four gets the full sums (combine_rows broadcasts).
-template <int NPTS>
-FHD_DEV void interp3(const float* f, const GridDev& g, const SrcWeights& w, bool act, int q, float out[3]) {
-#pragma unroll
-  for (int comp = 0; comp < 3; ++comp) {
-    const AxisWeights& wx = comp == 0 ? w.stg[0] : w.cen[0];
-    const AxisWeights& wy = comp == 1 ? w.stg[1] : w.cen[1];
-    const AxisWeights& wz = comp == 2 ? w.stg[2] : w.cen[2];
-    float r = 0.0f;
-    if (act && f) r = interp_row<NPTS>(f + (size_t)comp * g.N, g, wx, wy, wz, q);
-    out[comp] = combine_rows(r, wz);
-  }
-}
-
-template <int NPTS>
-FHD_DEV void weights_at(const GridDev& g, int4 c, float4 d, SrcWeights& w) {
-  const int4 cw = make_int4(wrapi(c.x, g.mx), wrapi(c.y, g.my), wrapi(c.z, g.mz), 0);
-  source_weights<NPTS>(cw, make_float3(d.x * g.idx, d.y * g.idy, d.z * g.idz), w, false);
+// J f at position (c, d), cells wrapped here.
+template <int NPTS, bool SMALL>
+FHD_DEV void interp_at(const float* f, const GridDev& g, int4 c, float4 d, int q, float out[3]) {
+  out[0] = out[1] = out[2] = 0.0f;
+  if (!f) return;
+  SrcWeights w;
+  source_weights<NPTS>(make_int4(wrapi(c.x, g.mx), wrapi(c.y, g.my), wrapi(c.z, g.mz), 0),
+                       make_float3(d.x * g.idx, d.y * g.idy, d.z * g.idz), w, false);
+  interp3<NPTS, SMALL, true>(f, g, w, q, out, Nothing());
 }
 
 FHD_DEV float4 f4_or_zero(const float4* p, int i) { return p ? p[i] : make_float4(0.f, 0.f, 0.f, 0.f); }
 
-template <int NPTS>
+template <int NPTS, bool SMALL>
 FHD_BODY void body_pvec(const PVecArgs& a, const Blk& b) {
   const int gid = xcd_item(b.x, b.nx) * blockDim.x + threadIdx.x;
   const int s = gid >> 2, q = gid & 3;
   const GridDev& g = a.g;
-  const bool act = s < a.np && q < NPTS;
-  SrcWeights w, w0;
-  int id = 0;
-  if (s < a.np) {
-    id = a.eval.id[s];
-    weights_at<NPTS>(g, a.eval.cell[s], a.eval.off[s], w);
-    if (a.f0) weights_at<NPTS>(g, a.cell0[id], a.off0[id], w0);
-  }
+  const int se = min(s, a.np - 1), qe = q < NPTS ? q : 0;
+  const int id = a.eval.id[se];
   float j1[3], j0[3] = {0.f, 0.f, 0.f};
-  interp3<NPTS>(a.f1, g, w, act, q, j1);
-  if (a.f0) interp3<NPTS>(a.f0, g, w0, act, q, j0);
+  interp_at<NPTS, SMALL>(a.f1, g, a.eval.cell[se], a.eval.off[se], qe, j1);
+  if (a.f0) interp_at<NPTS, SMALL>(a.f0, g, a.cell0[id], a.off0[id], qe, j0);
   if (s >= a.np || q != 0) return;
   const float4 A = f4_or_zero(a.A, id), B = f4_or_zero(a.B, id);
   a.out[id] = make_float4(a.a * A.x + a.b * B.x + a.c1 * j1[0] + a.c0 * j0[0],
@@ -914,38 +967,31 @@ FHD_BODY void body_pvec(const PVecArgs& a, const Blk& b) {
                              a.a2 * A2.z + a.b2 * B2.z + a.d1 * j1[2], 0.0f);
   }
 }
-FHD_KERNEL_PAIR((template <int NPTS>), 256, k_pvec, PVecArgs, body_pvec<NPTS>(a, b))
+FHD_KERNEL_PAIR((template <int NPTS, bool SMALL>), 256, k_pvec, PVecArgs, body_pvec<NPTS, SMALL>(a, b))
 
-template <int NPTS>
+template <int NPTS, bool SMALL>
 FHD_BODY void body_lag2(const Lag2Args& a, const Blk& b) {
   const int gid = xcd_item(b.x, b.nx) * blockDim.x + threadIdx.x;
   const int s = gid >> 2, q = gid & 3;
   const GridDev& g = a.g;
-  const bool act = s < a.np && q < NPTS;
-  SrcWeights w;
-  int id = 0;
-  if (s < a.np) {
-    id = a.eval.id[s];
-    weights_at<NPTS>(g, a.eval.cell[s], a.eval.off[s], w);
-  }
-  float uh[3];
-  interp3<NPTS>(a.fv, g, w, act, q, uh);
+  const int se = min(s, a.np - 1), qe = q < NPTS ? q : 0;
+  const int id = a.eval.id[se];
+  float uh[3], l[3];
+  interp_at<NPTS, SMALL>(a.fv, g, a.eval.cell[se], a.eval.off[se], qe, uh);
   // q' = q^n + hdt J(q^{n+1/2}) v_half, as (cell, offset)
-  if (s < a.np) {
+  {
     int4 c = a.cell0[id];
     const float4 o = a.off0[id];
     float ox = o.x + a.hdt * uh[0], oy = o.y + a.hdt * uh[1], oz = o.z + a.hdt * uh[2];
     renorm_axis(c.x, ox, g.dx, g.idx);
     renorm_axis(c.y, oy, g.dy, g.idy);
     renorm_axis(c.z, oz, g.dz, g.idz);
-    weights_at<NPTS>(g, c, make_float4(ox, oy, oz, 0.0f), w);
+    interp_at<NPTS, SMALL>(a.fl, g, c, make_float4(ox, oy, oz, 0.0f), qe, l);
   }
-  float l[3];
-  interp3<NPTS>(a.fl, g, w, act, q, l);
   if (s >= a.np || q != 0) return;
   a.out[id] = make_float4(l[0], l[1], l[2], 0.0f);
 }
-FHD_KERNEL_PAIR((template <int NPTS>), 256, k_lag2, Lag2Args, body_lag2<NPTS>(a, b))
+FHD_KERNEL_PAIR((template <int NPTS, bool SMALL>), 256, k_lag2, Lag2Args, body_lag2<NPTS, SMALL>(a, b))
 
 // ------------------------------- launchers -------------------------------
 static inline int nblk(int n, int b) { return (n + b - 1) / b; }
@@ -991,23 +1037,37 @@ void launch_wca_list(const WcaArgs& a, hipStream_t s) {
 void launch_bonded(const BondArgs& a, hipStream_t s) {
   if (a.np > 0) launch(k_bonded, k_bonded_b, FAM_BONDED, dim3((a.np + kBondThreads - 1) / kBondThreads), kBondThreads, a, s);
 }
+// The kernel of the stencil's points and, for boxes narrower than eight cells, the looping fold; V:
+// further template arguments.
+#define FHD_LAUNCH_STENCIL(kern, fam, grid, a, s, ...)                                                                 \
+  do {                                                                                                                 \
+    const bool small = (a).g.mx < 8 || (a).g.my < 8 || (a).g.mz < 8;                                                   \
+    if ((a).kernel_points == 4) {                                                                                      \
+      if (small) launch(kern<4, true __VA_ARGS__>, kern##_b<4, true __VA_ARGS__>, fam, grid, 256, a, s);               \
+      else launch(kern<4, false __VA_ARGS__>, kern##_b<4, false __VA_ARGS__>, fam, grid, 256, a, s);                   \
+    } else {                                                                                                           \
+      if (small) launch(kern<3, true __VA_ARGS__>, kern##_b<3, true __VA_ARGS__>, fam, grid, 256, a, s);               \
+      else launch(kern<3, false __VA_ARGS__>, kern##_b<3, false __VA_ARGS__>, fam, grid, 256, a, s);                   \
+    }                                                                                                                  \
+  } while (0)
 void launch_pvec(const PVecArgs& a, hipStream_t s) {
   if (a.np <= 0) return;
   const dim3 grid(nblk(4 * a.np, 256));
-  if (a.kernel_points == 4) launch(k_pvec<4>, k_pvec_b<4>, FAM_PVEC, grid, 256, a, s);
-  else launch(k_pvec<3>, k_pvec_b<3>, FAM_PVEC, grid, 256, a, s);
+  FHD_LAUNCH_STENCIL(k_pvec, FAM_PVEC, grid, a, s);
 }
 void launch_lag2(const Lag2Args& a, hipStream_t s) {
   if (a.np <= 0) return;
   const dim3 grid(nblk(4 * a.np, 256));
-  if (a.kernel_points == 4) launch(k_lag2<4>, k_lag2_b<4>, FAM_LAG2, grid, 256, a, s);
-  else launch(k_lag2<3>, k_lag2_b<3>, FAM_LAG2, grid, 256, a, s);
+  FHD_LAUNCH_STENCIL(k_lag2, FAM_LAG2, grid, a, s);
 }
+constexpr int kDeepParticles = 32768;
 void launch_interp(const InterpArgs& a, hipStream_t s) {
   if (a.np <= 0) return;
   const dim3 grid(nblk(4 * a.np, 256));
-  if (a.kernel_points == 4) launch(k_interp<4>, k_interp_b<4>, FAM_INTERP, grid, 256, a, s);
-  else launch(k_interp<3>, k_interp_b<3>, FAM_INTERP, grid, 256, a, s);
+  // Few particles: the launch waits for memory, and all rows in flight at once take a third of the
+  // round trips.  Many: the gathers' line traffic bounds it and the registers cost more waves.
+  if (a.np <= kDeepParticles) FHD_LAUNCH_STENCIL(k_interp, FAM_INTERP, grid, a, s, , true);
+  else FHD_LAUNCH_STENCIL(k_interp, FAM_INTERP, grid, a, s, , false);
 }
 
 }  // namespace fhd

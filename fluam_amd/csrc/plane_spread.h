@@ -37,17 +37,6 @@ namespace fhd {
 constexpr int kListCap = 6144;     // hits listed at once (also the sources scanned per chunk when more)
 constexpr int kOneLimb = 255;      // most sources per node for a single 32-bit sum
 
-// Fold an index within a few boxes of [0, m) into it.
-FHD_DEV int fold(int l, int m) {
-  if (l < 0) l += m;
-  else if (l >= m) l -= m;
-  if (m < 8) {
-    while (l < 0) l += m;
-    while (l >= m) l -= m;
-  }
-  return l;
-}
-
 // The key of a sorted slot: bits 0-8 its half cell along z (wrapped cell, sign of the offset), bit
 // 9 set when a displacement below `margin` may change it, bits 16 up its block of 4 x 4 columns.
 FHD_DEV unsigned plane_key(const GridDev& g, int cx, int cy, int cz, float dz, float margin) {

@@ -36,6 +36,9 @@ def rel(a, b):
     (ST, (72, 108, 8), 700, 3, {}),
     (ST, (128, 72, 8), 700, 4, {}),
     (QNB, (36, 48, 8), 400, 3, {"mass": 2.0}),
+    # more particles than the interpolation keeps all rows of in flight (32768)
+    (ST, (32, 16, 16), 33000, 4, {}),
+    (QNB, (24, 24, 16), 33000, 3, {}),
 ])
 def test_plane_spread_matches_oracle(scheme, cells, n, kernel, kw):
     print(f"[gpu-case] plane spread scheme={scheme} cells={cells} np={n} k={kernel} {kw}", flush=True)

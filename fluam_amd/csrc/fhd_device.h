@@ -24,20 +24,26 @@ FHD_DEV int fast_div(int n, uint32_t magic) { return magic ? (int)__umulhi((uint
 // average, and each transform multiplies by them on the way there and back.
 inline float2 unit_pair(double c, double s) {
   const float c0 = (float)c, s0 = (float)s;
-  const double uc = ldexp(1.0, ilogb(fabs(c) > 1e-9 ? c : 1e-9) - 23), us = ldexp(1.0, ilogb(fabs(s) > 1e-9 ? s : 1e-9) - 23);
   float2 best = make_float2(c0, s0);
   if (fabs(c) < 1e-9 || fabs(s) < 1e-9) return best;
+  // one ulp up or down of the larger, a few of the smaller (its steps are finer)
+  const bool cl = fabs(c) > fabs(s);
+  const float big = cl ? c0 : s0, small = cl ? s0 : c0;
+  const double eb = cl ? c : s, es = cl ? s : c;
   double least = 1.0;
-  for (int i = -4; i <= 4; ++i)
-    for (int j = -4; j <= 4; ++j) {
-      const float x = (float)(c0 + i * uc), y = (float)(s0 + j * us);
-      const double off = sqrt((x - c) * (x - c) + (y - s) * (y - s));
+  for (int i = -1; i <= 1; ++i) {
+    const float x = i == 0 ? big : nextafterf(big, i > 0 ? 2.0f : -2.0f);
+    float y = small;
+    for (int j = 0; j < 4; ++j) y = nextafterf(y, -2.0f);
+    for (int j = -4; j <= 4; ++j, y = nextafterf(y, 2.0f)) {
+      const double off = fabs(x - eb) + fabs(y - es);
       const double cost = fabs((double)x * x + (double)y * y - 1.0) + 0.1 * off;
-      if (off <= 6e-8 && cost < least) {
+      if (off <= 8e-8 && cost < least) {
         least = cost;
-        best = make_float2(x, y);
+        best = cl ? make_float2(x, y) : make_float2(y, x);
       }
     }
+  }
   return best;
 }
 

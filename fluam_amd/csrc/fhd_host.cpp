@@ -175,7 +175,7 @@ struct fhd_ctx {
   FftArgs fa;
   double dx, dy, dz, dV;
   // fields (3N each)
-  float *v = nullptr, *v2 = nullptr, *W = nullptr, *SF = nullptr, *adv[2] = {nullptr, nullptr};
+  float *v = nullptr, *v2 = nullptr, *W = nullptr, *B = nullptr, *adv[2] = {nullptr, nullptr};
   float* div = nullptr;
   float2* spec = nullptr;
   // Fourier tables
@@ -232,8 +232,8 @@ struct fhd_ctx {
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   int gperiod = 0, gphase = 0;
   bool own_stream = true;
-  int zchunk = 8;                        // W kernel: z planes per workgroup (schedule)
-  int zchunk_b = 8;                      // the same inside batched dispatches
+  int zchunk = 4;                        // W kernel: z planes per workgroup (schedule)
+  int zchunk_b = 4;                      // the same inside batched dispatches
   hipEvent_t done_ev = nullptr;          // fhd_record / fhd_query
   bool done_checked = false;             // error word read since the last fhd_record completed
   bool dev_error = false;                // fhd_query found a device error flag
@@ -374,7 +374,7 @@ void build_tables(fhd_ctx* c) {
 }
 
 void free_ctx(fhd_ctx* c) {
-  void* ptrs[] = {c->v, c->v2, c->W, c->SF, c->adv[0], c->adv[1], c->div, c->spec, c->twx, c->twy, c->twz,
+  void* ptrs[] = {c->v, c->v2, c->W, c->B, c->adv[0], c->adv[1], c->div, c->spec, c->twx, c->twy, c->twz,
                   c->ex, c->ey, c->ez, c->gx, c->gy, c->gz, c->cell[0], c->cell[1], c->off[0], c->off[1],
                   c->F[0], c->F[1], c->u, c->count, c->slot, c->tmp, c->start[0], c->start[1], c->sid[0],
                   c->sid[1], c->scell[0], c->scell[1], c->soff[0], c->soff[1], c->errd, c->key[0], c->key[1], c->rfd,
@@ -453,10 +453,18 @@ FluidWArgs base_w(fhd_ctx* c) {
 }
 
 // ---------------- schedule autotuner ----------------
-// The z-pass column tile (4, 8 or 16 columns) and the W kernel's z-chunk (4, 8 or 16 planes)
-// are timed once per grid shape on the first context of that shape and cached for the
-// process: a replica's schedule depends on its shape only, never on what else runs beside it,
-// and neither choice changes any result bit.
+// The z-pass column tile and the W kernel's chunk follow the grid's size; the radix plans of 48-,
+// 96- and 128-point columns and of 96 x 96 and 128 x 128 planes are timed once per grid shape on the
+// first context of that shape and cached for the process: a replica's schedule depends on its shape
+// only, never on what else runs beside it.
+
+// Columns of a z-pass workgroup: as many as leave the chip two workgroups per CU (fewer, longer rows
+// of a tile cost more than the columns save: per launch with 2, 4, 8, 16 columns 4.9, 5.1, 6.0, 7.5 us
+// at 32^3, 7.3, 6.4, 6.5, 8.0 at 64^3, 41, 31.5, 28.0, 28.0 at 128^3).
+int z_tile(int mx, int my) {
+  const int P = mx / 2 + 1;
+  return P / 8 * my >= 512 ? 8 : P / 4 * my >= 256 ? 4 : 2;
+}
 struct Sched {
   int btile, zchunk, zchunk_b, plan_xy, plan_xy_inv, plan_zs;
 };
@@ -488,20 +496,22 @@ float time_launches(fhd_ctx* c, const std::function<void()>& f, int reps) {
 void apply_schedule(fhd_ctx* c) {
   // keyed by shape and scheme: the W kernel is timed in the form the scheme launches
   const std::array<int, 4> key = {c->p.mx, c->p.my, c->p.mz, c->p.scheme};
-  const char* env = getenv("FHD_AUTOTUNE");  // 0: fixed defaults (8 columns, 8 planes)
+  const char* env = getenv("FHD_AUTOTUNE");  // 0: default radix plans
   const bool tune = !(env && env[0] == '0');
   std::lock_guard<std::mutex> lock(g_sched_mu);
   auto it = g_sched.find(key);
-  Sched sc = {8, 8, 8, 0, 0, 0};
+  // two planes per W workgroup: per launch with 1, 2, 4 planes 5.3, 5.2, 6.8 us at 32^3, 12.4, 7.5, 7.3 at
+  // 64^3, 13.9, 9.4, 11.9 at 96 x 48 x 64
+  Sched sc = {z_tile(c->p.mx, c->p.my), 2, 2, 0, 0, 0};
   if (it != g_sched.end()) {
     sc = it->second;
   } else if (tune) {
     // scratch runs on the context's own buffers before its state exists (contents irrelevant)
     float best = 1e30f;
     const bool stokes = c->p.scheme == FHD_SCHEME_STOKES_LIMIT;
-    // z pass: column tile and, for 48-, 96- and 128-point columns, the radix plan (128: 16 8,
-    // 8 16 or 4 4 8; 96: 16 2 3, 8 4 3 or 3 8 4; 48: 16 3, 3 16 or 4 4 3), timed in the form
-    // the scheme launches (the Stokes pass draws its stochastic stress)
+    // z pass of 48-, 96- and 128-point columns: the radix plan (128: 16 8, 8 16 or 4 4 8; 96: 16 2 3,
+    // 8 4 3 or 3 8 4; 48: 16 3, 3 16 or 4 4 3), timed in the form the scheme launches (the Stokes
+    // pass draws its stochastic stress)
     FftArgs za = c->fa;
     if (stokes) {
       za.stokes = 1;
@@ -509,15 +519,14 @@ void apply_schedule(fhd_ctx* c) {
       za.kn_f1 = za.kn_f4 = 1.0f;
       za.key = make_key(c);
     }
+    za.btile = sc.btile;
     const int mzp = c->p.mz;
-    const int nzp = (mzp == 48 || mzp == 96 || mzp == 128) ? 3 : 1;
-    for (int pz = 0; pz < nzp; ++pz)
-      for (int bt : {2, 4, 8, 16}) {  // 2: more column workgroups on small grids
-        za.btile = bt;
-        za.plan_zs = pz;
-        const float t = time_launches(c, [&] { launch_fft_z_solve(za, c->spec, c->s); }, 4);
-        if (t < best) { best = t; sc.btile = bt; sc.plan_zs = pz; }
-      }
+    const int nzp = (mzp == 48 || mzp == 96 || mzp == 128) ? 3 : 0;
+    for (int pz = 0; pz < nzp; ++pz) {
+      za.plan_zs = pz;
+      const float t = time_launches(c, [&] { launch_fft_z_solve(za, c->spec, c->s); }, 4);
+      if (t < best) { best = t; sc.plan_zs = pz; }
+    }
     c->fa.plan_zs = sc.plan_zs;
     // xy passes of 96 x 96 and 128 x 128 planes: the radix plans of the x and y transforms
     // (three each) of the LDS-stage kernels, and for 128 x 128 the register-transform kernels
@@ -536,27 +545,6 @@ void apply_schedule(fhd_ctx* c) {
       }
       c->fa.plan_xy = sc.plan_xy;
       c->fa.plan_xy_inv = sc.plan_xy_inv;
-    }
-    // W kernel (incompressible and QNB; the Stokes step has none): 2 planes per workgroup fill
-    // the chip on small grids (64^3: 512 workgroups) when the context launches alone; a
-    // batched dispatch already holds many contexts' workgroups, where the redundant halo planes
-    // of short chunks cost more, so it keeps the best of 4-16
-    best = 1e30f;
-    float best_b = 1e30f;
-    for (int zc : {2, 4, 8, 16}) {
-      if (stokes) break;
-      c->zchunk = zc;
-      FluidWArgs w = base_w(c);
-      w.noise = 1;
-      w.f1 = w.f4 = 1.0f;
-      w.v = c->v;
-      w.vadv = c->v;
-      w.lap_coef = 1.0f;
-      w.adv_coef = 1.0f;
-      w.trace_free = 1;
-      const float t = time_launches(c, [&] { launch_fluid_w(w, c->s); }, 4);
-      if (t < best) { best = t; sc.zchunk = zc; }
-      if (zc >= 4 && t < best_b) { best_b = t; sc.zchunk_b = zc; }
     }
     g_sched[key] = sc;
   }
@@ -797,11 +785,17 @@ void step_incompressible(fhd_ctx* c) {
   w.f1 = (float)sqrt(4.0 * p.temperature * p.shearviscosity * p.dt / (dV * rho * rho));
   w.f4 = (float)sqrt(2.0 * p.temperature * p.shearviscosity * p.dt / (dV * rho * rho));
   const float cn = (float)(0.5 * p.dt * p.shearviscosity / rho);
+  w.base_out = c->B;
   launch_fluid_w(w, c->s);
   mark(c, "fluid_w");
   fft_forward(c, c->W);
   fft_solve(c, 0, cn);
   fft_inverse(c, c->v2, c->v, 0.5f, 0.5f);  // v* = (v~ + v^n) / 2
+  // the second solve differs in its advection only
+  w.v = nullptr;
+  w.noise = 0;
+  w.base_out = nullptr;
+  w.base_in = c->B;
   w.vadv = c->v2;
   launch_fluid_w(w, c->s);
   mark(c, "fluid_w");
@@ -1771,7 +1765,7 @@ fhd_ctx* fhd_create(const fhd_params* pin) {
     c->v = dalloc<float>(N3);
     c->v2 = dalloc<float>(N3);
     c->W = dalloc<float>(N3);
-    c->SF = dalloc<float>(N3);
+    if (p.scheme == FHD_SCHEME_INCOMPRESSIBLE) c->B = dalloc<float>(N3);  // v + 1/2 dt nu L v + noise
     c->div = dalloc<float>(g.N);
     c->spec = dalloc<float2>(3 * (size_t)p.mz * p.my * g.P);
     if (p.scheme == FHD_SCHEME_QUASI_NEUTRALLY_BUOYANT) {
@@ -1801,7 +1795,6 @@ fhd_ctx* fhd_create(const fhd_params* pin) {
     c->step = p.initial_step;
     HIPCHK(hipMemcpy(c->v, v0.data(), N3 * sizeof(float), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(c->v2, 0, N3 * sizeof(float)));
-    HIPCHK(hipMemset(c->SF, 0, N3 * sizeof(float)));
     apply_schedule(c);
     c->np = p.np;
     if (c->np > 0) {

@@ -58,17 +58,19 @@ struct FluidWArgs {
   GridDev g;
   const float* v;          // W += v + lap_coef * L v (nullptr: term off)
   float lap_coef;
-  const float* vadv;       // W += adv_coef * A(vadv) (nullptr: off)
+  const float* vadv;       // W += adv_coef * A(vadv)
   float adv_coef;
   const float* adv_prev;   // W += adv_prev_coef * adv_prev (nullptr: off)
   float adv_prev_coef;
   float* adv_store;        // stores A(vadv) when non-null
-  int noise;               // 0 none, 1 Sigma_1, 2 Sigma_1 + Sigma_2
+  const float* base_in;    // W += base_in: the terms of an earlier pass (nullptr: none)
+  float* base_out;         // stores v + lap_coef L v + noise when non-null
+  int noise;               // 0 none, 1 Sigma_1
   int trace_free;
   float f1, f4;            // diagonal / off-diagonal noise prefactors
   Key key;
   float* W;
-  int zchunk;           // z planes per workgroup
+  int zchunk;           // z planes per workgroup (1, 2 or 4; others round down to these)
   int zchunk_b;         // the same when the launch is recorded into a batched dispatch
 };
 

@@ -1,11 +1,14 @@
 // fluid.hip -- the staggered-grid right-hand side W of each solve (fluam's kernelConstructW
 // family) with the stochastic stress generated in registers.
 //
-// One workgroup owns a 16 x 16 column of cells and marches up a chunk of z-planes.  The 6
-// stress normals of every cell of plane z+2 (plus the one-cell ring the divergence needs) are
-// drawn from the counter-based generator into an LDS ring of four planes while plane z's
-// stencil reads planes z-1..z+1, so each normal is drawn ~1.25 times instead of once per
-// neighbour that reads it.
+// One workgroup owns a 16 x 16 column of cells and ZC planes of it (ZC = 1, 2 or 4), one cell per
+// lane.  The velocities of its stencil are loaded first; under those loads the stress normals of the
+// ZC + 2 planes (with the one-cell ring the divergence needs) are drawn into LDS, spread over all
+// lanes; one barrier; then every lane takes its stencil.  Bound by the generator's instructions: at
+// ZC = 4 each normal is drawn 1.9 times.  A column of 256 lanes that marched up the planes, drawing
+// one plane per barrier with 62% of its lanes, took 10.1 us at 32^3 and 14.0 us at 64^3 per launch.
+// The second solve of an incompressible step has the same noise, so the first pass keeps the terms
+// both share and the second only adds its advection.
 //
 // Restates: kernelConstructW_1/_2 (src/kernelConstructW.cu:32-521), the QNB variants
 // (src/kernelConstructWQuasiNeutrallyBuoyant.cu:26-705,1366-2025) and
@@ -19,155 +22,144 @@ constexpr int TX = 16, TY = 16;
 constexpr int PX = TX + 2, PY = TY + 2;
 constexpr int PLANE = PX * PY;
 
-// stress slot components: 0 sXX, 1 XY, 2 XZ, 3 sYY, 4 YZ, 5 sZZ
-FHD_DEV void gen_plane(const FluidWArgs& a, const Key& key, float* slot, int x0, int y0, int zz) {
+// Draws the stress of items [0, ntot) of the planes zs - 1 .. zs + ZC: per plane the tile's cells and
+// its ring without corners.  Stress components: 0 sXX, 1 XY, 2 XZ, 3 sYY, 4 YZ, 5 sZZ.
+template <int ZC>
+FHD_DEV void draw_planes(const FluidWArgs& a, const Key& key, float (*nbuf)[6 * PLANE], int x0, int y0, int zs) {
   const GridDev& g = a.g;
-  // zz in [-1, mz], x0 + lx in [-1, mx], y0 + ly in [-1, my]: one conditional wrap each
-  const int z = zz < 0 ? zz + g.mz : (zz >= g.mz ? zz - g.mz : zz);
-  const int nown = TX * TY, ntot = nown + 2 * TX + 2 * TY;
-  for (int e = threadIdx.x; e < ntot; e += blockDim.x) {
+  constexpr int NOWN = TX * TY, NPL = NOWN + 2 * TX + 2 * TY;
+  for (int e = threadIdx.x; e < (ZC + 2) * NPL; e += 256 * ZC) {
+    const int pl = e / NPL, i = e - pl * NPL;
     int lx, ly;
-    if (e < nown) { lx = e % TX; ly = e / TX; }
+    if (i < NOWN) { lx = i % TX; ly = i / TX; }
     else {
-      int r = e - nown;
+      const int r = i - NOWN;
       if (r < TY) { lx = -1; ly = r; }
       else if (r < 2 * TY) { lx = TX; ly = r - TY; }
       else if (r < 2 * TY + TX) { lx = r - 2 * TY; ly = -1; }
       else { lx = r - 2 * TY - TX; ly = TY; }
     }
-    int x = x0 + lx, y = y0 + ly;
+    // one conditional wrap each, except in the planes above the box (not used) of a short last chunk
+    int x = x0 + lx, y = y0 + ly, z = zs - 1 + pl;
     x = x < 0 ? x + g.mx : (x >= g.mx ? x - g.mx : x);
     y = y < 0 ? y + g.my : (y >= g.my ? y - g.my : y);
-    uint32_t cell = (uint32_t)(x + g.mx * (y + g.my * z));
-    float n[12];
-    draw_normals4(key, cell, FHD_STREAM_FLUID, 0, &n[0]);
-    draw_normals4(key, cell, FHD_STREAM_FLUID, 1, &n[4]);
-    float s[6];
-    if (a.noise == 2) {
-      draw_normals4(key, cell, FHD_STREAM_FLUID, 2, &n[8]);
-#pragma unroll
-      for (int c = 0; c < 6; ++c) s[c] = n[c] + n[6 + c];
-    } else {
-#pragma unroll
-      for (int c = 0; c < 6; ++c) s[c] = n[c];
-    }
+    z = z < 0 ? z + g.mz : (z >= g.mz ? z - g.mz : z);
+    const uint32_t cell = (uint32_t)(x + g.mx * (y + g.my * z));
+    float s[8];
+    draw_normals4(key, cell, FHD_STREAM_FLUID, 0, &s[0]);
+    draw_normals4(key, cell, FHD_STREAM_FLUID, 1, &s[4]);
     if (a.trace_free) {
-      float tr = (s[0] + s[3] + s[5]) * (1.0f / 3.0f);
+      const float tr = (s[0] + s[3] + s[5]) * (1.0f / 3.0f);
       s[0] -= tr;
       s[3] -= tr;
       s[5] -= tr;
     }
-    int p = (lx + 1) + PX * (ly + 1);
+    const int p = (lx + 1) + PX * (ly + 1);
 #pragma unroll
-    for (int c = 0; c < 6; ++c) slot[c * PLANE + p] = s[c];
+    for (int c = 0; c < 6; ++c) nbuf[pl][c * PLANE + p] = s[c];
   }
 }
 
+// The seven values of a component around a cell: itself, x - 1, x + 1, y - 1, y + 1, z - 1, z + 1.
+FHD_DEV void load7(const float* f, const int n[7], float v[7]) {
+#pragma unroll
+  for (int k = 0; k < 7; ++k) v[k] = f[n[k]];
+}
+
+template <int ZC>
 FHD_BODY void body_fluid_w(const FluidWArgs& a, const Blk& b) {
-  // ring of four noise planes: while the stencil of plane z reads planes z - 1, z and z + 1,
-  // plane z + 2 is drawn into the fourth slot, so one barrier per plane suffices
-  constexpr int NR = 4;
-  __shared__ float nbuf[NR][6 * PLANE];
+  __shared__ float nbuf[ZC + 2][6 * PLANE];
   const GridDev& g = a.g;
   const Key key = resolve_key(a.key);
-  const int x0 = b.x * TX, y0 = b.y * TY;
-  const int zs = b.z * a.zchunk;
-  const int ze = min(zs + a.zchunk, g.mz);
-  const int lx = threadIdx.x % TX, ly = threadIdx.x / TX;
-  const int x = x0 + lx, y = y0 + ly;
-  const bool own = (x < g.mx) && (y < g.my);
+  const int x0 = b.x * TX, y0 = b.y * TY, zs = b.z * ZC;
+  const int lx = threadIdx.x % TX, ly = threadIdx.x / TX % TY, lz = threadIdx.x / (TX * TY);
+  const int x = x0 + lx, y = y0 + ly, z = zs + lz;
+  const bool own = x < g.mx && y < g.my && z < g.mz;
   const int N = g.N;
-  if (a.noise) {
-    gen_plane(a, key, nbuf[(zs - 1 + NR) % NR], x0, y0, zs - 1);
-    gen_plane(a, key, nbuf[zs % NR], x0, y0, zs);
-    gen_plane(a, key, nbuf[(zs + 1) % NR], x0, y0, zs + 1);
-  }
-  __syncthreads();
-  const int xm = wrapi(x - 1, g.mx), xp = wrapi(x + 1, g.mx);
-  const int ym = wrapi(y - 1, g.my), yp = wrapi(y + 1, g.my);
-  for (int z = zs; z < ze; ++z) {
-    if (a.noise && z + 2 <= ze) gen_plane(a, key, nbuf[(z + 2) % NR], x0, y0, z + 2);
-    if (own) {
-      const int zm = wrapi(z - 1, g.mz), zp = wrapi(z + 1, g.mz);
-      const int i = x + g.mx * (y + g.my * z);
-      float wx = 0.0f, wy = 0.0f, wz = 0.0f;
-      if (a.noise) {
-        const float* cur = nbuf[z % NR];
-        const float* prv = nbuf[(z - 1 + NR) % NR];
-        const float* nxt = nbuf[(z + 1) % NR];
-        const int p = (lx + 1) + PX * (ly + 1);
-        const float f1 = a.f1, f4 = a.f4;
-        wx = g.idx * f1 * (cur[0 * PLANE + p + 1] - cur[0 * PLANE + p]) +
-             g.idy * f4 * (cur[1 * PLANE + p] - cur[1 * PLANE + p - PX]) +
-             g.idz * f4 * (cur[2 * PLANE + p] - prv[2 * PLANE + p]);
-        wy = g.idy * f1 * (cur[3 * PLANE + p + PX] - cur[3 * PLANE + p]) +
-             g.idx * f4 * (cur[1 * PLANE + p] - cur[1 * PLANE + p - 1]) +
-             g.idz * f4 * (cur[4 * PLANE + p] - prv[4 * PLANE + p]);
-        wz = g.idz * f1 * (nxt[5 * PLANE + p] - cur[5 * PLANE + p]) +
-             g.idx * f4 * (cur[2 * PLANE + p] - cur[2 * PLANE + p - 1]) +
-             g.idy * f4 * (cur[4 * PLANE + p] - cur[4 * PLANE + p - PX]);
-      }
-      const int n0 = x + g.mx * (y + g.my * zm), n5 = x + g.mx * (y + g.my * zp);
-      const int n1 = x + g.mx * (ym + g.my * z), n4 = x + g.mx * (yp + g.my * z);
-      const int n2 = xm + g.mx * (y + g.my * z), n3 = xp + g.mx * (y + g.my * z);
-      if (a.v) {
-        const float* V = a.v;
-        const float ax = g.idx * g.idx, ay = g.idy * g.idy, az = g.idz * g.idz;
+  const int xm = x == 0 ? g.mx - 1 : x - 1, xp = x == g.mx - 1 ? 0 : x + 1;
+  const int ym = y == 0 ? g.my - 1 : y - 1, yp = y == g.my - 1 ? 0 : y + 1;
+  const int zm = z == 0 ? g.mz - 1 : z - 1, zp = z == g.mz - 1 ? 0 : z + 1;
+  const auto at = [&](int i, int j, int k) { return i + g.mx * (j + g.my * k); };
+  const int n[7] = {at(x, y, z), at(xm, y, z), at(xp, y, z), at(x, ym, z), at(x, yp, z), at(x, y, zm), at(x, y, zp)};
+  const int i = n[0];
+  float V[3][7], pxmy, pxmz, mxpy, pymz, mxpz, mypz, w[3] = {0.0f, 0.0f, 0.0f};
+  if (own) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const float* f = V + (size_t)c * N;
-          float fc = f[i];
-          float L = ax * (f[n3] - 2.0f * fc + f[n2]) + ay * (f[n4] - 2.0f * fc + f[n1]) +
-                    az * (f[n5] - 2.0f * fc + f[n0]);
-          float t = fc + a.lap_coef * L;
-          if (c == 0) wx += t; else if (c == 1) wy += t; else wz += t;
-        }
-      }
-      if (a.vadv) {
-        const float* VX = a.vadv;
-        const float* VY = a.vadv + N;
-        const float* VZ = a.vadv + 2 * (size_t)N;
-        const int pxmy = xp + g.mx * (ym + g.my * z), pxmz = xp + g.mx * (y + g.my * zm);
-        const int mxpy = xm + g.mx * (yp + g.my * z), mxpz = xm + g.mx * (y + g.my * zp);
-        const int pymz = x + g.mx * (yp + g.my * zm), mypz = x + g.mx * (ym + g.my * zp);
-        float vx = VX[i], vy = VY[i], vz = VZ[i];
-        float vx0 = VX[n0], vx1 = VX[n1], vx2 = VX[n2], vx3 = VX[n3], vx4 = VX[n4], vx5 = VX[n5];
-        float vy0 = VY[n0], vy1 = VY[n1], vy2 = VY[n2], vy3 = VY[n3], vy4 = VY[n4], vy5 = VY[n5];
-        float vz0 = VZ[n0], vz1 = VZ[n1], vz2 = VZ[n2], vz3 = VZ[n3], vz4 = VZ[n4], vz5 = VZ[n5];
-        // advection (dt/4) sum_b D_b[(v_a + v_a')(v_b + v_b')], src/kernelConstructW.cu:120-136
-        float Ax = g.idx * ((vx3 + vx) * (vx3 + vx) - (vx + vx2) * (vx + vx2)) +
-                   g.idy * ((vx4 + vx) * (vy3 + vy) - (vx + vx1) * (VY[pxmy] + vy1)) +
-                   g.idz * ((vx5 + vx) * (vz3 + vz) - (vx + vx0) * (VZ[pxmz] + vz0));
-        float Ay = g.idx * ((vy3 + vy) * (vx4 + vx) - (vy + vy2) * (VX[mxpy] + vx2)) +
-                   g.idy * ((vy4 + vy) * (vy4 + vy) - (vy + vy1) * (vy + vy1)) +
-                   g.idz * ((vy5 + vy) * (vz4 + vz) - (vy + vy0) * (VZ[pymz] + vz0));
-        float Az = g.idx * ((vz3 + vz) * (vx5 + vx) - (vz + vz2) * (VX[mxpz] + vx2)) +
-                   g.idy * ((vz4 + vz) * (vy5 + vy) - (vz + vz1) * (VY[mypz] + vy1)) +
-                   g.idz * ((vz5 + vz) * (vz5 + vz) - (vz + vz0) * (vz + vz0));
-        const float q = 0.25f;  // the dt factor is folded into adv_coef by the caller
-        Ax *= q; Ay *= q; Az *= q;
-        wx += a.adv_coef * Ax;
-        wy += a.adv_coef * Ay;
-        wz += a.adv_coef * Az;
-        if (a.adv_store) {
-          a.adv_store[i] = Ax;
-          a.adv_store[i + N] = Ay;
-          a.adv_store[i + 2 * (size_t)N] = Az;
-        }
-      }
-      if (a.adv_prev) {
-        wx += a.adv_prev_coef * a.adv_prev[i];
-        wy += a.adv_prev_coef * a.adv_prev[i + N];
-        wz += a.adv_prev_coef * a.adv_prev[i + 2 * (size_t)N];
-      }
-      a.W[i] = wx;
-      a.W[i + N] = wy;
-      a.W[i + 2 * (size_t)N] = wz;
+    for (int c = 0; c < 3; ++c) load7(a.vadv + (size_t)c * N, n, V[c]);
+    const float *VX = a.vadv, *VY = VX + N, *VZ = VY + N;
+    pxmy = VY[at(xp, ym, z)];
+    pxmz = VZ[at(xp, y, zm)];
+    mxpy = VX[at(xm, yp, z)];
+    pymz = VZ[at(x, yp, zm)];
+    mxpz = VX[at(xm, y, zp)];
+    mypz = VY[at(x, ym, zp)];
+    if (a.base_in) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) w[c] = a.base_in[i + (size_t)c * N];
     }
+  }
+  if (a.noise) {
+    draw_planes<ZC>(a, key, nbuf, x0, y0, zs);
     __syncthreads();
   }
+  if (!own) return;
+  if (a.noise) {
+    const float *cur = nbuf[lz + 1], *prv = nbuf[lz], *nxt = nbuf[lz + 2];
+    const int p = (lx + 1) + PX * (ly + 1);
+    const float f1 = a.f1, f4 = a.f4;
+    w[0] = g.idx * f1 * (cur[0 * PLANE + p + 1] - cur[0 * PLANE + p]) +
+           g.idy * f4 * (cur[1 * PLANE + p] - cur[1 * PLANE + p - PX]) +
+           g.idz * f4 * (cur[2 * PLANE + p] - prv[2 * PLANE + p]);
+    w[1] = g.idy * f1 * (cur[3 * PLANE + p + PX] - cur[3 * PLANE + p]) +
+           g.idx * f4 * (cur[1 * PLANE + p] - cur[1 * PLANE + p - 1]) +
+           g.idz * f4 * (cur[4 * PLANE + p] - prv[4 * PLANE + p]);
+    w[2] = g.idz * f1 * (nxt[5 * PLANE + p] - cur[5 * PLANE + p]) +
+           g.idx * f4 * (cur[2 * PLANE + p] - cur[2 * PLANE + p - 1]) +
+           g.idy * f4 * (cur[4 * PLANE + p] - cur[4 * PLANE + p - PX]);
+  }
+  if (a.v) {
+    const float ax = g.idx * g.idx, ay = g.idy * g.idy, az = g.idz * g.idz;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      float f[7];
+      if (a.v == a.vadv) {
+#pragma unroll
+        for (int k = 0; k < 7; ++k) f[k] = V[c][k];
+      } else {
+        load7(a.v + (size_t)c * N, n, f);
+      }
+      const float L = ax * (f[2] - 2.0f * f[0] + f[1]) + ay * (f[4] - 2.0f * f[0] + f[3]) +
+                      az * (f[6] - 2.0f * f[0] + f[5]);
+      w[c] += f[0] + a.lap_coef * L;
+    }
+  }
+  if (a.base_out) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) a.base_out[i + (size_t)c * N] = w[c];
+  }
+  // advection (1/4) sum_b D_b[(v_a + v_a')(v_b + v_b')], src/kernelConstructW.cu:120-136; the dt
+  // factor is folded into adv_coef by the caller
+  const float *vx = V[0], *vy = V[1], *vz = V[2];
+  const float Ax = g.idx * ((vx[2] + vx[0]) * (vx[2] + vx[0]) - (vx[0] + vx[1]) * (vx[0] + vx[1])) +
+                   g.idy * ((vx[4] + vx[0]) * (vy[2] + vy[0]) - (vx[0] + vx[3]) * (pxmy + vy[3])) +
+                   g.idz * ((vx[6] + vx[0]) * (vz[2] + vz[0]) - (vx[0] + vx[5]) * (pxmz + vz[5]));
+  const float Ay = g.idx * ((vy[2] + vy[0]) * (vx[4] + vx[0]) - (vy[0] + vy[1]) * (mxpy + vx[1])) +
+                   g.idy * ((vy[4] + vy[0]) * (vy[4] + vy[0]) - (vy[0] + vy[3]) * (vy[0] + vy[3])) +
+                   g.idz * ((vy[6] + vy[0]) * (vz[4] + vz[0]) - (vy[0] + vy[5]) * (pymz + vz[5]));
+  const float Az = g.idx * ((vz[2] + vz[0]) * (vx[6] + vx[0]) - (vz[0] + vz[1]) * (mxpz + vx[1])) +
+                   g.idy * ((vz[4] + vz[0]) * (vy[6] + vy[0]) - (vz[0] + vz[3]) * (mypz + vy[3])) +
+                   g.idz * ((vz[6] + vz[0]) * (vz[6] + vz[0]) - (vz[0] + vz[5]) * (vz[0] + vz[5]));
+  const float A[3] = {0.25f * Ax, 0.25f * Ay, 0.25f * Az};
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const size_t at_c = i + (size_t)c * N;
+    w[c] += a.adv_coef * A[c];
+    if (a.adv_prev) w[c] += a.adv_prev_coef * a.adv_prev[at_c];
+    if (a.adv_store) a.adv_store[at_c] = A[c];
+    a.W[at_c] = w[c];
+  }
 }
-FHD_KERNEL_PAIR((), 256, k_fluid_w, FluidWArgs, body_fluid_w(a, b))
+FHD_KERNEL_PAIR((template <int ZC>), 256 * ZC, k_fluid_w, FluidWArgs, body_fluid_w<ZC>(a, b))
 
 // Discrete staggered divergence (diagnostic), src/kernelUpdateVIncompressible.cu invariant.
 __global__ void k_divergence(GridDev g, const float* __restrict__ v, float* __restrict__ div) {
@@ -242,10 +234,12 @@ void launch_advance_step(unsigned long long* step, hipStream_t s) {
 }
 
 void launch_fluid_w(const FluidWArgs& a, hipStream_t s) {
-  FluidWArgs x = a;
-  if (t_recorder && x.zchunk_b > 0) x.zchunk = x.zchunk_b;
-  dim3 grid((x.g.mx + TX - 1) / TX, (x.g.my + TY - 1) / TY, (x.g.mz + x.zchunk - 1) / x.zchunk);
-  launch(k_fluid_w, k_fluid_w_b, FAM_FLUID_W, grid, 256, x, s);
+  const int want = t_recorder && a.zchunk_b > 0 ? a.zchunk_b : a.zchunk;
+  const int zc = want >= 4 ? 4 : want >= 2 ? 2 : 1;
+  const dim3 grid((a.g.mx + TX - 1) / TX, (a.g.my + TY - 1) / TY, (a.g.mz + zc - 1) / zc);
+  if (zc == 4) launch(k_fluid_w<4>, k_fluid_w_b<4>, FAM_FLUID_W, grid, 1024, a, s);
+  else if (zc == 2) launch(k_fluid_w<2>, k_fluid_w_b<2>, FAM_FLUID_W, grid, 512, a, s);
+  else launch(k_fluid_w<1>, k_fluid_w_b<1>, FAM_FLUID_W, grid, 256, a, s);
 }
 
 void launch_divergence(const GridDev& g, const float* v, float* div, hipStream_t s) {

@@ -418,15 +418,12 @@ void launch_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc&
 }
 // Columns per z-pass workgroup: the schedule's tile, as far as the largest class holds it.
 void launch_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s) {
-  const bool merged = t_recorder && fast_edge(a.g.mz);
-  if (!a.generic && !merged && fast_fft_z_solve(a, spec, s)) return;
+  if (!a.generic && fast_fft_z_solve(a, spec, s)) return;
   const int LS = a.g.mz | 1;
   const int most = kClassElems[2] / (3 * LS);  // >= 10: mz is at most 256
   const int want = a.btile < most ? a.btile : most;
   const int ntile = (a.g.P + want - 1) / want, T = (a.g.P + ntile - 1) / ntile;
-  FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, T};
-  // the radices the schedule chose for the context alone (48-point columns: fft_common.h's kPlan48)
-  if (merged && a.g.mz == 48 && a.plan_zs) x.f.lz = a.plan_zs == 1 ? line_plan(48, 3, 16, 1) : line_plan(48, 4, 4, 3);
+  const FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, T};
   FHD_LAUNCH_CLASS(lds_class(3 * T * LS), k_fft_z_solve, FAM_FFT_Z, dim3(ntile, a.g.my), x, s);
 }
 void launch_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha, float beta,

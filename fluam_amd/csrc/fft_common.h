@@ -32,6 +32,14 @@ FHD_DEV float2 turn16(float2 a, float p, float s, bool swap) {
                      fmaf(a.x, v, a.y * u) + fmaf(a.x, vl, a.y * ul));
 }
 
+// a (p + i s sqrt(3)/2) and a (s sqrt(3)/2 + i p)
+FHD_DEV float2 turn6(float2 a, float p, float s) {
+  return make_float2(fmaf(p, a.x, -s * mul_r3(a.y)), fmaf(p, a.y, s * mul_r3(a.x)));
+}
+FHD_DEV float2 turn12(float2 a, float s, float p) {
+  return make_float2(fmaf(-p, a.y, s * mul_r3(a.x)), fmaf(p, a.x, s * mul_r3(a.y)));
+}
+
 // In-register DFTs with kernel e^{s 2 pi i / R}.
 template <int R> struct Dft;
 template <> struct Dft<2> {
@@ -68,8 +76,7 @@ template <> struct Dft<6> {
     Dft<3>::run(e, s);
     Dft<3>::run(o, s);
     // w^k = e^{s 2 pi i k / 6}
-    const float c3 = 0.86602540378443864676f;
-    const float2 o1 = cmul(o[1], make_float2(0.5f, s * c3)), o2 = cmul(o[2], make_float2(-0.5f, s * c3));
+    const float2 o1 = turn6(o[1], 0.5f, s), o2 = turn6(o[2], -0.5f, s);
     v[0] = cadd(e[0], o[0]);
     v[3] = csub(e[0], o[0]);
     v[1] = cadd(e[1], o1);
@@ -124,6 +131,33 @@ template <> struct Dft<8> {
     v[6] = csub(e[2], o2);
     v[3] = cadd(e[3], o3);
     v[7] = csub(e[3], o3);
+  }
+};
+
+template <> struct Dft<12> {
+  static FHD_DEV void run(float2* v, float s) {
+    // four-point transforms of every third element, twiddles e^{s 2 pi i b k / 12}, three-point ones
+    float2 y[3][4];
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) y[b][k] = v[b + 3 * k];
+      Dft<4>::run(y[b], s);
+    }
+    y[1][1] = turn12(y[1][1], 1.0f, 0.5f * s);
+    y[1][2] = turn6(y[1][2], 0.5f, s);
+    y[1][3] = cmul_si(y[1][3], s);
+    y[2][1] = turn6(y[2][1], 0.5f, s);
+    y[2][2] = turn6(y[2][2], -0.5f, s);
+    y[2][3] = make_float2(-y[2][3].x, -y[2][3].y);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float2 t[3] = {y[0][k], y[1][k], y[2][k]};
+      Dft<3>::run(t, s);
+      v[k] = t[0];
+      v[k + 4] = t[1];
+      v[k + 8] = t[2];
+    }
   }
 };
 

@@ -102,97 +102,6 @@ FHD_BODY void body_fftC(const FftArgs& a, const float2* __restrict__ spec, float
 FHD_KERNEL_PAIR((template <int MX, int MY, int NT, int PX, int PY>), NT, k_fftC, FftPass,
                 body_fftC<MX, MY, NT, PX, PY>(a.f, a.spec, a.out, a.aux, a.alpha, a.beta, b))
 
-// ---------------- pass B: FFT along z, operator, inverse FFT along z ----------------
-// Workgroup (tile i, ky): kx columns i*T .. i*T+T-1, plus column ntile*T + i when P is not a
-// multiple of T (the Nyquist column for P = mx/2 + 1).  LDS lines: (c, t) at (c*(T+1)+t)*(MZ+1).
-template <int MZ, int NT, int TM, int PZ = 0>
-FHD_BODY void body_fftB(const FftArgs& a, float2* __restrict__ spec, int T, const Blk& b) {
-  // TM: room for T <= TM - 1 columns plus one extra column
-  constexpr int LS = MZ + 1;
-  __shared__ float2 buf[3 * TM * LS];
-  __shared__ float2 twz[MZ], ezs[MZ];
-  __shared__ float gzs[MZ];
-  const int P = a.g.P, my = a.g.my;
-  // neighbouring column tiles share the 128-byte lines of each z row: keep them on one XCD
-  const int item = xcd_item(b.x + b.nx * b.y, b.nx * b.ny);
-  const int ky = item / b.nx, tile = item - ky * b.nx;
-  const int ntile = P / T, rem = P - ntile * T;
-  const int TC = T + (tile < rem ? 1 : 0);
-  for (int i = threadIdx.x; i < MZ; i += NT) {
-    twz[i] = a.twz[i];
-    ezs[i] = a.ez[i];
-    gzs[i] = a.gz[i];
-  }
-  const size_t cstride = (size_t)my * MZ * P;
-  float2* base = spec + (size_t)ky * MZ * P;
-  // elements (c, z, t) on a TM-wide grid (t fastest, constant divisors); slots t >= TC idle.
-  // Every load of this lane is in flight before the first LDS write.
-  constexpr int EL = 3 * MZ * TM, NL = (EL + NT - 1) / NT;
-  const int ncomp = a.ncomp;
-  const int cs32 = (int)cstride;  // ncomp * cstride elements per ky row: far below 2^31 at every size
-  {
-    float2 v[NL];
-#pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      const int e = threadIdx.x + k * NT;
-      const int t = e % TM, r = e / TM, z = r % MZ, c = r / MZ;
-      if (e < EL && c < ncomp && t < TC) {
-        const int kx = t < T ? tile * T + t : ntile * T + tile;
-        v[k] = base[c * cs32 + z * P + kx];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      const int e = threadIdx.x + k * NT;
-      const int t = e % TM, r = e / TM, z = r % MZ, c = r / MZ;
-      if (e < EL && c < ncomp && t < TC) buf[(c * TM + t) * LS + z] = v[k];
-    }
-  }
-  __syncthreads();
-  const int lines = a.ncomp * TM;
-  if (a.zmode != 2) ffft<MZ, 1, NT, 3 * TM, 1, false, plan_choice(MZ, PZ)>(buf, lines, LS, twz);
-  if (a.zmode == 0) {
-    const float gy = a.gy[ky];
-    const float2 ey = a.ey[ky];
-    const Key key = a.knoise ? resolve_key(a.key) : a.key;
-    for (int e = threadIdx.x; e < MZ * TC; e += NT) {
-      const int t = e / MZ, z = e - t * MZ;
-      const int kx = t < T ? tile * T + t : ntile * T + tile;
-      const float gx = a.gx[kx];
-      const float2 ex = a.ex[kx];
-      const float gz = gzs[z];
-      const float2 ez = ezs[z];
-      const int i0 = (0 * TM + t) * LS + z, i1 = (1 * TM + t) * LS + z, i2 = (2 * TM + t) * LS + z;
-      float2 b0 = buf[i0], b1 = buf[i1], b2 = buf[i2];
-      solve_mode(a, key, kx, ky, z, gx, gy, gz, ex, ey, ez, b0, b1, b2);
-      buf[i0] = b0;
-      buf[i1] = b1;
-      buf[i2] = b2;
-    }
-    __syncthreads();
-  }
-  if (a.zmode != 1) ffft<MZ, 1, NT, 3 * TM, 1, true, plan_choice(MZ, PZ)>(buf, lines, LS, twz);
-  // the lane index, opaque to the compiler: the store indices are recomputed here rather than
-  // kept live in registers from the loads through both transforms
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));
-#pragma unroll
-  for (int k = 0; k < NL; ++k) {
-    const int e = tid + k * NT;
-    const int t = e % TM, r = e / TM, z = r % MZ, c = r / MZ;
-    if (e < EL && c < ncomp && t < TC) {
-      const int kx = t < T ? tile * T + t : ntile * T + tile;
-      base[c * cs32 + z * P + kx] = buf[(c * TM + t) * LS + z];
-    }
-  }
-}
-// 8 waves per SIMD (a 64-VGPR budget) where the LDS of that many workgroups fits in a CU
-constexpr int fftb_waves(int MZ, int NT, int TM) {
-  return (32 / (NT / 64)) * (3 * TM * (MZ + 1) * 8 + MZ * 20) <= 160 * 1024 ? 8 : 1;
-}
-FHD_KERNEL_PAIR_OCC((template <int MZ, int NT, int TM, int PZ>), NT, fftb_waves(MZ, NT, TM), k_fftB, FftPass,
-                body_fftB<MZ, NT, TM, PZ>(a.f, a.spec, a.T, b))
-
 // ---------------- dispatch ----------------
 template <int MX, int MY, int NT, int PX, int PY>
 static void launch_AC_plan(const FftPass& x, int which, int mz, hipStream_t s) {
@@ -285,65 +194,6 @@ bool fast_fft_xy_fwd(const FftArgs& a, const float* in, float2* spec, hipStream_
 bool fast_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha, float beta,
                      hipStream_t s) {
   return fast_AC(a, 1, nullptr, const_cast<float2*>(spec), out, aux, alpha, beta, s);
-}
-
-// Largest column-tile width T <= tmax whose leftover columns (P mod T) fit one per tile.
-static int column_tile(int P, int tmax) {
-  for (int T = tmax; T > 1; --T)
-    if (T <= P && P % T <= P / T) return T;
-  return 1;
-}
-
-template <int MZ, int NT, int PZ>
-static void launch_B_plan(const FftPass& x, int bt, dim3 grid, hipStream_t s) {
-  if (bt == 2) launch(k_fftB<MZ, NT, 3, PZ>, k_fftB_b<MZ, NT, 3, PZ>, FAM_FFT_Z, grid, NT, x, s);
-  else if (bt == 4) launch(k_fftB<MZ, NT, 5, PZ>, k_fftB_b<MZ, NT, 5, PZ>, FAM_FFT_Z, grid, NT, x, s);
-  else if (bt == 8) launch(k_fftB<MZ, NT, 9, PZ>, k_fftB_b<MZ, NT, 9, PZ>, FAM_FFT_Z, grid, NT, x, s);
-  else launch(k_fftB<MZ, NT, 17, PZ>, k_fftB_b<MZ, NT, 17, PZ>, FAM_FFT_Z, grid, NT, x, s);
-}
-// The z transform's radix plan (plan_choice index) comes from the autotuner for 48-, 96- and
-// 128-point columns.
-template <int MZ, int NT>
-static void launch_B_nt(const FftPass& x, int bt, dim3 grid, hipStream_t s) {
-  if constexpr (MZ == 48 || MZ == 96 || MZ == 128) {
-    if (x.f.plan_zs == 1) return launch_B_plan<MZ, NT, 1>(x, bt, grid, s);
-    if (x.f.plan_zs == 2) return launch_B_plan<MZ, NT, 2>(x, bt, grid, s);
-  }
-  launch_B_plan<MZ, NT, 0>(x, bt, grid, s);
-}
-
-// Column-tile width of the z pass: 2, 4, 8 or 16 (chosen per grid shape by the context's
-// schedule), with one extra LDS column for the leftover Nyquist column.
-template <int MZ>
-static bool launch_B2(const FftArgs& a, float2* spec, hipStream_t s) {
-  const int P = a.g.P;
-  const int bt = a.btile == 2 || a.btile == 4 || a.btile == 16 ? a.btile : 8;
-  const int T = column_tile(P, bt);
-  const dim3 grid(P / T, a.g.my);
-  const FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, T};
-  // 512 lanes halve each lane's column loads for a single context's pass from 64-point columns
-  // up (128^3: 29.6 vs 30.5 us per pass; 50 VGPRs); batched dispatches below 128 keep 256
-  if constexpr (MZ >= 64) {
-    if (MZ >= 128 || t_recorder == nullptr) {
-      launch_B_nt<MZ, 512>(x, bt, grid, s);
-      return true;
-    }
-  }
-  launch_B_nt<MZ, 256>(x, bt, grid, s);
-  return true;
-}
-
-bool fast_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s) {
-  switch (a.g.mz) {
-    case 16: return launch_B2<16>(a, spec, s);
-    case 24: return launch_B2<24>(a, spec, s);
-    case 32: return launch_B2<32>(a, spec, s);
-    case 48: return launch_B2<48>(a, spec, s);
-    case 64: return launch_B2<64>(a, spec, s);
-    case 96: return launch_B2<96>(a, spec, s);
-    case 128: return launch_B2<128>(a, spec, s);
-    default: return false;
-  }
 }
 
 }  // namespace fhd

@@ -11,8 +11,8 @@
 // contiguous range of items keeps neighbouring items, which share cache lines, on one L2.
 FHD_DEV int xcd_item(int b, int n) {
   constexpr int kXcd = 8;
-  if (n % kXcd) return b;
-  return (b % kXcd) * (n / kXcd) + b / kXcd;
+  const int x = b % kXcd;
+  return x * (n / kXcd) + min(x, n % kXcd) + b / kXcd;  // the first n % 8 ranges are one item longer
 }
 
 // n / d for n d < 2^32 by multiplication with ceil(2^32 / d) (0 stands for d = 1).

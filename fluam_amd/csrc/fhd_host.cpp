@@ -358,7 +358,6 @@ void build_tables(fhd_ctx* c) {
   a.btile = 8;
   a.plan_xy = 0;
   a.plan_xy_inv = 0;
-  a.plan_zs = 0;
   a.zmode = 0;
   a.ncomp = 3;
   a.knoise = 0;
@@ -453,20 +452,21 @@ FluidWArgs base_w(fhd_ctx* c) {
 }
 
 // ---------------- schedule autotuner ----------------
-// The z-pass column tile and the W kernel's chunk follow the grid's size; the radix plans of 48-,
-// 96- and 128-point columns and of 96 x 96 and 128 x 128 planes are timed once per grid shape on the
+// The z-pass column tile and the W kernel's chunk follow the grid's size; the radix plans of
+// 96 x 96 and 128 x 128 planes are timed once per grid shape on the
 // first context of that shape and cached for the process: a replica's schedule depends on its shape
 // only, never on what else runs beside it.
 
-// Columns of a z-pass workgroup: as many as leave the chip two workgroups per CU (fewer, longer rows
-// of a tile cost more than the columns save: per launch with 2, 4, 8, 16 columns 4.9, 5.1, 6.0, 7.5 us
-// at 32^3, 7.3, 6.4, 6.5, 8.0 at 64^3, 41, 31.5, 28.0, 28.0 at 128^3).
-int z_tile(int mx, int my) {
+// Columns of a z-pass workgroup: 4, fewer where that leaves the chip less than a workgroup per CU, and 8
+// where the grid still has four per CU and their LDS leaves room for five.  Per launch with 2, 4, 8
+// columns: 8.0, 8.0, 8.2 us at 32^3, 12.5, 11.1, 11.5 at 108 x 54 x 72, 10.5, 10.0, 11.1 at 128 x 64 x 32,
+// 27.6, 27.4, 26.4 at 128^3, 49.5, 46.7, 69.7 at 128 x 128 x 256.
+int z_tile(int mx, int my, int mz) {
   const int P = mx / 2 + 1;
-  return P / 8 * my >= 512 ? 8 : P / 4 * my >= 256 ? 4 : 2;
+  return P / 8 * my >= 1024 && mz <= 144 ? 8 : P / 4 * my >= 256 ? 4 : 2;
 }
 struct Sched {
-  int btile, zchunk, zchunk_b, plan_xy, plan_xy_inv, plan_zs;
+  int btile, zchunk, zchunk_b, plan_xy, plan_xy_inv;
 };
 std::mutex g_sched_mu;
 std::map<std::array<int, 4>, Sched> g_sched;
@@ -502,39 +502,17 @@ void apply_schedule(fhd_ctx* c) {
   auto it = g_sched.find(key);
   // two planes per W workgroup: per launch with 1, 2, 4 planes 5.3, 5.2, 6.8 us at 32^3, 12.4, 7.5, 7.3 at
   // 64^3, 13.9, 9.4, 11.9 at 96 x 48 x 64
-  Sched sc = {z_tile(c->p.mx, c->p.my), 2, 2, 0, 0, 0};
+  Sched sc = {z_tile(c->p.mx, c->p.my, c->p.mz), 2, 2, 0, 0};
   if (it != g_sched.end()) {
     sc = it->second;
   } else if (tune) {
     // scratch runs on the context's own buffers before its state exists (contents irrelevant)
-    float best = 1e30f;
-    const bool stokes = c->p.scheme == FHD_SCHEME_STOKES_LIMIT;
-    // z pass of 48-, 96- and 128-point columns: the radix plan (128: 16 8, 8 16 or 4 4 8; 96: 16 2 3,
-    // 8 4 3 or 3 8 4; 48: 16 3, 3 16 or 4 4 3), timed in the form the scheme launches (the Stokes
-    // pass draws its stochastic stress)
-    FftArgs za = c->fa;
-    if (stokes) {
-      za.stokes = 1;
-      za.knoise = 2;
-      za.kn_f1 = za.kn_f4 = 1.0f;
-      za.key = make_key(c);
-    }
-    za.btile = sc.btile;
-    const int mzp = c->p.mz;
-    const int nzp = (mzp == 48 || mzp == 96 || mzp == 128) ? 3 : 0;
-    for (int pz = 0; pz < nzp; ++pz) {
-      za.plan_zs = pz;
-      const float t = time_launches(c, [&] { launch_fft_z_solve(za, c->spec, c->s); }, 4);
-      if (t < best) { best = t; sc.plan_zs = pz; }
-    }
-    c->fa.plan_zs = sc.plan_zs;
     // xy passes of 96 x 96 and 128 x 128 planes: the radix plans of the x and y transforms
     // (three each) of the LDS-stage kernels, and for 128 x 128 the register-transform kernels
     // (plan 9), chosen for the forward and the inverse pass separately
     const bool sq128 = c->p.mx == 128 && c->p.my == 128, sq96 = c->p.mx == 96 && c->p.my == 96;
     if (sq128 || sq96) {
-      best = 1e30f;
-      float best_inv = 1e30f;
+      float best = 1e30f, best_inv = 1e30f;
       for (int pxy = 0; pxy < (sq128 ? 10 : 9); ++pxy) {  // 9: the register-transform kernels
         c->fa.plan_xy = c->fa.plan_xy_inv = pxy;
         const float tf = time_launches(c, [&] { launch_fft_xy_fwd(c->fa, c->W, c->spec, c->s); }, 4);
@@ -551,11 +529,10 @@ void apply_schedule(fhd_ctx* c) {
   c->fa.btile = sc.btile;
   c->fa.plan_xy = sc.plan_xy;
   c->fa.plan_xy_inv = sc.plan_xy_inv;
-  c->fa.plan_zs = sc.plan_zs;
   c->zchunk = sc.zchunk;
   c->zchunk_b = sc.zchunk_b;
   // explicit radix plans (tests and experiments): FHD_PLAN_XY in 0-9 (128 x 128 planes; 0-8
-  // for 96 x 96), FHD_PLAN_Z in 0-2 (48-, 96- and 128-point columns)
+  // for 96 x 96), FHD_PLAN_Z in 0-2 (accepted, no effect: the z pass has one plan per length)
   if (const char* e = getenv("FHD_PLAN_XY")) {
     const int v = atoi(e);
     if (v < 0 || v > 9) throw std::runtime_error("FHD_PLAN_XY must be 0-9");
@@ -564,7 +541,6 @@ void apply_schedule(fhd_ctx* c) {
   if (const char* e = getenv("FHD_PLAN_Z")) {
     const int v = atoi(e);
     if (v < 0 || v > 2) throw std::runtime_error("FHD_PLAN_Z must be 0-2");
-    c->fa.plan_zs = v;
   }
   // explicit schedule (tests and experiments): FHD_BTILE in {2, 4, 8, 16}, FHD_ZCHUNK >= 1
   if (const char* e = getenv("FHD_BTILE")) {
@@ -2202,7 +2178,7 @@ int fhd_get_schedule(const fhd_ctx* c, int out[6]) {
   if (!c || !out) return 0;
   out[0] = c->fa.btile;
   out[1] = c->fa.plan_xy;
-  out[2] = c->fa.plan_zs;
+  out[2] = 0;  // the z pass has one radix plan per length
   out[3] = c->zchunk;
   out[4] = c->zchunk_b;
   out[5] = c->fa.plan_xy_inv;

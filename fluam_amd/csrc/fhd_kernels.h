@@ -39,7 +39,6 @@ struct FftArgs {
   int btile;                      // kx columns per pass-B workgroup (2, 4, 8 or 16)
   int plan_xy;                    // radix plans of the forward xy pass (96 x 96, 128 x 128 planes): px + 3 py, 0 default
   int plan_xy_inv;                // the same for the inverse xy pass
-  int plan_zs;                    // radix plan of the z pass (128-point columns), 0 default
   int zmode;                      // 0: FFT_z, operator, inverse FFT_z; 1: FFT_z only; 2: inverse only
   int ncomp;                      // velocity components transformed (3; 1 for a single field, transform-only modes)
   int knoise;                     // Stokes: the kept part of the stress divergence, drawn in Fourier space
@@ -92,6 +91,7 @@ struct FftPass {
   const float* aux;
   float alpha, beta;
   int T;                // z pass: kx columns per workgroup
+  uint32_t mt, ml;      // fft_z.hip: fast_div's reciprocals of T and of ncomp T
 };
 
 // Tile decomposition used for particle binning and deterministic spreading.

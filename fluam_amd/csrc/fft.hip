@@ -20,13 +20,14 @@
 // elements in LDS, so a lane never holds more than 9 elements (64 VGPRs, the CU full of waves in
 // every class), every load of a lane is in flight at once, and the butterflies a lane may hold in
 // a stage are a constant per radix.  The radices go up to 16 (at most three stages for any length
-// up to 256), the divisions by runtime extents are multiplications by host-made reciprocals.
-// Bound by LDS and barrier latency, like the size-specialised passes.  Per launch (HIP events,
-// which add about 4 us), with 256 lanes, radices up to 8 and a load-wait-store loop per element
-// before, and now: 108 x 54 x 72 forward 33.6 -> 13.1, z 37.4 -> 15.0, inverse 34.8 -> 13.8 us;
-// 128 x 64 x 32 forward 28.9 -> 13.8 us; 256-point columns of 128 x 128 planes 181 -> 58 us.
-// Where a size-specialised instance exists it stays ahead (128^3: 20.7 / 28.0 / 19.2 against
-// 23.6 / 34.2 / 23.2 us; 64^3: 9.6 / 11.3 / 8.9 against 13.8 / 14.0 / 13.3), so those shapes keep it.
+// up to 256), the divisions by runtime extents are multiplications by host-made reciprocals, and the
+// y transform's last stage (the inverse's first) works on the modes in global memory.  Bound by LDS
+// and barrier latency, like the size-specialised passes.  Per launch (HIP events, which add about
+// 4 us), with 256 lanes, radices up to 8 and a load-wait-store loop per element at first, then with
+// every stage through LDS, and now: 108 x 54 x 72 forward 33.6, 13.5, 12.8, inverse 34.8, 13.0, 12.9 us;
+// 128 x 64 x 32 inverse 13.8, now 13.3, 96 x 48 x 64 13.1, now 12.5.  Where a size-specialised instance
+// exists it stays ahead (128^3 forward and inverse 20.7 / 19.2 against 23.6 / 23.2 us; 64^3 9.6 / 8.9
+// against 13.8 / 13.3), so those shapes keep it; the z pass is fft_z.hip's but for a few lengths.
 // The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
 // on the one alone and on the other in a merged batch), so the compiler must not choose which
 // products become fused multiply-adds: the fused ones are written out.
@@ -56,20 +57,32 @@ struct Lines {
 // into registers, the workgroup synchronises, then writes.  Consecutive lanes take butterfly j of
 // consecutive lines, which lie an odd number of elements apart or next to each other, so the
 // lanes of a wave use different LDS banks and share one twiddle.  INV: the adjoint stage of the
-// inverse transform (fft_stages.h).
-template <int R, int NT, bool INV>
-FHD_DEV void stockham_stage(float2* buf, const Lines& ln, int n, int Ns, uint32_t mns, const float2* tw, int twmul) {
+// inverse transform.  GIO: the modes lie in global memory, element e of line l at m.g[l + e m.gs], and
+// a transform of two stages runs the first one in place (all as in fft_stages.h).
+struct Modes {
+  float2* g;
+  int gs;
+};
+struct NotReady {
+  FHD_DEV void operator()() const {}
+};
+template <int R, int NT, bool INV, bool GIO, class Ready>
+FHD_DEV void stockham_stage(float2* buf, const Lines& ln, const LinePlan& p, int Ns, uint32_t mns, const float2* tw,
+                            int twmul, const Modes& m, const Ready& ready) {
   constexpr int KMAX = kmax_for(R);
   constexpr float s = INV ? 1.0f : -1.0f;
-  const int nbl = n / R;
+  const int n = p.n, nbl = n / R;
   const int total = ln.count * nbl;
   const int twstep = n / (Ns * R) * twmul;
+  const bool last = Ns * R == n, glob = GIO && last, inpl = GIO && p.nst == 2;
   // opaque to the compiler, which otherwise hoists the lane indices of every radix's stage out of
   // the stage loop and spills them (150 VGPRs)
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));
+  const int in_j = inpl && last ? R : 1, in_r = inpl && last ? ln.es : nbl * ln.es;
+  const int out_r = inpl && !last ? in_r : Ns * ln.es;
   float2 v[KMAX][R];
-  int to[KMAX];  // first element of the butterfly's outputs, -1: none
+  int to[KMAX], t1[KMAX];  // first element of the butterfly's outputs (-1: none), twiddle step
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     const int b = tid + k * NT;
@@ -78,39 +91,58 @@ FHD_DEV void stockham_stage(float2* buf, const Lines& ln, int n, int Ns, uint32_
       const int j = fast_div(b, ln.ml), l = b - j * ln.count;
       const int base = l * ln.ls;
       const int jn = Ns == 1 ? j : fast_div(j, mns), kk = j - jn * Ns;
-      const int t1 = kk * twstep;
-      const int spread = base + j * ln.es, packed = base + (jn * Ns * R + kk) * ln.es;
-      int at = INV ? packed : spread;
-      const int step = (INV ? Ns : nbl) * ln.es;
+      t1[k] = kk * twstep;
+      const int in = base + j * in_j * ln.es, out = inpl && !last ? in : base + (jn * Ns * R + kk) * ln.es;
+      if (GIO && INV && last) {
+        int at = l + j * m.gs;
 #pragma unroll
-      for (int r = 0; r < R; ++r, at += step) {
-        v[k][r] = buf[at];
-        if (!INV && Ns > 1 && r > 0) v[k][r] = cmul(v[k][r], tw[r * t1]);
+        for (int r = 0; r < R; ++r, at += nbl * m.gs) v[k][r] = m.g[at];
+      } else {
+        int at = INV ? out : in;
+        const int step = INV ? out_r : in_r;
+#pragma unroll
+        for (int r = 0; r < R; ++r, at += step) v[k][r] = buf[at];
+      }
+      to[k] = GIO && !INV && last ? l + j * m.gs : INV ? in : out;
+    }
+  }
+  if (GIO && INV && last) ready();
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    if (to[k] >= 0) {
+      if (!INV && Ns > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[k][r] = cmul(v[k][r], tw[r * t1[k]]);
       }
       Dft<R>::run(v[k], s);
       if (INV && Ns > 1) {
 #pragma unroll
-        for (int r = 1; r < R; ++r) v[k][r] = cmul(v[k][r], cconj(tw[r * t1]));
+        for (int r = 1; r < R; ++r) v[k][r] = cmul(v[k][r], cconj(tw[r * t1[k]]));
       }
-      to[k] = INV ? spread : packed;
     }
   }
-  __syncthreads();
+  if (!last && !inpl) __syncthreads();
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     if (to[k] >= 0) {
       int at = to[k];
-      const int step = (INV ? nbl : Ns) * ln.es;
+      if (GIO && !INV && last) {
 #pragma unroll
-      for (int r = 0; r < R; ++r, at += step) buf[at] = v[k][r];
+        for (int r = 0; r < R; ++r, at += nbl * m.gs) m.g[at] = v[k][r];
+      } else {
+        const int step = INV ? in_r : out_r;
+#pragma unroll
+        for (int r = 0; r < R; ++r, at += step) buf[at] = v[k][r];
+      }
     }
   }
-  __syncthreads();
+  if (!glob || INV) __syncthreads();
 }
 
 // Full FFT of every line: at most three stages, undone in reverse order by the inverse.
-template <int NT, bool INV>
-FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const float2* tw, int twmul) {
+template <int NT, bool INV, bool GIO, class Ready>
+FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const float2* tw, int twmul, const Modes& m,
+                     const Ready& ready) {
   int Ns = INV ? p.n : 1;
   for (int k = 0; k < p.nst; ++k) {
     const int st = INV ? p.nst - 1 - k : k;
@@ -118,16 +150,22 @@ FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const floa
     const uint32_t mns = p.mns[st];
     if (INV) Ns /= R;
     switch (R) {
-      case 16: stockham_stage<16, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
-      case 9: stockham_stage<9, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
-      case 8: stockham_stage<8, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
-      case 6: stockham_stage<6, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
-      case 4: stockham_stage<4, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
-      case 3: stockham_stage<3, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
-      default: stockham_stage<2, NT, INV>(buf, ln, p.n, Ns, mns, tw, twmul); break;
+#define FHD_STAGE(r) stockham_stage<r, NT, INV, GIO>(buf, ln, p, Ns, mns, tw, twmul, m, ready); break
+      case 16: FHD_STAGE(16);
+      case 9: FHD_STAGE(9);
+      case 8: FHD_STAGE(8);
+      case 6: FHD_STAGE(6);
+      case 4: FHD_STAGE(4);
+      case 3: FHD_STAGE(3);
+      default: FHD_STAGE(2);
+#undef FHD_STAGE
     }
     if (!INV) Ns *= R;
   }
+}
+template <int NT, bool INV>
+FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const float2* tw, int twmul) {
+  lds_fft<NT, INV, false>(buf, ln, p, tw, twmul, Modes{nullptr, 0}, NotReady{});
 }
 
 // ---------------------------------------------------------------------------------------
@@ -220,15 +258,11 @@ FHD_BODY void body_fft_xy_fwd(const FftArgs& a, const float* __restrict__ in, fl
   }
   __syncthreads();
   // y: columns kx = 0..P-1
-  lds_fft<NT, false>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1);
   float2* dst = spec + ((size_t)c * my * mz + z) * P;
-#pragma unroll
-  for (int k = 0; k < kPerLane; ++k) {
-    const int e = threadIdx.x + k * NT;
-    if (e < P * my) {
-      const int ky = fast_div(e, a.mdp), kx = e - ky * P;
-      dst[(size_t)ky * mz * P + kx] = buf[ky * PS + kx];
-    }
+  if (my > 1) {
+    lds_fft<NT, false, true>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1, Modes{dst, mz * P}, NotReady{});
+  } else if ((int)threadIdx.x < P) {
+    dst[threadIdx.x] = buf[threadIdx.x];
   }
 }
 FHD_KERNEL_PAIR_OCC((template <int NT, int ELEMS>), NT, 8, k_fft_xy_fwd, FftPass,
@@ -323,26 +357,18 @@ FHD_BODY void body_fft_xy_inv(const FftArgs& a, const float2* __restrict__ spec,
   __shared__ float2 twy[kMaxFftLen];
   const int z = b.x, c = b.y;
   const int mx = a.g.mx, my = a.g.my, mz = a.g.mz, P = a.g.P, h = mx / 2, PS = P | 1;
-  const float2* src = spec + ((size_t)c * my * mz + z) * P;
-  {
-    float2 v[kPerLane];
-#pragma unroll
-    for (int k = 0; k < kPerLane; ++k) {
-      const int e = threadIdx.x + k * NT;
-      const int ky = fast_div(e, a.mdp), kx = e - ky * P;
-      if (e < P * my) v[k] = src[(size_t)ky * mz * P + kx];
-    }
+  float2* src = const_cast<float2*>(spec) + ((size_t)c * my * mz + z) * P;
+  const auto tables = [&] {
     for (int i = threadIdx.x; i < mx; i += NT) twx[i] = a.twx[i];
     for (int i = threadIdx.x; i < my; i += NT) twy[i] = a.twy[i];
-#pragma unroll
-    for (int k = 0; k < kPerLane; ++k) {
-      const int e = threadIdx.x + k * NT;
-      const int ky = fast_div(e, a.mdp), kx = e - ky * P;
-      if (e < P * my) buf[ky * PS + kx] = v[k];
-    }
+    __syncthreads();
+  };
+  if (my > 1) {
+    lds_fft<NT, true, true>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1, Modes{src, mz * P}, tables);
+  } else {
+    if ((int)threadIdx.x < P) buf[threadIdx.x] = src[threadIdx.x];
+    tables();
   }
-  __syncthreads();
-  lds_fft<NT, true>(buf, Lines{P, a.mdp, 1, PS}, a.ly, twy, 1);
   // C2R packing: Z[k] = (X[k] + conj X[h-k]) + i (X[k] - conj X[h-k]) e^{+2 pi i k / mx}
   const int npair = h / 2 + 1;
   for (int e = threadIdx.x; e < my * npair; e += NT) {
@@ -416,7 +442,8 @@ void launch_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc&
   const FftSpread x{{a, in, spec, nullptr, nullptr, 0.0f, 0.0f, 0}, src};
   FHD_LAUNCH_CLASS(lds_class(a.g.my * (a.g.P | 1)), k_fft_spread_xy_fwd, FAM_FFT_XY_FWD, dim3(a.g.mz, a.ncomp), x, s);
 }
-// Columns per z-pass workgroup: the schedule's tile, as far as the largest class holds it.
+// Lengths without an instance in fft_z.hip, or all of them when the runtime-size kernels are forced.
+// Columns per workgroup: the schedule's tile, as far as the largest class holds it.
 void launch_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s) {
   if (!a.generic && fast_fft_z_solve(a, spec, s)) return;
   const int LS = a.g.mz | 1;

@@ -1,10 +1,8 @@
-// fft_fast.hip -- size-specialised versions of the three FFT passes (see fft.hip for the
-// algorithm).  Transform lengths, radix plans and LDS extents are template parameters, so every
+// fft_fast.hip -- size-specialised versions of the xy passes (see fft.hip for the algorithm).  Transform lengths, radix plans and LDS extents are template parameters, so every
 // index division in the Stockham stages is by a constant and the register arrays are sized for
 // the actual plane instead of the worst case.  Instantiated for xy planes mx x my with both
-// lengths in {16, 24, 32, 48, 64} or mx = my in {96, 128}, and z pencils of any of those
-// lengths; other shapes use the generic kernels, which share the spectrum layout
-// spec[c][ky][z][kx].
+// lengths in {16, 24, 32, 48, 64} or mx = my in {96, 128}; other shapes use the generic kernels,
+// which share the spectrum layout spec[c][ky][z][kx].
 // The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
 // on the one alone and on the other in a merged batch), so the compiler must not choose which
 // products become fused multiply-adds: the fused ones are written out.
@@ -30,28 +28,12 @@ FHD_BODY void body_fftC(const FftArgs& a, const float2* __restrict__ spec, float
   __shared__ float2 twx[MX];
   __shared__ float2 twy[MY];
   const int z = b.x, c = b.y, mz = a.g.mz;
-  for (int i = threadIdx.x; i < MX; i += NT) twx[i] = a.twx[i];
-  for (int i = threadIdx.x; i < MY; i += NT) twy[i] = a.twy[i];
-  const float2* src = spec + (size_t)c * MY * mz * P + (size_t)z * P;
-  constexpr int NL = (MY * P + NT - 1) / NT;
-  {
-    float2 v[NL];
-#pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      const int e = threadIdx.x + k * NT;
-      if (e < MY * P) {
-        const int ky = e / P, kx = e - ky * P;
-        v[k] = src[(size_t)ky * mz * P + kx];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < NL; ++k) {
-      const int e = threadIdx.x + k * NT;
-      if (e < MY * P) buf[e] = v[k];
-    }
-  }
-  __syncthreads();
-  ffft<MY, P, NT, P, 1, true, plan_choice(MY, PY)>(buf, P, 1, twy);
+  float2* src = const_cast<float2*>(spec) + (size_t)c * MY * mz * P + (size_t)z * P;
+  ffft_modes<MY, P, NT, P, 1, true, plan_choice(MY, PY)>(buf, P, 1, twy, src, mz * P, [&] {
+    for (int i = threadIdx.x; i < MX; i += NT) twx[i] = a.twx[i];
+    for (int i = threadIdx.x; i < MY; i += NT) twy[i] = a.twy[i];
+    __syncthreads();
+  });
   constexpr int NP = H / 2 + 1;
   for (int e = threadIdx.x; e < MY * NP; e += NT) {
     const int y = e / NP, k = e - y * NP;

@@ -1,5 +1,9 @@
 // fft_stages.h -- the Stockham stages and the forward xy pass of the size-specialised FFT kernels,
 // shared by the plain passes (fft_fast.hip) and the passes with spreading (fft_spread.hip).
+// Bound by LDS crossings and barriers: a plane crosses LDS ten times with six barriers.  Twelve and
+// ten, with every stage written, waited for and read back on both sides, took 20.0 us per inverse
+// launch at 128^3 (HIP events, which add about 4 us; now 18.3), 14.7 at 96^3 (14.1); 100 steps of
+// 128^3 Stokes 22.8 ms (now 22.0).
 #pragma once
 #include "fhd_device.h"
 #include "fhd_kernels.h"
@@ -18,64 +22,102 @@ namespace fhd {
 // where the forward stage writes, twiddles after the butterfly, writes where it reads).  The
 // inverse is then the exact adjoint of the forward transform with the table's rounded twiddles, so
 // their phase errors cancel over the round trip of a solve instead of adding up over the steps.
-template <int N, int R, int NS, int ES, int NT, int MAXL, int TWM, bool INV>
-FHD_DEV void fstage(float2* buf, int lines, int LS, const float2* tw) {
+// The last stage (the inverse's first) reads and writes the same elements, so nothing waits between.
+// GIO: it leaves LDS out on the side of the modes, which lie in global memory (`g`: element e of line
+// l at g[l + e gs]; of consecutive lines in consecutive words).  A transform of two stages then also
+// runs its first one in place: element j R1 + r stays at j + r R2, so the second stage's butterfly j
+// finds its elements at j R2 + r.  `ready` is called once the global loads are under way and ends with
+// a barrier.
+template <int N, int R, int NS, int ES, int NT, int MAXL, int TWM, bool INV, bool GIO, bool INPL, class Ready>
+FHD_DEV void fstage(float2* buf, int lines, int LS, const float2* tw, float2* g, int gs, const Ready& ready) {
   constexpr int NBL = N / R;
   constexpr int KMAX = (MAXL * NBL + NT - 1) / NT;
   constexpr int STRIDE = N / (NS * R);
+  constexpr bool LAST = NS * R == N, GLOB = GIO && LAST;
   constexpr float s = INV ? 1.0f : -1.0f;
+  // elements of butterfly j on the input side of the forward stage (NBL apart) and on its output side
+  // (NS apart in the sub-transform's block)
+  constexpr int IN_J = INPL && LAST ? R : 1, IN_R = INPL && LAST ? 1 : NBL;
+  constexpr bool OUT_IN = INPL && !LAST;
+  const auto in_at = [&](int j) { return j * IN_J; };
+  const auto out_at = [&](int j) { return OUT_IN ? in_at(j) : (j / NS) * NS * R + j % NS; };
+  constexpr int OUT_R = OUT_IN ? IN_R : NS;
   float2 v[KMAX][R];
-  int to[KMAX];  // first element of the butterfly's outputs, -1: none
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     const int b = threadIdx.x + k * NT;
-    const int j = b / MAXL;
-    const int l = b - j * MAXL;
-    to[k] = -1;
+    const int j = b / MAXL, l = b - j * MAXL;
     if (j < NBL && l < lines) {
-      const int base = l * LS;
-      const int kk = j % NS;
-      // spread: elements NBL apart; packed: elements NS apart in the sub-transform's block
-      const int spread = base + j * ES, packed = base + ((j / NS) * NS * R + kk) * ES;
+      const int base = l * LS + (INV ? out_at(j) : in_at(j)) * ES;
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float2 x = INV ? buf[packed + r * NS * ES] : buf[spread + r * NBL * ES];
-        if (!INV && NS > 1 && r > 0) x = cmul(x, tw[(kk * r * STRIDE) * TWM]);
-        v[k][r] = x;
+      for (int r = 0; r < R; ++r) v[k][r] = GLOB && INV ? g[l + (j + r * NBL) * gs] : buf[base + r * (INV ? OUT_R : IN_R) * ES];
+    }
+  }
+  if (GLOB && INV) ready();
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const int b = threadIdx.x + k * NT;
+    const int j = b / MAXL, l = b - j * MAXL;
+    if (j < NBL && l < lines) {
+      const int kk = j % NS;
+      if (!INV && NS > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[k][r] = cmul(v[k][r], tw[(kk * r * STRIDE) * TWM]);
       }
       Dft<R>::run(v[k], s);
       if (INV && NS > 1) {
 #pragma unroll
         for (int r = 1; r < R; ++r) v[k][r] = cmul(v[k][r], cconj(tw[(kk * r * STRIDE) * TWM]));
       }
-      to[k] = INV ? spread : packed;
     }
   }
-  __syncthreads();
+  if (!LAST && !INPL) __syncthreads();
 #pragma unroll
-  for (int k = 0; k < KMAX; ++k)
-    if (to[k] >= 0) {
+  for (int k = 0; k < KMAX; ++k) {
+    const int b = threadIdx.x + k * NT;
+    const int j = b / MAXL, l = b - j * MAXL;
+    if (j < NBL && l < lines) {
+      const int base = l * LS + (INV ? in_at(j) : out_at(j)) * ES;
 #pragma unroll
-      for (int r = 0; r < R; ++r) buf[to[k] + r * (INV ? NBL : NS) * ES] = v[k][r];
+      for (int r = 0; r < R; ++r) {
+        if (GLOB && !INV) g[l + (j + r * NBL) * gs] = v[k][r];
+        else buf[base + r * (INV ? IN_R : OUT_R) * ES] = v[k][r];
+      }
     }
-  __syncthreads();
+  }
+  if (!GLOB || INV) __syncthreads();
 }
 
-template <int N, int ST, int NS, int ES, int NT, int MAXL, int TWM, uint32_t PLAN, bool INV>
+struct NotReady {
+  FHD_DEV void operator()() const {}
+};
+constexpr int plan_stages(uint32_t plan, int n) {
+  int st = 0;
+  for (int done = 1; done < n; ++st) done *= plan_at(plan, n, st);
+  return st;
+}
+
+template <int N, int ST, int NS, int ES, int NT, int MAXL, int TWM, uint32_t PLAN, bool INV, bool GIO, class Ready>
 struct FStages {
-  static FHD_DEV void run(float2* buf, int lines, int LS, const float2* tw) {
+  static FHD_DEV void run(float2* buf, int lines, int LS, const float2* tw, float2* g, int gs, const Ready& ready) {
     constexpr int R = NS >= N ? 1 : plan_at(PLAN, N, ST);
+    constexpr bool INPL = GIO && plan_stages(PLAN, N) == 2;
     if constexpr (R > 1) {
-      if constexpr (!INV) fstage<N, R, NS, ES, NT, MAXL, TWM, INV>(buf, lines, LS, tw);
-      FStages<N, ST + 1, NS * R, ES, NT, MAXL, TWM, PLAN, INV>::run(buf, lines, LS, tw);
-      if constexpr (INV) fstage<N, R, NS, ES, NT, MAXL, TWM, INV>(buf, lines, LS, tw);
+      if constexpr (!INV) fstage<N, R, NS, ES, NT, MAXL, TWM, INV, GIO, INPL>(buf, lines, LS, tw, g, gs, ready);
+      FStages<N, ST + 1, NS * R, ES, NT, MAXL, TWM, PLAN, INV, GIO, Ready>::run(buf, lines, LS, tw, g, gs, ready);
+      if constexpr (INV) fstage<N, R, NS, ES, NT, MAXL, TWM, INV, GIO, INPL>(buf, lines, LS, tw, g, gs, ready);
     }
   }
 };
 
 template <int N, int ES, int NT, int MAXL, int TWM, bool INV, uint32_t PLAN>
 FHD_DEV void ffft(float2* buf, int lines, int LS, const float2* tw) {
-  FStages<N, 0, 1, ES, NT, MAXL, TWM, PLAN, INV>::run(buf, lines, LS, tw);
+  FStages<N, 0, 1, ES, NT, MAXL, TWM, PLAN, INV, false, NotReady>::run(buf, lines, LS, tw, nullptr, 0, NotReady{});
+}
+// The same with the modes in global memory (fstage's GIO).
+template <int N, int ES, int NT, int MAXL, int TWM, bool INV, uint32_t PLAN, class Ready = NotReady>
+FHD_DEV void ffft_modes(float2* buf, int lines, int LS, const float2* tw, float2* g, int gs, const Ready& ready = Ready{}) {
+  FStages<N, 0, 1, ES, NT, MAXL, TWM, PLAN, INV, true, Ready>::run(buf, lines, LS, tw, g, gs, ready);
 }
 
 // ---------------- pass A: real plane -> half spectrum (x) -> FFT along y ----------------
@@ -168,12 +210,8 @@ FHD_BODY void body_fftA(const FftArgs& a, const float* __restrict__ in, float2* 
     }
   }
   __syncthreads();
-  ffft<MY, P, NT, P, 1, false, plan_choice(MY, PY)>(buf, P, 1, twy);
-  float2* dst = spec + (size_t)c * MY * mz * P + (size_t)z * P;
-  for (int e = threadIdx.x; e < MY * P; e += NT) {
-    const int ky = e / P, kx = e - ky * P;
-    dst[(size_t)ky * mz * P + kx] = buf[e];
-  }
+  ffft_modes<MY, P, NT, P, 1, false, plan_choice(MY, PY)>(buf, P, 1, twy, spec + (size_t)c * MY * mz * P + (size_t)z * P,
+                                                          mz * P);
 }
 
 }  // namespace fhd

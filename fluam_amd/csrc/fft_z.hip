@@ -11,7 +11,7 @@
 // (128^3 Stokes 36 us per launch, this form 26.4).  Bound by the LDS crossings and, with noise, by the
 // Philox and Box-Muller arithmetic, with the memory round trips of the ends under other workgroups.
 // Per launch (HIP events, which add about 4 us), staged through LDS and now: Stokes 128^3 31 -> 26.4,
-// 128 x 128 x 256 69 -> 46.6, 128 x 64 x 32 13 -> 10.0, 32^3 9.6 -> 8.0; 108 x 54 x 72 19 -> 11.1.
+// 128 x 128 x 256 69 -> 46.6, 128 x 64 x 32 13 -> 10.0, 32^3 9.6 -> 8.0; 108 x 54 x 72 19 -> 11.0.
 #pragma clang fp contract(off)  // same bits from every instance (fft_fast.hip)
 #include "fhd_device.h"
 #include "fhd_kernels.h"

@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <string.h>
 
 #define FHD_DEV __device__ __forceinline__
 
@@ -30,17 +31,23 @@ inline float2 unit_pair(double c, double s) {
   const bool cl = fabs(c) > fabs(s);
   const float big = cl ? c0 : s0, small = cl ? s0 : c0;
   const double eb = cl ? c : s, es = cl ? s : c;
+  // neighbours by their bits: neither component is near zero
+  const auto ulps = [](float v, int n) {
+    int i;
+    memcpy(&i, &v, 4);
+    i += n;
+    memcpy(&v, &i, 4);
+    return v;
+  };
   double least = 1.0;
   for (int i = -1; i <= 1; ++i) {
-    const float x = i == 0 ? big : nextafterf(big, i > 0 ? 2.0f : -2.0f);
-    float y = small;
-    for (int j = 0; j < 4; ++j) y = nextafterf(y, -2.0f);
-    for (int j = -4; j <= 4; ++j, y = nextafterf(y, 2.0f)) {
-      const double off = fabs(x - eb) + fabs(y - es);
-      const double cost = fabs((double)x * x + (double)y * y - 1.0) + 0.1 * off;
+    const double x = ulps(big, i), offx = fabs(x - eb), x1 = x * x - 1.0;
+    for (int j = -4; j <= 4; ++j) {
+      const double y = ulps(small, j), off = offx + fabs(y - es);
+      const double cost = fabs(x1 + y * y) + 0.1 * off;
       if (off <= 8e-8 && cost < least) {
         least = cost;
-        best = cl ? make_float2(x, y) : make_float2(y, x);
+        best = cl ? make_float2((float)x, (float)y) : make_float2((float)y, (float)x);
       }
     }
   }

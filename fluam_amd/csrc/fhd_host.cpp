@@ -494,7 +494,7 @@ float time_launches(fhd_ctx* c, const std::function<void()>& f, int reps) {
 }
 
 void apply_schedule(fhd_ctx* c) {
-  // keyed by shape and scheme: the W kernel is timed in the form the scheme launches
+  // keyed by shape and scheme
   const std::array<int, 4> key = {c->p.mx, c->p.my, c->p.mz, c->p.scheme};
   const char* env = getenv("FHD_AUTOTUNE");  // 0: default radix plans
   const bool tune = !(env && env[0] == '0');

@@ -26,7 +26,7 @@ inline LinePlan line_plan(int n, int r0, int r1, int r2) {
   }
   return p;
 }
-// Lengths of the size-specialised passes: planes with both edges up to 64, columns up to 128.
+// Edges of the size-specialised planes and of the boxes that a merged batch gathers in one dispatch.
 inline bool fast_edge(int m) { return m == 16 || m == 24 || m == 32 || m == 48 || m == 64; }
 
 struct FftArgs {

@@ -350,8 +350,8 @@ FHD_KERNEL_PAIR_OCC((template <int NT, int ELEMS>), NT, 8, k_fft_z_solve, FftPas
 // Pass C: inverse FFT along y, C2R along x; out = alpha * result + beta * aux.
 // ---------------------------------------------------------------------------------------
 template <int NT, int ELEMS>
-FHD_BODY void body_fft_xy_inv(const FftArgs& a, const float2* __restrict__ spec, float* __restrict__ out,
-                              const float* __restrict__ aux, float alpha, float beta, const Blk& b) {
+FHD_BODY void body_fft_xy_inv(const FftArgs& a, const float2* __restrict__ spec, float* out,
+                              const float* aux, float alpha, float beta, const Blk& b) {
   __shared__ float2 buf[ELEMS];
   __shared__ float2 twx[kMaxFftLen];
   __shared__ float2 twy[kMaxFftLen];

@@ -167,8 +167,8 @@ FHD_BODY void body_fftA128(const FftArgs& a, const float* __restrict__ in, float
 FHD_KERNEL_PAIR((), kNT128, k_fftA128, FftPass, body_fftA128(a.f, a.in, a.spec, b))
 
 // ---------------- inverse: half spectrum -> real plane, out = alpha r + beta aux ----------------
-FHD_BODY void body_fftC128(const FftArgs& a, const float2* __restrict__ spec, float* __restrict__ out,
-                           const float* __restrict__ aux, float alpha, float beta, const Blk& b) {
+FHD_BODY void body_fftC128(const FftArgs& a, const float2* __restrict__ spec, float* out,
+                           const float* aux, float alpha, float beta, const Blk& b) {
   constexpr int H = kM / 2, P = H + 1;
   __shared__ float2 buf[H * kLS];
   __shared__ float2 tw[kM];

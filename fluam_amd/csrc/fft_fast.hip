@@ -21,8 +21,8 @@ FHD_KERNEL_PAIR((template <int MX, int MY, int NT, int PX, int PY>), NT, k_fftA,
 
 // ---------------- pass C: FFT along y (inverse) -> C2R along x -> out = alpha r + beta aux ----
 template <int MX, int MY, int NT, int PX = 0, int PY = 0>
-FHD_BODY void body_fftC(const FftArgs& a, const float2* __restrict__ spec, float* __restrict__ out,
-                        const float* __restrict__ aux, float alpha, float beta, const Blk& b) {
+FHD_BODY void body_fftC(const FftArgs& a, const float2* __restrict__ spec, float* out,
+                        const float* aux, float alpha, float beta, const Blk& b) {
   constexpr int H = MX / 2, P = H + 1;
   __shared__ float2 buf[MY * P];
   __shared__ float2 twx[MX];

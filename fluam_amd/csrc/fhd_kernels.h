@@ -55,15 +55,15 @@ struct FftArgs {
 
 struct FluidWArgs {
   GridDev g;
-  const float* v;          // W += v + lap_coef * L v (nullptr: term off)
-  float lap_coef;
+  const float* v;          // W += v_coef * v + lap_coef * L v (nullptr: term off)
+  float v_coef, lap_coef;
   const float* vadv;       // W += adv_coef * A(vadv)
   float adv_coef;
   const float* adv_prev;   // W += adv_prev_coef * adv_prev (nullptr: off)
   float adv_prev_coef;
   float* adv_store;        // stores A(vadv) when non-null
   const float* base_in;    // W += base_in: the terms of an earlier pass (nullptr: none)
-  float* base_out;         // stores v + lap_coef L v + noise when non-null
+  float* base_out;         // stores v_coef v + lap_coef L v + noise when non-null
   int noise;               // 0 none, 1 Sigma_1
   int trace_free;
   float f1, f4;            // diagonal / off-diagonal noise prefactors

@@ -130,7 +130,7 @@ FHD_BODY void body_fluid_w(const FluidWArgs& a, const Blk& b) {
       }
       const float L = ax * (f[2] - 2.0f * f[0] + f[1]) + ay * (f[4] - 2.0f * f[0] + f[3]) +
                       az * (f[6] - 2.0f * f[0] + f[5]);
-      w[c] += f[0] + a.lap_coef * L;
+      w[c] += a.v_coef * f[0] + a.lap_coef * L;
     }
   }
   if (a.base_out) {

@@ -1,0 +1,87 @@
+"""Rounding errors of whole runs against the FP64 oracle.
+
+The fluid's velocity is kept in 32 bits: 50 steps that each round it to 2.4e-8 of itself leave 1.7e-7,
+the steps' changes (a fifth of the velocity, through transforms good to 2e-7) 2.8e-7 and the noise's own
+6e-8: 3.4e-7 together.  Bound: three times that, 1e-6, for the field and for the root mean square over
+seeds of a particle's three numbers.  The kept part of the velocity is projected again step by step, so its
+divergence stays at the rounding error of the velocity, 6e-8 sqrt(6) / h of it, times 1 / sqrt(1 - s^2) =
+5.7 for a kept share s of 63/64: 8.4e-7 root mean square over the cells, and five times that at the worst of
+4096 of them."""
+import numpy as np
+import pytest
+
+import fluam_amd as F
+import oracle_lib as O
+from fluam_amd._abi import make_params, SCHEME_INCOMPRESSIBLE, SCHEME_QUASI_NEUTRALLY_BUOYANT
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+def pair(scheme, cells, seed, h, kT, dt, **kw):
+    """Both sides of a run that starts at thermal equilibrium."""
+    print(f"[gpu-case] precision scheme={scheme} cells={cells} seed={seed}", flush=True)
+    p = make_params(scheme, cells=cells, box=tuple(h * m for m in cells), temperature=kT, dt=dt, seed=seed, **kw)
+    rng = np.random.default_rng(seed)
+    v = rng.standard_normal(3 * cells[0] * cells[1] * cells[2]) * np.sqrt(kT / h ** 3)
+    v = v.astype(np.float32).astype(np.float64)
+    g, o = F.Simulation(p), O.Oracle(p)
+    g.set_velocity(v)
+    o.set_velocity(v)
+    return p, rng, g, o
+
+
+def test_particle_velocity_of_a_heavy_particle():
+    off = []
+    for seed in range(6):
+        p, rng, g, o = pair(SCHEME_QUASI_NEUTRALLY_BUOYANT, (32, 32, 32), 3 + seed, 10.0, 0.1, 0.25, np=1,
+                            kernel_points=3, mass=8000.0, initial_positions=1, nonbonded=0, cutoff=0.0)
+        q = rng.uniform(-150.0, 150.0, 3)
+        g.set_particles(q)
+        o.set_particles(q)
+        g.step(50)
+        g.sync()
+        o.step(50)
+        off.append(rel(g.particle_velocities(), o.particle_velocities()))
+        assert rel(g.velocity(), o.velocity()) < 1e-6
+    print("  u", " ".join("%.1e" % x for x in off), flush=True)
+    assert np.sqrt(np.mean(np.square(off))) < 1e-6
+
+
+@pytest.mark.parametrize("cells,h,dt", [
+    ((32, 32, 32), 10.0, 0.25),
+    ((48, 24, 16), 1.0, 0.05),
+    ((96, 96, 8), 10.0, 0.25),
+    ((128, 128, 4), 10.0, 0.25),  # in place, also by the kernels with the transform in registers
+    ((108, 54, 12), 10.0, 0.25),
+    ((16, 2, 1), 10.0, 0.25),
+])
+def test_incompressible_velocity(cells, h, dt):
+    p, _, g, o = pair(SCHEME_INCOMPRESSIBLE, cells, 7, h, 1e-3 * h ** 3, dt)
+    g.step(50)
+    g.sync()
+    o.step(50)
+    assert rel(g.velocity(), o.velocity()) < 1e-6
+
+
+@pytest.mark.parametrize("dt", [2.0, 40.0])
+def test_stiff_viscous_step(dt):
+    """Viscous numbers of order one and above: little or nothing of the velocity is kept out of the solve, and
+    the error is that of a solve of the whole velocity, 3.5e-6 over 50 steps, with the modes' 1 + x between."""
+    p, _, g, o = pair(SCHEME_INCOMPRESSIBLE, (24, 32, 16), 9, 1.0, 1e-6, dt)
+    g.step(50)
+    g.sync()
+    o.step(50)
+    assert rel(g.velocity(), o.velocity()) < 1e-5
+
+
+@pytest.mark.parametrize("scheme", [SCHEME_INCOMPRESSIBLE, SCHEME_QUASI_NEUTRALLY_BUOYANT])
+def test_kept_velocity_stays_divergence_free(scheme):
+    """1500 steps at the largest kept share (63/64)."""
+    p, _, g, o = pair(scheme, (16, 16, 16), 11, 10.0, 0.1, 0.25)
+    g.step(1500)
+    rms = np.sqrt(np.mean(np.square(g.velocity())))
+    assert g.max_divergence() * 10.0 / rms < 5 * 8.4e-7

@@ -3,7 +3,6 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include <string.h>
 
 #define FHD_DEV __device__ __forceinline__
 
@@ -19,40 +18,6 @@ FHD_DEV int xcd_item(int b, int n) {
 // n / d for n d < 2^32 by multiplication with ceil(2^32 / d) (0 stands for d = 1).
 __host__ FHD_DEV uint32_t fast_div_magic(int d) { return 0xFFFFFFFFu / (uint32_t)d + 1u; }
 FHD_DEV int fast_div(int n, uint32_t magic) { return magic ? (int)__umulhi((uint32_t)n, magic) : n; }
-
-// (c, s) of the unit circle in FP32, chosen among the neighbours within an ulp or so of the nearest
-// pair for the length closest to 1: rounded to nearest the table's entries are 2e-8 short on
-// average, and each transform multiplies by them on the way there and back.
-inline float2 unit_pair(double c, double s) {
-  const float c0 = (float)c, s0 = (float)s;
-  float2 best = make_float2(c0, s0);
-  if (fabs(c) < 1e-9 || fabs(s) < 1e-9) return best;
-  // one ulp up or down of the larger, a few of the smaller (its steps are finer)
-  const bool cl = fabs(c) > fabs(s);
-  const float big = cl ? c0 : s0, small = cl ? s0 : c0;
-  const double eb = cl ? c : s, es = cl ? s : c;
-  // neighbours by their bits: neither component is near zero
-  const auto ulps = [](float v, int n) {
-    int i;
-    memcpy(&i, &v, 4);
-    i += n;
-    memcpy(&v, &i, 4);
-    return v;
-  };
-  double least = 1.0;
-  for (int i = -1; i <= 1; ++i) {
-    const double x = ulps(big, i), offx = fabs(x - eb), x1 = x * x - 1.0;
-    for (int j = -4; j <= 4; ++j) {
-      const double y = ulps(small, j), off = offx + fabs(y - es);
-      const double cost = fabs(x1 + y * y) + 0.1 * off;
-      if (off <= 8e-8 && cost < least) {
-        least = cost;
-        best = cl ? make_float2((float)x, (float)y) : make_float2((float)y, (float)x);
-      }
-    }
-  }
-  return best;
-}
 
 // Device error flags (bits of the context's error word; cf. fluam's errorKernel,
 // src/allocateErrorArray.cu:22-32): a non-finite particle displacement, and a displacement of

@@ -315,7 +315,7 @@ void build_tables(fhd_ctx* c) {
     std::vector<float2> t(n);
     for (int k = 0; k < n; ++k) {
       double a = -2.0 * M_PI * (double)k / (double)n;
-      t[k] = unit_pair(cos(a), sin(a));
+      t[k] = make_float2((float)cos(a), (float)sin(a));
     }
     return t;
   };
@@ -328,7 +328,7 @@ void build_tables(fhd_ctx* c) {
     std::vector<float2> t(n);
     for (int k = 0; k < n; ++k) {
       double a = M_PI * (double)k / (double)n;
-      t[k] = unit_pair(cos(a), sin(a));
+      t[k] = make_float2((float)cos(a), (float)sin(a));
     }
     return t;
   };

@@ -34,6 +34,17 @@ def pair(scheme, cells, seed, h, kT, dt, **kw):
     return p, rng, g, o
 
 
+@pytest.mark.parametrize("mx", [16, 48, 54, 96, 128, 256])
+def test_forward_transform_of_a_point_gives_the_nearest_twiddles(mx):
+    """A point next to the origin transforms to e^{-2 pi i k / mx}: 32-bit twiddles rounded to nearest are off
+    by at most 2^-25 a component, 2^-25 / sqrt(3) root mean square, and nothing else rounds on the way."""
+    a = np.zeros((16, 16, mx))
+    a[0, 0, 1] = 1.0
+    off = F.fft_r2c(a)[0, 0] - np.exp(-2j * np.pi * np.arange(mx // 2 + 1) / mx)
+    assert max(abs(off.real).max(), abs(off.imag).max()) < 1.0001 * 2.0 ** -25
+    assert np.sqrt(np.mean(np.abs(off) ** 2)) < np.sqrt(2.0 / 3.0) * 2.0 ** -25
+
+
 def test_particle_velocity_of_a_heavy_particle():
     off = []
     for seed in range(6):

@@ -207,7 +207,7 @@ struct fhd_ctx {
   int4* scell[2] = {nullptr, nullptr};
   float4* soff[2] = {nullptr, nullptr};
   unsigned* key[2] = {nullptr, nullptr};  // plane_key of each sorted slot
-  float margin = 0.0f;     // most that a source's stencil is displaced along z
+  float margin = 0.0f;     // most that a source's stencil is displaced along an axis
   float4* rfd = nullptr;   // normals of the RFD displacement, by sorted slot of set 0
   int* errd = nullptr;
   // harmonic bonds (bondedForces); null when the run has none
@@ -686,6 +686,7 @@ PlaneSrc spread_values(fhd_ctx* c, int k, const float4* val, float coef) {
   memset(&p, 0, sizeof(p));
   p.t = c->t;
   p.kernel_points = c->p.kernel_points;
+  p.near = 1;
   p.out_coef = (float)(1.0 / c->dV);
   p.ngroups = 1;
   p.grp[0].set = sset(c, k);
@@ -876,6 +877,7 @@ void step_stokes(fhd_ctx* c) {
     r.disp = (float)(0.5 * p.rfd_delta);
     r.rfd_quirk = p.rfd_mode == FHD_RFD_REFERENCE;
     r.wide = (int)std::min(64.0, std::ceil(2.0 * c->margin / c->dz));
+    sp.near = c->margin <= std::min(c->dx, c->dy);
     spread_forward(c, sp, nullptr);
   } else {
     launch_zero_f(c->W, 3 * (size_t)c->g.N, c->s);

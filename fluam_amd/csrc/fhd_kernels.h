@@ -149,6 +149,7 @@ struct SpreadGroup {
 struct PlaneSrc {
   Tiles t;
   int kernel_points;
+  int near;             // no source is displaced by more than a cell along x or y
   int ngroups;
   SpreadGroup grp[2];
   float out_coef;       // multiplies the accumulated field

@@ -185,6 +185,15 @@ FHD_DEV void add_nodes(int* acc, int pitch, const GridDev& g, const AxisWeights&
   }
 }
 
+// Most that an axis of m cells contributes to what a source adds to a node, per unit of its value: one
+// weight (1/2 of 4 points, 2/3 of 3), or the sum of those that a narrow axis folds onto the node, which is
+// more only on an axis of one cell, where it is all of them.  deriv: derivative weights may take the
+// place of the plain ones (thermal drift: 1/2 and 1; folded onto one cell they cancel).
+template <int NPTS>
+FHD_DEV float axis_most(int m, bool deriv) {
+  return m == 1 ? 1.0f : NPTS == 4 ? 0.5f : deriv ? 1.0f : 2.0f / 3.0f;
+}
+
 struct PlaneLds {
   unsigned short list[kListCap];  // group 0's hits from the front, group 1's from the back
   int runs[2][6];
@@ -341,7 +350,6 @@ FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, con
   if (sweep == 0 && tid == 0) L.bound = L.most = 0;
   __syncthreads();
   const bool two = P.ngroups > 1;
-  const int wide = max(P.grp[0].wide, two ? P.grp[1].wide : 0);
   bool one;  // every group's sources have 16-bit indices
   {
     const PlaneRuns r0 = plane_runs(L, 0);
@@ -369,12 +377,12 @@ FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, con
   int nhit0 = uniform(L.n[0]);
   const int nhit1 = uniform(L.n[1]);
   one = one && nhit0 + nhit1 <= kListCap;
-  // most sources at a node: its stencils come from cells at most 2 + ceil(wide / 2) away, within
-  // one block of 4 each way while that is at most 3
+  // most sources at a node: its stencils come from cells at most 3 away, so from the blocks of 4 around
+  // its own, unless a pair is displaced by more than a cell along x or y
   const auto count_and_clear = [&] {
     if (sweep == 0) {
       int most = 0;
-      if (wide <= 2) {
+      if (P.near) {
         for (int e = tid; e < bx * by; e += NT) {
           const int y = e / bx, x = e - y * bx;
           int s = 0;
@@ -443,11 +451,13 @@ FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, con
   }
   __syncthreads();
   if (one) nhit0 = uniform(L.kept);
-  // contributions are below value x the largest product of weights: 1/2 each (4-point) or 2/3
-  // (3-point), with a derivative weight (at most 1/2 and 1) in place of one of them for the drift
+  // what a source adds to a node is below value x the product of its axes' most (axis_most)
   const float top = __int_as_float(uniform(L.bound));
   const bool bad = top > 3.0e38f;
-  const float m = bad ? 0.0f : top * (NPTS == 4 ? 0.1251f : P.grp[0].drift != 0.0f ? 0.4446f : 0.2964f);
+  const bool drift = P.grp[0].drift != 0.0f;
+  const float most = axis_most<NPTS>(g.mx, drift && C == 0) * axis_most<NPTS>(g.my, drift && C == 1) *
+                     axis_most<NPTS>(g.mz, drift && C == 2);
+  const float m = bad ? 0.0f : 1.001f * top * most;
   const int n = max(uniform(L.most), 1);
   int e2 = -90;
   if (m > 0.0f) {
@@ -455,7 +465,9 @@ FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, con
     frexpf(m, &e);  // m < 2^e
     e2 = max(e, -90);
   }
-  const int S = 30 - (31 - __clz(n));  // n 2^S <= 2^31
+  // n 2^S <= 2^31; a source's up to eight additions to a node round by half a unit each, which the
+  // thousandth above covers while S >= 13
+  const int S = 30 - (31 - __clz(n)) - (n > 65536 ? 1 : 0);
   const float scale = ldexpf(1.0f, S - e2);
   const float scale2 = sweep == 0 ? 0.0f : ldexpf(1.0f, S);
   for (int gi = 0; gi < P.ngroups; ++gi) {

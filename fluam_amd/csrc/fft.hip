@@ -176,9 +176,11 @@ FHD_DEV void lds_fft(float2* buf, const Lines& ln, const LinePlan& p, const floa
 template <int NT, int ELEMS, bool SP>
 FHD_BODY void body_fft_xy_fwd(const FftArgs& a, const float* __restrict__ in, float2* __restrict__ spec,
                               const Blk& b, const PlaneSrc* src_sp) {
-  __shared__ float2 buf[ELEMS];
-  // the twiddles of both transforms; before they are stored, plane_spread's lists
+  __shared__ __align__(16) float2 buf[ELEMS];  // plane_spread clears it 16 bytes at a time
+  // the twiddles of both transforms; before they are stored, plane_spread's lists (whose scales lie beyond
+  // the twiddles)
   constexpr int kTw = 2 * kMaxFftLen * sizeof(float2);
+  static_assert(offsetof(PlaneLds, scale) >= kTw, "the scales are read while the twiddles are stored");
   __shared__ __align__(16) unsigned char side[SP && (int)sizeof(PlaneLds) > kTw ? (int)sizeof(PlaneLds) : kTw];
   float2* const twx = reinterpret_cast<float2*>(side);
   float2* const twy = twx + kMaxFftLen;
@@ -206,27 +208,28 @@ FHD_BODY void body_fft_xy_fwd(const FftArgs& a, const float* __restrict__ in, fl
     // workgroup's own rows of the spectrum (at least mx floats each), written later
     float* part = reinterpret_cast<float*>(spec + ((size_t)c * my * mz + z) * P);
     int* acc = reinterpret_cast<int*>(buf);
-    float inv2, rest;
-    const float inv = plane_spread<NT>(acc, 2 * my * PS, 2 * PS, a.g, *src_sp, z, c, pl, 0, &inv2);
-    if (inv2 != 0.0f) {
+    const bool more = plane_spread<NT, false>(acc, 2 * my * PS, 2 * PS, a.g, *src_sp, z, c, pl);
+    const PlaneUnit unit = plane_unit(pl, *src_sp, a.g);
+    if (more) {
       for (int e = threadIdx.x; e < h * my; e += NT) {
-        const int y = fast_div(e, a.mdh);
-        const int2 q = *reinterpret_cast<const int2*>(&buf[e + y * (PS - h)]);
-        float* at = part + (size_t)y * mz * 2 * P + 2 * (e - y * h);
-        at[0] = inv * (float)q.x;
-        at[1] = inv * (float)q.y;
+        const int y = fast_div(e, a.mdh), x = e - y * h;
+        const int2 q = *reinterpret_cast<const int2*>(&buf[x + y * PS]);
+        const float f = unit.at(pl, 2 * x, y);
+        float* at = part + (size_t)y * mz * 2 * P + 2 * x;
+        at[0] = f * (float)q.x;
+        at[1] = f * (float)q.y;
       }
       __syncthreads();
-      plane_spread<NT>(acc, 2 * my * PS, 2 * PS, a.g, *src_sp, z, c, pl, 1, &rest);
+      plane_spread<NT, true>(acc, 2 * my * PS, 2 * PS, a.g, *src_sp, z, c, pl);
     }
-    const float f = inv2 != 0.0f ? inv2 : inv;
     for (int e = threadIdx.x; e < h * my; e += NT) {
-      const int y = fast_div(e, a.mdh);
-      float2* at_e = &buf[e + y * (PS - h)];
+      const int y = fast_div(e, a.mdh), x = e - y * h;
+      float2* at_e = &buf[x + y * PS];
       const int2 q = *reinterpret_cast<const int2*>(at_e);
+      const float f = unit.at(pl, 2 * x, y) * (more ? unit.rest : 1.0f);
       float2 r = make_float2(f * (float)q.x, f * (float)q.y);
-      if (inv2 != 0.0f) {
-        const float* at = part + (size_t)y * mz * 2 * P + 2 * (e - y * h);
+      if (more) {
+        const float* at = part + (size_t)y * mz * 2 * P + 2 * x;
         r = cadd(r, make_float2(at[0], at[1]));
       }
       *at_e = in ? cadd(r, src[e]) : r;

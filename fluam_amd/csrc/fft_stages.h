@@ -126,9 +126,10 @@ template <int MX, int MY, int NT, int PX, int PY, bool SP>
 FHD_BODY void body_fftA(const FftArgs& a, const float* __restrict__ in, float2* __restrict__ spec, const Blk& b,
                         const PlaneSrc* src_sp) {
   constexpr int H = MX / 2, P = H + 1;
-  __shared__ float2 buf[MY * P];
-  // the twiddles; before they are stored, plane_spread's lists
+  __shared__ __align__(16) float2 buf[MY * P];  // plane_spread clears it 16 bytes at a time
+  // the twiddles; before they are stored, plane_spread's lists (whose scales lie beyond the twiddles)
   constexpr int kTw = (MX + MY) * sizeof(float2);
+  static_assert(offsetof(PlaneLds, scale) >= kTw, "the scales are read while the twiddles are stored");
   __shared__ __align__(16) unsigned char side[SP && (int)sizeof(PlaneLds) > kTw ? (int)sizeof(PlaneLds) : kTw];
   float2* const twx = reinterpret_cast<float2*>(side);
   float2* const twy = twx + MX;
@@ -166,24 +167,25 @@ FHD_BODY void body_fftA(const FftArgs& a, const float* __restrict__ in, float2* 
     const auto at = [&](int e) { return (size_t)(e / (MX / 2)) * mz * 2 * P + 2 * (e % (MX / 2)); };
     int* acc = reinterpret_cast<int*>(buf);
     const float2* src2 = reinterpret_cast<const float2*>(src);
-    float inv2, rest;
-    const float inv = plane_spread<NT>(acc, 2 * MY * P, 2 * P, a.g, *src_sp, z, c, pl, 0, &inv2);
-    if (inv2 != 0.0f) {
+    const bool more = plane_spread<NT, false>(acc, 2 * MY * P, 2 * P, a.g, *src_sp, z, c, pl);
+    const PlaneUnit unit = plane_unit(pl, *src_sp, a.g);
+    if (more) {
       for (int e = threadIdx.x; e < MY * H; e += NT) {
         const int2 q = *reinterpret_cast<const int2*>(&buf[e / H * P + e % H]);
-        part[at(e)] = inv * (float)q.x;
-        part[at(e) + 1] = inv * (float)q.y;
+        const float f = unit.at(pl, 2 * (e % H), e / H);
+        part[at(e)] = f * (float)q.x;
+        part[at(e) + 1] = f * (float)q.y;
       }
       __syncthreads();
-      plane_spread<NT>(acc, 2 * MY * P, 2 * P, a.g, *src_sp, z, c, pl, 1, &rest);
+      plane_spread<NT, true>(acc, 2 * MY * P, 2 * P, a.g, *src_sp, z, c, pl);
     }
-    const float f = inv2 != 0.0f ? inv2 : inv;
 #pragma unroll 2
     for (int e = threadIdx.x; e < MY * H; e += NT) {
       float2* at_e = &buf[e / H * P + e % H];
       const int2 q = *reinterpret_cast<const int2*>(at_e);
+      const float f = unit.at(pl, 2 * (e % H), e / H) * (more ? unit.rest : 1.0f);
       float2 r = make_float2(f * (float)q.x, f * (float)q.y);
-      if (inv2 != 0.0f) r = cadd(r, make_float2(part[at(e)], part[at(e) + 1]));
+      if (more) r = cadd(r, make_float2(part[at(e)], part[at(e) + 1]));
       *at_e = in ? cadd(r, src2[e]) : r;
     }
   }

@@ -7,10 +7,11 @@
 // and src/kernelSpreadParticles.cu:3012-4082.
 //
 // The contributions are added as 32-bit fixed-point integers by LDS atomics: integer addition is
-// associative, so the field is bit-identical whatever order they arrive in.  The scale comes from
-// the plane's largest source value and from the largest number of sources whose stencils can meet
-// at one node (counted in blocks of 4 x 4 columns), so that no node's sum reaches 2^31; with more
-// than kOneLimb of them a second sweep adds what the first one's rounding left over.
+// associative, so the field is bit-identical whatever order they arrive in.  Every 4 x 4 block of columns
+// has its own scale, from the largest value among the sources that can reach it and from their number, so
+// that no node's sum reaches 2^31 and a weak force is rounded by its own neighbourhood's measure, not by
+// the plane's strongest; with more than kOneLimb sources in reach of a block a second sweep adds what the
+// first one's rounding left over.
 //
 // Bound by the latency of its dependent phases and, for the pairs, by the vector instructions of
 // the rows; a plane is one workgroup, so at 128^3 half the CUs hold two of the 384 planes and half
@@ -22,13 +23,14 @@
 //  1. scan: the sources sorted into the tile layers that can reach the plane are tested by a 4-byte
 //     key (their half cell along z and their 4 x 4 block of columns); the hits enter the plane's
 //     count and a list in LDS (ballot compaction).
-//  2. values: vector values are read for the bound, and the hits with a zero component (a particle
-//     with no WCA neighbour) leave the list.
+//  2. values: vector values are read for the blocks' counts and bounds, and the hits with a zero component
+//     (a particle with no WCA neighbour) leave the list.
 //  3. add: one lane per listed source computes its weights along x and y and its weight on this
 //     plane, and adds the 9 or 16 nodes of the row.  The two rows of a random-finite-difference
 //     pair have the same nodes but for the few particles within the displacement of a half cell's
 //     face, so their difference is added at once.
 #pragma once
+#include <stddef.h>
 #include "fhd_device.h"
 #include "fhd_kernels.h"
 
@@ -36,6 +38,7 @@ namespace fhd {
 
 constexpr int kListCap = 6144;     // hits listed at once (also the sources scanned per chunk when more)
 constexpr int kOneLimb = 255;      // most sources per node for a single 32-bit sum
+constexpr int kPlaneBlocks = 1024; // 4 x 4 blocks of the largest plane that can hold particles
 
 // The key of a sorted slot: bits 0-8 its half cell along z (wrapped cell, sign of the offset), bit
 // 9 set when a displacement below `margin` may change it, bits 16 up its block of 4 x 4 columns.
@@ -161,30 +164,6 @@ FHD_DEV int node_at(int b, int k, int m) {
   return n;
 }
 
-// Adds the nodes of a row (weights wx and wy times r), or of the difference of two rows on the same
-// nodes (PAIR: minus vx and vy times s).
-template <int NPTS, bool PAIR>
-FHD_DEV void add_nodes(int* acc, int pitch, const GridDev& g, const AxisWeights& wx, const AxisWeights& wy, float r,
-                       const AxisWeights& vx, const AxisWeights& vy, float s, float scale2) {
-  int xs[NPTS];
-#pragma unroll
-  for (int k = 0; k < NPTS; ++k) xs[k] = node_at(wx.base, k, g.mx);
-#pragma unroll
-  for (int ky = 0; ky < NPTS; ++ky) {
-    const int row = node_at(wy.base, ky, g.my) * pitch;
-    const float wyz = wy.w[ky] * r, vyz = PAIR ? vy.w[ky] * s : 0.0f;
-#pragma unroll
-    for (int kx = 0; kx < NPTS; ++kx) {
-      float v = wx.w[kx] * wyz;
-      if (PAIR) v = fmaf(-vx.w[kx], vyz, v);
-      // rounded: truncation would shift every sum toward zero (it tripled the velocity's error)
-      int n = (int)rintf(v);
-      if (scale2 != 0.0f) n = (int)rintf((v - (float)n) * scale2);
-      atomicAdd(&acc[row + xs[kx]], n);
-    }
-  }
-}
-
 // Most that an axis of m cells contributes to what a source adds to a node, per unit of its value: one
 // weight (1/2 of 4 points, 2/3 of 3), or the sum of those that a narrow axis folds onto the node, which is
 // more only on an axis of one cell, where it is all of them.  deriv: derivative weights may take the
@@ -199,15 +178,62 @@ struct PlaneLds {
   int runs[2][6];
   int n[2];   // the groups' hit counts
   int kept;   // group 0's hits with a value
-  int bound;  // largest value (float bits)
   int most;   // most sources that can meet at a node
+  int top;    // largest value (float bits)
+  int bad;    // an overflowed or NaN source
+  signed char scale[kPlaneBlocks];  // binary exponent of each 4 x 4 block's fixed-point scale
 };
+
+// Binary exponent of the fixed-point scale of nodes that at most n sources reach, each with less than t.
+FHD_DEV int count_exp(int n) {
+  // n 2^S <= 2^31; a source's up to eight additions to a node round by half a unit each, which the
+  // thousandth in plane_scale covers while S >= 13
+  n = max(n, 1);
+  return 30 - (31 - __clz(n)) - (n > 65536 ? 1 : 0);
+}
+FHD_DEV int plane_scale(int n, float t) {
+  int e = -90;
+  if (t > 0.0f) frexpf(1.001f * t, &e);  // t < 2^e
+  return count_exp(n) - max(e, -90);
+}
+
+// Adds the nodes of a row (weights wx and wy times r), or of the difference of two rows on the same
+// nodes (PAIR: minus vx and vy times s).  Four nodes lie in at most two blocks along an axis.
+template <int NPTS, bool PAIR>
+FHD_DEV void add_nodes(int* acc, int pitch, const GridDev& g, const PlaneLds& L, const AxisWeights& wx,
+                       const AxisWeights& wy, float r, const AxisWeights& vx, const AxisWeights& vy, float s,
+                       float scale2) {
+  const int nbx = (g.mx + 3) >> 2, nby = (g.my + 3) >> 2;
+  const int xa = wx.base >> 2, xb = xa + 1 == nbx ? 0 : xa + 1;
+  const int ya = wy.base >> 2, yb = ya + 1 == nby ? 0 : ya + 1;
+  const int aa = L.scale[xa + nbx * ya], ba = L.scale[xb + nbx * ya];
+  const int ab = L.scale[xa + nbx * yb], bb = L.scale[xb + nbx * yb];
+  int xs[NPTS];
+#pragma unroll
+  for (int k = 0; k < NPTS; ++k) xs[k] = node_at(wx.base, k, g.mx);
+#pragma unroll
+  for (int ky = 0; ky < NPTS; ++ky) {
+    const int y = node_at(wy.base, ky, g.my), row = y * pitch;
+    const bool own = y >> 2 == ya;
+    const int ea = own ? aa : ab, eb = own ? ba : bb;
+    const float wyz = wy.w[ky] * r, vyz = PAIR ? vy.w[ky] * s : 0.0f;
+#pragma unroll
+    for (int kx = 0; kx < NPTS; ++kx) {
+      float v = wx.w[kx] * wyz;
+      if (PAIR) v = fmaf(-vx.w[kx], vyz, v);
+      v = ldexpf(v, xs[kx] >> 2 == xa ? ea : eb);
+      // rounded: truncation would shift every sum toward zero (it tripled the velocity's error)
+      int n = (int)rintf(v);
+      if (scale2 != 0.0f) n = (int)rintf((v - (float)n) * scale2);
+      atomicAdd(&acc[row + xs[kx]], n);
+    }
+  }
+}
 
 FHD_DEV int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // Appends the kept entries of a wave's lanes to the front of the list.
-FHD_DEV void list_keep(PlaneLds& L, bool keep, int entry) {
-  const int lane = threadIdx.x & 63;
+FHD_DEV void list_keep(PlaneLds& L, int lane, bool keep, int entry) {
   const unsigned long long bal = __ballot(keep);
   if (bal == 0) return;
   int at = 0;
@@ -226,27 +252,27 @@ FHD_DEV PlaneRuns plane_runs(const PlaneLds& L, int gi) {
   return r;
 }
 
-// Lists the hits among sources [i0, i1) of group gi (entries relative to i0); `count`: also counts
-// them by block.  K keys of a lane are in flight at once.
+// Lists the hits among sources [i0, i1) of group gi (entries relative to i0); `pairs`: also counts
+// them, two each, by block (null: not).  K keys of a lane are in flight at once.
 template <int NT, int K>
-FHD_DEV void plane_keys(const SpreadGroup& G, const PlaneRuns& runs, int b, int i1, unsigned key[K]) {
+FHD_DEV void plane_keys(const SpreadGroup& G, const PlaneRuns& runs, int tid, int b, int i1, unsigned key[K]) {
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const int i = b + k * NT + (int)threadIdx.x;
+    const int i = b + k * NT + tid;
     key[k] = i < i1 ? G.key[runs.slot(i)] : ~0u;
   }
 }
 template <int NT, int K>
-FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, const unsigned key[K], int b, int i0, int z, int C,
-                        PlaneLds& L, int* blocks, bool count) {
+FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, const unsigned key[K], int b, int i0, int z, int C,
+                        PlaneLds& L, int* pairs) {
   const SpreadGroup& G = P.grp[gi];
-  const int lane = threadIdx.x & 63;
+  const int lane = tid & 63;
   unsigned long long bal[K];
   int total = 0;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const bool hit = key[k] != ~0u && row_hits(key[k] & 511, key[k] & 512 ? G.wide : 0, z, g.mz, P.kernel_points, C == 2);
-    if (hit && count) atomicAdd(&blocks[key[k] >> 16], G.mode == SRC_RFD ? 2 : 1);
+    if (hit && pairs) atomicAdd(&pairs[key[k] >> 16], 2);
     bal[k] = __ballot(hit);
     total += __popcll(bal[k]);
   }
@@ -258,19 +284,19 @@ FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, const unsig
   for (int k = 0; k < K; ++k) {
     const int mine = at + __popcll(bal[k] & ((1ull << lane) - 1ull));
     if ((bal[k] >> lane & 1) && mine < kListCap)
-      L.list[gi == 0 ? mine : kListCap - 1 - mine] = (unsigned short)(b + k * NT + (int)threadIdx.x - i0);
+      L.list[gi == 0 ? mine : kListCap - 1 - mine] = (unsigned short)(b + k * NT + tid - i0);
     at += __popcll(bal[k]);
   }
 }
 // from: the first source scanned (i0 or later).
 template <int NT>
-FHD_DEV void plane_scan(const GridDev& g, const PlaneSrc& P, int gi, const PlaneRuns& runs, int i0, int from, int i1,
-                        int z, int C, PlaneLds& L, int* blocks, bool count) {
+FHD_DEV void plane_scan(const GridDev& g, const PlaneSrc& P, int gi, int tid, const PlaneRuns& runs, int i0, int from, int i1,
+                        int z, int C, PlaneLds& L, int* pairs) {
   constexpr int K = 4;
   for (int b = from; b < i1; b += K * NT) {
     unsigned key[K];
-    plane_keys<NT, K>(P.grp[gi], runs, b, i1, key);
-    plane_test<NT, K>(g, P, gi, key, b, i0, z, C, L, blocks, count);
+    plane_keys<NT, K>(P.grp[gi], runs, tid, b, i1, key);
+    plane_test<NT, K>(g, P, gi, tid, key, b, i0, z, C, L, pairs);
   }
 }
 
@@ -281,8 +307,8 @@ FHD_DEV float src_value(const SpreadGroup& G, int j, int C) {
 
 // Adds source j's row to the plane.
 template <int NPTS>
-FHD_DEV void plane_add(int* acc, int pitch, const GridDev& g, const SpreadGroup& G, int j, int z, int C, float scale,
-                       float scale2) {
+FHD_DEV void plane_add(int* acc, int pitch, const GridDev& g, const PlaneLds& L, const SpreadGroup& G, int j, int z,
+                       int C, float scale2) {
   float v = src_value(G, j, C);
   v = fabsf(v) <= 3.0e38f ? v : 0.0f;  // the plane is marked already
   const int4 c = G.set.cell[j];
@@ -292,20 +318,20 @@ FHD_DEV void plane_add(int* acc, int pitch, const GridDev& g, const SpreadGroup&
     const bool face = a == C;
     return src_axis<NPTS>(ca, da, 0.0f, h, ih, m, face, false, v, face ? drift : 0.0f);
   };
-  float r = row_weight<NPTS>(axis(2, c.z, d.z, g.dz, g.idz, g.mz), z, g.mz) * scale;
+  float r = row_weight<NPTS>(axis(2, c.z, d.z, g.dz, g.idz, g.mz), z, g.mz);
   if (drift == 0.0f) r *= v;
   const AxisWeights wx = axis(0, c.x, d.x, g.dx, g.idx, g.mx), wy = axis(1, c.y, d.y, g.dy, g.idy, g.my);
-  add_nodes<NPTS, false>(acc, pitch, g, wx, wy, r, wx, wy, 0.0f, scale2);
+  add_nodes<NPTS, false>(acc, pitch, g, L, wx, wy, r, wx, wy, 0.0f, scale2);
 }
 
 // Adds the difference of both rows of RFD pair j.
 template <int NPTS>
-FHD_DEV void plane_add_pair(int* acc, int pitch, const GridDev& g, const SpreadGroup& G, int j, int z, int C, float scale,
-                            float scale2) {
+FHD_DEV void plane_add_pair(int* acc, int pitch, const GridDev& g, const PlaneLds& L, const SpreadGroup& G, int j, int z,
+                            int C, float scale2) {
   const int4 c = G.set.cell[j];
   const float4 d = G.set.off[j];
   const float4 w = G.val[j];
-  const float v = (C == 0 ? w.x : C == 1 ? w.y : w.z) * G.coef * scale;
+  const float v = (C == 0 ? w.x : C == 1 ? w.y : w.z) * G.coef;
   const bool quirk = G.rfd_quirk;
   const auto zw = [&](float s) {
     return v * row_weight<NPTS>(src_axis<NPTS>(c.z, d.z, s * w.z, g.dz, g.idz, g.mz, C == 2, quirk, 0.0f, 0.0f), z, g.mz);
@@ -316,40 +342,65 @@ FHD_DEV void plane_add_pair(int* acc, int pitch, const GridDev& g, const SpreadG
   const AxisWeights y0 = src_axis<NPTS>(c.y, d.y, G.disp * w.y, g.dy, g.idy, g.my, C == 1, quirk, 0.0f, 0.0f);
   const AxisWeights y1 = src_axis<NPTS>(c.y, d.y, -G.disp * w.y, g.dy, g.idy, g.my, C == 1, quirk, 0.0f, 0.0f);
   if (x0.base == x1.base && y0.base == y1.base) {
-    add_nodes<NPTS, true>(acc, pitch, g, x0, y0, r0, x1, y1, r1, scale2);
+    add_nodes<NPTS, true>(acc, pitch, g, L, x0, y0, r0, x1, y1, r1, scale2);
   } else {
-    add_nodes<NPTS, false>(acc, pitch, g, x0, y0, r0, x0, y0, 0.0f, scale2);
-    add_nodes<NPTS, false>(acc, pitch, g, x1, y1, -r1, x1, y1, 0.0f, scale2);
+    add_nodes<NPTS, false>(acc, pitch, g, L, x0, y0, r0, x0, y0, 0.0f, scale2);
+    add_nodes<NPTS, false>(acc, pitch, g, L, x1, y1, -r1, x1, y1, 0.0f, scale2);
   }
 }
-template <int NPTS, int NT>
-FHD_DEV void plane_add_list(int* acc, int pitch, const GridDev& g, const SpreadGroup& G, int gi, const PlaneRuns& runs,
-                            int i0, int nh, int z, int C, const PlaneLds& L, float scale, float scale2) {
-  for (int k = threadIdx.x; k < nh; k += NT) {
-    const int j = runs.slot(i0 + L.list[gi == 0 ? k : kListCap - 1 - k]);
-    if (G.mode == SRC_RFD) plane_add_pair<NPTS>(acc, pitch, g, G, j, z, C, scale, scale2);
-    else plane_add<NPTS>(acc, pitch, g, G, j, z, C, scale, scale2);
+template <int NPTS, int NT, bool PAIRS>
+FHD_DEV void plane_add_list(int* acc, int pitch, const GridDev& g, const SpreadGroup& G, int tid, const PlaneRuns& runs,
+                            int i0, int nh, int z, int C, const PlaneLds& L, float scale2) {
+  for (int k = tid; k < nh; k += NT) {
+    const int j = runs.slot(i0 + L.list[PAIRS ? kListCap - 1 - k : k]);
+    if (PAIRS) plane_add_pair<NPTS>(acc, pitch, g, L, G, j, z, C, scale2);
+    else plane_add<NPTS>(acc, pitch, g, L, G, j, z, C, scale2);
   }
 }
 
-// Accumulates the plane into acc (`words` words, row pitch `pitch`, cleared here) and returns what
-// the integers are to be multiplied by; *inv2 != 0: the caller takes these sums (times the returned
-// factor) and calls again with sweep 1 for the remainders, to be multiplied by *inv2.  Every lane
-// of the workgroup calls it; the plane is complete (barrier passed) on return.
-template <int NPTS, int NT>
-FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, const PlaneSrc& P, int z, int C,
-                           PlaneLds& L, int sweep, float* inv2) {
-  int* const blocks = acc;  // the block counts, until the plane is cleared
-  const int tid = threadIdx.x, lane = tid & 63;
+// Group 0 (vector values) or 1 (pairs): `nh` listed hits, or where they are more than the list holds
+// (`one` false) chunks of as many sources.
+template <int NPTS, int NT, bool PAIRS>
+FHD_DEV void plane_add_group(int* acc, int pitch, const GridDev& g, const PlaneSrc& P, int tid, int z, int C, PlaneLds& L,
+                             bool one, int nh, float scale2) {
+  const SpreadGroup& G = P.grp[PAIRS];
+  const PlaneRuns r = plane_runs(L, PAIRS);
+  const int all = one ? 1 : r.total();
+  for (int i0 = 0; i0 < all; i0 += kListCap) {
+    if (!one) {
+      __syncthreads();  // the previous chunk's list consumed
+      if (tid == 0) L.n[PAIRS] = 0;
+      __syncthreads();
+      plane_scan<NT>(g, P, PAIRS, tid, r, i0, i0, min(all, i0 + kListCap), z, C, L, nullptr);
+      __syncthreads();
+      nh = uniform(L.n[PAIRS]);
+    }
+    plane_add_list<NPTS, NT, PAIRS>(acc, pitch, g, G, tid, r, i0, nh, z, C, L, scale2);
+  }
+}
+
+// Accumulates the plane into acc (`words` words, row pitch `pitch`, cleared here) and returns whether a
+// second call (REST) is to follow, for what the rounding of this one's integers left over: the caller
+// adds the sums of both, times plane_unit.  Every lane of the workgroup calls it; the plane is complete
+// (barrier passed) on return.
+template <int NPTS, int NT, bool REST>
+FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, const PlaneSrc& P, int z, int C,
+                          PlaneLds& L) {
+  int tid = threadIdx.x;
+
+  const int lane = tid & 63;
   const int bx = (g.mx + 3) >> 2, by = (g.my + 3) >> 2;
+  // each block's sources and their largest value (float bits), until the scales are known
+  int *const count = acc, *const top = acc + bx * by;
+  const int head = !REST ? min(words, (2 * bx * by + 3) & ~3) : 0;
   if (tid < 12 && tid < 6 * P.ngroups) L.runs[tid >= 6][tid % 6] = run_bound(P.t, P.grp[tid >= 6], z, tid % 6);
-  if (sweep == 0)
-    for (int e = tid; e < bx * by; e += NT) blocks[e] = 0;
+  for (int e = tid; e < head; e += NT) acc[e] = 0;
   if (tid < 2) L.n[tid] = 0;
   if (tid == 0) L.kept = 0;
-  if (sweep == 0 && tid == 0) L.bound = L.most = 0;
+  if (!REST && tid == 0) L.most = L.top = L.bad = 0;
   __syncthreads();
   const bool two = P.ngroups > 1;
+  int* const pairs = !REST ? count : nullptr;
   bool one;  // every group's sources have 16-bit indices
   {
     const PlaneRuns r0 = plane_runs(L, 0);
@@ -357,19 +408,19 @@ FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, con
     // the first keys of both groups are in flight at once
     constexpr int K = 4;
     unsigned k0[K], k1[K];
-    plane_keys<NT, K>(P.grp[0], r0, 0, n0, k0);
+    plane_keys<NT, K>(P.grp[0], r0, tid, 0, n0, k0);
     PlaneRuns r1 = r0;
     int n1 = 0;
     if (two) {
       r1 = plane_runs(L, 1);
       n1 = r1.total();
-      plane_keys<NT, K>(P.grp[1], r1, 0, n1, k1);
+      plane_keys<NT, K>(P.grp[1], r1, tid, 0, n1, k1);
     }
-    plane_test<NT, K>(g, P, 0, k0, 0, 0, z, C, L, blocks, sweep == 0);
-    if (n0 > K * NT) plane_scan<NT>(g, P, 0, r0, 0, K * NT, n0, z, C, L, blocks, sweep == 0);
+    plane_test<NT, K>(g, P, 0, tid, k0, 0, 0, z, C, L, nullptr);
+    if (n0 > K * NT) plane_scan<NT>(g, P, 0, tid, r0, 0, K * NT, n0, z, C, L, nullptr);
     if (two) {
-      plane_test<NT, K>(g, P, 1, k1, 0, 0, z, C, L, blocks, sweep == 0);
-      if (n1 > K * NT) plane_scan<NT>(g, P, 1, r1, 0, K * NT, n1, z, C, L, blocks, sweep == 0);
+      plane_test<NT, K>(g, P, 1, tid, k1, 0, 0, z, C, L, pairs);
+      if (n1 > K * NT) plane_scan<NT>(g, P, 1, tid, r1, 0, K * NT, n1, z, C, L, pairs);
     }
     one = n0 <= 65536 && n1 <= 65536;
   }
@@ -377,46 +428,31 @@ FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, con
   int nhit0 = uniform(L.n[0]);
   const int nhit1 = uniform(L.n[1]);
   one = one && nhit0 + nhit1 <= kListCap;
-  // most sources at a node: its stencils come from cells at most 3 away, so from the blocks of 4 around
-  // its own, unless a pair is displaced by more than a cell along x or y
-  const auto count_and_clear = [&] {
-    if (sweep == 0) {
-      int most = 0;
-      if (P.near) {
-        for (int e = tid; e < bx * by; e += NT) {
-          const int y = e / bx, x = e - y * bx;
-          int s = 0;
-          for (int dy = -1; dy <= min(1, by - 2); ++dy) {
-            const int yy = y + dy < 0 ? by - 1 : y + dy >= by ? 0 : y + dy;
-            for (int dx = -1; dx <= min(1, bx - 2); ++dx) {
-              const int xx = x + dx < 0 ? bx - 1 : x + dx >= bx ? 0 : x + dx;
-              s += blocks[xx + bx * yy];
-            }
-          }
-          most = max(most, s);
-        }
-      } else {
-        most = nhit0 + 2 * nhit1;
-      }
-      most = wave_max_i32(most);
-      if (lane == 0) atomicMax(&L.most, most);
-    }
-    __syncthreads();
+  const auto clear = [&](int from, int to) {  // both multiples of 4, or the plane's end
     int4* acc4 = reinterpret_cast<int4*>(acc);
-    for (int e = tid; e < words / 4; e += NT) acc4[e] = make_int4(0, 0, 0, 0);
-    if (tid < (words & 3)) acc[(words & ~3) + tid] = 0;
+    for (int e = from / 4 + tid; e < to / 4; e += NT) acc4[e] = make_int4(0, 0, 0, 0);
+    if (tid < (to & 3)) acc[(to & ~3) + tid] = 0;
   };
-  // bound of the values: a pair's normals are below 5.8 (24-bit uniforms), vector values are read
-  // (under the count).  Group 0 holds vector values; its listed hits without one leave the list.
+  // Group 0 holds vector values: those of its hits enter their blocks' counts and bounds, and the listed
+  // hits without one leave the list.
   {
     const SpreadGroup& G = P.grp[0];
     const PlaneRuns r = plane_runs(L, 0);
     const float drift = fabsf(G.drift) * (C == 0 ? g.idx : C == 1 ? g.idy : g.idz);
-    float m = two ? 5.8f * fabsf(P.grp[1].coef) : 0.0f;
+    const auto enter = [&](float v, unsigned key) {
+      const float a = fabsf(v) + drift;
+      const bool fine = a <= 3.0e38f;
+      if (!fine) L.bad = 1;
+      if (!REST) {
+        atomicAdd(&count[key >> 16], 1);
+        atomicMax(&top[key >> 16], __float_as_int(fine ? a : 3.0e38f));
+      }
+    };
     if (one) {
       constexpr int K = (kListCap + NT - 1) / NT;
       constexpr int KF = 3;  // values of a lane in flight at once
       unsigned short e[KF];
+      unsigned key[KF];
       float v[KF];
       // rounds of KF x NT entries, each read in full before the shorter list overwrites it
       for (int k0 = 0; k0 < K * NT && (k0 == 0 || k0 < nhit0); k0 += KF * NT) {
@@ -426,79 +462,96 @@ FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, con
           v[k] = 0.0f;
           if (i < nhit0) {
             e[k] = L.list[i];
-            v[k] = src_value(G, r.slot(e[k]), C);
+            const int j = r.slot(e[k]);
+            key[k] = G.key[j];
+            v[k] = src_value(G, j, C);
           }
         }
-        if (k0 == 0) count_and_clear();
-        else __syncthreads();
+        if (k0 == 0) clear(head, words);
+        __syncthreads();
 #pragma unroll
         for (int k = 0; k < KF; ++k) {
-          const bool in = k0 + tid + k * NT < nhit0;
-          const float a = fabsf(v[k]) + drift;
-          if (in) m = fmaxf(m, a <= 3.0e38f ? a : 3.4e38f);  // overflowed or NaN: marks the plane
-          list_keep(L, in && (v[k] != 0.0f || drift != 0.0f), e[k]);
+          const bool keep = k0 + tid + k * NT < nhit0 && (v[k] != 0.0f || drift != 0.0f);
+          if (keep) enter(v[k], key[k]);
+          list_keep(L, lane, keep, e[k]);
         }
       }
     } else {
-      count_and_clear();
+      clear(head, words);
       for (int i = tid; i < r.total(); i += NT) {
-        const float a = fabsf(src_value(G, r.slot(i), C)) + drift;
-        m = fmaxf(m, a <= 3.0e38f ? a : 3.4e38f);
+        const int j = r.slot(i);
+        const unsigned key = G.key[j];
+        if (!row_hits(key & 511, key & 512 ? G.wide : 0, z, g.mz, NPTS, C == 2)) continue;
+        const float v = src_value(G, j, C);
+        if (v != 0.0f || drift != 0.0f) enter(v, key);
       }
     }
-    const int w = wave_max_i32(__float_as_int(m));
-    if (lane == 0) atomicMax(&L.bound, w);
   }
   __syncthreads();
   if (one) nhit0 = uniform(L.kept);
-  // what a source adds to a node is below value x the product of its axes' most (axis_most)
-  const float top = __int_as_float(uniform(L.bound));
-  const bool bad = top > 3.0e38f;
-  const bool drift = P.grp[0].drift != 0.0f;
-  const float most = axis_most<NPTS>(g.mx, drift && C == 0) * axis_most<NPTS>(g.my, drift && C == 1) *
-                     axis_most<NPTS>(g.mz, drift && C == 2);
-  const float m = bad ? 0.0f : 1.001f * top * most;
-  const int n = max(uniform(L.most), 1);
-  int e2 = -90;
-  if (m > 0.0f) {
-    int e;
-    frexpf(m, &e);  // m < 2^e
-    e2 = max(e, -90);
-  }
-  // n 2^S <= 2^31; a source's up to eight additions to a node round by half a unit each, which the
-  // thousandth above covers while S >= 13
-  const int S = 30 - (31 - __clz(n)) - (n > 65536 ? 1 : 0);
-  const float scale = ldexpf(1.0f, S - e2);
-  const float scale2 = sweep == 0 ? 0.0f : ldexpf(1.0f, S);
-  for (int gi = 0; gi < P.ngroups; ++gi) {
-    const SpreadGroup& G = P.grp[gi];
-    const PlaneRuns r = plane_runs(L, gi);
-    // more hits than the list holds: chunks of as many sources
-    const int all = one ? 1 : r.total(), step = one ? 1 : kListCap;
-    for (int i0 = 0; i0 < all; i0 += step) {
-      int nh = gi == 0 ? nhit0 : nhit1;
-      if (!one) {
-        __syncthreads();  // the previous chunk's list consumed
-        if (tid == 0) L.n[gi] = 0;
-        __syncthreads();
-        plane_scan<NT>(g, P, gi, r, i0, i0, min(all, i0 + step), z, C, L, blocks, false);
-        __syncthreads();
-        nh = uniform(L.n[gi]);
+  if (!REST) {
+    // The scale of a block's nodes: their sources lie in cells at most 3 away, so in the blocks around it,
+    // unless a pair is displaced by more than a cell along x or y (then the plane has one scale).  What a
+    // source adds to a node is below value x the product of its axes' most; a pair's normals are below 5.8
+    // (24-bit uniforms).
+    const bool drift = P.grp[0].drift != 0.0f;
+    const float most = axis_most<NPTS>(g.mx, drift && C == 0) * axis_most<NPTS>(g.my, drift && C == 1) *
+                       axis_most<NPTS>(g.mz, drift && C == 2);
+    const float pair = two ? 5.8f * fabsf(P.grp[1].coef) : 0.0f;
+    if (tid == 0 && !(pair <= 3.0e38f)) L.bad = 1;
+    const float floor = fminf(pair, 3.0e38f);
+    int n_most = 0, t_most = 0;
+    for (int e = tid; e < bx * by; e += NT) {
+      const int y = e / bx, x = e - y * bx;
+      int n = 0, t = 0;
+      for (int dy = -1; dy <= min(1, by - 2); ++dy) {
+        const int yy = y + dy < 0 ? by - 1 : y + dy >= by ? 0 : y + dy;
+        for (int dx = -1; dx <= min(1, bx - 2); ++dx) {
+          const int xx = x + dx < 0 ? bx - 1 : x + dx >= bx ? 0 : x + dx;
+          n += count[xx + bx * yy];
+          t = max(t, top[xx + bx * yy]);
+        }
       }
-      plane_add_list<NPTS, NT>(acc, pitch, g, G, gi, r, one ? 0 : i0, nh, z, C, L, scale, scale2);
+      if (P.near) L.scale[e] = (signed char)plane_scale(n, most * fmaxf(__int_as_float(t), floor));
+      n_most = max(n_most, n);
+      t_most = max(t_most, t);
     }
+    n_most = wave_max_i32(P.near ? n_most : nhit0 + 2 * nhit1);
+    if (lane == 0) atomicMax(&L.most, n_most);
+    if (!P.near) {
+      t_most = wave_max_i32(t_most);
+      if (lane == 0) atomicMax(&L.top, t_most);
+    }
+    __syncthreads();
+    clear(0, head);
+    if (!P.near) {
+      const int x = plane_scale(L.most, most * fmaxf(__int_as_float(L.top), floor));
+      for (int e = tid; e < bx * by; e += NT) L.scale[e] = (signed char)x;
+    }
+    __syncthreads();
   }
+  const float scale2 = !REST ? 0.0f : ldexpf(1.0f, count_exp(uniform(L.most)));
+  plane_add_group<NPTS, NT, false>(acc, pitch, g, P, tid, z, C, L, one, nhit0, scale2);
+  if (two) plane_add_group<NPTS, NT, true>(acc, pitch, g, P, tid, z, C, L, one, nhit1, scale2);
   __syncthreads();
-  // an overflowed or NaN source: the plane is written non-finite, which the interpolation flags
-  const float inv = bad ? __builtin_inff() : ldexpf(1.0f, e2 - S) * P.out_coef;
-  *inv2 = n > kOneLimb && !bad ? ldexpf(inv, -S) : 0.0f;
-  return inv;
+  return !REST && uniform(L.most) > kOneLimb && uniform(L.bad) == 0;
 }
-template <int NT>
-FHD_DEV float plane_spread(int* acc, int words, int pitch, const GridDev& g, const PlaneSrc& P, int z, int C,
-                           PlaneLds& L, int sweep, float* inv2) {
-  return P.kernel_points == 4 ? plane_spread<4, NT>(acc, words, pitch, g, P, z, C, L, sweep, inv2)
-                              : plane_spread<3, NT>(acc, words, pitch, g, P, z, C, L, sweep, inv2);
+template <int NT, bool REST>
+FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, const PlaneSrc& P, int z, int C,
+                          PlaneLds& L) {
+  return P.kernel_points == 4 ? plane_spread<4, NT, REST>(acc, words, pitch, g, P, z, C, L)
+                              : plane_spread<3, NT, REST>(acc, words, pitch, g, P, z, C, L);
+}
+
+// What the integers at node (x, y) are to be multiplied by, those of the second call by `rest` times as much.  A plane
+// with an overflowed or NaN source is written non-finite, which the interpolation flags.
+struct PlaneUnit {
+  float coef, rest;
+  int nbx;
+  FHD_DEV float at(const PlaneLds& L, int x, int y) const { return ldexpf(coef, -L.scale[(x >> 2) + nbx * (y >> 2)]); }
+};
+FHD_DEV PlaneUnit plane_unit(const PlaneLds& L, const PlaneSrc& P, const GridDev& g) {
+  return PlaneUnit{uniform(L.bad) ? __builtin_inff() : P.out_coef, ldexpf(1.0f, -count_exp(uniform(L.most))), (g.mx + 3) >> 2};
 }
 
 }  // namespace fhd

@@ -74,3 +74,52 @@ def test_one_axis_of_one_cell_without_forces(tmp_path):
 def test_displacements_across_flat_cells(tmp_path, kernel):
     """Displacements of up to 1.45 in cells of 0.25 x 0.25 x 2."""
     run(tmp_path, ST, (32, 24, 8), 500, kernel, 9, box=(8.0, 6.0, 16.0), rfd_delta=0.5)
+
+
+@pytest.mark.parametrize("scheme,cells,n,kernel,kw", [
+    (ST, (32, 32, 16), 600, 4, {}),    # one 32-bit sum
+    (ST, (16, 16, 8), 5000, 4, {}),    # two sums, every hit listed
+    (ST, (16, 16, 8), 20000, 3, {}),   # two sums, the list in chunks
+    (QNB, (32, 32, 16), 600, 3, {}),
+    (QNB, (16, 16, 8), 5000, 3, {}),
+    (QNB, (16, 16, 8), 20000, 4, {}),
+    (QNB, (8, 4, 2), 300, 4, {}),      # two sums in a box narrower than a stencil
+    (ST, (64, 16, 8), 9000, 4, {"rfd_delta": 2.5}),  # displaced beyond the neighbouring blocks: one scale
+    (ST, (72, 36, 8), 9000, 4, {}),    # runtime-size passes
+    (QNB, (128, 128, 4), 12000, 4, {}),
+])
+def test_crowded_planes_with_forces(tmp_path, scheme, cells, n, kernel, kw):
+    run(tmp_path, scheme, cells, n, kernel, 300 + kernel, **kw)
+
+
+def test_weak_forces_beside_a_strong_one(tmp_path):
+    """Thirty particles feel a force a millionth of that on one particle of the same plane, which sixty force-free ones
+    surround (so many sources in reach of a node take bits from its sum).  The Stokes flow is linear: what the
+    weak forces add to their particles' velocities is what they give alone, up to the rounding of the strong
+    one's field, about 2e-7 of its root mean square in each of the two runs subtracted; bound: three times that."""
+    m, rng = 128, np.random.default_rng(4)
+    q = np.zeros((91, 3))
+    q[1:61] = rng.uniform(-1.5, 1.5, (60, 3))
+    q[61:] = np.stack([*rng.uniform(12.0, 52.0, (2, 30)) * rng.choice([-1.0, 1.0], (2, 30)), rng.uniform(-0.5, 0.5, 30)], 1)
+    q += 0.3
+    pull = rng.standard_normal((91, 3))
+    pull /= np.linalg.norm(pull, axis=1)[:, None]
+
+    def velocities(name, strong, weak):
+        k = {**({0: 1.0} if strong else {}), **({i: 1e-6 for i in range(61, 91)} if weak else {})}
+        lines = ["0", str(len(k))] + [f"{i} {c} 0.0 " + " ".join(repr(float(x)) for x in q[i] + pull[i]) for i, c in k.items()]
+        (tmp_path / name).write_text("\n".join(lines) + "\n")
+        p = make_params(ST, cells=(m, m, m), np=91, kernel_points=4, nonbonded=0, temperature=0.0, dt=1e-4, seed=1,
+                        initial_positions=0, cutoff=0.0, bonded_forces=str(tmp_path / name))
+        print(f"[gpu-case] weak beside strong: {name}", flush=True)
+        g = F.Simulation(p)
+        g.set_particles(q.T.ravel())
+        g.step(1)
+        return g.particle_velocities().reshape(3, -1)[:, 61:], np.sqrt(np.mean(np.square(g.velocity())))
+
+    strong, rms = velocities("strong", True, False)
+    both, _ = velocities("both", True, True)
+    alone, _ = velocities("weak", False, True)
+    off = np.sqrt(np.mean(np.square(both - strong - alone)))
+    print(f"  off {off:.2e} of {np.sqrt(np.mean(np.square(alone))):.2e}, rms {rms:.2e}", flush=True)
+    assert off < 3.0 * np.sqrt(2.0) * 2e-7 * rms

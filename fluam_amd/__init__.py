@@ -288,7 +288,7 @@ class Simulation:
         return ms.value
 
     def schedule(self):
-        """The autotuned schedule: z-pass column tile, xy (forward, inverse) and z radix plans,
+        """The schedule in use: z-pass column tile, xy (forward, inverse) and z radix plans,
         W-kernel z chunks."""
         out = (C.c_int * 6)()
         if not lib().fhd_get_schedule(self.h, out):

@@ -447,11 +447,14 @@ void launch_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc&
 }
 // Lengths without an instance in fft_z.hip, or all of them when the runtime-size kernels are forced.
 // Columns per workgroup: the schedule's tile, as far as the largest class holds it.
+int z_columns(const FftArgs& a, int want) {
+  const int fast = a.generic ? 0 : fast_z_columns(a.g.mz, want);
+  const int most = kClassElems[2] / (3 * (a.g.mz | 1));  // >= 10: mz is at most 256
+  return fast ? fast : want < most ? want : most;
+}
 void launch_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s) {
   if (!a.generic && fast_fft_z_solve(a, spec, s)) return;
-  const int LS = a.g.mz | 1;
-  const int most = kClassElems[2] / (3 * LS);  // >= 10: mz is at most 256
-  const int want = a.btile < most ? a.btile : most;
+  const int LS = a.g.mz | 1, want = z_columns(a, a.btile);
   const int ntile = (a.g.P + want - 1) / want, T = (a.g.P + ntile - 1) / ntile;
   const FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, T};
   FHD_LAUNCH_CLASS(lds_class(3 * T * LS), k_fft_z_solve, FAM_FFT_Z, dim3(ntile, a.g.my), x, s);

@@ -15,7 +15,8 @@
 // real columns kx = 0 and kx = 64 share one complex column (their y transforms are the real
 // and imaginary parts of one complex transform, separated afterwards).  512 lanes per plane:
 // every lane has work in both transforms.  Same layouts, tables and results (to FP32
-// rounding) as the Stockham passes; the schedule autotuner times the two and keeps the faster.
+// rounding) as the Stockham passes; they run only when forced (FHD_PLAN_XY=9): 27.2 and
+// 32.4 us per launch at 128^3 against 20.1 and 20.6.
 // The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
 // on the one alone and on the other in a merged batch), so the compiler must not choose which
 // products become fused multiply-adds: the fused ones are written out.

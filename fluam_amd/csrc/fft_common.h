@@ -237,7 +237,7 @@ constexpr int plan_radix(int n, int st) {
 }
 
 // Explicit radix plans, 5 bits per stage from the first (0 ends the plan; plan 0 is the default
-// above).  The schedule autotuner picks those of 96 x 96 and 128 x 128 planes among the candidates below.
+// above).  Those of 96 x 96 and 128 x 128 planes are square_plan's, or forced with FHD_PLAN_XY.
 constexpr uint32_t plan2(int r0, int r1) { return (uint32_t)r0 | ((uint32_t)r1 << 5); }
 constexpr uint32_t plan3(int r0, int r1, int r2) { return plan2(r0, r1) | ((uint32_t)r2 << 10); }
 constexpr int plan_at(uint32_t plan, int n, int st) { return plan ? (int)((plan >> (5 * st)) & 31u) : plan_radix(n, st); }

@@ -92,10 +92,9 @@ static void launch_AC_plan(const FftPass& x, int which, int mz, hipStream_t s) {
   else
     launch(k_fftC<MX, MY, NT, PX, PY>, k_fftC_b<MX, MY, NT, PX, PY>, FAM_FFT_XY_INV, dim3(mz, x.f.ncomp), NT, x, s);
 }
-// The radix plans of the x and y transforms (plan_choice indices, px + 3 py) come from the
-// schedule autotuner for 96 x 96 and 128 x 128 planes, one for the forward and one for the
-// inverse pass (128 x 128 also has 9: the register-transform kernels of fft128.hip); other
-// planes use the default plan.
+// The radix plans of the x and y transforms (plan_choice indices, px + 3 py) are square_plan's and can
+// be forced for 96 x 96 and 128 x 128 planes (128 x 128 also has 9: the register-transform kernels of
+// fft128.hip); every other plane has plan 0.
 template <int MX, int MY, int NT>
 static void launch_AC_nt(const FftPass& x, int which, int mz, hipStream_t s) {
   if constexpr ((MX == 128 && MY == 128) || (MX == 96 && MY == 96)) {

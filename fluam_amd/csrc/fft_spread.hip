@@ -1,5 +1,5 @@
 // fft_spread.hip -- the forward xy pass with spreading for the plane shapes of fft_fast.hip: mx x my
-// with both lengths in {16, 24, 32, 48, 64} or mx = my in {96, 128}, default radix plans.
+// with both lengths in {16, 24, 32, 48, 64} or mx = my in {96, 128}.
 // The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
 // on the one alone and on the other in a merged batch), so the compiler must not choose which
 // products become fused multiply-adds: the fused ones are written out.
@@ -9,7 +9,8 @@
 namespace fhd {
 
 FHD_KERNEL_PAIR_OCC((template <int MX, int MY, int NT>), NT, 8, k_spread_fftA, FftSpread,
-                    body_fftA<MX, MY, NT, 0, 0, true>(a.p.f, a.p.in, a.p.spec, b, &a.s))
+                    body_fftA<MX, MY, NT, MX == MY ? square_plan(MX) % 3 : 0, MX == MY ? square_plan(MX) / 3 : 0, true>(
+                        a.p.f, a.p.in, a.p.spec, b, &a.s))
 
 
 // Lanes per plane workgroup as in the plain pass of a context launched alone; batched dispatches

@@ -197,10 +197,15 @@ FHD_BODY void body_z_merged(const FftPass& x, const Blk& b) {
 }
 FHD_KERNEL_PAIR_OCC((), kMergedLanes, 8, k_fftz_merged, FftPass, body_z_merged(a, b))
 
+int fast_z_columns(int mz, int want) {
+  if (mz > 256 || !zr1(mz)) return 0;
+  return want <= 2 ? 2 : want <= 4 ? 4 : 8;  // beyond 8 the workgroups are too few and too large
+}
+
 template <int N>
 static bool launch_z(const FftArgs& a, float2* spec, hipStream_t s) {
   const bool merged = t_recorder && zmerged(N);
-  const int tile = a.btile <= 2 ? 2 : a.btile <= 4 ? 4 : 8;  // beyond 8 the workgroups are too few and too large
+  const int tile = fast_z_columns(N, a.btile);
   const int most = merged ? kMergedLanes / zr1(N) / a.ncomp : tile * 3 / a.ncomp;
   const int ntile = (a.g.P + most - 1) / most, T = (a.g.P + ntile - 1) / ntile;
   const FftPass x{a, nullptr, spec, nullptr, nullptr, 0.0f, 0.0f, T, fast_div_magic(T), fast_div_magic(a.ncomp * T)};

@@ -13,9 +13,6 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
-#include <array>
-#include <functional>
-#include <map>
 #include <mutex>
 #include <stdexcept>
 #include <fstream>
@@ -451,11 +448,10 @@ FluidWArgs base_w(fhd_ctx* c) {
   return w;
 }
 
-// ---------------- schedule autotuner ----------------
-// The z-pass column tile and the W kernel's chunk follow the grid's size; the radix plans of
-// 96 x 96 and 128 x 128 planes are timed once per grid shape on the
-// first context of that shape and cached for the process: a replica's schedule depends on its shape
-// only, never on what else runs beside it.
+// ---------------- schedule ----------------
+// The z-pass column tile and the W kernel's chunk follow the grid's size; the radix plans are one per plane
+// shape (square_plan) and column length.  So a replica's schedule depends on its shape only, and a run's bits
+// on nothing but its inputs: plans round differently, so none is chosen by timing.
 
 // Columns of a z-pass workgroup: 4, fewer where that leaves the chip less than a workgroup per CU, and 8
 // where the grid still has four per CU and their LDS leaves room for five.  Per launch with 2, 4, 8
@@ -465,78 +461,22 @@ int z_tile(int mx, int my, int mz) {
   const int P = mx / 2 + 1;
   return P / 8 * my >= 1024 && mz <= 144 ? 8 : P / 4 * my >= 256 ? 4 : 2;
 }
-struct Sched {
-  int btile, zchunk, zchunk_b, plan_xy, plan_xy_inv;
-};
-std::mutex g_sched_mu;
-std::map<std::array<int, 4>, Sched> g_sched;
-
-// Shortest of three timed rounds of reps launches (one warm-up launch first), so one slow
-// round does not decide the schedule.
-float time_launches(fhd_ctx* c, const std::function<void()>& f, int reps) {
-  hipEvent_t a, b;
-  HIPCHK(hipEventCreate(&a));
-  HIPCHK(hipEventCreate(&b));
-  f();  // warm-up
-  float best = 1e30f;
-  for (int round = 0; round < 3; ++round) {
-    HIPCHK(hipEventRecord(a, c->s));
-    for (int k = 0; k < reps; ++k) f();
-    HIPCHK(hipEventRecord(b, c->s));
-    HIPCHK(hipEventSynchronize(b));
-    float ms = 0.0f;
-    HIPCHK(hipEventElapsedTime(&ms, a, b));
-    best = std::min(best, ms);
-  }
-  (void)hipEventDestroy(a);
-  (void)hipEventDestroy(b);
-  return best;
-}
-
+// Two planes per W workgroup: per launch with 1, 2, 4 planes 5.3, 5.2, 6.8 us at 32^3, 12.4, 7.5, 7.3 at
+// 64^3, 13.9, 9.4, 11.9 at 96 x 48 x 64.
 void apply_schedule(fhd_ctx* c) {
-  // keyed by shape and scheme
-  const std::array<int, 4> key = {c->p.mx, c->p.my, c->p.mz, c->p.scheme};
-  const char* env = getenv("FHD_AUTOTUNE");  // 0: default radix plans
-  const bool tune = !(env && env[0] == '0');
-  std::lock_guard<std::mutex> lock(g_sched_mu);
-  auto it = g_sched.find(key);
-  // two planes per W workgroup: per launch with 1, 2, 4 planes 5.3, 5.2, 6.8 us at 32^3, 12.4, 7.5, 7.3 at
-  // 64^3, 13.9, 9.4, 11.9 at 96 x 48 x 64
-  Sched sc = {z_tile(c->p.mx, c->p.my, c->p.mz), 2, 2, 0, 0};
-  if (it != g_sched.end()) {
-    sc = it->second;
-  } else if (tune) {
-    // scratch runs on the context's own buffers before its state exists (contents irrelevant)
-    // xy passes of 96 x 96 and 128 x 128 planes: the radix plans of the x and y transforms
-    // (three each) of the LDS-stage kernels, and for 128 x 128 the register-transform kernels
-    // (plan 9), chosen for the forward and the inverse pass separately
-    const bool sq128 = c->p.mx == 128 && c->p.my == 128, sq96 = c->p.mx == 96 && c->p.my == 96;
-    if (sq128 || sq96) {
-      float best = 1e30f, best_inv = 1e30f;
-      for (int pxy = 0; pxy < (sq128 ? 10 : 9); ++pxy) {  // 9: the register-transform kernels
-        c->fa.plan_xy = c->fa.plan_xy_inv = pxy;
-        const float tf = time_launches(c, [&] { launch_fft_xy_fwd(c->fa, c->W, c->spec, c->s); }, 4);
-        const float ti =
-            time_launches(c, [&] { launch_fft_xy_inv(c->fa, c->spec, c->W, nullptr, 1.0f, 0.0f, c->s); }, 4);
-        if (tf < best) { best = tf; sc.plan_xy = pxy; }
-        if (ti < best_inv) { best_inv = ti; sc.plan_xy_inv = pxy; }
-      }
-      c->fa.plan_xy = sc.plan_xy;
-      c->fa.plan_xy_inv = sc.plan_xy_inv;
-    }
-    g_sched[key] = sc;
-  }
-  c->fa.btile = sc.btile;
-  c->fa.plan_xy = sc.plan_xy;
-  c->fa.plan_xy_inv = sc.plan_xy_inv;
-  c->zchunk = sc.zchunk;
-  c->zchunk_b = sc.zchunk_b;
-  // explicit radix plans (tests and experiments): FHD_PLAN_XY in 0-9 (128 x 128 planes; 0-8
-  // for 96 x 96), FHD_PLAN_Z in 0-2 (accepted, no effect: the z pass has one plan per length)
+  c->fa.btile = z_tile(c->p.mx, c->p.my, c->p.mz);
+  c->zchunk = c->zchunk_b = 2;
+  const int edge = c->p.mx == c->p.my && !c->fa.generic ? c->p.mx : 0;
+  c->fa.plan_xy = c->fa.plan_xy_inv = square_plan(edge);
+  // explicit radix plans (tests and experiments): FHD_PLAN_XY in 0-9 (passes without spreading of 128 x 128
+  // planes; 0-8 for 96 x 96), FHD_PLAN_Z in 0-2 (accepted, no effect: the z pass has one plan per length)
   if (const char* e = getenv("FHD_PLAN_XY")) {
     const int v = atoi(e);
     if (v < 0 || v > 9) throw std::runtime_error("FHD_PLAN_XY must be 0-9");
-    c->fa.plan_xy = c->fa.plan_xy_inv = v;
+    if (edge == 128 || (edge == 96 && v < 9)) {
+      if (c->p.np == 0) c->fa.plan_xy = v;
+      c->fa.plan_xy_inv = v;
+    }
   }
   if (const char* e = getenv("FHD_PLAN_Z")) {
     const int v = atoi(e);
@@ -546,12 +486,12 @@ void apply_schedule(fhd_ctx* c) {
   if (const char* e = getenv("FHD_BTILE")) {
     const int v = atoi(e);
     if (v != 2 && v != 4 && v != 8 && v != 16) throw std::runtime_error("FHD_BTILE must be 2, 4, 8 or 16");
-    c->fa.btile = v;
+    c->fa.btile = z_columns(c->fa, v);
   }
   if (const char* e = getenv("FHD_ZCHUNK")) {
     const int v = atoi(e);
     if (v < 1) throw std::runtime_error("FHD_ZCHUNK must be at least 1");
-    c->zchunk = c->zchunk_b = v;
+    c->zchunk = c->zchunk_b = v >= 4 ? 4 : v >= 2 ? 2 : 1;
   }
 }
 
@@ -2345,6 +2285,7 @@ int fhd_fft_r2c_noalloc(int mx, int my, int mz, const float* in, float* out_spec
     const float* gt = reinterpret_cast<const float*>(tab + 6 * kMaxFftLen);
     a.gx = gt; a.gy = gt + kMaxFftLen; a.gz = gt + 2 * kMaxFftLen;
     fill_plans(a, mx, my, mz);
+    a.plan_xy = square_plan(mx == my ? mx : 0);
     a.btile = 8;
     a.zmode = 1;
     a.ncomp = 1;

@@ -29,6 +29,12 @@ inline LinePlan line_plan(int n, int r0, int r1, int r2) {
 // Edges of the size-specialised planes and of the boxes that a merged batch gathers in one dispatch.
 inline bool fast_edge(int m) { return m == 16 || m == 24 || m == 32 || m == 48 || m == 64; }
 
+// The radix plans (px + 3 py) of the xy passes of m x m planes, one for both directions: an inverse with
+// the forward pass's plan undoes its rounded twiddles.  Per launch (HIP events, which add about 4 us), plan 0
+// and this one: 96^3 forward 14.6, 14.0 and inverse 15.2, 14.4 us (the others up to 15), 128^3 20.3, 20.2
+// and 20.8, 19.9 us (the others 20.4-21.6; 9, with the transform in registers, 27.2 and 32.4).
+constexpr int square_plan(int m) { return m == 96 ? 3 : m == 128 ? 2 : 0; }
+
 struct FftArgs {
   GridDev g;
   const float2 *twx, *twy, *twz;  // e^{-2 pi i m / m_a}, m < m_a
@@ -37,7 +43,7 @@ struct FftArgs {
   LinePlan lx, ly, lz;            // transforms of mx/2, my and mz points (runtime-size kernels)
   uint32_t mdh, mdp, mdy;         // fast_div's reciprocals of mx/2, P and my
   int btile;                      // kx columns per pass-B workgroup (2, 4, 8 or 16)
-  int plan_xy;                    // radix plans of the forward xy pass (96 x 96, 128 x 128 planes): px + 3 py, 0 default
+  int plan_xy;                    // radix plans of the forward xy pass (96 x 96, 128 x 128 planes): px + 3 py
   int plan_xy_inv;                // the same for the inverse xy pass
   int zmode;                      // 0: FFT_z, operator, inverse FFT_z; 1: FFT_z only; 2: inverse only
   int ncomp;                      // velocity components transformed (3; 1 for a single field, transform-only modes)
@@ -303,6 +309,7 @@ struct FftSpread {
 bool fast_fft_xy_fwd(const FftArgs& a, const float* in, float2* spec, hipStream_t s);
 bool fast_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc& src, float2* spec, hipStream_t s);
 bool fast_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s);
+int fast_z_columns(int mz, int want);  // 0: not a length of fft_z.hip
 bool fast_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha, float beta,
                      hipStream_t s);
 
@@ -313,6 +320,8 @@ void launch_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc&
 // The 128 x 128 xy passes with the transforms in registers (which 0: forward, 1: inverse).
 void launch_fft128_xy(const FftPass& x, int which, int mz, hipStream_t s);
 void launch_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s);
+// The column tile that the z pass of these lengths runs with when asked for `want`.
+int z_columns(const FftArgs& a, int want);
 void launch_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha,
                        float beta, hipStream_t s);
 void launch_fluid_w(const FluidWArgs& a, hipStream_t s);

@@ -162,13 +162,13 @@ int fhd_get_np(const fhd_ctx* c);
 int fhd_time_steps(fhd_ctx* c, int nsteps, double* ms);
 int fhd_profile_kernels(fhd_ctx* c, int nsteps, double* kern_ms, char* kern_names, int nkern);
 
-/* The schedule of the context's grid shape (no fluam counterpart), by rule but for the xy radix plans of
- * 128 x 128 and 96 x 96 planes, which are timed: out[0] the z-pass column tile, out[1] the forward xy pass's radix plan (x plan + 3 y plan, 0-8, for 128 x 128
- * planes: x 16 4 | 4 16 | 8 8, y 16 8 | 8 16 | 4 4 8, and 9: the transforms in registers; for
- * 96 x 96 planes: x 16 3 | 3 16 | 4 4 3, y 16 2 3 | 8 4 3 | 3 8 4; 0 elsewhere), out[2] the z
- * pass's radix plan (always 0: one plan per length), out[3]
- * and out[4] the W kernel's z chunk alone and in batched dispatches, out[5] the inverse xy pass's
- * radix plan (the same candidates as out[1]). */
+/* The schedule that the context's passes run with, by rule from its grid's shape (no fluam counterpart):
+ * out[0] the z-pass column tile, out[1] the forward xy pass's radix plan (x plan + 3 y plan; 2 for
+ * 128 x 128 planes and 3 for 96 x 96, unless another is forced with FHD_PLAN_XY and the pass has no
+ * spreading; 128 x 128: x 16 4 | 4 16 | 8 8, y 16 8 | 8 16 | 4 4 8, and 9: the transforms in registers;
+ * 96 x 96: x 16 3 | 3 16 | 4 4 3, y 16 2 3 | 8 4 3 | 3 8 4; 0 for other planes), out[2] the z pass's
+ * radix plan (always 0: one plan per length), out[3] and out[4] the W kernel's z chunk alone and in
+ * batched dispatches, out[5] the inverse xy pass's radix plan (the same candidates as out[1]). */
 int fhd_get_schedule(const fhd_ctx* c, int out[6]);
 
 /* Divergence diagnostics of the current velocity: max |D v| over cells, in units of

@@ -87,10 +87,14 @@ FHD_KERNEL_PAIR((template <int MX, int MY, int NT, int PX, int PY>), NT, k_fftC,
 // ---------------- dispatch ----------------
 template <int MX, int MY, int NT, int PX, int PY>
 static void launch_AC_plan(const FftPass& x, int which, int mz, hipStream_t s) {
-  if (which == 0)
-    launch(k_fftA<MX, MY, NT, PX, PY>, k_fftA_b<MX, MY, NT, PX, PY>, FAM_FFT_XY_FWD, dim3(mz, x.f.ncomp), NT, x, s);
-  else
-    launch(k_fftC<MX, MY, NT, PX, PY>, k_fftC_b<MX, MY, NT, PX, PY>, FAM_FFT_XY_INV, dim3(mz, x.f.ncomp), NT, x, s);
+  // merged batches hold the smaller planes as runtime-size passes (merged_plane)
+  BatchedFn ba = nullptr, bc = nullptr;
+  if constexpr (MX > 64) {
+    ba = k_fftA_b<MX, MY, NT, PX, PY>;
+    bc = k_fftC_b<MX, MY, NT, PX, PY>;
+  }
+  if (which == 0) launch(k_fftA<MX, MY, NT, PX, PY>, ba, FAM_FFT_XY_FWD, dim3(mz, x.f.ncomp), NT, x, s);
+  else launch(k_fftC<MX, MY, NT, PX, PY>, bc, FAM_FFT_XY_INV, dim3(mz, x.f.ncomp), NT, x, s);
 }
 // The radix plans of the x and y transforms (plan_choice indices, px + 3 py) are square_plan's and can
 // be forced for 96 x 96 and 128 x 128 planes (128 x 128 also has 9: the register-transform kernels of
@@ -121,21 +125,19 @@ static void launch_AC_nt(const FftPass& x, int which, int mz, hipStream_t s) {
 // Lanes per plane workgroup.  A single context's pass has only 3 mz plane workgroups, and more
 // lanes per plane cover more of the plane load and store latency: 1024 from 64^2 up (128^3:
 // 25.4 vs 26.1 / 27.3 us per pass with 512; 58-60 VGPRs, two workgroups per CU by LDS).  A
-// batched dispatch already holds the planes of many contexts, and below 128^2 those pack
-// better as 512-lane workgroups (ensemble step 2.30 vs 2.41 ms).
+// batched dispatch already holds the planes of many contexts, and 96^2 planes pack better there as
+// 512-lane workgroups.
 template <int MX, int MY>
 static bool launch_AC(const FftArgs& a, int which, const float* in, float2* spec, float* out, const float* aux,
                       float alpha, float beta, hipStream_t s) {
   const FftPass x{a, in, spec, out, aux, alpha, beta, 0};
-  if constexpr (MX * MY >= 64 * 64) {
-    if (MX * MY >= 128 * 128 || t_recorder == nullptr) {
-      launch_AC_nt<MX, MY, 1024>(x, which, a.g.mz, s);
+  if constexpr (MX == 96) {
+    if (t_recorder) {
+      launch_AC_nt<MX, MY, 512>(x, which, a.g.mz, s);
       return true;
     }
-    launch_AC_nt<MX, MY, 512>(x, which, a.g.mz, s);
-  } else {
-    launch_AC_nt<MX, MY, 256>(x, which, a.g.mz, s);
   }
+  launch_AC_nt<MX, MY, MX * MY >= 64 * 64 ? 1024 : 256>(x, which, a.g.mz, s);
   return true;
 }
 

@@ -12,13 +12,15 @@ FHD_KERNEL_PAIR_OCC((template <int MX, int MY, int NT>), NT, 8, k_spread_fftA, F
                     body_fftA<MX, MY, NT, MX == MY ? square_plan(MX) % 3 : 0, MX == MY ? square_plan(MX) / 3 : 0, true>(
                         a.p.f, a.p.in, a.p.spec, b, &a.s))
 
-
-// Lanes per plane workgroup as in the plain pass of a context launched alone; batched dispatches
-// take the same, so a replica's kernel does not depend on the batch.
+// Lanes per plane workgroup as in the plain pass of a context launched alone.  Merged batches hold the planes
+// with both edges in the list above as runtime-size passes (merged_plane; the same radices and written-out
+// fused operations give the same bits), so only the larger squares have a batched form.
 template <int MX, int MY>
 static bool launch_plane(const FftSpread& x, hipStream_t s) {
   constexpr int NT = MX * MY >= 64 * 64 ? 1024 : 256;
-  launch(k_spread_fftA<MX, MY, NT>, k_spread_fftA_b<MX, MY, NT>, FAM_FFT_XY_FWD, dim3(x.p.f.g.mz, x.p.f.ncomp), NT, x, s);
+  BatchedFn batched = nullptr;
+  if constexpr (MX > 64) batched = k_spread_fftA_b<MX, MY, NT>;
+  launch(k_spread_fftA<MX, MY, NT>, batched, FAM_FFT_XY_FWD, dim3(x.p.f.g.mz, x.p.f.ncomp), NT, x, s);
   return true;
 }
 template <int MX>

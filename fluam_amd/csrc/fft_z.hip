@@ -197,6 +197,13 @@ FHD_BODY void body_z_merged(const FftPass& x, const Blk& b) {
 }
 FHD_KERNEL_PAIR_OCC((), kMergedLanes, 8, k_fftz_merged, FftPass, body_z_merged(a, b))
 
+// The lengths of the merged kernel have no batched form of their own.
+template <int N, int T>
+static BatchedFn z_batched() {
+  if constexpr (zmerged(N)) return nullptr;
+  else return k_fftz_b<N, T>;
+}
+
 int fast_z_columns(int mz, int want) {
   if (mz > 256 || !zr1(mz)) return 0;
   return want <= 2 ? 2 : want <= 4 ? 4 : 8;  // beyond 8 the workgroups are too few and too large
@@ -216,7 +223,7 @@ static bool launch_z(const FftArgs& a, float2* spec, hipStream_t s) {
       return true;
     }
   }
-#define FHD_Z(t) launch(k_fftz<N, t>, k_fftz_b<N, t>, FAM_FFT_Z, grid, zlanes(N, t), x, s)
+#define FHD_Z(t) launch(k_fftz<N, t>, z_batched<N, t>(), FAM_FFT_Z, grid, zlanes(N, t), x, s)
   if (tile == 2) FHD_Z(2);
   else if (tile == 4) FHD_Z(4);
   else FHD_Z(8);

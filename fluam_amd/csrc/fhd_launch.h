@@ -100,10 +100,12 @@ struct Recorder {
 // Installed by the batch code while it records a context's step on this thread.
 extern thread_local Recorder* t_recorder;
 
+// batched: null where a merged batch takes another kernel.
 template <class A>
 void launch(void (*single)(A), BatchedFn batched, int family, dim3 grid, int threads, const A& a, hipStream_t s) {
   if ((size_t)grid.x * grid.y * grid.z == 0) return;
   if (Recorder* r = t_recorder) {
+    if (!batched) throw std::logic_error("a kernel without a batched form was recorded");
     LaunchRecord rec;
     rec.family = family;
     rec.fn = reinterpret_cast<const void*>(batched);

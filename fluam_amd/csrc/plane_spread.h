@@ -264,7 +264,7 @@ FHD_DEV void plane_keys(const SpreadGroup& G, const PlaneRuns& runs, int tid, in
 }
 template <int NT, int K>
 FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, const unsigned key[K], int b, int i0, int z, int C,
-                        PlaneLds& L, int* pairs) {
+                        PlaneLds& L, int2* pairs) {
   const SpreadGroup& G = P.grp[gi];
   const int lane = tid & 63;
   unsigned long long bal[K];
@@ -272,7 +272,7 @@ FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, co
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const bool hit = key[k] != ~0u && row_hits(key[k] & 511, key[k] & 512 ? G.wide : 0, z, g.mz, P.kernel_points, C == 2);
-    if (hit && pairs) atomicAdd(&pairs[key[k] >> 16], 2);
+    if (hit && pairs) atomicAdd(&pairs[key[k] >> 16].x, 2);
     bal[k] = __ballot(hit);
     total += __popcll(bal[k]);
   }
@@ -291,7 +291,7 @@ FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, co
 // from: the first source scanned (i0 or later).
 template <int NT>
 FHD_DEV void plane_scan(const GridDev& g, const PlaneSrc& P, int gi, int tid, const PlaneRuns& runs, int i0, int from, int i1,
-                        int z, int C, PlaneLds& L, int* pairs) {
+                        int z, int C, PlaneLds& L, int2* pairs) {
   constexpr int K = 4;
   for (int b = from; b < i1; b += K * NT) {
     unsigned key[K];
@@ -390,8 +390,8 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
 
   const int lane = tid & 63;
   const int bx = (g.mx + 3) >> 2, by = (g.my + 3) >> 2;
-  // each block's sources and their largest value (float bits), until the scales are known
-  int *const count = acc, *const top = acc + bx * by;
+  // each block's sources (x) and their largest value (y, float bits), until the scales are known
+  int2* const block = reinterpret_cast<int2*>(acc);
   const int head = !REST ? min(words, (2 * bx * by + 3) & ~3) : 0;
   if (tid < 12 && tid < 6 * P.ngroups) L.runs[tid >= 6][tid % 6] = run_bound(P.t, P.grp[tid >= 6], z, tid % 6);
   for (int e = tid; e < head; e += NT) acc[e] = 0;
@@ -400,7 +400,7 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
   if (!REST && tid == 0) L.most = L.top = L.bad = 0;
   __syncthreads();
   const bool two = P.ngroups > 1;
-  int* const pairs = !REST ? count : nullptr;
+  int2* const pairs = !REST ? block : nullptr;
   bool one;  // every group's sources have 16-bit indices
   {
     const PlaneRuns r0 = plane_runs(L, 0);
@@ -444,8 +444,8 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
       const bool fine = a <= 3.0e38f;
       if (!fine) L.bad = 1;
       if (!REST) {
-        atomicAdd(&count[key >> 16], 1);
-        atomicMax(&top[key >> 16], __float_as_int(fine ? a : 3.0e38f));
+        atomicAdd(&block[key >> 16].x, 1);
+        atomicMax(&block[key >> 16].y, __float_as_int(fine ? a : 3.0e38f));
       }
     };
     if (one) {
@@ -503,15 +503,22 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
     int n_most = 0, t_most = 0;
     for (int e = tid; e < bx * by; e += NT) {
       const int y = e / bx, x = e - y * bx;
+      // the rows and columns around it, each once: of two there is no third, of one no second
+      const int ys[3] = {y, y == 0 ? by - 1 : y - 1, y == by - 1 ? 0 : y + 1};
+      const int xs[3] = {x, x == 0 ? bx - 1 : x - 1, x == bx - 1 ? 0 : x + 1};
+      int2 around[3][3];
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) around[dy][dx] = block[xs[dx] + bx * ys[dy]];
       int n = 0, t = 0;
-      for (int dy = -1; dy <= min(1, by - 2); ++dy) {
-        const int yy = y + dy < 0 ? by - 1 : y + dy >= by ? 0 : y + dy;
-        for (int dx = -1; dx <= min(1, bx - 2); ++dx) {
-          const int xx = x + dx < 0 ? bx - 1 : x + dx >= bx ? 0 : x + dx;
-          n += count[xx + bx * yy];
-          t = max(t, top[xx + bx * yy]);
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          n += dy < by && dx < bx ? around[dy][dx].x : 0;
+          t = max(t, around[dy][dx].y);
         }
-      }
       if (P.near) L.scale[e] = (signed char)plane_scale(n, most * fmaxf(__int_as_float(t), floor));
       n_most = max(n_most, n);
       t_most = max(t_most, t);

@@ -764,7 +764,7 @@ struct Nothing {
 };
 
 // Four lanes per particle: lane q sums z-row q of the stencil, the rows are combined across the quad,
-// then lane 0 applies the position update.  Below ~32,000 particles the launch is a chain of memory
+// then lane 0 applies the position update.  Below ~20,000 particles the launch is a chain of memory
 // round trips (position, rows, update): with the rows of all three components in flight, no branch
 // around the loads and the update's loads under them, 32^3 with 1,024 particles went from 10.6 to
 // 6.0 us per launch, 64^3 with 4,096 from 8.4 to 6.9 (two fields 16 to 10), 64^3 with 16,384 (4-point)
@@ -1060,7 +1060,11 @@ void launch_lag2(const Lag2Args& a, hipStream_t s) {
   const dim3 grid(nblk(4 * a.np, 256));
   FHD_LAUNCH_STENCIL(k_lag2, FAM_LAG2, grid, a, s);
 }
-constexpr int kDeepParticles = 32768;
+// Per launch (HIP events, which add about 4 us) component by component and with all rows in flight, Stokes
+// 4-point: 64^3 with 8,192 particles 11.0, 10.6 us, with 16,384 11.0, 10.8, with 24,576 13.0, 13.2; 128^3
+// with 16,384 13.4, 13.4, with 24,576 15.6, 16.2, with 65,536 22.9, 23.9.  Inertial 3-point: 64^3 with
+// 16,384 11.2, 10.5; 128^3 with 16,384 13.3, 12.9, with 24,576 15.4, 15.8.
+constexpr int kDeepParticles = 16384;
 void launch_interp(const InterpArgs& a, hipStream_t s) {
   if (a.np <= 0) return;
   const dim3 grid(nblk(4 * a.np, 256));

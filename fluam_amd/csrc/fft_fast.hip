@@ -174,6 +174,21 @@ static bool fast_AC(const FftArgs& a, int which, const float* in, float2* spec, 
 bool fast_fft_xy_fwd(const FftArgs& a, const float* in, float2* spec, hipStream_t s) {
   return fast_AC(a, 0, in, spec, nullptr, nullptr, 0.0f, 0.0f, s);
 }
+bool fast_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc& src, float2* spec, hipStream_t s) {
+  const FftSpread x{{a, in, spec, nullptr, nullptr, 0.0f, 0.0f, 0}, src};
+  switch (a.g.mx) {
+#define FHD_SPREAD(mx) case mx: return launch_spread_rect<mx>(x, s)
+    FHD_SPREAD(16);
+    FHD_SPREAD(24);
+    FHD_SPREAD(32);
+    FHD_SPREAD(48);
+    FHD_SPREAD(64);
+    FHD_SPREAD(96);
+    FHD_SPREAD(128);
+#undef FHD_SPREAD
+    default: return false;
+  }
+}
 bool fast_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha, float beta,
                      hipStream_t s) {
   return fast_AC(a, 1, nullptr, const_cast<float2*>(spec), out, aux, alpha, beta, s);

@@ -1,5 +1,6 @@
 // fft_spread.hip -- the forward xy pass with spreading for the plane shapes of fft_fast.hip: mx x my
-// with both lengths in {16, 24, 32, 48, 64} or mx = my in {96, 128}.
+// with both lengths in {16, 24, 32, 48, 64} or mx = my in {96, 128}.  Compiled once per mx
+// (FHD_SPREAD_MX): these are the largest kernels of the library.
 // The runtime-size and the size-specialised FFT kernels have to give the same bits (a replica runs
 // on the one alone and on the other in a merged batch), so the compiler must not choose which
 // products become fused multiply-adds: the fused ones are written out.
@@ -24,31 +25,20 @@ static bool launch_plane(const FftSpread& x, hipStream_t s) {
   return true;
 }
 template <int MX>
-static bool launch_rect(const FftSpread& x, hipStream_t s) {
-  switch (x.p.f.g.my) {
-    case 16: return launch_plane<MX, 16>(x, s);
-    case 24: return launch_plane<MX, 24>(x, s);
-    case 32: return launch_plane<MX, 32>(x, s);
-    case 48: return launch_plane<MX, 48>(x, s);
-    case 64: return launch_plane<MX, 64>(x, s);
-    default: return false;
+bool launch_spread_rect(const FftSpread& x, hipStream_t s) {
+  if constexpr (MX > 64) {
+    return x.p.f.g.my == MX && launch_plane<MX, MX>(x, s);
+  } else {
+    switch (x.p.f.g.my) {
+      case 16: return launch_plane<MX, 16>(x, s);
+      case 24: return launch_plane<MX, 24>(x, s);
+      case 32: return launch_plane<MX, 32>(x, s);
+      case 48: return launch_plane<MX, 48>(x, s);
+      case 64: return launch_plane<MX, 64>(x, s);
+      default: return false;
+    }
   }
 }
-
-bool fast_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc& src, float2* spec, hipStream_t s) {
-  const FftSpread x{{a, in, spec, nullptr, nullptr, 0.0f, 0.0f, 0}, src};
-  if (a.g.mx == a.g.my) {
-    if (a.g.mx == 96) return launch_plane<96, 96>(x, s);
-    if (a.g.mx == 128) return launch_plane<128, 128>(x, s);
-  }
-  switch (a.g.mx) {
-    case 16: return launch_rect<16>(x, s);
-    case 24: return launch_rect<24>(x, s);
-    case 32: return launch_rect<32>(x, s);
-    case 48: return launch_rect<48>(x, s);
-    case 64: return launch_rect<64>(x, s);
-    default: return false;
-  }
-}
+template bool launch_spread_rect<FHD_SPREAD_MX>(const FftSpread&, hipStream_t);
 
 }  // namespace fhd

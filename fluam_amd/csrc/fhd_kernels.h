@@ -308,6 +308,7 @@ struct FftSpread {
 // Size-specialised FFT passes (fft_fast.hip); return false when the shape has no specialisation.
 bool fast_fft_xy_fwd(const FftArgs& a, const float* in, float2* spec, hipStream_t s);
 bool fast_fft_spread_xy_fwd(const FftArgs& a, const float* in, const PlaneSrc& src, float2* spec, hipStream_t s);
+template <int MX> bool launch_spread_rect(const FftSpread& x, hipStream_t s);  // fft_spread.hip, a unit per mx
 bool fast_fft_z_solve(const FftArgs& a, float2* spec, hipStream_t s);
 int fast_z_columns(int mz, int want);  // 0: not a length of fft_z.hip
 bool fast_fft_xy_inv(const FftArgs& a, const float2* spec, float* out, const float* aux, float alpha, float beta,

@@ -2372,19 +2372,22 @@ namespace {
 long long ctx_bytes(const fhd_params& p) {
   const long long N = (long long)p.mx * p.my * p.mz, N3 = 3 * N;
   const long long P = p.mx / 2 + 1;
-  long long b = 6 * N3 * 4 + N * 4 + 3LL * p.mz * p.my * P * 8;  // v v2 W SF adv[2], div, spectrum
-  b += 3LL * (p.mx + p.my + p.mz) * 20;                            // tables
+  const bool qnb = p.scheme == FHD_SCHEME_QUASI_NEUTRALLY_BUOYANT, heavy = qnb && p.np > 0 && p.mass != 0.0;
+  // v, v2, W; the incompressible step's shared terms; two advection fields; the excess-mass field
+  const int fields = 3 + (p.scheme == FHD_SCHEME_INCOMPRESSIBLE ? 1 : 0) + (qnb ? 2 : 0) + (heavy ? 1 : 0);
+  long long b = fields * N3 * 4 + N * 4 + 3LL * p.mz * p.my * P * 8;  // and divergence, spectrum
+  b += 3LL * (p.mx + p.my + p.mz) * 20;                               // tables
   if (p.np > 0) {
     const long long np = p.np;
     const int te[3] = {tile_edge(p.mx), tile_edge(p.my), tile_edge(p.mz)};
     long long nt = 1;
     const int m[3] = {p.mx, p.my, p.mz};
     for (int a = 0; a < 3; ++a) nt *= te[a] > 0 ? m[a] / te[a] : 1;
-    b += 2 * np * (16 + 16 + 16 + 4 + 16 + 16) + 2 * (nt + 1) * 4;  // positions, forces, sorted sets
-    b += np * 16 + nt * 4 + 2 * np * 4;                               // u, counts, slots, scratch
-    b += 2 * np * 4;                                                  // plane keys
-    if (p.scheme == FHD_SCHEME_STOKES_LIMIT) b += np * 16;            // RFD normals
-    if (p.scheme == FHD_SCHEME_QUASI_NEUTRALLY_BUOYANT && p.mass != 0.0) b += N3 * 4 + 5 * np * 16;
+    b += 2 * np * (5 * 16 + 2 * 4) + 2 * (nt + 1) * 4;                   // positions, forces, sorted sets with their keys
+    b += np * 16 + 2 * nt * 4 + 3 * np * 4;                             // u, counts, slots, scratch
+    if (p.nonbonded && p.cutoff > 0) b += np * (4LL * kNbCap + 4 + 32);  // neighbour lists
+    if (p.scheme == FHD_SCHEME_STOKES_LIMIT) b += np * 16;              // RFD normals
+    if (heavy) b += 5 * np * 16;
   }
   return b;
 }

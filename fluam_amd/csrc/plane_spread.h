@@ -10,8 +10,8 @@
 // associative, so the field is bit-identical whatever order they arrive in.  Every 4 x 4 block of columns
 // has its own scale, from the largest value among the sources that can reach it and from their number, so
 // that no node's sum reaches 2^31 and a weak force is rounded by its own neighbourhood's measure, not by
-// the plane's strongest; with more than kOneLimb sources in reach of a block a second sweep adds what the
-// first one's rounding left over.
+// the plane's strongest; where that leaves a row less than 23 bits (255 forces or some 15,000 pairs in
+// reach of a block) a second sweep adds what the first one's rounding left over.
 //
 // Bound by the latency of its dependent phases and, for the pairs, by the vector instructions of
 // the rows; a plane is one workgroup, so at 128^3 half the CUs hold two of the 384 planes and half
@@ -37,7 +37,6 @@
 namespace fhd {
 
 constexpr int kListCap = 6144;     // hits listed at once (also the sources scanned per chunk when more)
-constexpr int kOneLimb = 255;      // most sources per node for a single 32-bit sum
 constexpr int kPlaneBlocks = 1024; // 4 x 4 blocks of the largest plane that can hold particles
 
 // The key of a sorted slot: bits 0-8 its half cell along z (wrapped cell, sign of the offset), bit
@@ -177,25 +176,62 @@ struct PlaneLds {
   unsigned short list[kListCap];  // group 0's hits from the front, group 1's from the back
   int runs[2][6];
   int n[2];   // the groups' hit counts
-  int kept;   // group 0's hits with a value
-  int most;   // most sources that can meet at a node
+  int kept;   // group 0's hits with a value (in chunks: whether there are any)
+  int most;   // most additions that can meet at a node
   int top;    // largest value (float bits)
+  int more;   // the remainders are to be summed as well
   int bad;    // an overflowed or NaN source
   signed char scale[kPlaneBlocks];  // binary exponent of each 4 x 4 block's fixed-point scale
 };
 
-// Binary exponent of the fixed-point scale of nodes that at most n sources reach, each with less than t.
-FHD_DEV int count_exp(int n) {
-  // n 2^S <= 2^31; a source's up to eight additions to a node round by half a unit each, which the
-  // thousandth in plane_scale covers while S >= 13
-  n = max(n, 1);
-  return 30 - (31 - __clz(n)) - (n > 65536 ? 1 : 0);
+// Bounds per plane and component: what a source adds to a node is below its value times `most`; one row of
+// a pair below `row`, and the two rows' difference, their weights being Lipschitz, below `diff` (a hundredth
+// of it at the default displacement).
+struct PlaneBounds {
+  float most, row, diff;
+};
+template <int NPTS>
+FHD_DEV PlaneBounds plane_bounds(const GridDev& g, const PlaneSrc& P, int C) {
+  const int m[3] = {g.mx, g.my, g.mz};
+  const float ih[3] = {g.idx, g.idy, g.idz};
+  const bool two = P.ngroups > 1, drift = P.grp[0].drift != 0.0f;
+  PlaneBounds b{1.0f, 0.0f, 0.0f};
+  // a pair's normals are below 5.8 (24-bit uniforms)
+  const float apart = two ? 2.0f * 5.8f * fabsf(P.grp[1].disp) : 0.0f;
+  float w[3], d[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    w[a] = axis_most<NPTS>(m[a], drift && a == C);
+    // slopes are at most 1/2 and 1; a narrow axis folds two weights onto a node
+    d[a] = m[a] == 1 ? 0.0f : fminf(w[a], (NPTS == 4 ? 0.5f : 1.0f) * (m[a] < NPTS ? 2.0f : 1.0f) * apart * ih[a]);
+    b.most *= w[a];
+  }
+  if (two) {
+    const float v = fminf(5.8f * fabsf(P.grp[1].coef), 3.0e38f);
+    b.row = v * b.most;
+    b.diff = v * fminf(b.most, d[0] * w[1] * w[2] + w[0] * d[1] * w[2] + w[0] * w[1] * d[2]);
+  }
+  return b;
 }
-FHD_DEV int plane_scale(int n, float t) {
-  int e = -90;
-  if (t > 0.0f) frexpf(1.001f * t, &e);  // t < 2^e
-  return count_exp(n) - max(e, -90);
+// Binary exponent x of the fixed-point scale of nodes that `nf` values of at most t and `np` pairs reach:
+// no node's sum passes 2^31, no single row's value 2^30.  A hundredth is left for what the additions round,
+// at most eight of them from a source.  more: the largest row keeps less than 23 bits, so the remainders
+// are to be summed as well.
+FHD_DEV int block_scale(const PlaneBounds& b, int nf, int np, float t, bool& more) {
+  const float down = 9.31322575e-10f;  // 2^-30: counts times values stay finite
+  const float value = t * b.most * down;
+  const float row = 1.01f * fmaxf(value, np ? b.row * down : 0.0f);
+  const float sum = 1.01f * fmaf((float)nf, value, (float)np * (b.diff * down));
+  int er = -200, es = -200;
+  if (row > 0.0f) frexpf(row, &er);  // row < 2^er
+  if (sum > 0.0f) frexpf(sum, &es);
+  er = max(er + 30, -90);
+  const int x = min(30 - er, 1 - es) - (nf + np > 1 << 18 ? 1 : 0);
+  more |= x < 23 - er;
+  return x;
 }
+// Binary exponent of the scale of the remainders, which are at most half a unit each.
+FHD_DEV int rest_exp(int most) { return 27 - (31 - __clz(max(most, 1))); }
 
 // Adds the nodes of a row (weights wx and wy times r), or of the difference of two rows on the same
 // nodes (PAIR: minus vx and vy times s).  Four nodes lie in at most two blocks along an axis.
@@ -252,8 +288,12 @@ FHD_DEV PlaneRuns plane_runs(const PlaneLds& L, int gi) {
   return r;
 }
 
-// Lists the hits among sources [i0, i1) of group gi (entries relative to i0); `pairs`: also counts
-// them, two each, by block (null: not).  K keys of a lane are in flight at once.
+// Component C of source j's value.
+FHD_DEV float src_value(const SpreadGroup& G, int j, int C) {
+  return G.coef * reinterpret_cast<const float*>(G.val + G.set.id[j])[C];
+}
+
+// The keys of sources [b, b + K NT) of a group, K of a lane in flight at once.
 template <int NT, int K>
 FHD_DEV void plane_keys(const SpreadGroup& G, const PlaneRuns& runs, int tid, int b, int i1, unsigned key[K]) {
 #pragma unroll
@@ -262,18 +302,18 @@ FHD_DEV void plane_keys(const SpreadGroup& G, const PlaneRuns& runs, int tid, in
     key[k] = i < i1 ? G.key[runs.slot(i)] : ~0u;
   }
 }
+FHD_DEV bool key_hits(unsigned key, const SpreadGroup& G, int z, int mz, int npts, bool stag) {
+  return key != ~0u && row_hits(key & 511, key & 512 ? G.wide : 0, z, mz, npts, stag);
+}
+// Lists the marked sources (entries relative to i0).
 template <int NT, int K>
-FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, const unsigned key[K], int b, int i0, int z, int C,
-                        PlaneLds& L, int2* pairs) {
-  const SpreadGroup& G = P.grp[gi];
+FHD_DEV void plane_list(PlaneLds& L, int gi, int tid, const bool hit[K], int b, int i0) {
   const int lane = tid & 63;
   unsigned long long bal[K];
   int total = 0;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const bool hit = key[k] != ~0u && row_hits(key[k] & 511, key[k] & 512 ? G.wide : 0, z, g.mz, P.kernel_points, C == 2);
-    if (hit && pairs) atomicAdd(&pairs[key[k] >> 16].x, 2);
-    bal[k] = __ballot(hit);
+    bal[k] = __ballot(hit[k]);
     total += __popcll(bal[k]);
   }
   if (total == 0) return;
@@ -283,26 +323,32 @@ FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, co
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int mine = at + __popcll(bal[k] & ((1ull << lane) - 1ull));
-    if ((bal[k] >> lane & 1) && mine < kListCap)
-      L.list[gi == 0 ? mine : kListCap - 1 - mine] = (unsigned short)(b + k * NT + tid - i0);
+    if (hit[k] && mine < kListCap) L.list[gi == 0 ? mine : kListCap - 1 - mine] = (unsigned short)(b + k * NT + tid - i0);
     at += __popcll(bal[k]);
   }
+}
+// Lists the hits among the keys, and counts pairs by block (block null: not).
+template <int NT, int K>
+FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, const unsigned key[K], int b, int i0, int z,
+                        int C, PlaneLds& L, int4* block) {
+  bool hit[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    hit[k] = key_hits(key[k], P.grp[gi], z, g.mz, P.kernel_points, C == 2);
+    if (hit[k] && gi == 1 && block) atomicAdd(&block[key[k] >> 16].y, 1);
+  }
+  plane_list<NT, K>(L, gi, tid, hit, b, i0);
 }
 // from: the first source scanned (i0 or later).
 template <int NT>
 FHD_DEV void plane_scan(const GridDev& g, const PlaneSrc& P, int gi, int tid, const PlaneRuns& runs, int i0, int from, int i1,
-                        int z, int C, PlaneLds& L, int2* pairs) {
+                        int z, int C, PlaneLds& L, int4* block) {
   constexpr int K = 4;
   for (int b = from; b < i1; b += K * NT) {
     unsigned key[K];
     plane_keys<NT, K>(P.grp[gi], runs, tid, b, i1, key);
-    plane_test<NT, K>(g, P, gi, tid, key, b, i0, z, C, L, pairs);
+    plane_test<NT, K>(g, P, gi, tid, key, b, i0, z, C, L, block);
   }
-}
-
-// Component C of source j's value.
-FHD_DEV float src_value(const SpreadGroup& G, int j, int C) {
-  return G.coef * reinterpret_cast<const float*>(G.val + G.set.id[j])[C];
 }
 
 // Adds source j's row to the plane.
@@ -359,22 +405,43 @@ FHD_DEV void plane_add_list(int* acc, int pitch, const GridDev& g, const SpreadG
 }
 
 // Group 0 (vector values) or 1 (pairs): `nh` listed hits, or where they are more than the list holds
-// (`one` false) chunks of as many sources.
+// (`one` false) as many at a time as it does, of group 0 those with a value.
 template <int NPTS, int NT, bool PAIRS>
 FHD_DEV void plane_add_group(int* acc, int pitch, const GridDev& g, const PlaneSrc& P, int tid, int z, int C, PlaneLds& L,
                              bool one, int nh, float scale2) {
   const SpreadGroup& G = P.grp[PAIRS];
   const PlaneRuns r = plane_runs(L, PAIRS);
-  const int all = one ? 1 : r.total();
-  for (int i0 = 0; i0 < all; i0 += kListCap) {
-    if (!one) {
-      __syncthreads();  // the previous chunk's list consumed
-      if (tid == 0) L.n[PAIRS] = 0;
-      __syncthreads();
-      plane_scan<NT>(g, P, PAIRS, tid, r, i0, i0, min(all, i0 + kListCap), z, C, L, nullptr);
+  if (one) {
+    plane_add_list<NPTS, NT, PAIRS>(acc, pitch, g, G, tid, r, 0, nh, z, C, L, scale2);
+    return;
+  }
+  constexpr int K = 4;
+  const int all = nh ? r.total() : 0;
+  for (int i = 0; i < all;) {
+    __syncthreads();  // the last entries consumed
+    if (tid == 0) L.n[PAIRS] = 0;
+    __syncthreads();
+    const int i0 = i;
+    do {
+      unsigned key[K];
+      bool hit[K];
+      float v[K];
+      plane_keys<NT, K>(G, r, tid, i, all, key);
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        hit[k] = key_hits(key[k], G, z, g.mz, NPTS, C == 2);
+        if (!PAIRS) v[k] = hit[k] ? src_value(G, r.slot(i + k * NT + tid), C) : 0.0f;
+      }
+      if (!PAIRS) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) hit[k] = hit[k] && (v[k] != 0.0f || G.drift != 0.0f);
+      }
+      plane_list<NT, K>(L, PAIRS, tid, hit, i, i0);
+      i += K * NT;
       __syncthreads();
       nh = uniform(L.n[PAIRS]);
-    }
+      __syncthreads();  // read by every wave before the next entries are counted
+    } while (i < all && nh + K * NT <= kListCap && i + K * NT - i0 <= 65536);
     plane_add_list<NPTS, NT, PAIRS>(acc, pitch, g, G, tid, r, i0, nh, z, C, L, scale2);
   }
 }
@@ -390,17 +457,16 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
 
   const int lane = tid & 63;
   const int bx = (g.mx + 3) >> 2, by = (g.my + 3) >> 2;
-  // each block's sources (x) and their largest value (y, float bits), until the scales are known
-  int2* const block = reinterpret_cast<int2*>(acc);
-  const int head = !REST ? min(words, (2 * bx * by + 3) & ~3) : 0;
+  // each block's values (x), pairs (y) and largest value (z, float bits), until the scales are known
+  int4* const block = reinterpret_cast<int4*>(acc);
+  const int head = !REST ? 4 * bx * by : 0;  // a block has four words of the plane at least
   if (tid < 12 && tid < 6 * P.ngroups) L.runs[tid >= 6][tid % 6] = run_bound(P.t, P.grp[tid >= 6], z, tid % 6);
   for (int e = tid; e < head; e += NT) acc[e] = 0;
   if (tid < 2) L.n[tid] = 0;
   if (tid == 0) L.kept = 0;
-  if (!REST && tid == 0) L.most = L.top = L.bad = 0;
+  if (!REST && tid == 0) L.most = L.top = L.more = L.bad = 0;
   __syncthreads();
   const bool two = P.ngroups > 1;
-  int2* const pairs = !REST ? block : nullptr;
   bool one;  // every group's sources have 16-bit indices
   {
     const PlaneRuns r0 = plane_runs(L, 0);
@@ -416,6 +482,7 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
       n1 = r1.total();
       plane_keys<NT, K>(P.grp[1], r1, tid, 0, n1, k1);
     }
+    int4* const pairs = !REST ? block : nullptr;
     plane_test<NT, K>(g, P, 0, tid, k0, 0, 0, z, C, L, nullptr);
     if (n0 > K * NT) plane_scan<NT>(g, P, 0, tid, r0, 0, K * NT, n0, z, C, L, nullptr);
     if (two) {
@@ -425,7 +492,7 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
     one = n0 <= 65536 && n1 <= 65536;
   }
   __syncthreads();
-  int nhit0 = uniform(L.n[0]);
+  const int nhit0 = uniform(L.n[0]);
   const int nhit1 = uniform(L.n[1]);
   one = one && nhit0 + nhit1 <= kListCap;
   const auto clear = [&](int from, int to) {  // both multiples of 4, or the plane's end
@@ -445,7 +512,7 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
       if (!fine) L.bad = 1;
       if (!REST) {
         atomicAdd(&block[key >> 16].x, 1);
-        atomicMax(&block[key >> 16].y, __float_as_int(fine ? a : 3.0e38f));
+        atomicMax(&block[key >> 16].z, __float_as_int(fine ? a : 3.0e38f));
       }
     };
     if (one) {
@@ -478,49 +545,56 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
       }
     } else {
       clear(head, words);
-      for (int i = tid; i < r.total(); i += NT) {
-        const int j = r.slot(i);
-        const unsigned key = G.key[j];
-        if (!row_hits(key & 511, key & 512 ? G.wide : 0, z, g.mz, NPTS, C == 2)) continue;
-        const float v = src_value(G, j, C);
-        if (v != 0.0f || drift != 0.0f) enter(v, key);
+      constexpr int K = 4;
+      for (int b = 0; b < r.total(); b += K * NT) {
+        unsigned key[K];
+        float v[K];
+        plane_keys<NT, K>(G, r, tid, b, r.total(), key);
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          if (!key_hits(key[k], G, z, g.mz, NPTS, C == 2)) key[k] = ~0u;
+          v[k] = key[k] != ~0u ? src_value(G, r.slot(b + k * NT + tid), C) : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+          if (key[k] != ~0u && (v[k] != 0.0f || drift != 0.0f)) {
+            enter(v[k], key[k]);
+            L.kept = 1;
+          }
       }
     }
   }
   __syncthreads();
-  if (one) nhit0 = uniform(L.kept);
+  const int nval = uniform(L.kept);
   if (!REST) {
     // The scale of a block's nodes: their sources lie in cells at most 3 away, so in the blocks around it,
-    // unless a pair is displaced by more than a cell along x or y (then the plane has one scale).  What a
-    // source adds to a node is below value x the product of its axes' most; a pair's normals are below 5.8
-    // (24-bit uniforms).
-    const bool drift = P.grp[0].drift != 0.0f;
-    const float most = axis_most<NPTS>(g.mx, drift && C == 0) * axis_most<NPTS>(g.my, drift && C == 1) *
-                       axis_most<NPTS>(g.mz, drift && C == 2);
-    const float pair = two ? 5.8f * fabsf(P.grp[1].coef) : 0.0f;
-    if (tid == 0 && !(pair <= 3.0e38f)) L.bad = 1;
-    const float floor = fminf(pair, 3.0e38f);
+    // unless a pair is displaced by more than a cell along x or y (then the plane has one scale).
+    const PlaneBounds bounds = plane_bounds<NPTS>(g, P, C);
+    if (tid == 0 && two && !(5.8f * fabsf(P.grp[1].coef) <= 3.0e38f)) L.bad = 1;
+    bool more = false;
     int n_most = 0, t_most = 0;
     for (int e = tid; e < bx * by; e += NT) {
       const int y = e / bx, x = e - y * bx;
       // the rows and columns around it, each once: of two there is no third, of one no second
       const int ys[3] = {y, y == 0 ? by - 1 : y - 1, y == by - 1 ? 0 : y + 1};
       const int xs[3] = {x, x == 0 ? bx - 1 : x - 1, x == bx - 1 ? 0 : x + 1};
-      int2 around[3][3];
+      int4 around[3][3];
 #pragma unroll
       for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
         for (int dx = 0; dx < 3; ++dx) around[dy][dx] = block[xs[dx] + bx * ys[dy]];
-      int n = 0, t = 0;
+      int nf = 0, np = 0, t = 0;
 #pragma unroll
       for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
         for (int dx = 0; dx < 3; ++dx) {
-          n += dy < by && dx < bx ? around[dy][dx].x : 0;
-          t = max(t, around[dy][dx].y);
+          const bool in = dy < by && dx < bx;
+          nf += in ? around[dy][dx].x : 0;
+          np += in ? around[dy][dx].y : 0;
+          t = max(t, around[dy][dx].z);
         }
-      if (P.near) L.scale[e] = (signed char)plane_scale(n, most * fmaxf(__int_as_float(t), floor));
-      n_most = max(n_most, n);
+      if (P.near) L.scale[e] = (signed char)block_scale(bounds, nf, np, __int_as_float(t), more);
+      n_most = max(n_most, nf + 2 * np);
       t_most = max(t_most, t);
     }
     n_most = wave_max_i32(P.near ? n_most : nhit0 + 2 * nhit1);
@@ -529,19 +603,21 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
       t_most = wave_max_i32(t_most);
       if (lane == 0) atomicMax(&L.top, t_most);
     }
+    if (more) L.more = 1;
     __syncthreads();
     clear(0, head);
     if (!P.near) {
-      const int x = plane_scale(L.most, most * fmaxf(__int_as_float(L.top), floor));
+      const int x = block_scale(bounds, nval ? nhit0 : 0, nhit1, __int_as_float(L.top), more);
       for (int e = tid; e < bx * by; e += NT) L.scale[e] = (signed char)x;
+      if (more) L.more = 1;
     }
     __syncthreads();
   }
-  const float scale2 = !REST ? 0.0f : ldexpf(1.0f, count_exp(uniform(L.most)));
-  plane_add_group<NPTS, NT, false>(acc, pitch, g, P, tid, z, C, L, one, nhit0, scale2);
+  const float scale2 = !REST ? 0.0f : ldexpf(1.0f, rest_exp(uniform(L.most)));
+  plane_add_group<NPTS, NT, false>(acc, pitch, g, P, tid, z, C, L, one, nval, scale2);
   if (two) plane_add_group<NPTS, NT, true>(acc, pitch, g, P, tid, z, C, L, one, nhit1, scale2);
   __syncthreads();
-  return !REST && uniform(L.most) > kOneLimb && uniform(L.bad) == 0;
+  return !REST && uniform(L.more) != 0 && uniform(L.bad) == 0;
 }
 template <int NT, bool REST>
 FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, const PlaneSrc& P, int z, int C,
@@ -558,7 +634,7 @@ struct PlaneUnit {
   FHD_DEV float at(const PlaneLds& L, int x, int y) const { return ldexpf(coef, -L.scale[(x >> 2) + nbx * (y >> 2)]); }
 };
 FHD_DEV PlaneUnit plane_unit(const PlaneLds& L, const PlaneSrc& P, const GridDev& g) {
-  return PlaneUnit{uniform(L.bad) ? __builtin_inff() : P.out_coef, ldexpf(1.0f, -count_exp(uniform(L.most))), (g.mx + 3) >> 2};
+  return PlaneUnit{uniform(L.bad) ? __builtin_inff() : P.out_coef, ldexpf(1.0f, -rest_exp(uniform(L.most))), (g.mx + 3) >> 2};
 }
 
 }  // namespace fhd

@@ -87,6 +87,8 @@ def test_displacements_across_flat_cells(tmp_path, kernel):
     (ST, (64, 16, 8), 9000, 4, {"rfd_delta": 2.5}),  # displaced beyond the neighbouring blocks: one scale
     (ST, (72, 36, 8), 9000, 4, {}),    # runtime-size passes
     (QNB, (128, 128, 4), 12000, 4, {}),
+    (ST, (64, 64, 16), 140000, 4, {}),   # more sources in reach of a plane than 16 bits index
+    (QNB, (48, 24, 16), 140000, 3, {}),
 ])
 def test_crowded_planes_with_forces(tmp_path, scheme, cells, n, kernel, kw):
     run(tmp_path, scheme, cells, n, kernel, 300 + kernel, **kw)

@@ -36,7 +36,7 @@
 
 namespace fhd {
 
-constexpr int kListCap = 6144;     // hits listed at once (also the sources scanned per chunk when more)
+constexpr int kListCap = 6144;     // most hits listed
 constexpr int kPlaneBlocks = 1024; // 4 x 4 blocks of the largest plane that can hold particles
 
 // The key of a sorted slot: bits 0-8 its half cell along z (wrapped cell, sign of the offset), bit
@@ -173,10 +173,13 @@ FHD_DEV float axis_most(int m, bool deriv) {
 }
 
 struct PlaneLds {
-  unsigned short list[kListCap];  // group 0's hits from the front, group 1's from the back
+  union {
+    unsigned short list[kListCap];  // group 0's hits from the front, group 1's from the back
+    int slots[kListCap / 2];        // without a list: a share of each wave for its next hits
+  };
   int runs[2][6];
   int n[2];   // the groups' hit counts
-  int kept;   // group 0's hits with a value (in chunks: whether there are any)
+  int kept;   // group 0's hits with a value (without a list: whether there are any)
   int most;   // most additions that can meet at a node
   int top;    // largest value (float bits)
   int more;   // the remainders are to be summed as well
@@ -305,9 +308,9 @@ FHD_DEV void plane_keys(const SpreadGroup& G, const PlaneRuns& runs, int tid, in
 FHD_DEV bool key_hits(unsigned key, const SpreadGroup& G, int z, int mz, int npts, bool stag) {
   return key != ~0u && row_hits(key & 511, key & 512 ? G.wide : 0, z, mz, npts, stag);
 }
-// Lists the marked sources (entries relative to i0).
+// Lists the marked sources.
 template <int NT, int K>
-FHD_DEV void plane_list(PlaneLds& L, int gi, int tid, const bool hit[K], int b, int i0) {
+FHD_DEV void plane_list(PlaneLds& L, int gi, int tid, const bool hit[K], int b) {
   const int lane = tid & 63;
   unsigned long long bal[K];
   int total = 0;
@@ -323,13 +326,13 @@ FHD_DEV void plane_list(PlaneLds& L, int gi, int tid, const bool hit[K], int b, 
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int mine = at + __popcll(bal[k] & ((1ull << lane) - 1ull));
-    if (hit[k] && mine < kListCap) L.list[gi == 0 ? mine : kListCap - 1 - mine] = (unsigned short)(b + k * NT + tid - i0);
+    if (hit[k] && mine < kListCap) L.list[gi == 0 ? mine : kListCap - 1 - mine] = (unsigned short)(b + k * NT + tid);
     at += __popcll(bal[k]);
   }
 }
 // Lists the hits among the keys, and counts pairs by block (block null: not).
 template <int NT, int K>
-FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, const unsigned key[K], int b, int i0, int z,
+FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, const unsigned key[K], int b, int z,
                         int C, PlaneLds& L, int4* block) {
   bool hit[K];
 #pragma unroll
@@ -337,17 +340,16 @@ FHD_DEV void plane_test(const GridDev& g, const PlaneSrc& P, int gi, int tid, co
     hit[k] = key_hits(key[k], P.grp[gi], z, g.mz, P.kernel_points, C == 2);
     if (hit[k] && gi == 1 && block) atomicAdd(&block[key[k] >> 16].y, 1);
   }
-  plane_list<NT, K>(L, gi, tid, hit, b, i0);
+  plane_list<NT, K>(L, gi, tid, hit, b);
 }
-// from: the first source scanned (i0 or later).
 template <int NT>
-FHD_DEV void plane_scan(const GridDev& g, const PlaneSrc& P, int gi, int tid, const PlaneRuns& runs, int i0, int from, int i1,
+FHD_DEV void plane_scan(const GridDev& g, const PlaneSrc& P, int gi, int tid, const PlaneRuns& runs, int from, int i1,
                         int z, int C, PlaneLds& L, int4* block) {
   constexpr int K = 4;
   for (int b = from; b < i1; b += K * NT) {
     unsigned key[K];
     plane_keys<NT, K>(P.grp[gi], runs, tid, b, i1, key);
-    plane_test<NT, K>(g, P, gi, tid, key, b, i0, z, C, L, block);
+    plane_test<NT, K>(g, P, gi, tid, key, b, z, C, L, block);
   }
 }
 
@@ -394,55 +396,71 @@ FHD_DEV void plane_add_pair(int* acc, int pitch, const GridDev& g, const PlaneLd
     add_nodes<NPTS, false>(acc, pitch, g, L, x1, y1, -r1, x1, y1, 0.0f, scale2);
   }
 }
+// The next source for this lane (-1: none) of those of a group that hit the plane, gathered without the list:
+// each wave takes its share of the keys (from b on), collects their hits (of group 0 those with a value) in
+// LDS (n of them) and hands them out whenever it has one for every lane.  No barrier, so the waves cover each
+// other's loads.  False when nothing is left.
 template <int NPTS, int NT, bool PAIRS>
-FHD_DEV void plane_add_list(int* acc, int pitch, const GridDev& g, const SpreadGroup& G, int tid, const PlaneRuns& runs,
-                            int i0, int nh, int z, int C, const PlaneLds& L, float scale2) {
-  for (int k = tid; k < nh; k += NT) {
-    const int j = runs.slot(i0 + L.list[PAIRS ? kListCap - 1 - k : k]);
-    if (PAIRS) plane_add_pair<NPTS>(acc, pitch, g, L, G, j, z, C, scale2);
-    else plane_add<NPTS>(acc, pitch, g, L, G, j, z, C, scale2);
+FHD_DEV bool plane_gather(const SpreadGroup& G, const PlaneRuns& r, int all, int lane, int* slots, int mz, int z, int C,
+                          int& b, int& n, int& j) {
+  constexpr int K = 2;
+  static_assert(64 * K + 63 <= kListCap / 2 / (NT / 64), "a wave's share holds what it collects");
+  while (n < 64 && b < all) {
+    int slot[K];
+    unsigned key[K];
+    float v[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = b + k * 64 + lane;
+      slot[k] = r.slot(i);
+      key[k] = i < all ? G.key[slot[k]] : ~0u;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (!key_hits(key[k], G, z, mz, NPTS, C == 2)) key[k] = ~0u;
+      if (!PAIRS) v[k] = key[k] != ~0u ? src_value(G, slot[k], C) : 0.0f;
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const bool hit = key[k] != ~0u && (PAIRS || v[k] != 0.0f || G.drift != 0.0f);
+      const unsigned long long bal = __ballot(hit);
+      if (hit) slots[n + __popcll(bal & ((1ull << lane) - 1ull))] = slot[k];
+      n += __popcll(bal);
+    }
+    b += NT * K;
   }
+  if (n == 0) return false;
+  const int take = min(n, 64);
+  n -= take;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  j = lane < take ? slots[n + lane] : -1;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  return true;
 }
 
-// Group 0 (vector values) or 1 (pairs): `nh` listed hits, or where they are more than the list holds
-// (`one` false) as many at a time as it does, of group 0 those with a value.
+// Adds the rows of group 0 (vector values) or 1 (pairs): `nh` listed sources, or (`one` false) all that hit.
 template <int NPTS, int NT, bool PAIRS>
 FHD_DEV void plane_add_group(int* acc, int pitch, const GridDev& g, const PlaneSrc& P, int tid, int z, int C, PlaneLds& L,
                              bool one, int nh, float scale2) {
   const SpreadGroup& G = P.grp[PAIRS];
   const PlaneRuns r = plane_runs(L, PAIRS);
-  if (one) {
-    plane_add_list<NPTS, NT, PAIRS>(acc, pitch, g, G, tid, r, 0, nh, z, C, L, scale2);
-    return;
-  }
-  constexpr int K = 4;
-  const int all = nh ? r.total() : 0;
-  for (int i = 0; i < all;) {
-    __syncthreads();  // the last entries consumed
-    if (tid == 0) L.n[PAIRS] = 0;
-    __syncthreads();
-    const int i0 = i;
-    do {
-      unsigned key[K];
-      bool hit[K];
-      float v[K];
-      plane_keys<NT, K>(G, r, tid, i, all, key);
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        hit[k] = key_hits(key[k], G, z, g.mz, NPTS, C == 2);
-        if (!PAIRS) v[k] = hit[k] ? src_value(G, r.slot(i + k * NT + tid), C) : 0.0f;
-      }
-      if (!PAIRS) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) hit[k] = hit[k] && (v[k] != 0.0f || G.drift != 0.0f);
-      }
-      plane_list<NT, K>(L, PAIRS, tid, hit, i, i0);
-      i += K * NT;
-      __syncthreads();
-      nh = uniform(L.n[PAIRS]);
-      __syncthreads();  // read by every wave before the next entries are counted
-    } while (i < all && nh + K * NT <= kListCap && i + K * NT - i0 <= 65536);
-    plane_add_list<NPTS, NT, PAIRS>(acc, pitch, g, G, tid, r, i0, nh, z, C, L, scale2);
+  const int all = r.total(), lane = tid & 63, wave = uniform(tid >> 6);
+  int n = 0, b = one ? wave * 64 : wave * 128;
+  for (;;) {
+    int j = -1;
+    if (one) {
+      if (b >= nh) break;
+      if (b + lane < nh) j = r.slot(L.list[PAIRS ? kListCap - 1 - b - lane : b + lane]);
+      b += NT;
+    } else if (!plane_gather<NPTS, NT, PAIRS>(G, r, all, lane, L.slots + wave * (kListCap / 2 / (NT / 64)), g.mz, z, C, b, n, j)) {
+      break;
+    }
+    if (j >= 0) {
+      if (PAIRS) plane_add_pair<NPTS>(acc, pitch, g, L, G, j, z, C, scale2);
+      else plane_add<NPTS>(acc, pitch, g, L, G, j, z, C, scale2);
+    }
   }
 }
 
@@ -467,34 +485,32 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
   if (!REST && tid == 0) L.most = L.top = L.more = L.bad = 0;
   __syncthreads();
   const bool two = P.ngroups > 1;
-  bool one;  // every group's sources have 16-bit indices
-  {
+  // sources in reach, of which the plane is hit by about five in fourteen (five planes of the one or two
+  // layers of eight): with three times what the list holds they are not listed
+  const int n0 = plane_runs(L, 0).total(), n1 = two ? plane_runs(L, 1).total() : 0;
+  const bool listed = n0 + n1 <= 3 * kListCap;
+  int4* const pairs = !REST ? block : nullptr;
+  if (listed) {
     const PlaneRuns r0 = plane_runs(L, 0);
-    const int n0 = r0.total();
     // the first keys of both groups are in flight at once
     constexpr int K = 4;
     unsigned k0[K], k1[K];
     plane_keys<NT, K>(P.grp[0], r0, tid, 0, n0, k0);
     PlaneRuns r1 = r0;
-    int n1 = 0;
     if (two) {
       r1 = plane_runs(L, 1);
-      n1 = r1.total();
       plane_keys<NT, K>(P.grp[1], r1, tid, 0, n1, k1);
     }
-    int4* const pairs = !REST ? block : nullptr;
-    plane_test<NT, K>(g, P, 0, tid, k0, 0, 0, z, C, L, nullptr);
-    if (n0 > K * NT) plane_scan<NT>(g, P, 0, tid, r0, 0, K * NT, n0, z, C, L, nullptr);
+    plane_test<NT, K>(g, P, 0, tid, k0, 0, z, C, L, nullptr);
+    if (n0 > K * NT) plane_scan<NT>(g, P, 0, tid, r0, K * NT, n0, z, C, L, nullptr);
     if (two) {
-      plane_test<NT, K>(g, P, 1, tid, k1, 0, 0, z, C, L, pairs);
-      if (n1 > K * NT) plane_scan<NT>(g, P, 1, tid, r1, 0, K * NT, n1, z, C, L, pairs);
+      plane_test<NT, K>(g, P, 1, tid, k1, 0, z, C, L, pairs);
+      if (n1 > K * NT) plane_scan<NT>(g, P, 1, tid, r1, K * NT, n1, z, C, L, pairs);
     }
-    one = n0 <= 65536 && n1 <= 65536;
   }
   __syncthreads();
-  const int nhit0 = uniform(L.n[0]);
-  const int nhit1 = uniform(L.n[1]);
-  one = one && nhit0 + nhit1 <= kListCap;
+  const int nhit0 = listed ? uniform(L.n[0]) : n0, nhit1 = listed ? uniform(L.n[1]) : n1;  // at most
+  const bool one = listed && nhit0 + nhit1 <= kListCap;
   const auto clear = [&](int from, int to) {  // both multiples of 4, or the plane's end
     int4* acc4 = reinterpret_cast<int4*>(acc);
     for (int e = from / 4 + tid; e < to / 4; e += NT) acc4[e] = make_int4(0, 0, 0, 0);
@@ -546,10 +562,10 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
     } else {
       clear(head, words);
       constexpr int K = 4;
-      for (int b = 0; b < r.total(); b += K * NT) {
+      for (int b = 0; b < n0; b += K * NT) {
         unsigned key[K];
         float v[K];
-        plane_keys<NT, K>(G, r, tid, b, r.total(), key);
+        plane_keys<NT, K>(G, r, tid, b, n0, key);
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           if (!key_hits(key[k], G, z, g.mz, NPTS, C == 2)) key[k] = ~0u;
@@ -561,6 +577,17 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
             enter(v[k], key[k]);
             L.kept = 1;
           }
+      }
+      if (two && !listed && !REST) {
+        const SpreadGroup& G1 = P.grp[1];
+        const PlaneRuns r1 = plane_runs(L, 1);
+        for (int b = 0; b < n1; b += K * NT) {
+          unsigned key[K];
+          plane_keys<NT, K>(G1, r1, tid, b, n1, key);
+#pragma unroll
+          for (int k = 0; k < K; ++k)
+            if (key_hits(key[k], G1, z, g.mz, NPTS, C == 2)) atomicAdd(&block[key[k] >> 16].y, 1);
+        }
       }
     }
   }
@@ -614,7 +641,7 @@ FHD_DEV bool plane_spread(int* acc, int words, int pitch, const GridDev& g, cons
     __syncthreads();
   }
   const float scale2 = !REST ? 0.0f : ldexpf(1.0f, rest_exp(uniform(L.most)));
-  plane_add_group<NPTS, NT, false>(acc, pitch, g, P, tid, z, C, L, one, nval, scale2);
+  if (nval) plane_add_group<NPTS, NT, false>(acc, pitch, g, P, tid, z, C, L, one, nval, scale2);
   if (two) plane_add_group<NPTS, NT, true>(acc, pitch, g, P, tid, z, C, L, one, nhit1, scale2);
   __syncthreads();
   return !REST && uniform(L.more) != 0 && uniform(L.bad) == 0;

@@ -16,19 +16,25 @@
 // Bound by the latency of its dependent phases and, for the pairs, by the vector instructions of
 // the rows; a plane is one workgroup, so at 128^3 half the CUs hold two of the 384 planes and half
 // one.  Per launch at 128^3 with 65,536 particles (rocprof): first solve (vector values, most of
-// them zero) 34 us, second (values and pairs) 50 us, where the transform alone takes 17.7 us; a
+// them zero) 32 us, second (values and pairs) 52 us, where the transform alone takes 16 us; a
 // separate record pass, a spread of 8^3 tiles and the transform took 44 and 69 us.  64^3 with 16,384
-// particles: 16 and 23 us against 22 and 37; 32^3 with 1,024: 12 and 16 us against 16 and 21.
+// particles: 16 and 24 us against 22 and 37; 32^3 with 1,024: 10 and 14 us against 16 and 21.  At the
+// 64 registers that let two planes share a CU the 128 x 128 kernel spills 11 VGPRs, smaller ones none.
 //
 //  1. scan: the sources sorted into the tile layers that can reach the plane are tested by a 4-byte
-//     key (their half cell along z and their 4 x 4 block of columns); the hits enter the plane's
-//     count and a list in LDS (ballot compaction).
+//     key (their half cell along z and their 4 x 4 block of columns); the hits enter a list in LDS
+//     (ballot compaction), pairs their block's count.
 //  2. values: vector values are read for the blocks' counts and bounds, and the hits with a zero component
 //     (a particle with no WCA neighbour) leave the list.
-//  3. add: one lane per listed source computes its weights along x and y and its weight on this
+//  3. scales: each block's, from the counts and bounds of the blocks around it.
+//  4. add: one lane per listed source computes its weights along x and y and its weight on this
 //     plane, and adds the 9 or 16 nodes of the row.  The two rows of a random-finite-difference
 //     pair have the same nodes but for the few particles within the displacement of a half cell's
 //     face, so their difference is added at once.
+// Planes with more hits than the list holds do without it: they read the values of all sources in
+// reach, and each wave then collects the hits of its own share of the keys and adds a row per lane.  128^3
+// with 524,288 particles: 300 us per launch (their average), where listing them piece by piece took 384,
+// and the record pass, the spread and the transform 297; 64^3 with 131,072: 147, 179 and 157 us.
 #pragma once
 #include <stddef.h>
 #include "fhd_device.h"

@@ -249,10 +249,23 @@ struct GridDev {
 
 // Particle position: integer cell (unwrapped) + offset from the cell centre in
 // [-h/2, h/2) per axis.  The unwrapped coordinate is (c + 1/2) h - L/2 + d.
-struct PartPos {
-  int4* cell;    // x, y, z, w unused
-  float4* off;   // x, y, z, w unused
-};
+// Between steps a position also carries what its offset's rounding left off, as 16-bit multiples of
+// 2^(ilogb(h) - 39) (half an ulp of an offset is at most 2^14 of them): x and y in the cell's w, z in the
+// offset's.  Without it a run's positions wander by the rounding of every step, which the forces of close
+// pairs multiply by 25 (100 steps of 64^3: forces off by 3.0e-6).
+FHD_DEV float low_part(int bits, int shift, float quantum) { return (float)(short)(bits >> shift) * quantum; }
+// b + t, rounded; `e`: the rounding error (Knuth's two-sum).
+FHD_DEV float two_sum(float b, float t, float& e) {
+  const float s = b + t, bb = s - b;
+  e = (b - (s - bb)) + (t - bb);
+  return s;
+}
+// The low part's multiple: a little below half an ulp and cut, so that it never reaches the rounding's tie
+// and a position read out and set again is split as it was.
+FHD_DEV int low_bits(float e, float inverse) {
+  const float q = e * (0.999f * inverse);
+  return (int)fminf(fmaxf(q, -32767.0f), 32767.0f);
+}
 
 // Square root of x in [0.25, 4] to within half an ulp or so: the hardware reciprocal root and one
 // Newton step (sqrtf's correct rounding over the full range costs three times the instructions).

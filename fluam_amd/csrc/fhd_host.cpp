@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <memory>
 #include <mutex>
 #include <stdexcept>
 #include <fstream>
@@ -393,17 +394,26 @@ void free_ctx(fhd_ctx* c) {
   if (c->s && c->own_stream) (void)hipStreamDestroy(c->s);
 }
 
-// Host position <-> (cell, offset).
-void to_cell(double q, double L, double h, int& cc, float& d) {
+// Host position <-> (cell, offset); returns what the offset's rounding left off.
+double to_cell(double q, double L, double h, int& cc, float& d) {
   double t = (q + 0.5 * L) / h;
   double f = floor(t);
   cc = (int)f;
   double off = q - ((f + 0.5) * h - 0.5 * L);
   d = (float)off;
-  if (d >= 0.5f * (float)h) { cc += 1; d -= (float)h; }
-  if (d < -0.5f * (float)h) { cc -= 1; d += (float)h; }
+  const float hf = (float)h;
+  const bool up = d >= 0.5f * hf, down = d < -0.5f * hf;
+  if (__builtin_expect(up || down, 0)) {
+    const int n = up ? 1 : -1;
+    cc += n;
+    d -= n * hf;
+    off -= n * h;
+  }
+  return off - (double)d;
 }
 double from_cell(int cc, float d, double L, double h) { return ((double)cc + 0.5) * h - 0.5 * L + (double)d; }
+// Quantum of the offsets' low parts (low_part in fhd_device.h).
+double low_quantum(double h) { return ldexp(1.0, ilogb(h) - 39); }
 
 void initial_positions(const fhd_params& p, std::vector<double>& q);
 
@@ -648,6 +658,11 @@ InterpArgs interp_base(fhd_ctx* c, int eval_set) {
   a.nb = nb_list(c);
   const double move = 0.45 * c->nb_skin;
   a.nb_move2 = (float)(move * move);
+  const double h[3] = {c->dx, c->dy, c->dz};
+  for (int k = 0; k < 3; ++k) {
+    a.low[k] = (float)low_quantum(h[k]);
+    a.ilow[k] = 1.0f / a.low[k];  // exact: a power of two
+  }
   a.np = c->np;
   return a;
 }
@@ -831,6 +846,7 @@ void step_stokes(fhd_ctx* c) {
     ia.base_off = c->off[0];
     ia.out_cell = c->cell[0];
     ia.out_off = c->off[0];
+    ia.low_out = 1;
     skin_to_full(c, ia);
     ia.f1 = c->v;
     ia.a1 = (float)dt;
@@ -1055,6 +1071,7 @@ void step_qnb(fhd_ctx* c) {
     ia.base_off = c->off[0];
     ia.out_cell = c->cell[0];
     ia.out_off = c->off[0];
+    ia.low_out = 1;
     skin_to_full(c, ia);
     ia.f1 = c->v;
     ia.a1 = (float)(0.5 * dt);
@@ -1943,24 +1960,31 @@ int fhd_get_velocity(fhd_ctx* c, double* v) {
 int fhd_set_particles(fhd_ctx* c, const double* q) {
   CTX_TRY(c, {
     const int np = c->np;
-    std::vector<int4> hc(np);
-    std::vector<float4> ho(np);
+    std::unique_ptr<int4[]> hc(new int4[np]);
+    std::unique_ptr<float4[]> ho(new float4[np]);
     const double L[3] = {c->p.lx, c->p.ly, c->p.lz}, h[3] = {c->dx, c->dy, c->dz};
+    double part[3];  // low parts per unit of length
+    for (int a = 0; a < 3; ++a) part[a] = 1.0 / low_quantum(h[a]);
     for (int i = 0; i < np; ++i) {
-      int cc[3];
+      int cc[3], low[3];
       float d[3];
       for (int a = 0; a < 3; ++a) {
         double qa = q[(size_t)a * np + i];
         if (!std::isfinite(qa)) throw std::runtime_error("non-finite particle position");
-        to_cell(qa, L[a], h[a], cc[a], d[a]);
+        const double left = to_cell(qa, L[a], h[a], cc[a], d[a]) * part[a];  // below 2^16
+        const int n = (int)(left + 65536.5) - 65536;
+        low[a] = std::min(32767, std::max(-32767, n));
       }
-      hc[i] = make_int4(cc[0], cc[1], cc[2], 0);
-      ho[i] = make_float4(d[0], d[1], d[2], 0.0f);
+      float lz;
+      const int bits = low[2] & 0xFFFF;
+      memcpy(&lz, &bits, sizeof(lz));
+      hc[i] = make_int4(cc[0], cc[1], cc[2], (low[0] & 0xFFFF) | (int)((unsigned)low[1] << 16));
+      ho[i] = make_float4(d[0], d[1], d[2], lz);
     }
     HIPCHK(hipStreamSynchronize(c->s));
     if (np > 0) {
-      HIPCHK(hipMemcpy(c->cell[0], hc.data(), np * sizeof(int4), hipMemcpyHostToDevice));
-      HIPCHK(hipMemcpy(c->off[0], ho.data(), np * sizeof(float4), hipMemcpyHostToDevice));
+      HIPCHK(hipMemcpy(c->cell[0], hc.get(), np * sizeof(int4), hipMemcpyHostToDevice));
+      HIPCHK(hipMemcpy(c->off[0], ho.get(), np * sizeof(float4), hipMemcpyHostToDevice));
       const int one = 1;  // the sorted copies are stale: sort again before the next use
       HIPCHK(hipMemcpy(c->sflag, &one, sizeof(int), hipMemcpyHostToDevice));
       if (c->nb_flag) HIPCHK(hipMemcpy(c->nb_flag, &one, sizeof(int), hipMemcpyHostToDevice));  // and rebuild the lists
@@ -1979,10 +2003,13 @@ int fhd_get_particles(fhd_ctx* c, double* q) {
       HIPCHK(hipMemcpy(hc.data(), c->cell[0], np * sizeof(int4), hipMemcpyDeviceToHost));
       HIPCHK(hipMemcpy(ho.data(), c->off[0], np * sizeof(float4), hipMemcpyDeviceToHost));
     }
+    const double low[3] = {low_quantum(c->dx), low_quantum(c->dy), low_quantum(c->dz)};
     for (int i = 0; i < np; ++i) {
-      q[i] = from_cell(hc[i].x, ho[i].x, c->p.lx, c->dx);
-      q[np + i] = from_cell(hc[i].y, ho[i].y, c->p.ly, c->dy);
-      q[2 * (size_t)np + i] = from_cell(hc[i].z, ho[i].z, c->p.lz, c->dz);
+      int lz;
+      memcpy(&lz, &ho[i].w, sizeof(lz));
+      q[i] = from_cell(hc[i].x, ho[i].x, c->p.lx, c->dx) + (short)hc[i].w * low[0];
+      q[np + i] = from_cell(hc[i].y, ho[i].y, c->p.ly, c->dy) + (short)(hc[i].w >> 16) * low[1];
+      q[2 * (size_t)np + i] = from_cell(hc[i].z, ho[i].z, c->p.lz, c->dz) + (short)lz * low[2];
     }
   });
   return 1;

@@ -200,6 +200,8 @@ struct InterpArgs {
   const float4* base_off;
   int4* out_cell;        // out = base + a1 J f1 + a2 J f2 + extra (by id)
   float4* out_off;
+  float low[3], ilow[3]; // quantum of the offsets' low parts (low_part) and its inverse
+  int low_out;           // 1: out keeps the low parts (the set that is the next update's base)
   SkinArgs sk;           // sorted copies of out, kept current (s_cell null: none)
   const float* f1; float a1;
   const float* f2; float a2;

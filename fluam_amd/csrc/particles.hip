@@ -843,12 +843,35 @@ FHD_DEV void interp_finish(const InterpArgs& a, int s, int id, const InterpPre& 
       if (!(fabsf(disp[1]) < 16777216.0f * g.dy)) disp[1] = 0.0f;
       if (!(fabsf(disp[2]) < 16777216.0f * g.dz)) disp[2] = 0.0f;
     }
-    float ox = bo.x + disp[0], oy = bo.y + disp[1], oz = bo.z + disp[2];
+    float ex, ey, ez;
+    float ox = two_sum(bo.x, disp[0] + low_part(bc.w, 0, a.low[0]), ex);
+    float oy = two_sum(bo.y, disp[1] + low_part(bc.w, 16, a.low[1]), ey);
+    float oz = two_sum(bo.z, disp[2] + low_part(__float_as_int(bo.w), 0, a.low[2]), ez);
     renorm_axis(bc.x, ox, g.dx, g.idx);
     renorm_axis(bc.y, oy, g.dy, g.idy);
     renorm_axis(bc.z, oz, g.dz, g.idz);
+    bc.w = 0;
+    float low_z = 0.0f;
+    if (a.low_out) {
+      // an offset that moved to another cell has a finer ulp: its low part's upper bits belong to it
+      const auto settle = [](float& o, float& e, float h) {
+        float r;
+        const float s = two_sum(o, e, r);
+        if (fabsf(s) < 0.5f * h) {
+          o = s;
+          e = r;
+        }
+      };
+      if (bc.x != pre.bc.x || bc.y != pre.bc.y || bc.z != pre.bc.z) {
+        settle(ox, ex, g.dx);
+        settle(oy, ey, g.dy);
+        settle(oz, ez, g.dz);
+      }
+      bc.w = (low_bits(ex, a.ilow[0]) & 0xFFFF) | (low_bits(ey, a.ilow[1]) << 16);
+      low_z = __int_as_float(low_bits(ez, a.ilow[2]) & 0xFFFF);
+    }
     a.out_cell[id] = bc;
-    a.out_off[id] = make_float4(ox, oy, oz, 0.0f);
+    a.out_off[id] = make_float4(ox, oy, oz, low_z);
     if (a.nb.flag) {
       // the WCA neighbour lists hold every pair that was within rc + skin at the build; they
       // stay complete while no particle has moved more than half a skin from where it was then

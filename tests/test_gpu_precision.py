@@ -12,7 +12,8 @@ import pytest
 
 import fluam_amd as F
 import oracle_lib as O
-from fluam_amd._abi import make_params, SCHEME_INCOMPRESSIBLE, SCHEME_QUASI_NEUTRALLY_BUOYANT
+from fluam_amd._abi import (make_params, SCHEME_INCOMPRESSIBLE, SCHEME_QUASI_NEUTRALLY_BUOYANT,
+                            SCHEME_STOKES_LIMIT)
 
 pytestmark = pytest.mark.gpu
 
@@ -96,3 +97,52 @@ def test_kept_velocity_stays_divergence_free(scheme):
     g.step(1500)
     rms = np.sqrt(np.mean(np.square(g.velocity())))
     assert g.max_divergence() * 10.0 / rms < 5 * 8.4e-7
+
+
+def lattice(rng, cells, h, n):
+    """n sites of a lattice of 1.25 cells, displaced by up to 0.12: pairs within the WCA range, none inside."""
+    m = [int(c / 1.25) for c in cells]
+    at = np.stack(np.unravel_index(rng.choice(m[0] * m[1] * m[2], n, replace=False), m), 1)
+    box = np.array(cells, dtype=np.float64)
+    return ((((at + 0.5) / m - 0.5) * box + rng.uniform(-0.12, 0.12, (n, 3))) * h).T.ravel()
+
+
+@pytest.mark.parametrize("scheme,h,kernel", [(SCHEME_STOKES_LIMIT, 1.0, 3), (SCHEME_STOKES_LIMIT, 0.7, 4),
+                                             (SCHEME_QUASI_NEUTRALLY_BUOYANT, 1.0, 3)])
+def test_forces_of_close_pairs_after_100_steps(scheme, h, kernel):
+    """The offset of the evaluated position is rounded once (2^-26 to 2^-25 of a cell, 1.2e-8 root mean square a
+    coordinate, 2.4e-8 sigma of a pair's distance), and a pair at contact changes its force by about 25 times that
+    part: 6e-7.  Bound: three times that; a run that rounds its positions at every step is ten steps' root away."""
+    cells, n = (32, 24, 32), 800
+    rng = np.random.default_rng(17)
+    q = lattice(rng, cells, h, n)
+    print(f"[gpu-case] precision forces scheme={scheme} h={h}", flush=True)
+    p = make_params(scheme, cells=cells, box=tuple(h * m for m in cells), np=n, kernel_points=kernel,
+                    temperature=1e-3, dt=0.05 * h * h, seed=23, initial_positions=1, wca_sigma=h,
+                    cutoff=2.0 ** (1.0 / 6.0) * h)
+    g, o = F.Simulation(p), O.Oracle(p)
+    g.set_particles(q)
+    o.set_particles(q)
+    assert np.abs(g.particles() - q).max() < 2.0 ** -38 * h
+    g.step(100)
+    g.sync()
+    o.step(100)
+    e = rel(g.forces(), o.forces())
+    print(f"  forces {e:.1e}, positions {np.abs(g.particles() - o.particles()).max() / h:.1e}", flush=True)
+    assert e < 1.8e-6
+
+
+def test_positions_resume_with_their_low_parts():
+    """Positions read out and set again are the same state, in cells that are no power of two."""
+    cells, h, n = (16, 24, 16), 0.3, 200
+    p = make_params(SCHEME_STOKES_LIMIT, cells=cells, box=tuple(h * m for m in cells), np=n, kernel_points=3,
+                    temperature=1e-3, dt=0.05, seed=5, initial_positions=0, nonbonded=0, cutoff=0.0)
+    print("[gpu-case] precision resume", flush=True)
+    a, b = F.Simulation(p), F.Simulation(p)
+    for _ in range(6):
+        q = a.particles()
+        b.set_particles(q)
+        assert np.array_equal(b.particles(), q)
+        a.step(1)
+        b.step(1)
+        assert np.array_equal(a.particles(), b.particles())

@@ -78,8 +78,8 @@ def test_displacements_across_flat_cells(tmp_path, kernel):
 
 @pytest.mark.parametrize("scheme,cells,n,kernel,kw", [
     (ST, (32, 32, 16), 600, 4, {}),    # one 32-bit sum
-    (ST, (16, 16, 8), 5000, 4, {}),    # two sums, every hit listed
-    (ST, (16, 16, 8), 20000, 3, {}),   # two sums, the list in chunks
+    (ST, (16, 16, 8), 5000, 4, {}),    # two sums, more hits than the list holds
+    (ST, (16, 16, 8), 20000, 3, {}),   # two sums, not listed
     (QNB, (32, 32, 16), 600, 3, {}),
     (QNB, (16, 16, 8), 5000, 3, {}),
     (QNB, (16, 16, 8), 20000, 4, {}),
@@ -87,11 +87,30 @@ def test_displacements_across_flat_cells(tmp_path, kernel):
     (ST, (64, 16, 8), 9000, 4, {"rfd_delta": 2.5}),  # displaced beyond the neighbouring blocks: one scale
     (ST, (72, 36, 8), 9000, 4, {}),    # runtime-size passes
     (QNB, (128, 128, 4), 12000, 4, {}),
-    (ST, (64, 64, 16), 140000, 4, {}),   # more sources in reach of a plane than 16 bits index
+    (ST, (64, 64, 16), 140000, 4, {}),
     (QNB, (48, 24, 16), 140000, 3, {}),
 ])
 def test_crowded_planes_with_forces(tmp_path, scheme, cells, n, kernel, kw):
     run(tmp_path, scheme, cells, n, kernel, 300 + kernel, **kw)
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+def test_crowded_replicas_equal_alone(mode):
+    """Planes without a list, in boxes that a merged batch gives to the runtime-size passes."""
+    ps = [make_params(ST, cells=c, np=n, kernel_points=k, nonbonded=0, temperature=1e-3, dt=0.05, seed=40 + n,
+                      initial_positions=0, cutoff=0.0)
+          for c, n, k in (((16, 16, 16), 9000, 4), ((32, 16, 24), 14000, 3), ((32, 32, 32), 40, 4), ((64, 64, 16), 30000, 4))]
+    print(f"[gpu-case] crowded replicas mode={mode}", flush=True)
+    b = F.Batch(ps)
+    b.set_mode(mode)
+    b.step(3)
+    b.sync()
+    for p, r in zip(ps, b.replicas):
+        alone = F.Simulation(p)
+        alone.step(3)
+        assert np.array_equal(alone.velocity(), r.velocity())
+        assert np.array_equal(alone.particles(), r.particles())
+    b.close()
 
 
 def test_weak_forces_beside_a_strong_one(tmp_path):

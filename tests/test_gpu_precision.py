@@ -63,15 +63,19 @@ def test_particle_velocity_of_a_heavy_particle():
     assert np.sqrt(np.mean(np.square(off))) < 1e-6
 
 
-@pytest.mark.parametrize("cells,h,dt", [
-    ((32, 32, 32), 10.0, 0.25),
-    ((48, 24, 16), 1.0, 0.05),
-    ((96, 96, 8), 10.0, 0.25),
-    ((128, 128, 4), 10.0, 0.25),  # in place, also by the kernels with the transform in registers
-    ((108, 54, 12), 10.0, 0.25),
-    ((16, 2, 1), 10.0, 0.25),
+@pytest.mark.parametrize("cells,h,dt,plan", [
+    ((32, 32, 32), 10.0, 0.25, None),
+    ((48, 24, 16), 1.0, 0.05, None),
+    ((96, 96, 8), 10.0, 0.25, None),
+    ((128, 128, 4), 10.0, 0.25, None),
+    ((128, 128, 4), 10.0, 0.25, 9),  # the kernels with the transform in registers
+    ((108, 54, 12), 10.0, 0.25, None),
+    ((16, 2, 1), 10.0, 0.25, None),
 ])
-def test_incompressible_velocity(cells, h, dt):
+def test_incompressible_velocity(cells, h, dt, plan, monkeypatch):
+    """Every inverse pass adds the kept velocity in place."""
+    if plan is not None:
+        monkeypatch.setenv("FHD_PLAN_XY", str(plan))
     p, _, g, o = pair(SCHEME_INCOMPRESSIBLE, cells, 7, h, 1e-3 * h ** 3, dt)
     g.step(50)
     g.sync()
